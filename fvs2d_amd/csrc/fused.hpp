@@ -232,21 +232,7 @@ __device__ __forceinline__ void boundary_flux(const Phys &P, double t, int c, in
 // gather of the block's face fluxes from LDS in the reference's per-cell
 // order (src/residual.f90:97-101,153-155), -R/vol (164-166), local time step
 // (src/runge_kutta.f90:433), stage update, next primitive state, and the
-// last stage's squared increments (per-block sums for the residual norm)
-// fixed-shape tree over NT threads (deterministic); with NT = 2 kBlock the
-// upper half contributes exact zeros, so the sums equal the kBlock tree's
-template <int NT>
-__device__ __forceinline__ void block_sum4_t(double v[4], double *red) {
-  const int t = threadIdx.x;
-  for (int k = 0; k < 4; ++k) red[k * NT + t] = v[k];
-  __syncthreads();
-  for (int s = NT / 2; s > 0; s >>= 1) {
-    if (t < s)
-      for (int k = 0; k < 4; ++k) red[k * NT + t] = red[k * NT + t] + red[k * NT + t + s];
-    __syncthreads();
-  }
-  for (int k = 0; k < 4; ++k) v[k] = red[k * NT];
-}
+// last stage's squared increments (sums per 64-cell slice for the residual norm)
 
 // The cell-side inputs of the stage update, loaded before the face fluxes
 // are complete (their latency overlaps the barrier): the cell's gather
@@ -296,15 +282,14 @@ __device__ __forceinline__ const unsigned *active_mask(const int *blist, int nbl
   return reinterpret_cast<const unsigned *>(blist + nbl);
 }
 
-// NT threads per workgroup, CB cells per block (CB <= NT); instance masks
-// exist for 256-cell blocks only
-template <int NT, int CB = kBlock>
+// CB cells per block, one per thread (further threads of the workgroup idle);
+// instance masks exist for 256-cell blocks only
+template <int CB = kBlock>
 __device__ __forceinline__ void block_update_finish(int N, int lb, const Upd &A, const UpdIn &in,
                                                     const double *__restrict__ lF, const double *__restrict__ lS,
                                                     double *__restrict__ Ua, double *__restrict__ Ub,
                                                     double *__restrict__ Facc, double *__restrict__ Wout,
-                                                    double *__restrict__ dtl, double *__restrict__ part,
-                                                    double *__restrict__ d2out, double *__restrict__ red,
+                                                    double *__restrict__ dtl, const NormOut &norm,
                                                     const unsigned *__restrict__ amask) {
   const int i = lb * CB + threadIdx.x;
   double d2[4] = {0, 0, 0, 0};
@@ -370,7 +355,6 @@ __device__ __forceinline__ void block_update_finish(int N, int lb, const Upd &A,
           d2[v] = d * d;
         }
       }
-      if (d2out) st4(d2out, i, d2);
     } else if (A.mode == M_SSP3 && on) {
       st4(Ub, i, un);
     }
@@ -380,12 +364,7 @@ __device__ __forceinline__ void block_update_finish(int N, int lb, const Upd &A,
       st4(Wout, i, w);
     }
   }
-  if (A.last) {
-    __syncthreads();  // red may alias the face fluxes just gathered
-    block_sum4_t<NT>(d2, red);
-    if (threadIdx.x == 0)
-      for (int v = 0; v < 4; ++v) part[4 * lb + v] = d2[v];
-  }
+  if (A.last && threadIdx.x < CB) slice_norms(norm, i, N, d2);
 }
 
 // fused face fluxes (LDS) + ordered gather + stage update; reads the stage's
@@ -411,11 +390,11 @@ __global__ __launch_bounds__(BS) void k_flux_update(int N, int nb, int gw, int m
                                                         const double *__restrict__ vol, double *__restrict__ Ua,
                                                         double *__restrict__ Ub, double *__restrict__ Facc,
                                                         double *__restrict__ Wout, double *__restrict__ dtl,
-                                                        double *__restrict__ part, const int *__restrict__ blist,
-                                                        const double *__restrict__ pinf_inst,
-                                                        double *__restrict__ d2out, int phi_one, int cons) {
+                                                        NormOut norm, const int *__restrict__ blist,
+                                                        const double *__restrict__ pinf_inst, int phi_one,
+                                                        int cons) {
   extern __shared__ double lds[];
-  double *lF = lds;             // [maxf][4] flux*area (later the block reduction)
+  double *lF = lds;             // [maxf][4] flux*area
   double *lS = lds + 4 * maxf;  // [maxf]    wave speed*area, only when the stage sets local time steps
   const bool ws = A.steady && A.first;
   __shared__ double sG[8 * BS];  // gradients of the block's own cells
@@ -519,8 +498,8 @@ __global__ __launch_bounds__(BS) void k_flux_update(int N, int nb, int gw, int m
     }
   }
   __syncthreads();
-  block_update_finish<BS, BS>(N, lb, A, in, lF, lS, Ua, Ub, Facc, Wout, dtl, part, d2out, lF,
-                              blist ? active_mask(blist, nbl) : nullptr);
+  block_update_finish<BS>(N, lb, A, in, lF, lS, Ua, Ub, Facc, Wout, dtl, norm,
+                          blist ? active_mask(blist, nbl) : nullptr);
 }
 
 // Whole RK stage in one kernel per 256-cell block: the block stages, in LDS,
@@ -751,7 +730,8 @@ struct StageArgs {
   const double *vol;
   const int *ioff, *frz;
   int ninst;
-  double *Ua, *Ub, *Facc, *dtl, *part;
+  double *Ua, *Ub, *Facc, *dtl;
+  NormOut norm;
   const int *blist, *binst;
   const double *pinf_inst;
 };
@@ -759,7 +739,7 @@ struct StageArgs {
 // One 256-cell block lb of a whole RK stage (see above).
 template <int LIM, int PMODE>
 __device__ __forceinline__ void stage_block(const StageArgs &a, int lb, const Upd &A, const double *__restrict__ Win,
-                                            double *__restrict__ Wout, double *__restrict__ d2out) {
+                                            double *__restrict__ Wout) {
   extern __shared__ double lds[];
   const int N = a.N, max1 = a.max1, max2 = a.max2, maxf = a.maxf;
   double *lW = lds;                                   // [max2][4]
@@ -812,62 +792,96 @@ __device__ __forceinline__ void stage_block(const StageArgs &a, int lb, const Up
     lS[f] = wsa;
   }
   __syncthreads();
-  // the staged states are no longer read: their LDS holds the reduction
   {
     UpdIn in;
     const int ic = lb * kBlock + threadIdx.x;
     if (threadIdx.x < kBlock && ic < N)
       block_update_load(N, ic, a.gw, A, a.lgat, a.vol, a.Ua, a.Ub, a.Facc, a.dtl, in);
-    block_update_finish<kStageThreads>(N, lb, A, in, lF, lS, a.Ua, a.Ub, a.Facc, Wout, a.dtl, a.part, d2out, lds,
-                                       a.blist ? active_mask(a.blist, nbl) : nullptr);
+    block_update_finish(N, lb, A, in, lF, lS, a.Ua, a.Ub, a.Facc, Wout, a.dtl, a.norm,
+                        a.blist ? active_mask(a.blist, nbl) : nullptr);
   }
 }
 
 template <int LIM, int PMODE>
 __global__ __launch_bounds__(kStageThreads) void k_stage(StageArgs a, Upd A, const double *__restrict__ Win,
-                                                         double *__restrict__ Wout, double *__restrict__ d2out) {
+                                                         double *__restrict__ Wout) {
   const int lb = a.blist ? a.blist[blockIdx.x] : xcd_block(a.nb);
   const int nbl = a.nb < 0 ? -a.nb : a.nb;
   if (lb >= nbl) return;  // the whole workgroup leaves before any barrier
-  stage_block<LIM, PMODE>(a, lb, A, Win, Wout, d2out);
+  stage_block<LIM, PMODE>(a, lb, A, Win, Wout);
 }
 
-// Thread t's share of an instance's squared increments: cells a + t, a + t
-// + kBlock, ... < b added in that order, with kInstLoads loads in flight
-// before their adds (an instance holds up to 2^18 cells, one workgroup walks
-// it, and the loads' latency would otherwise be paid once per cell)
-constexpr int kInstLoads = 8;
-__device__ __forceinline__ void inst_share(int a, int b, int t, const double *__restrict__ d2, double s[4]) {
-  for (int i0 = a + t; i0 < b; i0 += kInstLoads * kBlock) {
-    double q[kInstLoads][4];
-#pragma unroll
-    for (int u = 0; u < kInstLoads; ++u) {
-      const int i = i0 + u * kBlock;
-      if (i < b) ld4(d2, i, q[u]);
-    }
-#pragma unroll
-    for (int u = 0; u < kInstLoads; ++u)
-      if (i0 + u * kBlock < b)
-        for (int v = 0; v < 4; ++v) s[v] = s[v] + q[u][v];
+// Residual norms of one step of instance k from the step's partials (fixed
+// order: kBlock threads over the whole slices of its cells, its cells in
+// slices shared with other instances, then a tree).  red: 4 kBlock doubles of
+// LDS; threads past kBlock only keep the barriers.
+struct InstNorms {
+  int ninst, ng, nsplit;     // instances, slices and shared slices
+  const int *off;            // first cell of each instance
+  const int *split;
+  const int *act;            // NULL: all active
+  double *last;              // norms of the last step each instance took
+};
+__device__ __forceinline__ void inst_norm_row(const InstNorms &I, int k, const double *__restrict__ part,
+                                              const double *__restrict__ d2, bool keep_last,
+                                              double *__restrict__ out, double *red) {
+  const int t = threadIdx.x;
+  // an instance that is masked out repeats the norms of its last step
+  if (I.act && !I.act[k]) {
+    if (t < 4) out[t] = I.last[4 * k + t];
+    return;
   }
+  const int a = I.off[k], b = I.off[k + 1];
+  const int g0 = (a + kSlice - 1) / kSlice, g1 = b / kSlice;  // whole slices [g0, g1)
+  if (t < kBlock) {
+    double s[4] = {0, 0, 0, 0};
+    for (int p0 = g0 + t; p0 < g1; p0 += kNormLoads * kBlock) {
+      double q[kNormLoads][4];
+#pragma unroll
+      for (int u = 0; u < kNormLoads; ++u) {
+        const int p = p0 + u * kBlock;
+        if (p < g1) ld4(part, p, q[u]);
+        else q[u][0] = q[u][1] = q[u][2] = q[u][3] = 0.0;
+      }
+#pragma unroll
+      for (int u = 0; u < kNormLoads; ++u)
+        for (int v = 0; v < 4; ++v) s[v] = s[v] + q[u][v];
+    }
+    // cells of the first and the last slice where it is shared (threads 0..63
+    // and 64..127; one slice holding the whole instance counts once)
+    const int head = a / kSlice, tail = b / kSlice, l = t & 63;
+    const int g = t < kSlice ? head : tail;
+    const int i = g * kSlice + l;
+    const bool shared = t < kSlice ? a % kSlice != 0 : t < 2 * kSlice && b % kSlice != 0 && tail >= g0;
+    if (shared && i >= a && i < b) {
+      double q[4];
+      ld4(d2, long(I.split[g]) * kSlice + l, q);
+      for (int v = 0; v < 4; ++v) s[v] = s[v] + q[v];
+    }
+    for (int v = 0; v < 4; ++v) red[v * kBlock + t] = s[v];
+  }
+  __syncthreads();
+  for (int h = kBlock / 2; h > 0; h >>= 1) {
+    if (t < h)
+      for (int v = 0; v < 4; ++v) red[v * kBlock + t] = red[v * kBlock + t] + red[v * kBlock + t + h];
+    __syncthreads();
+  }
+  if (t < 4) {
+    const double n = sqrt(red[t * kBlock] / double(b - a));
+    out[t] = n;
+    if (keep_last) I.last[4 * k + t] = n;
+  }
+  __syncthreads();
 }
 
-// per-instance residual norms of one step from the per-cell squared
-// increments: one workgroup per instance, fixed-shape tree (deterministic)
-__global__ __launch_bounds__(kBlock) void k_inst_norms(int ninst, const int *__restrict__ off,
+// per-instance norms of the pending steps: one workgroup per instance and step
+__global__ __launch_bounds__(kBlock) void k_inst_norms(InstNorms I, int rows, const double *__restrict__ part,
                                                        const double *__restrict__ d2, const int *__restrict__ ctr,
                                                        double *__restrict__ out) {
   __shared__ double red[4 * kBlock];
-  const int k = blockIdx.x;
-  if (k >= ninst) return;
-  const int a = off[k], b = off[k + 1];
-  double s[4] = {0, 0, 0, 0};
-  inst_share(a, b, threadIdx.x, d2, s);
-  block_sum4(s, red);
-  if (threadIdx.x == 0) {
-    double *o = out + 4 * (long(ctr ? ctr[0] : 0) * ninst + k);
-    for (int v = 0; v < 4; ++v) o[v] = sqrt(s[v] / double(b - a));
-  }
+  const int k = blockIdx.x, r = blockIdx.y;
+  inst_norm_row(I, k, part + 4 * long(r) * I.ng, d2 + 4 * long(r) * I.nsplit * kSlice, r == rows - 1,
+                out + 4 * ((long(ctr[0]) + r) * I.ninst + k), red);
 }
 
 __global__ void k_counter(int *__restrict__ ctr, int value, int add) {
@@ -948,79 +962,14 @@ __device__ __forceinline__ bool grid_barrier(unsigned *bar, unsigned nwg, unsign
   return ok != 0;
 }
 
-// The whole-mesh residual norms of one step (k_norm_final's summation:
-// kNormThreads partial sums over strided partials, then its tree), computed
-// by NT threads that each play kNormThreads / NT of its threads, so the bits
-// are those of k_norm_final.  red: 4 kNormThreads doubles of LDS.
-template <int NT>
-__device__ __forceinline__ void norm_sum_block(int nparts, int N, const double *__restrict__ part,
-                                               double *__restrict__ out, double *red) {
-  constexpr int R = kNormThreads / NT;
-  for (int r = 0; r < R; ++r) {
-    const int vt = threadIdx.x + r * NT;
-    double s[4] = {0, 0, 0, 0};
-    for (int p0 = vt; p0 < nparts; p0 += kNormLoads * kNormThreads) {
-      double q[kNormLoads][4];
-#pragma unroll
-      for (int u = 0; u < kNormLoads; ++u) {
-        const int p = p0 + u * kNormThreads;
-        if (p < nparts) ld4(part, p, q[u]);
-        else q[u][0] = q[u][1] = q[u][2] = q[u][3] = 0.0;
-      }
-#pragma unroll
-      for (int u = 0; u < kNormLoads; ++u)
-        for (int v = 0; v < 4; ++v) s[v] = s[v] + q[u][v];
-    }
-    for (int v = 0; v < 4; ++v) red[v * kNormThreads + vt] = s[v];
-  }
-  __syncthreads();
-  for (int h = kNormThreads / 2; h > 0; h >>= 1) {
-    for (int r = 0; r < R; ++r) {
-      const int vt = threadIdx.x + r * NT;
-      if (vt < h)
-        for (int v = 0; v < 4; ++v)
-          red[v * kNormThreads + vt] = red[v * kNormThreads + vt] + red[v * kNormThreads + vt + h];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0)
-    for (int v = 0; v < 4; ++v) out[v] = sqrt(red[v * kNormThreads] / double(N));
-  __syncthreads();
-}
-
-// Instance k's residual norms of one step with k_inst_norms' summation (the
-// first kBlock threads of the workgroup play its threads).  red: 4 kBlock
-// doubles of LDS.
-__device__ __forceinline__ void inst_norm_block(int k, const int *__restrict__ off, const double *__restrict__ d2,
-                                                double *__restrict__ out, double *red) {
-  const int t = threadIdx.x;
-  const int a = off[k], b = off[k + 1];
-  if (t < kBlock) {
-    double s[4] = {0, 0, 0, 0};
-    inst_share(a, b, t, d2, s);
-    for (int v = 0; v < 4; ++v) red[v * kBlock + t] = s[v];
-  }
-  __syncthreads();
-  for (int h = kBlock / 2; h > 0; h >>= 1) {
-    if (t < h)
-      for (int v = 0; v < 4; ++v) red[v * kBlock + t] = red[v * kBlock + t] + red[v * kBlock + t + h];
-    __syncthreads();
-  }
-  if (t == 0)
-    for (int v = 0; v < 4; ++v) out[v] = sqrt(red[v * kBlock] / double(b - a));
-  __syncthreads();
-}
-
 struct PersistCtl {
   Upd A[4];                 // the stages of one step
   int nst, nsteps, nlaunch;  // stages per step, steps, launch blocks
   double *W0, *W1;          // primitive states: stage k of the launch reads W0 when k is even
-  double *d2buf;            // per-cell squared increments of a step's last stage
   double *dn;               // whole-mesh norms, one row per step (NULL: none)
-  int nparts;
+  int ng;                   // 64-cell slices
   double *dinst;            // per-instance norms (NULL: none)
-  int ninst;
-  const int *inst_off;
+  InstNorms inst;
   int *ctr;                 // output row of the first step; advanced by nsteps at the end
   unsigned *bar;
   int *err;
@@ -1042,7 +991,7 @@ __global__ __launch_bounds__(kStageThreads) void k_steps_persistent(StageArgs a,
       double *Wout = par ? c.W0 : c.W1;
       for (int q = blockIdx.x; q < c.nlaunch; q += gridDim.x) {
         const int lb = a.blist ? a.blist[q] : q;
-        stage_block<LIM, PMODE>(a, lb, A, Win, Wout, A.last ? c.d2buf : nullptr);
+        stage_block<LIM, PMODE>(a, lb, A, Win, Wout);
         __syncthreads();  // the next block's staging overwrites this one's LDS
       }
       ok = grid_barrier(c.bar, gridDim.x, gen, c.spin, c.err);
@@ -1052,10 +1001,11 @@ __global__ __launch_bounds__(kStageThreads) void k_steps_persistent(StageArgs a,
     // this step's norms; the partials and increments they read are next
     // written by the last stage of the next step, two or more barriers later
     const long row = long(row0) + s;
-    if (c.dn && blockIdx.x == 0) norm_sum_block<kStageThreads>(c.nparts, a.N, a.part, c.dn + 4 * row, lds);
+    if (c.dn && blockIdx.x == 0) norm_row<kStageThreads>(c.ng, a.N, a.norm.part, c.dn + 4 * row, lds);
     if (c.dinst)
-      for (int k = blockIdx.x; k < c.ninst; k += gridDim.x)
-        inst_norm_block(k, c.inst_off, c.d2buf, c.dinst + 4 * (row * c.ninst + k), lds);
+      for (int k = blockIdx.x; k < c.inst.ninst; k += gridDim.x)
+        inst_norm_row(c.inst, k, a.norm.part, a.norm.d2, s == c.nsteps - 1,
+                      c.dinst + 4 * (row * c.inst.ninst + k), lds);
   }
   if (ok) ok = grid_barrier(c.bar, gridDim.x, gen, c.spin, c.err);
   if (ok && blockIdx.x == 0 && threadIdx.x == 0) c.ctr[0] = row0 + c.nsteps;

@@ -633,6 +633,48 @@ __device__ __forceinline__ void block_sum4(double v[4], double *red) {
   for (int k = 0; k < 4; ++k) v[k] = red[k * kBlock];
 }
 
+// Where a step's last stage leaves the squared increments of the residual
+// norm: one sum of four per 64-cell slice (a wavefront's cells, added by a
+// fixed cross-lane tree, so the sums do not depend on the block size or the
+// kernel), and, in batches, the single cells of the slices that hold cells of
+// more than one instance (split[slice] = their index, -1 for whole slices).
+// Wavefront sums need no LDS and no barrier; the tree over a whole block that
+// they replace took nine barriers.
+struct NormOut {
+  double *part;
+  const int *split;
+  double *d2;
+};
+
+// Sum over the wavefront's lanes of v[0..3]: lanes 16 k .. 16 k + 15 return
+// the sum of v[k].  The first two exchanges halve the values a lane carries, so
+// seven cross-lane moves of a double do instead of 24.
+__device__ __forceinline__ double wave_sum4(const double v[4]) {
+  const int lane = threadIdx.x & 63;
+  const bool up = lane & 32, odd = lane & 16;
+  double a = up ? v[2] : v[0], b = up ? v[3] : v[1];
+  a = a + __shfl_xor(up ? v[0] : v[2], 32, 64);
+  b = b + __shfl_xor(up ? v[1] : v[3], 32, 64);
+  double s = odd ? b : a;
+  s = s + __shfl_xor(odd ? a : b, 16, 64);
+  for (int k = 8; k > 0; k >>= 1) s = s + __shfl_xor(s, k, 64);
+  return s;
+}
+
+// the slice of cell i (i - lane is a multiple of 64; every lane of the
+// wavefront calls this, lanes past the last cell with zeros)
+__device__ __forceinline__ void slice_norms(const NormOut &o, int i, int N, const double d2[4]) {
+  const int lane = threadIdx.x & 63, i0 = i - lane;
+  if (i0 >= N) return;
+  const int g = i0 / kSlice;
+  const double s = wave_sum4(d2);
+  if ((lane & 15) == 0) o.part[4 * long(g) + (lane >> 4)] = s;
+  if (o.split) {
+    const int k = o.split[g];
+    if (k >= 0) st4(o.d2, long(k) * kSlice + lane, d2);
+  }
+}
+
 // gather (src/residual.f90:97-101,153-155 in the reference's per-cell order),
 // -R/vol (164-166), local time step (src/runge_kutta.f90:433) and stage update
 __global__ __launch_bounds__(kBlock) void k_update(int nbx, int N, int gw, Upd A, const int *__restrict__ gat,
@@ -641,8 +683,7 @@ __global__ __launch_bounds__(kBlock) void k_update(int nbx, int N, int gw, Upd A
                                                    double *__restrict__ Ub, double *__restrict__ Facc,
                                                    double *__restrict__ W, double *__restrict__ dtl,
                                                    double *__restrict__ rout, double *__restrict__ wsout,
-                                                   double *__restrict__ part) {
-  __shared__ double red[4 * kBlock];
+                                                   NormOut norm) {
   const int nb = nblk(N), lb = xcd_block(nbx);
   if (lb >= nb) return;
   const int i = lb * kBlock + threadIdx.x;
@@ -718,50 +759,54 @@ __global__ __launch_bounds__(kBlock) void k_update(int nbx, int N, int gw, Upd A
       st4(W, i, w);
     }
   }
-  if (A.mode != M_RESID && A.last) {
-    block_sum4(d2, red);
-    if (threadIdx.x == 0)
-      for (int v = 0; v < 4; ++v) part[4 * lb + v] = d2[v];
-  }
+  if (A.mode != M_RESID && A.last) slice_norms(norm, i, N, d2);
 }
 
-// residual norms of one step: sqrt(sum_i (U-U0)^2 / N) per variable
-// (src/runge_kutta.f90:169-184), partials summed in block order
+// Residual norms of one step: sqrt(sum_i (U-U0)^2 / N) per variable
+// (src/runge_kutta.f90:169-184) from the step's slice sums: kNormThreads
+// partial sums over strided slices (kNormLoads loads in flight before their
+// adds; absent ones are exact zeros), then a tree.  NT threads each play
+// kNormThreads / NT of them, so the bits do not depend on NT.  red: 4
+// kNormThreads doubles of LDS.
 constexpr int kNormThreads = 1024;
-// (bump: also advance the step counter, which the caller then skips)
 constexpr int kNormLoads = 8;
-__global__ __launch_bounds__(kNormThreads) void k_norm_final(int nparts, int N, const double *__restrict__ part,
-                                                             double *__restrict__ out, int *__restrict__ ctr,
-                                                             int bump) {
-  __shared__ double red[4 * kNormThreads];
-  const int t = threadIdx.x;
-  double s[4] = {0, 0, 0, 0};
-  // thread t adds partials t, t + 1024, ... in that order; eight loads are in
-  // flight before the adds (absent ones are exact zeros)
-  for (int p0 = t; p0 < nparts; p0 += kNormLoads * kNormThreads) {
-    double q[kNormLoads][4];
+template <int NT>
+__device__ __forceinline__ void norm_row(int ng, int N, const double *__restrict__ part, double *__restrict__ out,
+                                         double *red) {
+  static_assert(kNormThreads % NT == 0, "every thread plays the same number of partial sums");
+  for (int vt = threadIdx.x; vt < kNormThreads; vt += NT) {
+    double s[4] = {0, 0, 0, 0};
+    for (int p0 = vt; p0 < ng; p0 += kNormLoads * kNormThreads) {
+      double q[kNormLoads][4];
 #pragma unroll
-    for (int u = 0; u < kNormLoads; ++u) {
-      const int p = p0 + u * kNormThreads;
-      if (p < nparts) ld4(part, p, q[u]);
-      else q[u][0] = q[u][1] = q[u][2] = q[u][3] = 0.0;
+      for (int u = 0; u < kNormLoads; ++u) {
+        const int p = p0 + u * kNormThreads;
+        if (p < ng) ld4(part, p, q[u]);
+        else q[u][0] = q[u][1] = q[u][2] = q[u][3] = 0.0;
+      }
+#pragma unroll
+      for (int u = 0; u < kNormLoads; ++u)
+        for (int v = 0; v < 4; ++v) s[v] = s[v] + q[u][v];
     }
-#pragma unroll
-    for (int u = 0; u < kNormLoads; ++u)
-      for (int v = 0; v < 4; ++v) s[v] = s[v] + q[u][v];
+    for (int v = 0; v < 4; ++v) red[v * kNormThreads + vt] = s[v];
   }
-  for (int v = 0; v < 4; ++v) red[v * kNormThreads + t] = s[v];
   __syncthreads();
   for (int h = kNormThreads / 2; h > 0; h >>= 1) {
-    if (t < h)
-      for (int v = 0; v < 4; ++v) red[v * kNormThreads + t] = red[v * kNormThreads + t] + red[v * kNormThreads + t + h];
+    for (int vt = threadIdx.x; vt < h; vt += NT)
+      for (int v = 0; v < 4; ++v)
+        red[v * kNormThreads + vt] = red[v * kNormThreads + vt] + red[v * kNormThreads + vt + h];
     __syncthreads();
   }
-  if (t == 0) {
-    double *o = out + 4 * (ctr ? ctr[0] : 0);
-    for (int v = 0; v < 4; ++v) o[v] = sqrt(red[v * kNormThreads] / double(N));
-    if (bump && ctr) ctr[0] = ctr[0] + 1;
-  }
+  if (threadIdx.x < 4) out[threadIdx.x] = sqrt(red[threadIdx.x * kNormThreads] / double(N));
+  __syncthreads();
+}
+
+// the pending steps' norms, one workgroup per step
+__global__ __launch_bounds__(kNormThreads) void k_norms(int ng, int N, const double *__restrict__ part,
+                                                        const int *__restrict__ ctr, double *__restrict__ out) {
+  __shared__ double red[4 * kNormThreads];
+  const int r = blockIdx.x;
+  norm_row<kNormThreads>(ng, N, part + 4 * long(r) * ng, out + 4 * (long(ctr[0]) + r), red);
 }
 
 // isentropic-vortex error over interior cells (src/mms.f90:315-361)
@@ -947,6 +992,14 @@ static __device__ __align__(256) double scratch[kScratchDoubles];
 
 namespace {
 constexpr int kMaxDevices = 64;
+// steps whose norm sums may be pending, and the memory their slice sums may
+// take (32 B per 64 cells and step: all 32 rows up to 4M cells)
+constexpr int kNormRows = 32;
+constexpr long kNormBytes = 64L << 20;
+// steps a captured graph covers: enough that its norm launches cost little
+// (0.5 us a step), few enough nodes that recapturing it (after every chunk of
+// a batched solve that froze or finished an instance) stays cheap
+constexpr int kGraphSteps = 8;
 double *g_scratch_ptr[kMaxDevices] = {};
 std::mutex g_scratch_mu;
 
@@ -1073,7 +1126,7 @@ struct fvs_ctx {
   // blist: nblk(N) entries of launch-block list, then 8 words per block of
   // active-cell bits (masked batches)
   int *dinst_off = nullptr, *dbinst = nullptr, *dwoff = nullptr, *blist = nullptr;
-  double *dpinf_inst = nullptr, *d2buf = nullptr, *dmach_aoa = nullptr, *dforces = nullptr;
+  double *dpinf_inst = nullptr, *dmach_aoa = nullptr, *dforces = nullptr;
   int nact = 0;                      // active blocks (0 = all, no list)
   // step counter for norm outputs (graph replays), graph mode switch
   int *dctr = nullptr;
@@ -1107,7 +1160,13 @@ struct fvs_ctx {
   // W does not hold the primitive state of U0 (the conservative-stage path
   // writes none); refreshed by the first caller that reads W
   bool w_stale = false;
-  int nparts = 0;
+  // residual norms: each step's slice sums go to one of norm_rows rows of part
+  // (and, in batches, the cells of the nsplit slices shared by instances to
+  // d2s); one launch reduces all pending rows.  norm_row is the row of the
+  // step being launched
+  int ng = 0, norm_rows = 1, norm_row = 0, nsplit = 0;
+  int *dsplit = nullptr, *dact = nullptr;
+  double *d2s = nullptr, *dlast = nullptr, *vpart = nullptr;
   bool have_state = false;
   double last_ms = 0.0;
   // the device the context was created on, and the address of `scratch` there
@@ -1469,8 +1528,6 @@ int setup_stage(fvs_ctx &C, const std::vector<int> &boff, const std::vector<int>
   max1 += max1 & 1;  // keep the LDS arrays after lP 16-byte aligned
   const int max2n = max2;
   if (size_t(6) * max2n * sizeof(double) > C.lds_max) return 0;
-  // k_stage's block reduction reuses the staged-state area: 4 x 512 doubles
-  max2 = std::max(max2, kStageThreads);
   const size_t lds = (size_t(6) * max2 + size_t(9) * max1 + size_t(5) * C.maxf) * sizeof(double);
   if (int rc = C.upload(C.s2off, s2off)) return rc;
   if (int rc = C.upload(C.s2n1, s2n1)) return rc;
@@ -1776,9 +1833,8 @@ int setup_device(fvs_ctx &C) {
     std::vector<short> lgat;
     int maxf = 0;
     block_lists(kBlock, boff, bfaces, lgat, maxf);
-    // LDS of k_flux_update: face fluxes (at least the 4 x 256 reduction) +
-    // the block's gradients and states
-    if (size_t(std::max(5 * maxf, 4 * kBlock)) * sizeof(double) + 12 * kBlock * sizeof(double) <= 64 * 1024) {
+    // LDS of k_flux_update: face fluxes + the block's gradients and states
+    if (size_t(5) * maxf * sizeof(double) + 12 * kBlock * sizeof(double) <= 64 * 1024) {
       C.maxf = maxf;
       C.nlisted = long(bfaces.size());
       if (int rc = C.upload(C.boff, boff)) return rc;
@@ -2028,8 +2084,11 @@ int setup_device(fvs_ctx &C) {
   if (int rc = C.alloc(C.WSA, size_t(Fi + Fb))) return rc;
   if (int rc = C.alloc(C.rout, n4)) return rc;
   if (int rc = C.alloc(C.wsout, N)) return rc;
-  C.nparts = std::max(nblk(N, kSmallBlock), nblk(std::max(C.ncell_intr, 1)));
-  if (int rc = C.alloc(C.part, 13 * size_t(C.nparts))) return rc;
+  // as many rows as fit kNormBytes, at least one
+  C.ng = nblk(N, kSlice);
+  C.norm_rows = int(std::max<long>(1, std::min<long>(kNormRows, kNormBytes / (32L * C.ng))));
+  if (int rc = C.alloc(C.part, 4 * size_t(C.ng) * C.norm_rows)) return rc;
+  if (int rc = C.alloc(C.vpart, 13 * size_t(nblk(std::max(C.ncell_intr, 1))))) return rc;
   if (int rc = C.alloc(C.small, 64)) return rc;
   if (int rc = C.alloc(C.dctr, 1)) return rc;
   if (int rc = C.alloc(C.pbar, 2)) return rc;
@@ -2061,7 +2120,17 @@ int setup_device(fvs_ctx &C) {
     if (int rc = C.upload(C.dmach_aoa, C.mach_aoa)) return rc;
     if (int rc = C.upload(C.dwoff, woff)) return rc;
     HIPC(hipMemcpyAsync(C.wall, wsorted.data(), wsorted.size() * sizeof(int), hipMemcpyHostToDevice, C.stream));
-    if (int rc = C.alloc(C.d2buf, n4)) return rc;
+    // slices that are not all one instance's cells
+    std::vector<int> split(C.ng, -1);
+    for (int g = 0; g < C.ng; ++g) {
+      const int i0 = g * kSlice, i1 = i0 + kSlice;
+      const int k = int(std::upper_bound(off.begin(), off.end(), i0) - off.begin());  // off[k] ends i0's instance
+      if (off[k] < i1) split[g] = C.nsplit++;
+    }
+    if (int rc = C.upload(C.dsplit, split)) return rc;
+    if (int rc = C.alloc(C.d2s, 4 * size_t(kSlice) * C.nsplit * C.norm_rows)) return rc;
+    if (int rc = C.alloc(C.dact, C.ninst)) return rc;
+    if (int rc = C.upload(C.dlast, std::vector<double>(4 * size_t(C.ninst), 0.0))) return rc;
     if (int rc = C.alloc(C.dforces, 4 * size_t(C.ninst))) return rc;
     if (int rc = C.alloc(C.blist, 9 * size_t(nblk(N)))) return rc;
   }
@@ -2223,11 +2292,20 @@ int launch_fluxes(fvs_ctx &C, double t) {
   return 0;
 }
 
+// where the last stage of the step being launched leaves its norm sums
+NormOut norm_out(const fvs_ctx &C) {
+  NormOut o;
+  o.part = C.part + 4 * size_t(C.ng) * C.norm_row;
+  o.split = C.dsplit;
+  o.d2 = C.d2s + 4 * size_t(kSlice) * C.nsplit * C.norm_row;
+  return o;
+}
+
 int launch_update(fvs_ctx &C, const Upd &A) {
   ProfScope ps(C, KC_UPDATE);
   hipLaunchKernelGGL(k_update, dim3(xcd_grid(nblk(C.N))), dim3(kBlock), 0, C.stream, xcd_arg(nblk(C.N), C.xcd_upd),
                      C.N, C.GW, A, C.gat, C.FA, C.WSA, C.vol,
-                     C.U0, C.Ub, C.Facc, C.W, C.dtl, C.rout, C.wsout, C.part);
+                     C.U0, C.Ub, C.Facc, C.W, C.dtl, C.rout, C.wsout, norm_out(C));
   HIPC(hipGetLastError());
   return 0;
 }
@@ -2247,20 +2325,20 @@ int launch_flux_update(fvs_ctx &C, const Upd &A, double t, const double *uin = n
     const int phi_one = (C.opt.limiter == 0 && C.opt.recon != 1) ? 1 : 0;
     if (C.small_blocks) {
       const int nb = nblk(C.N, kSmallBlock);
-      const size_t lds = size_t(std::max(per * C.maxf_s, 4 * kSmallBlock)) * sizeof(double);
+      const size_t lds = size_t(per) * C.maxf_s * sizeof(double);
       hipLaunchKernelGGL(k_flux_update<kSmallBlock>, dim3(xcd_grid(nb)), dim3(kSmallBlock), lds, C.stream, C.N,
                          xcd_arg(nb, C.xcd_fused), C.GW, C.maxf_s, A, C.P, t, C.boff_s, C.lrec_s, C.lgeo_s,
                          C.nlisted_s, C.lgat_s, cons ? uin : C.W, C.grad, C.phi, C.vol, C.U0, cons ? uout : C.Ub,
-                         C.Facc, cons ? nullptr : C.Walt, C.dtl, C.part, nullptr, nullptr,
-                         A.last ? C.d2buf : nullptr, phi_one, cons ? 1 : 0);
+                         C.Facc, cons ? nullptr : C.Walt, C.dtl, norm_out(C), nullptr, nullptr, phi_one,
+                         cons ? 1 : 0);
     } else {
       const int nb = nblk(C.N);
-      const size_t lds = size_t(std::max(per * C.maxf, 4 * kBlock)) * sizeof(double);
+      const size_t lds = size_t(per) * C.maxf * sizeof(double);
       hipLaunchKernelGGL(k_flux_update<kBlock>, dim3(C.nact ? C.nact : xcd_grid(nb)), dim3(kBlock), lds, C.stream,
                          C.N, xcd_arg(nb, C.xcd_fused), C.GW, C.maxf, A, C.P, t, C.boff, C.lrec, C.lgeo, C.nlisted,
                          C.lgat, cons ? uin : C.W, C.grad, C.phi, C.vol, C.U0, cons ? uout : C.Ub, C.Facc,
-                         cons ? nullptr : C.Walt, C.dtl, C.part, C.nact ? C.blist : nullptr,
-                         C.ninst > 0 ? C.dpinf_inst : nullptr, A.last ? C.d2buf : nullptr, phi_one, cons ? 1 : 0);
+                         cons ? nullptr : C.Walt, C.dtl, norm_out(C), C.nact ? C.blist : nullptr,
+                         C.ninst > 0 ? C.dpinf_inst : nullptr, phi_one, cons ? 1 : 0);
     }
   }
   HIPC(hipGetLastError());
@@ -2311,7 +2389,7 @@ StageArgs stage_args(const fvs_ctx &C, double t) {
   a.Ub = C.Ub;
   a.Facc = C.Facc;
   a.dtl = C.dtl;
-  a.part = C.part;
+  a.norm = norm_out(C);
   a.blist = C.nact ? C.blist : nullptr;
   a.binst = C.dbinst;
   a.pinf_inst = C.dpinf_inst;
@@ -2330,8 +2408,7 @@ int launch_stage(fvs_ctx &C, const Upd &A, double t) {
   const bool lim = C.opt.limiter > 0 && !C.limiter_frozen;
   const dim3 g(C.nact ? C.nact : xcd_grid(nb)), b(kStageThreads);
   const StageArgs a = stage_args(C, t);
-  double *d2 = A.last ? C.d2buf : nullptr;
-#define FVS_STAGE(L, PM) hipLaunchKernelGGL((k_stage<L, PM>), g, b, lds, C.stream, a, A, C.W, C.Walt, d2)
+#define FVS_STAGE(L, PM) hipLaunchKernelGGL((k_stage<L, PM>), g, b, lds, C.stream, a, A, C.W, C.Walt)
   if (lim) {
     if (C.pmode == 0) FVS_STAGE(1, 0);
     else if (C.pmode == 1) FVS_STAGE(1, 1);
@@ -2354,8 +2431,8 @@ int launch_vortex_err(fvs_ctx &C, double t, double *dst) {
   if (n == 0) return 0;
   const int nb = nblk(n);
   hipLaunchKernelGGL(k_vortex_err, dim3(nb), dim3(kBlock), 0, C.stream, n, C.P, t, C.cell_intr, C.cx, C.cy, C.U0,
-                     C.part);
-  hipLaunchKernelGGL(k_vortex_final, dim3(1), dim3(64), 0, C.stream, nb, n, C.part, C.cell_intr, C.cx, C.cy,
+                     C.vpart);
+  hipLaunchKernelGGL(k_vortex_final, dim3(1), dim3(64), 0, C.stream, nb, n, C.vpart, C.cell_intr, C.cx, C.cy,
                      C.iperm[0], dst);
   HIPC(hipGetLastError());
   return 0;
@@ -2909,10 +2986,23 @@ int fvs_roe_flux_batch(int n, double gamma, const double *pL, const double *pR, 
 
 namespace {
 
+InstNorms inst_norms_of(const fvs_ctx &C) {
+  InstNorms I;
+  I.ninst = C.ninst;
+  I.ng = C.ng;
+  I.nsplit = C.nsplit;
+  I.off = C.dinst_off;
+  I.split = C.dsplit;
+  I.act = C.nact ? C.dact : nullptr;
+  I.last = C.dlast;
+  return I;
+}
+
 // The stage sequence of one time step (src/runge_kutta.f90:120-418 and the
-// SSP-RK3 of this library).  Norm outputs go to dn / dinst at the step index
-// held in the device counter, which the step advances; so the same launch
-// sequence can be captured once in a HIP graph and replayed.
+// SSP-RK3 of this library).  Its norm sums go to row norm_row of the pending
+// norms; launch_norms reduces them to the output rows the device counter
+// names, so a sequence of steps and their norms can be captured once in a HIP
+// graph and replayed.
 // SSP-RK3 stages on conservative states (no primitive-state traffic): the
 // fused path with the staged-halo LSQ gradient, an unlimited Green-Gauss
 // gradient (kernel_path 3 keeps primitive states) or a first-order
@@ -2979,7 +3069,7 @@ Upd stage_upd(const fvs_options &o, int k, double told, double &ts) {
   return A;
 }
 
-int launch_step(fvs_ctx &C, double told, double *dn, double *dinst) {
+int launch_step(fvs_ctx &C, double told) {
   const fvs_options &o = C.opt;
   const int nst = (o.rk_scheme == FVS_RK_SSP3) ? 3 : 4;
   for (int k = 0; k < nst; ++k) {
@@ -3002,21 +3092,26 @@ int launch_step(fvs_ctx &C, double told, double *dn, double *dinst) {
     }
     if (rc) return rc;
   }
-  // the step counter (the norms' output row) advances after its last reader
-  const bool inst = dinst && C.ninst > 0;
-  if (!C.nact) {
+  HIPC(hipGetLastError());
+  return 0;
+}
+
+// Norms of the steps whose slice sums are pending (rows 0 .. rows - 1), to the
+// output rows from the device's step counter on, which then advances.  One
+// launch of one workgroup per step (and instance): a reduction of its own after
+// every step left the chip idle meanwhile, 3.2 of 47 us per step on 8,192
+// cells and 70 of 580 us on a batch of 12 O-grids (983,040 cells).
+int launch_norms(fvs_ctx &C, int rows, double *dn, double *dinst) {
+  if (rows <= 0) return 0;
+  {
     ProfScope ps(C, KC_NORM);
-    // one partial sum per launch block of the last stage
-    const int nparts = (C.fused && !C.stage && C.small_blocks) ? nblk(C.N, kSmallBlock) : nblk(C.N);
-    hipLaunchKernelGGL(k_norm_final, dim3(1), dim3(kNormThreads), 0, C.stream, nparts, C.N, C.part, dn, C.dctr,
-                       inst ? 0 : 1);
+    if (dn && !C.nact)
+      hipLaunchKernelGGL(k_norms, dim3(rows), dim3(kNormThreads), 0, C.stream, C.ng, C.N, C.part, C.dctr, dn);
+    if (dinst && C.ninst > 0)
+      hipLaunchKernelGGL(k_inst_norms, dim3(C.ninst, rows), dim3(kBlock), 0, C.stream, inst_norms_of(C), rows, C.part,
+                         C.d2s, C.dctr, dinst);
   }
-  if (inst) {
-    ProfScope ps(C, KC_NORM);
-    hipLaunchKernelGGL(k_inst_norms, dim3(C.ninst), dim3(kBlock), 0, C.stream, C.ninst, C.dinst_off, C.d2buf, C.dctr,
-                       dinst);
-  }
-  if (C.nact || inst) hipLaunchKernelGGL(k_counter, dim3(1), dim3(1), 0, C.stream, C.dctr, 1, 1);
+  hipLaunchKernelGGL(k_counter, dim3(1), dim3(1), 0, C.stream, C.dctr, rows, 1);
   HIPC(hipGetLastError());
   return 0;
 }
@@ -3045,7 +3140,11 @@ int ensure_graph(fvs_ctx &C, int gsteps, double t1, double *dn, double *dinst) {
   int rc = 0;
   // t1 is baked into the captured launches; only time-dependent boundary
   // data read it, and those never run from a graph
-  for (int g = 0; g < gsteps && !rc; ++g) rc = launch_step(C, t1, dn, dinst);
+  for (int g = 0; g < gsteps && !rc; ++g) {
+    C.norm_row = g;
+    rc = launch_step(C, t1);
+  }
+  if (!rc) rc = launch_norms(C, gsteps, dn, dinst);
   hipError_t e = hipStreamEndCapture(C.stream, &graph);
   if (rc) {
     if (graph) (void)hipGraphDestroy(graph);
@@ -3078,17 +3177,16 @@ int launch_persistent(fvs_ctx &C, double t1, int nsteps, double *dn, double *din
   c.nlaunch = C.nact ? C.nact : nblk(C.N);
   c.W0 = C.W;
   c.W1 = C.Walt;
-  c.d2buf = C.d2buf;
   c.dn = C.nact ? nullptr : dn;
-  c.nparts = nblk(C.N);
+  c.ng = C.ng;
   const bool inst = dinst && C.ninst > 0;
   c.dinst = inst ? dinst : nullptr;
-  c.ninst = C.ninst;
-  c.inst_off = C.dinst_off;
+  c.inst = inst_norms_of(C);
   c.ctr = C.dctr;
   c.bar = C.pbar;
   c.err = C.perr;
   c.spin = 1u << 22;
+  C.norm_row = 0;
   StageArgs a = stage_args(C, t1);
   a.nb = nblk(C.N);  // plain numbering: the persistent loop walks the blocks itself
   const size_t lds = std::max(stage_lds(C), size_t(4) * kNormThreads * sizeof(double));
@@ -3130,21 +3228,30 @@ int run_steps(fvs_ctx &C, double t1, int nsteps, double *dn, double *dv, double 
     return launch_persistent(C, t1, nsteps, dn, dinst);
   int s = 0;
   // graph replay: one captured graph covers an even number of stages so the
-  // primitive-state buffers are back in place after each replay
+  // primitive-state buffers are back in place after each replay, and as many
+  // steps as kGraphSteps and the norm rows allow (at most half the call's, so
+  // that it is replayed)
   if (graph_ok && C.use_graph && !C.profiling && !dv && !time_dependent(C)) {
-    const int gsteps = (nst % 2 == 0) ? 1 : 2;
-    if (nsteps >= 2 * gsteps) {
+    int gsteps = (nst % 2 == 0) ? 1 : 2;
+    while (2 * gsteps <= std::min({kGraphSteps, C.norm_rows, nsteps / 2})) gsteps *= 2;
+    if (nsteps >= 2 * gsteps && gsteps <= C.norm_rows) {
       if (int rc = ensure_graph(C, gsteps, t1, dn, dinst)) return rc;
       hipError_t e = hipSuccess;
       for (; s + gsteps <= nsteps && e == hipSuccess; s += gsteps) e = hipGraphLaunch(C.gexec, C.stream);
       if (e != hipSuccess) return fail(FVS_EHIP, std::string("graph launch: ") + hipGetErrorString(e));
     }
   }
+  int pending = 0;
   for (; s < nsteps; ++s) {
     const double told = t1 + double(s) * dt;
-    if (int rc = launch_step(C, told, dn, dinst)) return rc;
+    C.norm_row = pending;
+    if (int rc = launch_step(C, told)) return rc;
     if (dv)
       if (int rc = launch_vortex_err(C, told + dt, dv + kVerr * size_t(s))) return rc;
+    if (++pending == C.norm_rows || s + 1 == nsteps) {
+      if (int rc = launch_norms(C, pending, dn, dinst)) return rc;
+      pending = 0;
+    }
   }
   // the conservative stages wrote no primitive state: W is refreshed by the
   // next caller that reads it, not inside the timed steps
@@ -3164,7 +3271,7 @@ int integrate(fvs_ctx *C, double t1, int nsteps, double *norms, double *verr, do
   const bool want_inst = inst_norms && C->ninst > 0;
   if (want_inst)
     if (int rc = C->grow(C->di_buf, C->di_cap, size_t(nsteps) * C->ninst * 4)) return rc;
-  double *dn = C->dn_buf, *dv = verr ? C->dv_buf : nullptr, *di = want_inst ? C->di_buf : nullptr;
+  double *dn = want_inst && !norms ? nullptr : C->dn_buf, *dv = verr ? C->dv_buf : nullptr, *di = want_inst ? C->di_buf : nullptr;
   const bool timers = C->phase_timing && !C->profiling;
   if (timers) {
     C->profiling = true;
@@ -3326,6 +3433,9 @@ int fvs_batch_set_active(fvs_ctx *C, const int *active) try {
   // masked cells are not updated, so on the primitive-state paths their W
   // lags the stage parity; a resumed instance starts from its own state
   refresh_prim(*C);
+  std::vector<int> act(C->ninst);
+  for (int k = 0; k < C->ninst; ++k) act[k] = active[k] != 0;
+  HIPC(hipMemcpyAsync(C->dact, act.data(), act.size() * sizeof(int), hipMemcpyHostToDevice, C->stream));
   HIPC(hipGetLastError());
   HIPC(hipStreamSynchronize(C->stream));
   C->nact = all ? 0 : int(list.size());
@@ -3485,7 +3595,7 @@ int fvs_kernel_times(fvs_ctx *C, double t1, int nsteps, double *ms, double *byte
   else state = (32 + 32 + 64 + 64 + 64 + 64 + 32 + 32 + 32) / 4.0;
   if (C->opt.steady) state += (8.0 + 8.0 * (nst - 1)) / nst;
   const double bup = N * (C->GW * 4.0 + 8 + 32 + state) + (Fi + Fb) * 40.0;
-  const double bno = 4.0 * 8 * nblk(C->N) + 32;
+  const double bno = 32.0 * C->ng * std::min(C->norm_rows, nsteps);  // slice sums of the steps one launch reduces
   // fused: the listed face records (cells + 7 geometry values; a face on
   // a block border is listed, and stored, once per block), the stage's W and
   // grad once (phi unless there is no limiter), the cell-side traffic of the
