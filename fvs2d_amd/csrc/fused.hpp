@@ -56,6 +56,18 @@ __device__ __forceinline__ void lsq_apply_ginv(double G11, double G12, double G2
   }
 }
 
+// instance of cell i by bisection of the offset table (ioff[0] = 0 <= i <
+// ioff[ninst])
+__device__ __forceinline__ int instance_of(const int *__restrict__ ioff, int ninst, int i) {
+  int lo = 0, hi = ninst;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (ioff[mid] <= i) lo = mid;
+    else hi = mid;
+  }
+  return lo;
+}
+
 // PMODE: 0 -> p = 0, 1 -> p = 1, 2 -> p = 2, 3 -> general p (pow)
 template <int LIM, int PMODE>
 __global__ __launch_bounds__(kBlock) void k_grad_lsqc(int N, int nb, const double *__restrict__ W,
@@ -146,15 +158,7 @@ __global__ __launch_bounds__(kBlock) void k_grad_lsqc(int N, int nb, const doubl
     // batch mode with some instances frozen: find the cell's instance in the
     // offset table (ioff[0] = 0 <= i < ioff[ninst] = N) and keep its value
     bool keep = false;
-    if (ioff) {
-      int lo = 0, hi = ninst;
-      while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (ioff[mid] <= i) lo = mid;
-        else hi = mid;
-      }
-      keep = frz[lo] != 0;
-    }
+    if (ioff) keep = frz[instance_of(ioff, ninst, i)] != 0;
     if (!keep) phi[i] = cell_limiter(lt, nvrt[i], N, i, loff, vol[i], w, mn, mx, gx, gy);
   }
 }
@@ -282,34 +286,34 @@ __device__ __forceinline__ const unsigned *active_mask(const int *blist, int nbl
   return reinterpret_cast<const unsigned *>(blist + nbl);
 }
 
-// CB cells per block, one per thread (further threads of the workgroup idle);
-// instance masks exist for 256-cell blocks only
-template <int CB = kBlock>
-__device__ __forceinline__ void block_update_finish(int N, int lb, const Upd &A, const UpdIn &in,
-                                                    const double *__restrict__ lF, const double *__restrict__ lS,
-                                                    double *__restrict__ Ua, double *__restrict__ Ub,
-                                                    double *__restrict__ Facc, double *__restrict__ Wout,
-                                                    double *__restrict__ dtl, const NormOut &norm,
-                                                    const unsigned *__restrict__ amask) {
-  const int i = lb * CB + threadIdx.x;
+// Gather, update and norm sums of cell i, one per thread (valid: i < N; whole
+// wavefronts call this): flux(f, fa) gives the flux * area of the block's face
+// f, speed(f) its wave speed * area.  amask (batches with masked instances): bit
+// i of its words is set when cell i belongs to an active instance; a masked
+// cell keeps its state (the update is computed, nothing is stored) and
+// contributes zero increments.
+template <class Flux, class Speed>
+__device__ __forceinline__ void cell_update(int N, int i, bool valid, const Upd &A, const UpdIn &in, Flux flux,
+                                            Speed speed, double *__restrict__ Ua, double *__restrict__ Ub,
+                                            double *__restrict__ Facc, double *__restrict__ Wout,
+                                            double *__restrict__ dtl, const NormOut &norm,
+                                            const unsigned *__restrict__ amask) {
   double d2[4] = {0, 0, 0, 0};
-  // amask (batches with masked instances): bit l of the block's eight words
-  // is set when its cell l belongs to an active instance; a masked cell
-  // keeps its state (the update is computed, nothing is stored) and
-  // contributes zero increments
-  const bool on = !amask || threadIdx.x >= CB || ((amask[8 * lb + (threadIdx.x >> 5)] >> (threadIdx.x & 31)) & 1u);
-  if (threadIdx.x < CB && i < N) {
+  const bool on = !amask || !valid || ((amask[i >> 5] >> (i & 31)) & 1u);
+  if (valid) {
     double acc[4] = {0.0, 0.0, 0.0, 0.0}, wacc = 0.0;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const int s = in.sv[k];
       if (s == 0) break;
       const int f = (s > 0 ? s : -s) - 1;
+      double fa[4];
+      flux(f, fa);
       if (s > 0)
-        for (int v = 0; v < 4; ++v) acc[v] = acc[v] + lF[4 * f + v];
+        for (int v = 0; v < 4; ++v) acc[v] = acc[v] + fa[v];
       else
-        for (int v = 0; v < 4; ++v) acc[v] = acc[v] - lF[4 * f + v];
-      if (A.steady && A.first) wacc = wacc + lS[f];
+        for (int v = 0; v < 4; ++v) acc[v] = acc[v] - fa[v];
+      if (A.steady && A.first) wacc = wacc + speed(f);
     }
     const double V = in.V;
     double R[4];
@@ -364,7 +368,25 @@ __device__ __forceinline__ void block_update_finish(int N, int lb, const Upd &A,
       st4(Wout, i, w);
     }
   }
-  if (A.last && threadIdx.x < CB) slice_norms(norm, i, N, d2);
+  if (A.last) slice_norms(norm, i, N, d2);
+}
+
+// the same for a 256-, 128-cell block with its face fluxes as [f][4] and wave
+// speeds as [f] in LDS
+template <int CB = kBlock>
+__device__ __forceinline__ void block_update_finish(int N, int lb, const Upd &A, const UpdIn &in,
+                                                    const double *__restrict__ lF, const double *__restrict__ lS,
+                                                    double *__restrict__ Ua, double *__restrict__ Ub,
+                                                    double *__restrict__ Facc, double *__restrict__ Wout,
+                                                    double *__restrict__ dtl, const NormOut &norm,
+                                                    const unsigned *__restrict__ amask) {
+  const int i = lb * CB + threadIdx.x;
+  if (threadIdx.x < CB)
+    cell_update(N, i, i < N, A, in,
+                [&](int f, double fa[4]) __attribute__((always_inline)) {
+                  for (int v = 0; v < 4; ++v) fa[v] = lF[4 * f + v];
+                },
+                [&](int f) __attribute__((always_inline)) { return lS[f]; }, Ua, Ub, Facc, Wout, dtl, norm, amask);
 }
 
 // fused face fluxes (LDS) + ordered gather + stage update; reads the stage's
@@ -502,24 +524,6 @@ __global__ __launch_bounds__(BS) void k_flux_update(int N, int nb, int gw, int m
                           blist ? active_mask(blist, nbl) : nullptr);
 }
 
-// Whole RK stage in one kernel per 256-cell block: the block stages, in LDS,
-// the state and centre of every cell its gradients read (C2: the block's
-// cells, then the other cells of its faces -- together C1 -- then the rest
-// of their stencils), computes the gradient (and limiter) of the C1 cells
-// from LDS, the fluxes of its faces from LDS, and the gather + update of its
-// own cells, with 512 threads per 256-cell block.  Halo gradients are
-// recomputed by every block that needs them
-// (about 19% more gradients on triangle meshes), so gradients never travel
-// through HBM.  Arithmetic and summation order are those of k_grad_lsqc and
-// k_flux_update, so the results are bit-identical to them.
-//
-// Per block b: C2 cells s2list[s2off[b] .. s2off[b+1]), the first s2n1[b]
-// of them C1 (its own cells first, in order); C1 stencils in slices of 64
-// cells (slice sl0[b] + q/64, width slw, entries slid[sleo + k*64 + q%64] =
-// local C2 index << 4 | periodic-shift code); listed face f's cells as local
-// indices blf[f] = c1 | c2 << 16 (c2 = 0xffff on a boundary face).
-// phisrc: 0 -> limiter values 1 (no limiter), 1 -> read phi (frozen); with
-// LIM the limiter is evaluated and written for the block's own cells.
 // One stencil entry of an LDS-staged LSQ gradient: local code (index << 4 |
 // periodic shift) of neighbour j of the cell at centre ci with state w.
 // The term itself is the shared lsq_term.
@@ -559,46 +563,13 @@ __device__ __forceinline__ double grad_finish(int id, int N, const double w[4], 
     g8[4 + v] = gy[v];
   }
   bool keep = !LIM;
-  if (LIM && ioff) {
-    int lo = 0, hi = ninst;
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (ioff[mid] <= id) lo = mid;
-      else hi = mid;
-    }
-    keep = frz[lo] != 0;
-  }
+  if (LIM && ioff) keep = frz[instance_of(ioff, ninst, id)] != 0;
   if (!keep) {
     const double ph = cell_limiter(lt, nvrt[id], N, id, loff, vol[id], w, mn, mx, gx, gy);
     if (own) phi[id] = ph;
     return ph;
   }
   return phisrc == 1 ? phi[id] : 1.0;
-}
-
-// Gradient of local cell q (global id) from states and centres staged in
-// LDS, with its stencil as local codes (index << 4 | periodic shift) in a
-// 64-cell slice starting at sl (width wid).  Same arithmetic and order as
-// k_grad_lsqc.
-template <int LIM, int PMODE>
-__device__ __forceinline__ double lds_gradient(int q, int id, int N, const double *__restrict__ lW,
-                                               const double2 *__restrict__ lX, const unsigned short *__restrict__ sl,
-                                               int wid, const ShiftTable &st, double p,
-                                               const double *__restrict__ ginv, double g8[8], int phisrc,
-                                               double *__restrict__ phi, int lt, const int *__restrict__ nvrt,
-                                               const double2 *__restrict__ loff, const double *__restrict__ vol,
-                                               const int *__restrict__ ioff, const int *__restrict__ frz, int ninst,
-                                               bool own) {
-  const int l = q % kSlice;
-  const double2 ci = lX[q];
-  double w[4], sx[4] = {0, 0, 0, 0}, sy[4] = {0, 0, 0, 0}, mn[4], mx[4];
-  ld4(lW, q, w);
-  for (int v = 0; v < 4; ++v) mn[v] = mx[v] = w[v];
-  for (int k = 0; k < wid; ++k)
-    lds_accum<LIM, PMODE>(sl[long(k) * kSlice + l], ci, w, lW, lX, st, p, sx, sy, mn, mx);
-  const double G[3] = {ginv[id], ginv[N + id], ginv[2 * long(N) + id]};
-  return grad_finish<LIM>(id, N, w, sx, sy, mn, mx, G, g8, phisrc, phi, lt, nvrt, loff, vol, ioff, frz, ninst,
-                          own);
 }
 
 // LSQ gradient (and limiter) of the block's own cells with the cells its
@@ -697,118 +668,6 @@ __global__ __launch_bounds__(BS, LIM ? 1 : 7) void k_grad_lsqh(int N, int nb, in
   double g8[8];
   grad_finish<LIM>(id, N, w, sx, sy, mn, mx, G, g8, 0, phi, lt, nvrt, loff, vol, ioff, frz, ninst, true);
   st8(grad, id, g8);
-}
-
-constexpr int kStageThreads = 2 * kBlock;  // two threads per cell: each phase fits one round
-
-// Everything k_stage reads besides the stage's own update constants and its
-// input / output primitive states (one struct, so the same block body serves
-// the per-stage launch and the persistent whole-step kernel).
-struct StageArgs {
-  int N, nb, gw, maxf, max1, max2;
-  Phys P;
-  double t;
-  const int *boff, *bfaces;
-  const unsigned *blf;
-  const short *lgat;
-  int Fi;
-  const double *fgeo;
-  const int *btype;
-  const double *bgeo;
-  const int *s2off, *s2n1, *s2list, *sl0, *slw;
-  const long *sleo;
-  const unsigned short *slid;
-  const double2 *cxy;
-  const double *ginv;
-  ShiftTable st;
-  double p;
-  int phisrc;
-  double *phi;
-  int lt;
-  const int *nvrt;
-  const double2 *loff;
-  const double *vol;
-  const int *ioff, *frz;
-  int ninst;
-  double *Ua, *Ub, *Facc, *dtl;
-  NormOut norm;
-  const int *blist, *binst;
-  const double *pinf_inst;
-};
-
-// One 256-cell block lb of a whole RK stage (see above).
-template <int LIM, int PMODE>
-__device__ __forceinline__ void stage_block(const StageArgs &a, int lb, const Upd &A, const double *__restrict__ Win,
-                                            double *__restrict__ Wout) {
-  extern __shared__ double lds[];
-  const int N = a.N, max1 = a.max1, max2 = a.max2, maxf = a.maxf;
-  double *lW = lds;                                   // [max2][4]
-  double2 *lX = reinterpret_cast<double2 *>(lds + 4 * max2);  // [max2]
-  double *lG = lds + 6 * max2;                        // [max1][8]
-  double *lP = lG + 8 * max1;                         // [max1]
-  double *lF = lP + max1;                             // [maxf][4]
-  double *lS = lF + 4 * maxf;                         // [maxf]
-  const int nbl = a.nb < 0 ? -a.nb : a.nb;
-  const int o2 = a.s2off[lb], n2 = a.s2off[lb + 1] - o2, n1 = a.s2n1[lb];
-  const int i0 = lb * kBlock, nown = (N - i0 < kBlock) ? N - i0 : kBlock;
-  // stage the state and centres of C2
-  for (int q = threadIdx.x; q < n2; q += kStageThreads) {
-    const int id = a.s2list[o2 + q];
-    double w[4];
-    ld4(Win, id, w);
-    st4(lW, q, w);
-    lX[q] = a.cxy[id];
-  }
-  __syncthreads();
-  // gradients (and limiter values) of C1 from LDS
-  for (int q = threadIdx.x; q < n1; q += kStageThreads) {
-    const int id = a.s2list[o2 + q];
-    const int si = a.sl0[lb] + q / kSlice;
-    double g8[8];
-    const double ph = lds_gradient<LIM, PMODE>(q, id, N, lW, lX, a.slid + a.sleo[si], a.slw[si], a.st, a.p, a.ginv,
-                                               g8, a.phisrc, a.phi, a.lt, a.nvrt, a.loff, a.vol, a.ioff, a.frz,
-                                               a.ninst, q < nown);
-    st8(lG, q, g8);
-    lP[q] = ph;
-  }
-  __syncthreads();
-  // face fluxes from LDS
-  const int f0 = a.boff[lb], nf = a.boff[lb + 1] - f0;
-  for (int f = threadIdx.x; f < nf; f += kStageThreads) {
-    const int slot = a.bfaces[f0 + f];
-    const unsigned pr = a.blf[f0 + f];
-    const int la = int(pr & 0xffffu), lc = int(pr >> 16);
-    double fa[4], wsa, g[8];
-    if (slot < a.Fi) {
-      ld8(a.fgeo, slot, g);
-      interior_flux(a.P, make_int2(la, lc), g, lW, lG, lP, fa, wsa);
-    } else {
-      const int b = slot - a.Fi;
-      ld8(a.bgeo, b, g);
-      boundary_flux(a.P, a.t, la, a.btype[b], g, lW, lG, lP, fa, wsa,
-                    a.binst ? a.pinf_inst + 4 * a.binst[b] : a.P.pinf);
-    }
-    for (int v = 0; v < 4; ++v) lF[4 * f + v] = fa[v];
-    lS[f] = wsa;
-  }
-  __syncthreads();
-  {
-    UpdIn in;
-    const int ic = lb * kBlock + threadIdx.x;
-    if (threadIdx.x < kBlock && ic < N)
-      block_update_load(N, ic, a.gw, A, a.lgat, a.vol, a.Ua, a.Ub, a.Facc, a.dtl, in);
-    block_update_finish(N, lb, A, in, lF, lS, a.Ua, a.Ub, a.Facc, Wout, a.dtl, a.norm,
-                        a.blist ? active_mask(a.blist, nbl) : nullptr);
-  }
-}
-
-template <int LIM, int PMODE>
-__global__ __launch_bounds__(kStageThreads) void k_stage(StageArgs a, Upd A, const double *__restrict__ Win,
-                                                         double *__restrict__ Wout) {
-  const int lb = a.blist ? a.blist[blockIdx.x] : xcd_block(a.nb);
-  const int nbl = a.nb < 0 ? -a.nb : a.nb;
-  if (lb >= nbl) return;  // the whole workgroup leaves before any barrier
-  stage_block<LIM, PMODE>(a, lb, A, Win, Wout);
 }
 
 // Residual norms of one step of instance k from the step's partials (fixed
@@ -920,100 +779,3 @@ __global__ void k_wall_forces_inst(int ninst, const int *__restrict__ woff, cons
   out[4 * k + 3] = cn1 * sn + ca1 * c;
 }
 
-// ---------------------------------------------------------------------------
-// Persistent whole-step kernel: one cooperative launch runs nsteps time steps
-// of the whole-stage block body over the launch-block list (the ragged batch's
-// active blocks, or every block), with a grid-wide barrier after each stage
-// and the step's residual norms reduced in the same launch.
-// ---------------------------------------------------------------------------
-
-// Grid-wide barrier of a co-resident launch: thread 0 of each workgroup
-// counts itself in bar[0]; the last one resets the count and advances the
-// generation bar[1]; the others poll the generation.  Each poll is bounded
-// (spin polls, or as soon as another workgroup has given up and set *err):
-// a workgroup that gives up records it in *err and returns false, so every
-// wave of the launch ends.
-__device__ __forceinline__ bool grid_barrier(unsigned *bar, unsigned nwg, unsigned &gen, unsigned spin, int *err) {
-  __shared__ int ok;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    ok = 1;
-    __threadfence();
-    const unsigned arrived = atomicAdd(&bar[0], 1u);
-    if (arrived == nwg - 1) {
-      atomicExch(&bar[0], 0u);
-      __threadfence();
-      atomicAdd(&bar[1], 1u);
-    } else {
-      unsigned n = 0;
-      while (__hip_atomic_load(&bar[1], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) == gen) {
-        __builtin_amdgcn_s_sleep(2);
-        if (++n >= spin || __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
-          atomicExch(err, 1);
-          ok = 0;
-          break;
-        }
-      }
-    }
-    gen = gen + 1;
-    __threadfence();
-  }
-  __syncthreads();
-  return ok != 0;
-}
-
-struct PersistCtl {
-  Upd A[4];                 // the stages of one step
-  int nst, nsteps, nlaunch;  // stages per step, steps, launch blocks
-  double *W0, *W1;          // primitive states: stage k of the launch reads W0 when k is even
-  double *dn;               // whole-mesh norms, one row per step (NULL: none)
-  int ng;                   // 64-cell slices
-  double *dinst;            // per-instance norms (NULL: none)
-  InstNorms inst;
-  int *ctr;                 // output row of the first step; advanced by nsteps at the end
-  unsigned *bar;
-  int *err;
-  unsigned spin;
-};
-
-template <int LIM, int PMODE>
-__global__ __launch_bounds__(kStageThreads) void k_steps_persistent(StageArgs a, PersistCtl c) {
-  extern __shared__ double lds[];
-  unsigned gen = 0;
-  if (threadIdx.x == 0) gen = __hip_atomic_load(&c.bar[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const int row0 = c.ctr[0];  // block 0 writes the counter only after the last barrier
-  int par = 0;
-  bool ok = true;
-  for (int s = 0; s < c.nsteps && ok; ++s) {
-    for (int k = 0; k < c.nst && ok; ++k) {
-      const Upd A = c.A[k];
-      const double *Win = par ? c.W1 : c.W0;
-      double *Wout = par ? c.W0 : c.W1;
-      for (int q = blockIdx.x; q < c.nlaunch; q += gridDim.x) {
-        const int lb = a.blist ? a.blist[q] : q;
-        stage_block<LIM, PMODE>(a, lb, A, Win, Wout);
-        __syncthreads();  // the next block's staging overwrites this one's LDS
-      }
-      ok = grid_barrier(c.bar, gridDim.x, gen, c.spin, c.err);
-      par ^= 1;
-    }
-    if (!ok) break;
-    // this step's norms; the partials and increments they read are next
-    // written by the last stage of the next step, two or more barriers later
-    const long row = long(row0) + s;
-    if (c.dn && blockIdx.x == 0) norm_row<kStageThreads>(c.ng, a.N, a.norm.part, c.dn + 4 * row, lds);
-    if (c.dinst)
-      for (int k = blockIdx.x; k < c.inst.ninst; k += gridDim.x)
-        inst_norm_row(c.inst, k, a.norm.part, a.norm.d2, s == c.nsteps - 1,
-                      c.dinst + 4 * (row * c.inst.ninst + k), lds);
-  }
-  if (ok) ok = grid_barrier(c.bar, gridDim.x, gen, c.spin, c.err);
-  if (ok && blockIdx.x == 0 && threadIdx.x == 0) c.ctr[0] = row0 + c.nsteps;
-}
-
-__global__ void k_barrier_reset(unsigned *bar, int *err) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    bar[0] = 0u;
-    err[0] = 0;
-  }
-}

@@ -124,13 +124,9 @@ __global__ void k_prim(int N, double g, const double *__restrict__ U, double *__
 // which can differ from the reference's minimum only where two candidates
 // are within rounding of each other.  Van Albada divides per face as
 // written.
-__device__ __forceinline__ double cell_limiter(int lt, int nf, int N, int i, const double2 *__restrict__ off,
-                                               double vol, const double w[4], const double mn[4],
-                                               const double mx[4], const double gx[4], const double gy[4]) {
-  // face offsets in registers: every index below is a compile-time constant
-  double2 o[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) o[k] = (k < nf) ? off[long(k) * N + i] : make_double2(0.0, 0.0);
+__device__ __forceinline__ double cell_limiter_v(int lt, int nf, const double2 o[4], double vol, const double w[4],
+                                                 const double mn[4], const double mx[4], const double gx[4],
+                                                 const double gy[4]) {
   if (lt == 3) {
     double phi = 0.0;
 #pragma unroll
@@ -180,6 +176,17 @@ __device__ __forceinline__ double cell_limiter(int lt, int nf, int N, int i, con
     }
   }
   return bn / bd;
+}
+
+// the same with the cell's face offsets loaded here (into registers: every
+// index is a compile-time constant)
+__device__ __forceinline__ double cell_limiter(int lt, int nf, int N, int i, const double2 *__restrict__ off,
+                                               double vol, const double w[4], const double mn[4],
+                                               const double mx[4], const double gx[4], const double gy[4]) {
+  double2 o[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) o[k] = (k < nf) ? off[long(k) * N + i] : make_double2(0.0, 0.0);
+  return cell_limiter_v(lt, nf, o, vol, w, mn, mx, gx, gy);
 }
 
 // LSQ gradient (src/gradient_lsq.f90:371-419): grad_i = sum_j cw_j (q_j - q_i),
@@ -977,6 +984,7 @@ __global__ void k_fill(long n, double v, double *__restrict__ p) {
 // host side
 // ---------------------------------------------------------------------------
 #include "fused.hpp"
+#include "stage.hpp"
 
 }  // namespace
 
@@ -996,6 +1004,14 @@ constexpr int kMaxDevices = 64;
 // take (32 B per 64 cells and step: all 32 rows up to 4M cells)
 constexpr int kNormRows = 32;
 constexpr long kNormBytes = 64L << 20;
+// The whole-stage kernel's blocks per range of a block's cells, past which the
+// two kernels per stage are used (ranges cut in half have halos larger than
+// themselves), and the cell count up to which latency decides instead.  In the
+// reference order, where every range is cut, us per step whole / two kernels:
+// 8,192 cells 34 / 43, 131,072 cells 77 / 79 (limited 115 / 90), 980,000 cells
+// 533 / 389.
+constexpr double kStageMostBlocks = 1.5;
+constexpr int kStageSmallMesh = 1 << 15;
 // steps a captured graph covers: enough that its norm launches cost little
 // (0.5 us a step), few enough nodes that recapturing it (after every chunk of
 // a batched solve that froze or finished an instance) stays cheap
@@ -1090,15 +1106,19 @@ struct fvs_ctx {
   bool xcd_grad = false, xcd_flux = false, xcd_upd = false, xcd_fused = true;
   // limiter values frozen at their last evaluation (steady convergence aid)
   bool limiter_frozen = false;
-  // whole-stage kernel (k_stage): per-block C2 lists, local stencils and face cells
-  bool stage = false, halo = false;  // k_stage in use; per-block data built (k_grad_lsqh)
-  bool use_halo = true;              // gradient from the staged halo (autotuned)
-  int max1 = 0, max2 = 0, max2n = 0;
-  int *s2off = nullptr, *s2n1 = nullptr, *s2list = nullptr, *sl0 = nullptr, *slw = nullptr;
-  long *sleo = nullptr;
-  unsigned short *slid = nullptr;
-  unsigned *blf = nullptr;
-  long nslid = 0, nlist2 = 0, nslid_own = 0;
+  // whole stage in one kernel (k_stage): block lists, block size (0: none), each
+  // block's first cell and count, and what the lists hold in all.  use_stage:
+  // the time loop runs it (else the two kernels per stage, whose lists
+  // two_kernel_lists builds when first asked for); sweep: direction of the next
+  // launch over the blocks; slist: blocks with active cells (masked batches)
+  StageLists SL{};
+  int stage_bs = 0, sweep = 0, nslist = 0;
+  std::vector<int2> stage_cells;
+  long stage_words = 0, stage_faces = 0, stage_halo = 0;
+  bool use_stage = true, two_kernel = false;
+  int *slist = nullptr;
+  bool halo = false;     // staged-halo lists built (k_grad_lsqh)
+  bool use_halo = true;  // gradient from the staged halo (autotuned)
   // staged-halo gradient (k_grad_lsqh): per block, the cells outside it that
   // its stencils read (ascending), and every stencil entry as a 16-bit local
   // index (own cells 0..255, halo 256..) << 4 | periodic-shift code, two
@@ -1417,138 +1437,6 @@ bool pack_sell(int N, const std::vector<int> &perm, const std::vector<int> &iper
   return true;
 }
 
-// Per-block data of the whole-stage kernel (k_stage).  For block b: C1 =
-// its own cells (in order) then the other cells of its listed faces
-// (ascending); C2 = C1 then the remaining cells of the C1 stencils
-// (ascending); the C1 stencils re-expressed as local C2 indices (<< 4, with
-// the periodic-shift code in the low bits), in slices of 64 C1 cells padded
-// with the cell itself; each listed face's cells as local indices.  The
-// stencil entries keep the order of the global stencil, so the gradients are
-// bit-identical to k_grad_lsqc's.  C.halo (k_grad_lsqh, the default
-// gradient) is set when every block fits 4095 local cells and its staged
-// halo 64 KiB; C.stage (k_stage) with kernel_path 2 when its whole LDS
-// layout fits 64 KiB too.
-int setup_stage(fvs_ctx &C, const std::vector<int> &boff, const std::vector<int> &bfaces,
-                const std::vector<int2> &fic, const std::vector<int> &fbc, const std::vector<int> &off,
-                const std::vector<int> &wid, const std::vector<int> &nb, const std::vector<unsigned> &code) {
-  const int N = C.N, Fi = C.Fi, nbk = nblk(N);
-  std::vector<int> s2off(nbk + 1, 0), s2n1(nbk, 0), s2list, sl0(nbk + 1, 0), slw;
-  std::vector<long> sleo;
-  std::vector<unsigned short> slid;
-  std::vector<unsigned> blf(bfaces.size(), 0u);
-  std::vector<int> lmap(N, -1), c1, extra;
-  int max1 = 0, max2 = 0;
-  long eo = 0, eo_own = 0;
-  for (int b = 0; b < nbk; ++b) {
-    const int i0 = b * kBlock, i1 = std::min(N, i0 + kBlock);
-    c1.clear();
-    extra.clear();
-    for (int i = i0; i < i1; ++i) c1.push_back(i);
-    for (int f = boff[b]; f < boff[b + 1]; ++f) {
-      const int sl = bfaces[f];
-      if (sl >= Fi) continue;
-      const int a = fic[sl].x, c = fic[sl].y;
-      if (a < i0 || a >= i1) extra.push_back(a);
-      if (c < i0 || c >= i1) extra.push_back(c);
-    }
-    std::sort(extra.begin(), extra.end());
-    extra.erase(std::unique(extra.begin(), extra.end()), extra.end());
-    c1.insert(c1.end(), extra.begin(), extra.end());
-    const int n1 = int(c1.size());
-    for (int q = 0; q < n1; ++q) lmap[c1[q]] = q;
-    extra.clear();
-    for (int q = 0; q < n1; ++q) {
-      const int i = c1[q], sg = i / kSlice, l = i % kSlice;
-      for (int k = 0; k < wid[sg]; ++k) {
-        const int j = nb[off[sg] + long(k) * kSlice + l];
-        if (lmap[j] == -1) {
-          lmap[j] = -2;
-          extra.push_back(j);
-        }
-      }
-    }
-    std::sort(extra.begin(), extra.end());
-    for (size_t k = 0; k < extra.size(); ++k) lmap[extra[k]] = n1 + int(k);
-    const int n2 = n1 + int(extra.size());
-    bool fits = n2 <= 4095;
-    const int ns = (n1 + kSlice - 1) / kSlice;
-    for (int tq = 0; tq < ns && fits; ++tq) {
-      int w = 0;
-      for (int q = tq * kSlice; q < std::min(n1, (tq + 1) * kSlice); ++q) w = std::max(w, wid[c1[q] / kSlice]);
-      slw.push_back(w);
-      sleo.push_back(eo);
-      if (tq * kSlice < i1 - i0) eo_own += long(w) * kSlice;
-      slid.resize(size_t(eo + long(w) * kSlice), 0);
-      for (int l = 0; l < kSlice; ++l) {
-        const int q = tq * kSlice + l;
-        if (q >= n1) continue;
-        const int i = c1[q], sg = i / kSlice, li = i % kSlice;
-        for (int k = 0; k < w; ++k) {
-          unsigned v = unsigned(q) << 4;  // padding: the cell itself, no shift
-          if (k < wid[sg]) {
-            const unsigned cd = code[off[sg] + long(k) * kSlice + li];
-            v = (unsigned(lmap[int(cd & 0x07ffffffu)]) << 4) | (cd >> 27);
-          }
-          slid[size_t(eo + long(k) * kSlice + l)] = static_cast<unsigned short>(v);
-        }
-      }
-      eo += long(w) * kSlice;
-    }
-    if (!fits) return 0;
-    sl0[b + 1] = sl0[b] + ns;
-    for (int f = boff[b]; f < boff[b + 1]; ++f) {
-      const int sl = bfaces[f];
-      if (sl < Fi) blf[f] = unsigned(lmap[fic[sl].x]) | (unsigned(lmap[fic[sl].y]) << 16);
-      else blf[f] = unsigned(lmap[fbc[sl - Fi]]) | (0xffffu << 16);
-    }
-    // every local index the kernel reads stays inside the block's arrays
-    for (int tq = 0; tq < ns; ++tq) {
-      const int si = sl0[b] + tq;
-      for (int l = 0; l < kSlice && tq * kSlice + l < n1; ++l)
-        for (int k = 0; k < slw[si]; ++k)
-          if (int(slid[size_t(sleo[si] + long(k) * kSlice + l)] >> 4) >= n2)
-            return fail(FVS_EINVAL, "stage set-up: stencil entry outside the block's cell list");
-    }
-    for (int f = boff[b]; f < boff[b + 1]; ++f) {
-      const int a = int(blf[f] & 0xffffu), c = int(blf[f] >> 16);
-      if (a >= n1 || (bfaces[f] < Fi ? c >= n1 : c != 0xffff))
-        return fail(FVS_EINVAL, "stage set-up: face cell outside the block's gradient cells");
-    }
-    for (int q = 0; q < i1 - i0; ++q)
-      if (c1[q] != i0 + q) return fail(FVS_EINVAL, "stage set-up: own cells not first");
-    s2list.insert(s2list.end(), c1.begin(), c1.end());
-    s2list.insert(s2list.end(), extra.begin(), extra.end());
-    s2off[b + 1] = int(s2list.size());
-    s2n1[b] = n1;
-    max1 = std::max(max1, n1);
-    max2 = std::max(max2, n2);
-    for (int c : c1) lmap[c] = -1;
-    for (int c : extra) lmap[c] = -1;
-  }
-  max1 += max1 & 1;  // keep the LDS arrays after lP 16-byte aligned
-  const int max2n = max2;
-  if (size_t(6) * max2n * sizeof(double) > C.lds_max) return 0;
-  const size_t lds = (size_t(6) * max2 + size_t(9) * max1 + size_t(5) * C.maxf) * sizeof(double);
-  if (int rc = C.upload(C.s2off, s2off)) return rc;
-  if (int rc = C.upload(C.s2n1, s2n1)) return rc;
-  if (int rc = C.upload(C.s2list, s2list)) return rc;
-  if (int rc = C.upload(C.sl0, sl0)) return rc;
-  if (int rc = C.upload(C.slw, slw)) return rc;
-  if (int rc = C.upload(C.sleo, sleo)) return rc;
-  if (int rc = C.upload(C.slid, slid)) return rc;
-  if (int rc = C.upload(C.blf, blf)) return rc;
-  C.max1 = max1;
-  C.max2 = max2;
-  C.max2n = max2n;
-  C.nslid = long(slid.size());
-  C.nlist2 = long(s2list.size());
-  C.nslid_own = eo_own;
-  // the device's per-workgroup LDS limit (160 KiB on gfx950): blocks of
-  // stretched cells (O-grids) have larger halos
-  C.stage = lds <= C.lds_max;
-  return 0;
-}
-
 // Lists of the staged-halo gradient k_grad_lsqh (see the fvs_ctx fields).
 // Local entries keep the order of the global stencil, so the gradients are
 // bit-identical to k_grad_lsqc's.  Enabled (C.halo) when every block's local
@@ -1665,6 +1553,141 @@ int setup_grad_halo(fvs_ctx &C, const std::vector<int> &off, const std::vector<i
   return 0;
 }
 
+#include "stage_setup.hpp"
+
+// the time loop's stages run the whole-stage kernel
+bool whole_stage(const fvs_ctx &C) { return C.stage_bs != 0 && C.use_stage; }
+
+// Per-block face lists of the fused flux + update kernel (256-cell blocks and,
+// for single meshes, the 128-cell ones the autotuner tries): every face slot
+// touching block b's cells, ascending (interior slots, then boundary slots), its
+// record in list order, and each cell's faces as signed local indices in the
+// gather order.
+int flux_lists(fvs_ctx &C, const StageMesh &M) {
+  const int N = C.N, Fi = C.Fi, gw = C.GW;
+  // per-block lists for blocks of bs cells: boff, bfaces, lgat and the
+  // largest list (maxf)
+  auto block_lists = [&](int bs, std::vector<int> &boff, std::vector<int> &bfaces, std::vector<short> &lgat,
+                         int &maxf) {
+    const int nbk = nblk(N, bs);
+    boff.assign(nbk + 1, 0);
+    bfaces.clear();
+    lgat.assign(size_t(gw) * N, 0);
+    // blocks in contiguous parts on the host's cores; each part's lists in
+    // block order, joined afterwards
+    const long np = parallel_parts(nbk, 64);
+    std::vector<std::vector<int>> pf(np);
+    std::vector<int> pmax(np, 0);
+    parallel_for(nbk, 64, [&](long t, long b0, long b1) {
+      std::vector<int> loc;
+      for (long b = b0; b < b1; ++b) {
+        loc.clear();
+        const int i0 = int(b) * bs, i1 = std::min(N, i0 + bs);
+        for (int i = i0; i < i1; ++i)
+          for (int k = 0; k < gw; ++k) {
+            const int sg = M.gat[size_t(k) * N + i];
+            if (sg) loc.push_back((sg > 0 ? sg : -sg) - 1);
+          }
+        std::sort(loc.begin(), loc.end());
+        loc.erase(std::unique(loc.begin(), loc.end()), loc.end());
+        for (int i = i0; i < i1; ++i)
+          for (int k = 0; k < gw; ++k) {
+            const int sg = M.gat[size_t(k) * N + i];
+            if (!sg) continue;
+            const int slot = (sg > 0 ? sg : -sg) - 1;
+            const int li = int(std::lower_bound(loc.begin(), loc.end(), slot) - loc.begin()) + 1;
+            lgat[size_t(k) * N + i] = short(sg > 0 ? li : -li);
+          }
+        pf[t].insert(pf[t].end(), loc.begin(), loc.end());
+        boff[b + 1] = int(loc.size());
+        pmax[t] = std::max(pmax[t], int(loc.size()));
+      }
+    });
+    for (int b = 0; b < nbk; ++b) boff[b + 1] += boff[b];
+    bfaces.reserve(size_t(boff[nbk]));
+    for (auto &v : pf) bfaces.insert(bfaces.end(), v.begin(), v.end());
+    maxf = *std::max_element(pmax.begin(), pmax.end());
+  };
+  // the listed faces' records in list order: cells and 7 geometry planes
+  auto upload_records = [&](const std::vector<int> &bfaces, int2 *&dlrec, double *&dlgeo) -> int {
+    const size_t L = bfaces.size();
+    std::vector<int2> lrec(L);
+    std::vector<double> lgeo(7 * L);
+    parallel_for(long(L), 4096, [&](long, long f0, long f1) {
+      for (long f = f0; f < f1; ++f) {
+        const int sl = bfaces[f];
+        const double *g;
+        if (sl < Fi) {
+          lrec[f] = M.fic[sl];
+          g = &M.fig[8 * size_t(sl)];
+        } else {
+          const int bq = sl - Fi;
+          const int inst = C.ninst > 0 ? C.inst_of_real[C.perm[M.fbc[bq]]] : 0;
+          lrec[f] = make_int2(M.fbc[bq], -1 - (M.fbt[bq] | (inst << 2)));
+          g = &M.fbg[8 * size_t(bq)];
+        }
+        for (int k = 0; k < 7; ++k) lgeo[size_t(k) * L + f] = g[k];
+      }
+    });
+    if (int rc = C.upload(dlrec, lrec)) return rc;
+    return C.upload(dlgeo, lgeo);
+  };
+  std::vector<int> boff, bfaces;
+  std::vector<short> lgat;
+  block_lists(kBlock, boff, bfaces, lgat, C.maxf);
+  C.nlisted = long(bfaces.size());
+  if (int rc = C.upload(C.boff, boff)) return rc;
+  if (int rc = C.upload(C.lgat, lgat)) return rc;
+  if (int rc = upload_records(bfaces, C.lrec, C.lgeo)) return rc;
+  HIPC(hipStreamSynchronize(C.stream));  // the host arrays are reused
+  // 128-cell blocks: single meshes of at least 64 of them (batches keep the
+  // 256-cell blocks their instance masks are built for)
+  if (C.ninst == 0 && C.opt.kernel_path != 2 && N >= 64 * kSmallBlock) {
+    block_lists(kSmallBlock, boff, bfaces, lgat, C.maxf_s);
+    C.nlisted_s = long(bfaces.size());
+    if (int rc = C.upload(C.boff_s, boff)) return rc;
+    if (int rc = C.upload(C.lgat_s, lgat)) return rc;
+    if (int rc = upload_records(bfaces, C.lrec_s, C.lgeo_s)) return rc;
+    HIPC(hipStreamSynchronize(C.stream));
+    C.have_small = true;
+  }
+  return 0;
+}
+
+// Lists of the two-kernel stage (fused flux + update, staged-halo LSQ gradient)
+// for a context whose time loop runs the whole-stage kernel, when a call selects
+// the two kernels: built from the arrays on the device.
+int two_kernel_lists(fvs_ctx &C) {
+  if (C.two_kernel || !C.stage_bs) return 0;
+  const size_t N = C.N, Fi = C.Fi, Fb = C.Fb, ns = (N + kSlice - 1) / kSlice;
+  auto fetch = [&](auto &v, const void *src, size_t n) -> hipError_t {
+    v.resize(n);
+    return n ? hipMemcpyAsync(v.data(), src, n * sizeof(v[0]), hipMemcpyDeviceToHost, C.stream) : hipSuccess;
+  };
+  std::vector<int> gat, fbc, fbt, off, wid;
+  std::vector<int2> fic;
+  std::vector<double> fig, fbg;
+  std::vector<unsigned> code;
+  HIPC(fetch(gat, C.gat, size_t(C.GW) * N));
+  HIPC(fetch(fic, C.fi_cells, Fi));
+  HIPC(fetch(fig, C.fi_geo, 8 * Fi));
+  HIPC(fetch(fbc, C.fb_cell, Fb));
+  HIPC(fetch(fbt, C.fb_type, Fb));
+  HIPC(fetch(fbg, C.fb_geo, 8 * Fb));
+  HIPC(fetch(off, C.soff, ns + 1));
+  HIPC(fetch(wid, C.swid, ns));
+  HIPC(hipStreamSynchronize(C.stream));
+  HIPC(fetch(code, C.sid, size_t(off[ns])));
+  HIPC(hipStreamSynchronize(C.stream));
+  const StageMesh M{gat, fic, fig, fbc, fbt, fbg, off, wid, code};
+  if (int rc = flux_lists(C, M)) return rc;
+  if (C.opt.kernel_path != 3)
+    if (int rc = setup_grad_halo(C, off, wid, code)) return rc;
+  HIPC(hipStreamSynchronize(C.stream));
+  C.two_kernel = true;
+  return 0;
+}
+
 int setup_device(fvs_ctx &C) {
   MeshPrep &m = C.mp;
   const int N = C.N = m.ncells;
@@ -1756,108 +1779,9 @@ int setup_device(fvs_ctx &C) {
     }
   });
   if (int rc = C.upload(C.gat, gat)) return rc;
-  // per-block face lists for the fused flux + update kernel: every face slot
-  // touching block b's cells, ascending (interior slots, then boundary slots),
-  // and each cell's faces as signed local indices in the gather order
-  std::vector<int> h_boff, h_bfaces;
-  // per-block lists for blocks of bs cells: boff, bfaces, lgat and the
-  // largest list (maxf)
-  auto block_lists = [&](int bs, std::vector<int> &boff, std::vector<int> &bfaces, std::vector<short> &lgat,
-                         int &maxf) {
-    const int nbk = nblk(N, bs);
-    boff.assign(nbk + 1, 0);
-    bfaces.clear();
-    lgat.assign(size_t(gw) * N, 0);
-    // blocks in contiguous parts on the host's cores; each part's lists in
-    // block order, joined afterwards
-    const long np = parallel_parts(nbk, 64);
-    std::vector<std::vector<int>> pf(np);
-    std::vector<int> pmax(np, 0);
-    parallel_for(nbk, 64, [&](long t, long b0, long b1) {
-      std::vector<int> loc;
-      for (long b = b0; b < b1; ++b) {
-        loc.clear();
-        const int i0 = int(b) * bs, i1 = std::min(N, i0 + bs);
-        for (int i = i0; i < i1; ++i)
-          for (int k = 0; k < gw; ++k) {
-            const int sg = gat[size_t(k) * N + i];
-            if (sg) loc.push_back((sg > 0 ? sg : -sg) - 1);
-          }
-        std::sort(loc.begin(), loc.end());
-        loc.erase(std::unique(loc.begin(), loc.end()), loc.end());
-        for (int i = i0; i < i1; ++i)
-          for (int k = 0; k < gw; ++k) {
-            const int sg = gat[size_t(k) * N + i];
-            if (!sg) continue;
-            const int slot = (sg > 0 ? sg : -sg) - 1;
-            const int li = int(std::lower_bound(loc.begin(), loc.end(), slot) - loc.begin()) + 1;
-            lgat[size_t(k) * N + i] = short(sg > 0 ? li : -li);
-          }
-        pf[t].insert(pf[t].end(), loc.begin(), loc.end());
-        boff[b + 1] = int(loc.size());
-        pmax[t] = std::max(pmax[t], int(loc.size()));
-      }
-    });
-    for (int b = 0; b < nbk; ++b) boff[b + 1] += boff[b];
-    bfaces.reserve(size_t(boff[nbk]));
-    for (auto &v : pf) bfaces.insert(bfaces.end(), v.begin(), v.end());
-    maxf = *std::max_element(pmax.begin(), pmax.end());
-  };
-  // the listed faces' records in list order: cells and 7 geometry planes
-  auto upload_records = [&](const std::vector<int> &bfaces, int2 *&dlrec, double *&dlgeo) -> int {
-    const size_t L = bfaces.size();
-    std::vector<int2> lrec(L);
-    std::vector<double> lgeo(7 * L);
-    parallel_for(long(L), 4096, [&](long, long f0, long f1) {
-      for (long f = f0; f < f1; ++f) {
-        const int sl = bfaces[f];
-        const double *g;
-        if (sl < Fi) {
-          lrec[f] = fic[sl];
-          g = &fig[8 * size_t(sl)];
-        } else {
-          const int bq = sl - Fi;
-          const int inst = C.ninst > 0 ? C.inst_of_real[P[fbc[bq]]] : 0;
-          lrec[f] = make_int2(fbc[bq], -1 - (fbt[bq] | (inst << 2)));
-          g = &fbg[8 * size_t(bq)];
-        }
-        for (int k = 0; k < 7; ++k) lgeo[size_t(k) * L + f] = g[k];
-      }
-    });
-    if (int rc = C.upload(dlrec, lrec)) return rc;
-    return C.upload(dlgeo, lgeo);
-  };
-  // (the fused update gathers at most 4 faces per cell: triangles and quads)
-  if ((C.opt.kernel_path == 0 || C.opt.kernel_path == 2 || C.opt.kernel_path == 3) && gw <= 4) {
-    std::vector<int> boff, bfaces;
-    std::vector<short> lgat;
-    int maxf = 0;
-    block_lists(kBlock, boff, bfaces, lgat, maxf);
-    // LDS of k_flux_update: face fluxes + the block's gradients and states
-    if (size_t(5) * maxf * sizeof(double) + 12 * kBlock * sizeof(double) <= 64 * 1024) {
-      C.maxf = maxf;
-      C.nlisted = long(bfaces.size());
-      if (int rc = C.upload(C.boff, boff)) return rc;
-      if (int rc = C.upload(C.bfaces, bfaces)) return rc;
-      if (int rc = C.upload(C.lgat, lgat)) return rc;
-      if (int rc = upload_records(bfaces, C.lrec, C.lgeo)) return rc;
-      C.fused = true;
-      h_boff.swap(boff);
-      h_bfaces.swap(bfaces);
-    }
-    // the same lists for blocks of kSmallBlock cells, a launch shape the
-    // autotuner tries (single meshes of at least 64 blocks: batches keep the
-    // 256-cell blocks their instance masks are built for)
-    if (C.fused && C.ninst == 0 && C.opt.kernel_path != 2 && N >= 64 * kSmallBlock) {
-      block_lists(kSmallBlock, boff, bfaces, lgat, maxf);
-      C.maxf_s = maxf;
-      C.nlisted_s = long(bfaces.size());
-      if (int rc = C.upload(C.boff_s, boff)) return rc;
-      if (int rc = C.upload(C.lgat_s, lgat)) return rc;
-      if (int rc = upload_records(bfaces, C.lrec_s, C.lgeo_s)) return rc;
-      C.have_small = true;
-    }
-  }
+  // the fused update gathers at most 4 faces per cell (triangles and quads),
+  // whose face fluxes, with the block's gradients and states, fit 64 KiB of LDS
+  C.fused = C.opt.kernel_path != 1 && gw <= 4;
   // limiter face offsets (xf - xc) per local edge, in the cell's own frame
   if (C.opt.limiter > 0) {
     std::vector<double2> lo(4 * size_t(N), make_double2(0.0, 0.0));
@@ -1964,10 +1888,11 @@ int setup_device(fvs_ctx &C) {
         if (int rc = C.upload(C.ginv, gi)) return rc;
         if (int rc = C.upload(C.sid, code)) return rc;
         C.lsqc = true;
-        if (C.opt.recon != 1 && C.opt.kernel_path != 3)
+        // the whole stage in one kernel, or the lists of two kernels per stage
+        if (C.fused && C.opt.recon != 1 && C.opt.kernel_path != 3)
+          if (int rc = setup_stage(C, {gat, fic, fig, fbc, fbt, fbg, off, wid, code})) return rc;
+        if (!C.stage_bs && C.opt.recon != 1 && C.opt.kernel_path != 3)
           if (int rc = setup_grad_halo(C, off, wid, code)) return rc;
-        if (C.fused && C.opt.recon != 1 && C.opt.kernel_path == 2)
-          if (int rc = setup_stage(C, h_boff, h_bfaces, fic, fbc, off, wid, nb, code)) return rc;
       }
     }
     // a limited Green-Gauss gradient takes its bounds from a staged halo of
@@ -1978,6 +1903,12 @@ int setup_device(fvs_ctx &C) {
       std::vector<unsigned> code(nb.begin(), nb.end());
       if (int rc = setup_grad_halo(C, off, wid, code)) return rc;
     }
+  }
+  if (C.fused && !C.stage_bs) {
+    const std::vector<int> none;
+    const std::vector<unsigned> nocode;
+    if (int rc = flux_lists(C, {gat, fic, fig, fbc, fbt, fbg, none, none, nocode})) return rc;
+    C.two_kernel = true;
   }
   if (C.opt.grad_method == 1) {
     std::vector<double2> c0(N), cn(size_t(C.NFW) * N, make_double2(0.0, 0.0));
@@ -2346,32 +2277,15 @@ int launch_flux_update(fvs_ctx &C, const Upd &A, double t, const double *uin = n
   return 0;
 }
 
-// arguments of the whole-stage block body for the current context state
-StageArgs stage_args(const fvs_ctx &C, double t) {
-  StageArgs a;
+// arguments of the whole-stage block body for the current context state; uout:
+// where conservative stage states go
+StageIn stage_in(const fvs_ctx &C, double t, double *uout) {
+  StageIn a;
   a.N = C.N;
-  a.nb = xcd_arg(nblk(C.N), C.xcd_fused);
   a.gw = C.GW;
-  a.maxf = C.maxf;
-  a.max1 = C.max1;
-  a.max2 = C.max2;
   a.P = C.P;
   a.t = t;
-  a.boff = C.boff;
-  a.bfaces = C.bfaces;
-  a.blf = C.blf;
-  a.lgat = C.lgat;
-  a.Fi = C.Fi;
-  a.fgeo = C.fi_geo;
-  a.btype = C.fb_type;
-  a.bgeo = C.fb_geo;
-  a.s2off = C.s2off;
-  a.s2n1 = C.s2n1;
-  a.s2list = C.s2list;
-  a.sl0 = C.sl0;
-  a.slw = C.slw;
-  a.sleo = C.sleo;
-  a.slid = C.slid;
+  a.S = C.SL;
   a.cxy = C.cxy;
   a.ginv = C.ginv;
   a.st = C.shifts;
@@ -2386,43 +2300,57 @@ StageArgs stage_args(const fvs_ctx &C, double t) {
   a.frz = C.dfrz;
   a.ninst = C.ninst;
   a.Ua = C.U0;
-  a.Ub = C.Ub;
+  a.Ub = uout ? uout : C.Ub;
   a.Facc = C.Facc;
   a.dtl = C.dtl;
   a.norm = norm_out(C);
-  a.blist = C.nact ? C.blist : nullptr;
-  a.binst = C.dbinst;
-  a.pinf_inst = C.dpinf_inst;
+  a.blist = C.nact ? C.slist : nullptr;
+  // the active-cell bits follow the list of 256-cell blocks, one per device cell
+  a.amask = C.nact ? reinterpret_cast<const unsigned *>(C.blist + nblk(C.N)) : nullptr;
+  a.pinf_inst = C.ninst > 0 ? C.dpinf_inst : nullptr;
+  const int nb = int(C.stage_cells.size());
+  a.nb = C.nact ? C.nslist : xcd_arg(nb, C.xcd_fused);
+  a.down = C.sweep;
   return a;
 }
 
-size_t stage_lds(const fvs_ctx &C) {
-  return (size_t(6) * C.max2 + size_t(9) * C.max1 + size_t(5) * C.maxf) * sizeof(double);
+// LDS of a block: the wave speeds only where the stage sets local time steps,
+// the limiter values only with a limiter
+template <class SH>
+size_t stage_lds(const fvs_ctx &C, bool speeds) {
+  return size_t(speeds ? SH::END : (C.opt.limiter > 0 ? SH::S : SH::P));
 }
 
-// whole stage in one kernel (k_stage); swaps the primitive buffers
-int launch_stage(fvs_ctx &C, const Upd &A, double t) {
+// whole stage in one kernel: uin / uout as in launch_flux_update
+int launch_stage(fvs_ctx &C, const Upd &A, double t, const double *uin = nullptr, double *uout = nullptr) {
   ProfScope ps(C, KC_FUSED);
-  const int nb = nblk(C.N);
-  const size_t lds = stage_lds(C);
-  const bool lim = C.opt.limiter > 0 && !C.limiter_frozen;
-  const dim3 g(C.nact ? C.nact : xcd_grid(nb)), b(kStageThreads);
-  const StageArgs a = stage_args(C, t);
-#define FVS_STAGE(L, PM) hipLaunchKernelGGL((k_stage<L, PM>), g, b, lds, C.stream, a, A, C.W, C.Walt)
-  if (lim) {
-    if (C.pmode == 0) FVS_STAGE(1, 0);
-    else if (C.pmode == 1) FVS_STAGE(1, 1);
-    else if (C.pmode == 2) FVS_STAGE(1, 2);
-    else FVS_STAGE(1, 3);
+  const bool cons = uin != nullptr, lim = C.opt.limiter > 0 && !C.limiter_frozen;
+  C.sweep ^= 1;
+  const StageIn a = stage_in(C, t, uout);
+  const dim3 g(C.nact ? C.nslist : xcd_grid(int(C.stage_cells.size())));
+  const double *in = cons ? uin : C.W;
+  double *out = cons ? nullptr : C.Walt;
+#define FVS_STAGE(SH, L, PM)                                                                                     \
+  hipLaunchKernelGGL((k_stage<SH, L, PM>), g, dim3(SH::NT), stage_lds<SH>(C, A.steady && A.first), C.stream, a, A, \
+                     in, out, cons ? 1 : 0)
+#define FVS_STAGE_PM(SH, L)                     \
+  do {                                          \
+    if (C.pmode == 0) FVS_STAGE(SH, L, 0);      \
+    else if (C.pmode == 1) FVS_STAGE(SH, L, 1); \
+    else if (C.pmode == 2) FVS_STAGE(SH, L, 2); \
+    else FVS_STAGE(SH, L, 3);                   \
+  } while (0)
+  if (C.stage_bs == StageLarge::BS) {
+    if (lim) FVS_STAGE_PM(StageLarge, 1);
+    else FVS_STAGE_PM(StageLarge, 0);
   } else {
-    if (C.pmode == 0) FVS_STAGE(0, 0);
-    else if (C.pmode == 1) FVS_STAGE(0, 1);
-    else if (C.pmode == 2) FVS_STAGE(0, 2);
-    else FVS_STAGE(0, 3);
+    if (lim) FVS_STAGE_PM(StageSmall, 1);
+    else FVS_STAGE_PM(StageSmall, 0);
   }
+#undef FVS_STAGE_PM
 #undef FVS_STAGE
   HIPC(hipGetLastError());
-  std::swap(C.W, C.Walt);
+  if (!cons) std::swap(C.W, C.Walt);
   return 0;
 }
 
@@ -3003,17 +2931,19 @@ InstNorms inst_norms_of(const fvs_ctx &C) {
 // norms; launch_norms reduces them to the output rows the device counter
 // names, so a sequence of steps and their norms can be captured once in a HIP
 // graph and replayed.
-// SSP-RK3 stages on conservative states (no primitive-state traffic): the
-// fused path with the staged-halo LSQ gradient, an unlimited Green-Gauss
-// gradient (kernel_path 3 keeps primitive states) or a first-order
+// Stages on conservative states (no primitive-state traffic; SSP-RK3 and the
+// two-register form): the whole-stage kernel (kernel_path 2 keeps primitive
+// states), or the fused path with the staged-halo LSQ gradient, an unlimited
+// Green-Gauss gradient (kernel_path 3 keeps primitive states) or a first-order
 // reconstruction
 bool cons_stages(const fvs_ctx &C) {
+  if (C.opt.rk_scheme != FVS_RK_SSP3 && C.opt.rk_scheme != FVS_RK_SSP42_SO) return false;
+  if (whole_stage(C)) return C.opt.kernel_path != 2;
   // Green-Gauss gradients: unlimited, or limited with the bounds from the
   // staged halo (where the stage states are converted once, as staged)
   const bool gg = (C.opt.grad_method == 1 || C.opt.grad_method == 2) && C.opt.kernel_path != 3 &&
                   (C.opt.limiter == 0 || (C.halo && C.use_halo));
-  return C.fused && !C.stage && (C.opt.rk_scheme == FVS_RK_SSP3 || C.opt.rk_scheme == FVS_RK_SSP42_SO) &&
-         (C.opt.recon == 1 || (C.opt.grad_method == 3 && C.halo && C.use_halo) || gg);
+  return C.fused && (C.opt.recon == 1 || (C.opt.grad_method == 3 && C.halo && C.use_halo) || gg);
 }
 
 // Update constants of stage k of a step starting at told, and the stage's
@@ -3076,14 +3006,16 @@ int launch_step(fvs_ctx &C, double told) {
     double ts = told;
     const Upd A = stage_upd(o, k, told, ts);
     int rc;
-    if (C.stage) {
-      rc = launch_stage(C, A, ts);
-    } else if (cons_stages(C)) {
+    if (cons_stages(C)) {
       // the stage input and output states (a stage's output never
       // overwrites a state its neighbouring blocks still read)
       double *const in3[3] = {C.U0, C.Ub, C.Uc}, *const out3[3] = {C.Ub, C.Uc, C.U0};
       double *const in4[4] = {C.U0, C.Ub, C.Uc, C.Ub}, *const out4[4] = {C.Ub, C.Uc, C.Ub, C.U0};
-      rc = nst == 3 ? launch_flux_update(C, A, ts, in3[k], out3[k]) : launch_flux_update(C, A, ts, in4[k], out4[k]);
+      const double *in = nst == 3 ? in3[k] : in4[k];
+      double *out = nst == 3 ? out3[k] : out4[k];
+      rc = whole_stage(C) ? launch_stage(C, A, ts, in, out) : launch_flux_update(C, A, ts, in, out);
+    } else if (whole_stage(C)) {
+      rc = launch_stage(C, A, ts);
     } else if (C.fused) {
       rc = launch_flux_update(C, A, ts);
     } else {
@@ -3174,7 +3106,7 @@ int launch_persistent(fvs_ctx &C, double t1, int nsteps, double *dn, double *din
     c.A[k] = stage_upd(o, k, t1, ts);
   }
   c.nsteps = nsteps;
-  c.nlaunch = C.nact ? C.nact : nblk(C.N);
+  c.nlaunch = C.nact ? C.nslist : int(C.stage_cells.size());
   c.W0 = C.W;
   c.W1 = C.Walt;
   c.dn = C.nact ? nullptr : dn;
@@ -3187,9 +3119,8 @@ int launch_persistent(fvs_ctx &C, double t1, int nsteps, double *dn, double *din
   c.err = C.perr;
   c.spin = 1u << 22;
   C.norm_row = 0;
-  StageArgs a = stage_args(C, t1);
-  a.nb = nblk(C.N);  // plain numbering: the persistent loop walks the blocks itself
-  const size_t lds = std::max(stage_lds(C), size_t(4) * kNormThreads * sizeof(double));
+  StageIn a = stage_in(C, t1, nullptr);
+  const size_t lds = std::max(size_t(StageSmall::END), size_t(4) * kNormThreads * sizeof(double));
   const bool lim = o.limiter > 0 && !C.limiter_frozen;
   const void *fn = nullptr;
 #define FVS_PK(L, PM) fn = reinterpret_cast<const void *>(&k_steps_persistent<L, PM>)
@@ -3206,12 +3137,12 @@ int launch_persistent(fvs_ctx &C, double t1, int nsteps, double *dn, double *din
   }
 #undef FVS_PK
   int per_cu = 0;
-  HIPC(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kStageThreads, lds));
+  HIPC(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, StageSmall::NT, lds));
   if (per_cu < 1) return fail(FVS_ESTATE, "persistent launch: the whole-stage kernel does not fit on a compute unit");
   const int grid = std::min(c.nlaunch, per_cu * C.ncu);
   hipLaunchKernelGGL(k_barrier_reset, dim3(1), dim3(64), 0, C.stream, C.pbar, C.perr);
   void *args[] = {&a, &c};
-  HIPC(hipLaunchCooperativeKernel(fn, dim3(grid), dim3(kStageThreads), args, unsigned(lds), C.stream));
+  HIPC(hipLaunchCooperativeKernel(fn, dim3(grid), dim3(StageSmall::NT), args, unsigned(lds), C.stream));
   C.persist_ran = true;
   if ((nsteps * c.nst) % 2) std::swap(C.W, C.Walt);
   return 0;
@@ -3224,7 +3155,7 @@ int run_steps(fvs_ctx &C, double t1, int nsteps, double *dn, double *dv, double 
   if (!cons) ensure_prim(C);  // the stages read W
   hipLaunchKernelGGL(k_counter, dim3(1), dim3(1), 0, C.stream, C.dctr, 0, 0);
   HIPC(hipGetLastError());
-  if (graph_ok && C.use_persistent && C.stage && !C.profiling && !dv && !time_dependent(C))
+  if (graph_ok && C.use_persistent && !C.profiling && !dv && !time_dependent(C))
     return launch_persistent(C, t1, nsteps, dn, dinst);
   int s = 0;
   // graph replay: one captured graph covers an even number of stages so the
@@ -3362,9 +3293,16 @@ int fvs_set_phase_timers(fvs_ctx *C, int on) try {
 int fvs_phase_times(const fvs_ctx *C, double *sec4) try {
   if (!C || !sec4) return fail(FVS_EINVAL, "null argument");
   const double *t = C->phase_ms;
-  sec4[0] = t[KC_GRAD] * 1e-3;                                    // gradient, limiter fused in
-  sec4[1] = 0.0;                                                  // limiter: inside the gradient launches
-  sec4[2] = (t[KC_FLUX_INT] + t[KC_FLUX_BND] + t[KC_FUSED]) * 1e-3;  // face fluxes (+ fused stage update)
+  // whole-stage launches: their time in the proportion of the floating-point
+  // operations, about 18 per stencil entry against 300 per face and 60 per cell
+  double share = 0.0;
+  if (whole_stage(*C)) {
+    const double g = 36.0 * double(C->stage_words), f = 300.0 * double(C->stage_faces) + 60.0 * C->N;
+    share = g / (g + f);
+  }
+  sec4[0] = (t[KC_GRAD] + share * t[KC_FUSED]) * 1e-3;  // gradient, limiter fused in
+  sec4[1] = 0.0;                                        // limiter: inside the gradient phase
+  sec4[2] = (t[KC_FLUX_INT] + t[KC_FLUX_BND] + (1.0 - share) * t[KC_FUSED]) * 1e-3;  // face fluxes (+ fused update)
   sec4[3] = (t[KC_UPDATE] + t[KC_NORM]) * 1e-3;                   // stage updates, residual norms
   return 0;
 } catch (...) {
@@ -3373,9 +3311,9 @@ int fvs_phase_times(const fvs_ctx *C, double *sec4) try {
 
 int fvs_set_persistent(fvs_ctx *C, int on) try {
   if (!C) return fail(FVS_EINVAL, "null context");
-  if (on && !C->stage)
+  if (on && !(C->opt.kernel_path == 2 && C->stage_bs == StageSmall::BS))
     return fail(FVS_ESTATE, "persistent launches run the whole-stage kernel: create the context with kernel_path 2 "
-                            "(LSQ gradient, triangle-sized blocks)");
+                            "(LSQ gradient)");
   C->use_persistent = on != 0;
   return 0;
 } catch (...) {
@@ -3427,6 +3365,21 @@ int fvs_batch_set_active(fvs_ctx *C, const int *active) try {
       if (on) list.push_back(b);
     }
     if (list.empty()) list.push_back(0);
+    if (C->stage_bs) {
+      std::vector<int> sl;
+      for (size_t b = 0; b < C->stage_cells.size(); ++b) {
+        const int i0 = C->stage_cells[b].x, i1 = i0 + C->stage_cells[b].y;
+        unsigned any = 0;  // blocks start on whole 64-cell slices
+        for (int w = i0 / 32; w < (i1 + 31) / 32; ++w) any |= mask[w];
+        if (any) sl.push_back(int(b));
+      }
+      if (sl.empty()) sl.push_back(0);
+      if (!C->slist)
+        if (int rc = C->alloc(C->slist, C->stage_cells.size())) return rc;
+      HIPC(hipMemcpyAsync(C->slist, sl.data(), sl.size() * sizeof(int), hipMemcpyHostToDevice, C->stream));
+      HIPC(hipStreamSynchronize(C->stream));
+      C->nslist = int(sl.size());
+    }
     HIPC(hipMemcpyAsync(C->blist, list.data(), list.size() * sizeof(int), hipMemcpyHostToDevice, C->stream));
     HIPC(hipMemcpyAsync(C->blist + nb, mask.data(), mask.size() * sizeof(unsigned), hipMemcpyHostToDevice, C->stream));
   }
@@ -3614,13 +3567,19 @@ int fvs_kernel_times(fvs_ctx *C, double t1, int nsteps, double *ms, double *byte
     if (C->opt.steady) st3 += (8.0 + 8.0 * (nst - 1)) / nst;
     bfu = nlisted * (8 + 56) + N * (32 + 64 + (phi1 ? 0 : 8)) + N * (C->GW * 2.0 + 8 + st3);
   }
-  // whole stage: own states, centres and G^-1 once, the per-block cell lists
-  // and local stencils, face records and block lists once, limiter inputs,
+  // whole stage: states, centres and G^-1 once, the block lists, limiter inputs,
   // the update's cell-side traffic
-  const double bst = N * (32 + 16 + 24) + 2.0 * double(C->nslid) + 4.0 * double(C->nlist2) + (Fi + Fb) * 56 +
-                     8.0 * double(C->nlisted) + (lim ? N * (8 + 4) + 16.0 * (3 * m.ntri + 4 * m.nquad) : 0.0) +
-                     N * (C->GW * 2.0 + 8 + 32 + state);
-  const double b5[KC_N] = {bg, bfi, bfb, bup, bno, C->stage ? bst : bfu};
+  double bst = N * (32 + 16 + 24 + C->GW * 2.0 + 8) + 4.0 * double(C->stage_words) + 4.0 * double(C->stage_halo) +
+               44.0 * double(C->stage_faces) + (lim ? N * (8 + 4) + 16.0 * (3 * m.ntri + 4 * m.nquad) : 0.0);
+  if (cons_stages(*C)) {
+    double st3 = (32 + 64 + 64) / 3.0;  // new states, and the step-start state after the first stage
+    if (C->opt.rk_scheme == FVS_RK_SSP42_SO) st3 = (32 + 32 + 32 + 64) / 4.0;
+    bst += N * st3;
+    if (C->opt.steady) bst += N * (8.0 + 8.0 * (nst - 1)) / nst;
+  } else {
+    bst += N * (32 + state);
+  }
+  const double b5[KC_N] = {bg, bfi, bfb, bup, bno, whole_stage(*C) ? bst : bfu};
   for (int k = 0; k < KC_N; ++k) {
     ms[k] = cnt[k] ? tot[k] / cnt[k] : 0.0;
     bytes[k] = b5[k];
@@ -3684,9 +3643,11 @@ int fvs_autotune(fvs_ctx *C, int nsteps, int *choice4, double *best_ms) try {
   };
   bool *knobs[7] = {&C->xcd_grad, &C->xcd_flux,  &C->xcd_upd,   &C->xcd_fused,
                     &C->use_halo, &C->small_blocks, &C->small_grad};
-  const bool lsq_halo = C->halo && !C->stage && C->opt.recon != 1 && C->opt.grad_method == 3;
-  const bool used[7] = {C->opt.recon != 1, !C->fused, !C->fused, C->fused && !C->stage,
-                        C->halo && !C->stage && C->opt.recon != 1, C->have_small && C->fused && !C->stage,
+  // the whole-stage kernel has its workgroup numbering only
+  const bool two = !whole_stage(*C);
+  const bool lsq_halo = C->halo && two && C->opt.recon != 1 && C->opt.grad_method == 3;
+  const bool used[7] = {two && C->opt.recon != 1, !C->fused, !C->fused, C->fused,
+                        C->halo && two && C->opt.recon != 1, C->have_small && two && C->fused,
                         lsq_halo && C->have_small_grad};
   double best = 0.0;
   // warm-up: the first few dozen launches after the device was idle run
@@ -3724,9 +3685,13 @@ int fvs_autotune(fvs_ctx *C, int nsteps, int *choice4, double *best_ms) try {
   if (rc) return rc;
   if (choice4) {
     for (int k = 0; k < 4; ++k) choice4[k] = *knobs[k] ? 1 : 0;
-    if (C->halo && C->use_halo) choice4[0] |= 2;
-    if (C->halo && C->use_halo && C->have_small_grad && C->small_grad) choice4[0] |= 4;
-    if (C->small_blocks) choice4[3] |= 4;
+    if (whole_stage(*C)) {
+      choice4[3] |= 8;
+    } else {
+      if (C->halo && C->use_halo) choice4[0] |= 2;
+      if (C->halo && C->use_halo && C->have_small_grad && C->small_grad) choice4[0] |= 4;
+      if (C->small_blocks) choice4[3] |= 4;
+    }
   }
   if (best_ms) *best_ms = best;
   return 0;
@@ -3737,16 +3702,23 @@ int fvs_autotune(fvs_ctx *C, int nsteps, int *choice4, double *best_ms) try {
 int fvs_set_launch_choices(fvs_ctx *C, const int *choice4) try {
   if (!C || !choice4) return fail(FVS_EINVAL, "null argument");
   const bool halo = (choice4[0] & 2) != 0, small = (choice4[3] & 4) != 0, small_grad = (choice4[0] & 4) != 0;
+  const bool whole = (choice4[3] & 8) != 0;
+  if (whole && !C->stage_bs) return fail(FVS_EINVAL, "launch choices: no whole-stage lists for this context");
+  if (whole && (halo || small || small_grad))
+    return fail(FVS_EINVAL, "launch choices: the whole-stage kernel has no gradient or block-size choice");
+  if (!whole)
+    if (int rc = two_kernel_lists(*C)) return rc;
   if (halo && !C->halo) return fail(FVS_EINVAL, "launch choices: no staged-halo gradient data for this context");
   if (small_grad && !(halo && C->have_small_grad))
     return fail(FVS_EINVAL, "launch choices: no 128-cell staged-halo gradient lists for this context");
-  if (small && !(C->have_small && C->fused && !C->stage))
+  if (small && !(C->have_small && C->fused))
     return fail(FVS_EINVAL, "launch choices: no 128-cell block lists for this context");
   C->xcd_grad = (choice4[0] & 1) != 0;
   C->xcd_flux = (choice4[1] & 1) != 0;
   C->xcd_upd = (choice4[2] & 1) != 0;
   C->xcd_fused = (choice4[3] & 1) != 0;
-  C->use_halo = halo;
+  if (!whole) C->use_halo = halo;
+  C->use_stage = whole;
   C->small_grad = small_grad;
   C->small_blocks = small;
   C->launch_gen++;

@@ -1,0 +1,284 @@
+// Host side of the whole-stage kernel: its block lists (included by fvs_api.hip
+// after the context).
+
+// local index of a cell in a block (keys: id | periodic shift << 27), open
+// addressing
+class LocalMap {
+  std::vector<unsigned> key;
+  std::vector<int> val, used;
+  unsigned mask = 0;
+
+ public:
+  void reset(size_t most) {
+    size_t n = 256;
+    while (n < 2 * most) n *= 2;
+    if (n > key.size()) {
+      key.assign(n, ~0u);
+      val.resize(n);
+      mask = unsigned(n - 1);
+    } else {
+      for (int h : used) key[h] = ~0u;
+    }
+    used.clear();
+  }
+  // the entry of k, created (fresh) if there is none
+  int &at(unsigned k, bool &fresh) {
+    unsigned h = (k * 2654435761u >> 8) & mask;
+    while (key[h] != ~0u && key[h] != k) h = (h + 1) & mask;
+    fresh = key[h] == ~0u;
+    if (fresh) {
+      key[h] = k;
+      used.push_back(int(h));
+    }
+    return val[h];
+  }
+};
+
+// the mesh as the block lists read it (device cell order)
+struct StageMesh {
+  const std::vector<int> &gat;       // gw x N signed face slots
+  const std::vector<int2> &fic;      // interior faces' cells
+  const std::vector<double> &fig;    // and geometry, 8 per face
+  const std::vector<int> &fbc, &fbt;  // boundary faces
+  const std::vector<double> &fbg;
+  const std::vector<int> &off, &wid;  // stencils in 64-cell slices
+  const std::vector<unsigned> &code;  // id | periodic shift << 27
+};
+
+// the blocks cut from one contiguous part of the cells
+template <class SH>
+struct StageCut {
+  const fvs_ctx &C;
+  const StageMesh &M;
+  const int cw;       // code words of the widest stencil
+  short *const lgat;  // gw x N signed 1-based local faces
+  std::vector<StageBlock> blk;
+  std::vector<unsigned> halo, face, code;
+  std::vector<int> slot, nf, width;
+  bool shift_ok = true;  // every periodic shift of a face is in the table
+
+  // byte offset of the local cell with index q, of which the first n1 have gradients
+  static int offset(int q, int n1) {
+    if (q < n1) return 16 * q;
+    const int r = q - n1;
+    return r < SH::C1 ? SH::R2 + 16 * r : SH::FAR + 16 * (r - SH::C1);
+  }
+
+  // cells [i0, i1) as one block; false (nothing added) when it does not fit.
+  // Ring 2 may spill to far cells only where the block cannot be cut.
+  bool block(int i0, int i1) {
+    const int N = C.N, Fi = C.Fi, gw = C.GW;
+    loc.clear();
+    for (int i = i0; i < i1; ++i)
+      for (int k = 0; k < gw; ++k)
+        if (const int sg = M.gat[size_t(k) * N + i]) loc.push_back((sg > 0 ? sg : -sg) - 1);
+    std::sort(loc.begin(), loc.end());
+    loc.erase(std::unique(loc.begin(), loc.end()), loc.end());
+    if (int(loc.size()) > SH::F) return false;
+    r1.clear();
+    for (int f : loc) {
+      if (f >= Fi) continue;
+      for (int c : {M.fic[f].x, M.fic[f].y})
+        if (c < i0 || c >= i1) r1.push_back(c);
+    }
+    std::sort(r1.begin(), r1.end());
+    r1.erase(std::unique(r1.begin(), r1.end()), r1.end());
+    const int base = nblk(i1 - i0, kSlice) * kSlice, n1 = base + int(r1.size());
+    if (n1 > SH::C1) return false;
+    map.reset(size_t(n1) * (2 * cw + 1));
+    bool fresh;
+    for (int i = i0; i < i1; ++i) map.at(unsigned(i), fresh) = i - i0;
+    hal.assign(r1.begin(), r1.end());
+    for (size_t k = 0; k < r1.size(); ++k) map.at(unsigned(r1[k]), fresh) = base + int(k);
+    const size_t c0 = code.size();
+    code.resize(c0 + size_t(SH::NSL) * cw * kSlice, 0u);
+    int w2[SH::NSL];
+    for (int s = 0; s < SH::NSL; ++s) {
+      w2[s] = 0;
+      for (int l = 0; l < kSlice; ++l) {
+        const int q = s * kSlice + l;
+        const int i = q < base ? (i0 + q < i1 ? i0 + q : -1) : (q < n1 ? r1[q - base] : -1);
+        if (i < 0) continue;
+        const int sg = i / kSlice, li = i % kSlice;
+        w2[s] = std::max(w2[s], (M.wid[sg] + 1) / 2);
+        for (int k = 0; k < 2 * cw; ++k) {
+          int v = q;  // past the cell's own stencil: the cell itself (a zero term)
+          if (k < M.wid[sg]) {
+            const unsigned key = M.code[M.off[sg] + long(k) * kSlice + li];
+            int &x = map.at(key, fresh);
+            if (fresh) {
+              x = base + int(hal.size());
+              hal.push_back(key);
+            }
+            v = x;
+          }
+          code[c0 + (size_t(s) * cw + k / 2) * kSlice + l] |= unsigned(offset(v, n1)) << (16 * (k & 1));
+        }
+      }
+    }
+    const int nl = base + int(hal.size());
+    if (nl - n1 > SH::C1 && (i1 - i0 > kSlice || offset(nl - 1, n1) > 0xfff0)) {
+      code.resize(c0);
+      return false;
+    }
+    blk.push_back({i0, i1 - i0, base, int(r1.size()), int(hal.size()), {0, 0, 0}});
+    width.insert(width.end(), w2, w2 + SH::NSL);
+    halo.insert(halo.end(), hal.begin(), hal.end());
+    nf.push_back(int(loc.size()));
+    slot.insert(slot.end(), loc.begin(), loc.end());
+    for (int f : loc) {
+      if (f >= Fi) {
+        face.push_back(16 * unsigned(map.at(unsigned(M.fbc[f - Fi]), fresh)) | 0xffffu << 16);
+        continue;
+      }
+      const unsigned l = unsigned(map.at(unsigned(M.fic[f].x), fresh)), r = unsigned(map.at(unsigned(M.fic[f].y), fresh));
+      const double sx = C.mp.esx[C.mp.edge_intr[f]], sy = C.mp.esy[C.mp.edge_intr[f]];
+      unsigned sh = 0;
+      if (sx != 0.0 || sy != 0.0) {
+        while (sh < 15 && !(C.shifts.sx[sh] == sx && C.shifts.sy[sh] == sy)) ++sh;
+        shift_ok = shift_ok && sh < 15;
+        ++sh;
+      }
+      face.push_back(16 * l | (16 * r | (sh & 15u)) << 16);
+    }
+    for (int i = i0; i < i1; ++i)
+      for (int k = 0; k < gw; ++k)
+        if (const int sg = M.gat[size_t(k) * N + i]) {
+          const int li = int(std::lower_bound(loc.begin(), loc.end(), (sg > 0 ? sg : -sg) - 1) - loc.begin()) + 1;
+          lgat[size_t(k) * N + i] = short(sg > 0 ? li : -li);
+        }
+    return true;
+  }
+
+  // cells [i0, i1) as one block or cut in two, down to one slice
+  bool place(int i0, int i1) {
+    if (block(i0, i1)) return true;
+    if (i1 - i0 <= kSlice) return false;
+    int h = kSlice;
+    while (2 * h < i1 - i0) h *= 2;
+    return place(i0, i0 + h) && place(i0 + h, i1);
+  }
+  bool place_range(long b) { return place(int(b) * SH::BS, std::min(C.N, int(b + 1) * SH::BS)); }
+
+  StageCut(const fvs_ctx &c, const StageMesh &m, int w, short *g) : C(c), M(m), cw(w), lgat(g) {}
+
+ private:
+  LocalMap map;
+  std::vector<int> loc, r1;
+  std::vector<unsigned> hal;
+};
+
+int code_words(const StageMesh &M) { return std::max(1, (*std::max_element(M.wid.begin(), M.wid.end()) + 1) / 2); }
+
+// Blocks per range of SH::BS cells, from up to 256 ranges spread over the cells
+// (a large number when one does not fit at all)
+template <class SH>
+double stage_blocks_per_range(const fvs_ctx &C, const StageMesh &M) {
+  const long nr = nblk(C.N, SH::BS), step = std::max(1L, nr / 256);
+  std::vector<short> lgat(size_t(C.GW) * C.N, 0);
+  StageCut<SH> cut(C, M, code_words(M), lgat.data());
+  long ranges = 0;
+  for (long b = step / 2; b < nr; b += step, ++ranges)
+    if (!cut.place_range(b)) return 1e9;
+  return double(cut.blk.size()) / double(std::max(1L, ranges));
+}
+
+// Cuts all cells into blocks of shape SH and uploads the lists; C.stage_bs stays
+// 0 when a slice does not fit, or when so many ranges had to be cut that the
+// two-kernel path is faster.
+template <class SH>
+int setup_stage_blocks(fvs_ctx &C, const StageMesh &M) {
+  const int N = C.N, Fi = C.Fi, cw = code_words(M);
+  const long nr = nblk(N, SH::BS), np = parallel_parts(nr, 64);
+  std::vector<short> lgat(size_t(C.GW) * N, 0);
+  std::vector<StageCut<SH>> parts(np, StageCut<SH>(C, M, cw, lgat.data()));
+  std::vector<char> ok(np, 1);
+  parallel_for(nr, 64, [&](long t, long b0, long b1) {
+    for (long b = b0; b < b1 && ok[t]; ++b) ok[t] = parts[t].place_range(b) && parts[t].shift_ok;
+  });
+  std::vector<size_t> start(np + 1, 0);
+  int hs = 1, fs = 1;
+  for (long t = 0; t < np; ++t) {
+    if (!ok[t]) return 0;
+    start[t + 1] = start[t] + parts[t].blk.size();
+    for (const StageBlock &d : parts[t].blk) hs = std::max(hs, d.nh);
+    for (int n : parts[t].nf) fs = std::max(fs, n);
+  }
+  const size_t nb = start[np];
+  if (N > kStageSmallMesh && double(nb) > kStageMostBlocks * double(nr)) return 0;
+  hs = (hs + 31) / 32 * 32;  // strides of whole cache lines
+  fs = (fs + 15) / 16 * 16;
+  std::vector<StageBlock> blk(nb);
+  std::vector<int> halo(nb * hs), bcode(nb * fs), width(nb * SH::NSL);
+  std::vector<unsigned> code(nb * SH::NSL * cw * kSlice), face(nb * fs);
+  std::vector<double> geo(nb * fs * 5);
+  run_threads(int(np), [&](int t) {
+    const StageCut<SH> &p = parts[t];
+    size_t ho = 0, fo = 0;
+    std::copy(p.blk.begin(), p.blk.end(), blk.begin() + start[t]);
+    std::copy(p.width.begin(), p.width.end(), width.begin() + start[t] * SH::NSL);
+    std::copy(p.code.begin(), p.code.end(), code.begin() + start[t] * SH::NSL * cw * kSlice);
+    for (size_t k = 0; k < p.blk.size(); ++k) {
+      const size_t b = start[t] + k;
+      const int nh = p.blk[k].nh, nf = p.nf[k];
+      std::fill(std::copy(p.halo.begin() + ho, p.halo.begin() + ho + nh, halo.begin() + b * hs),
+                halo.begin() + (b + 1) * hs, -1);
+      std::fill(std::copy(p.face.begin() + fo, p.face.begin() + fo + nf, face.begin() + b * fs),
+                face.begin() + (b + 1) * fs, ~0u);
+      double *q = &geo[b * fs * 5];
+      for (int e = 0; e < nf; ++e) {
+        const int f = p.slot[fo + e], bq = f - Fi;
+        const double *g = f < Fi ? &M.fig[8 * size_t(f)] : &M.fbg[8 * size_t(bq)];
+        q[2 * e] = g[0];
+        q[2 * e + 1] = g[1];
+        q[2 * (fs + e)] = f < Fi ? C.mp.ex[C.mp.edge_intr[f]] : g[5];
+        q[2 * (fs + e) + 1] = f < Fi ? C.mp.ey[C.mp.edge_intr[f]] : g[6];
+        q[4 * fs + e] = g[2];
+        if (f >= Fi)
+          bcode[b * fs + e] = M.fbt[bq] | ((C.ninst > 0 ? C.inst_of_real[C.perm[M.fbc[bq]]] : 0) << 2);
+      }
+      ho += size_t(nh);
+      fo += size_t(nf);
+    }
+  });
+  StageBlock *dblk;
+  int *dhalo, *dbcode, *dwidth;
+  unsigned *dcode, *dface;
+  double *dgeo;
+  short *dlgat;
+  if (int rc = C.upload(dblk, blk)) return rc;
+  if (int rc = C.upload(dhalo, halo)) return rc;
+  if (int rc = C.upload(dbcode, bcode)) return rc;
+  if (int rc = C.upload(dwidth, width)) return rc;
+  if (int rc = C.upload(dcode, code)) return rc;
+  if (int rc = C.upload(dface, face)) return rc;
+  if (int rc = C.upload(dgeo, geo)) return rc;
+  if (int rc = C.upload(dlgat, lgat)) return rc;
+  HIPC(hipStreamSynchronize(C.stream));  // the host arrays end here
+  C.SL = {dblk, dhalo, dcode, dwidth, dface, dgeo, dbcode, dlgat, hs, cw, fs};
+  C.stage_bs = SH::BS;
+  C.stage_words = C.stage_faces = C.stage_halo = 0;
+  for (const StageCut<SH> &p : parts) {
+    C.stage_faces += long(p.face.size());
+    C.stage_halo += long(p.halo.size());
+    for (int w : p.width) C.stage_words += long(w) * kSlice;
+  }
+  C.stage_cells.clear();
+  for (const StageBlock &d : blk) C.stage_cells.push_back(make_int2(d.i0, d.n0));
+  return 0;
+}
+
+// The block shape: 128-cell blocks, unless many of them do not fit (O-grids,
+// whose stretched blocks have large halos) and the mesh is large enough for a
+// 256-cell block on every CU.  Measured, us per step in 128- / 256-cell blocks:
+// 2,097,152-cell vortex (nothing cut) 390 / 410; O-grids, limited, 128x64 (11%
+// more blocks) 39 / 45, 256x128 69 / 70, 300x150 79 / 75, 512x256 (19% more) 153 /
+// 143; a batch of 12 O-grids (18% more) 443 / 396.
+int setup_stage(fvs_ctx &C, const StageMesh &M) {
+  const bool large = C.opt.kernel_path != 2 && C.N >= 256 * StageLarge::BS;
+  if (large && stage_blocks_per_range<StageSmall>(C, M) > 1.05) {
+    if (int rc = setup_stage_blocks<StageLarge>(C, M)) return rc;
+    if (C.stage_bs) return 0;
+  }
+  return setup_stage_blocks<StageSmall>(C, M);
+}

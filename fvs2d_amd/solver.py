@@ -60,7 +60,7 @@ class Scheme:
     dt: float = 0.01
     cfl: float = 1.0
     reorder: int = 0          # device cell order: 0 reference, 1 Morton, 2 coordinate bisection
-    kernel_path: int = 0      # 0 fastest available, 1 face-flux buffer, 2 whole stage, 3 no block halo
+    kernel_path: int = 0      # 0 fastest available, 1 face-flux buffer, 2 whole stage (primitive), 3 no block halo
 
     def to_c(self) -> _lib.Options:
         o = _lib.Options()
@@ -482,8 +482,9 @@ class Solver:
         0), for the LSQ gradient or a limited Green-Gauss gradient's limiter
         whether it reads its stencil from a per-block halo staged in LDS (bit
         1), and for the fused flux kernel and the staged-halo LSQ gradient 128-
-        or 256-cell blocks (bit 2); the state is left as it was.  Returns
-        (choices, best ms per step)."""
+        or 256-cell blocks (bit 2); bit 3 of the fused choice says that a whole
+        stage is one kernel, whose numbering is then the only choice.  The
+        state is left as it was.  Returns (choices, best ms per step)."""
         ch = np.zeros(4, np.int32)
         best = np.zeros(1)
         check(self._L.fvs_autotune(self._h, nsteps, ptr(ch), ptr(best)))

@@ -66,17 +66,19 @@ typedef struct {
   int reorder;          /* device cell order: 0 reference order, 1 Morton (Z-curve)
                            blocks, 2 recursive coordinate bisection (compact
                            blocks on graded meshes); results are the same  */
-  int kernel_path;      /* 0: fastest available (fused LDS flux+update, centroid LSQ;
-                              SSP-RK3 stages read conservative stage states and
-                              write no primitive state, with the LSQ gradient or an
-                              unlimited Green-Gauss one);
+  int kernel_path;      /* 0: fastest available (LSQ gradients: the whole stage in one
+                              kernel where the cell order gives compact blocks, else a
+                              gradient and a fused flux+update kernel; SSP-RK3 stages
+                              read conservative stage states and write no primitive
+                              state, with the LSQ gradient or an unlimited Green-Gauss
+                              one);
                            1: face-flux buffer kernels only;
-                           2: whole stage in one kernel (gradients recomputed per
-                              block from LDS; LSQ, centroid form, triangle-sized
-                              blocks; falls back to 0 where it does not apply);
-                           3: as 0 without the per-block halo data (the LSQ
-                              gradient gathers its stencil cell by cell) and with
-                              SSP-RK3 stages on primitive states */
+                           2: the whole stage in one kernel on primitive states
+                              (LSQ, centroid form; falls back to 0 where it does not
+                              apply), which fvs_set_persistent needs;
+                           3: two kernels per stage without the per-block halo data
+                              (the LSQ gradient gathers its stencil cell by cell) and
+                              with SSP-RK3 stages on primitive states */
 } fvs_options;
 
 const char *fvs_last_error(void);
@@ -131,7 +133,8 @@ int fvs_set_phase_timers(fvs_ctx *ctx, int on);
  * evaluated inside the gradient launches, so its time is here), limiter
  * (always 0 for that reason), face fluxes (with the stage update where it is
  * fused into the flux launch), Runge-Kutta (separate stage-update launches
- * and the residual-norm reduction). */
+ * and the residual-norm reduction).  A launch of a whole stage is divided
+ * between gradient and face fluxes in the proportion of their operations. */
 int fvs_phase_times(const fvs_ctx *ctx, double *sec4);
 /* Launch mode, no reference counterpart: on != 0 runs each
  * fvs_time_integration call (or batch call) as one persistent cooperative
@@ -281,18 +284,21 @@ int fvs_batch_freeze_limiter(fvs_ctx *ctx, const int *frozen);
  * gather+update, fused flux+update], the faster of plain and XCD-aware
  * workgroup numbering, and the faster of 256 and 128 cells per workgroup for
  * the fused flux + update kernel and for the staged-halo LSQ gradient
- * (single meshes of at least 8,192 cells).  The state is restored
+ * (single meshes of at least 8,192 cells).  Where a stage is one kernel, its
+ * workgroup numbering is the only choice.  The state is restored
  * afterwards.  choice4 (may be NULL) receives the choices (bit 0 set =
  * XCD-aware; for the gradient, bit 1 set = the LSQ gradient, or a limited
  * Green-Gauss gradient's limiter, reads its stencil from a per-block halo
  * staged in LDS, the other candidate it tries, and bit 2 set = that LSQ
  * gradient on 128-cell workgroups; for the fused kernel, bit 2 set = 128-cell
- * workgroups), best_ms (may be NULL) the chosen setting's mean
+ * workgroups and bit 3 set = the whole stage in one kernel), best_ms (may be NULL) the chosen setting's mean
  * time per step over its last two trials. */
 int fvs_autotune(fvs_ctx *ctx, int nsteps, int *choice4, double *best_ms);
 /* Applies launch choices in fvs_autotune's choice4 encoding (for instance
  * choices an earlier fvs_autotune returned), without timing anything; a
- * choice this context has no data for fails with FVS_EINVAL.  No reference
+ * choice this context has no data for fails with FVS_EINVAL.  Without the
+ * whole-stage bit a context of one kernel per stage changes to two, whose
+ * lists the first such call builds.  No reference
  * counterpart. */
 int fvs_set_launch_choices(fvs_ctx *ctx, const int *choice4);
 /* wall-clock of the last fvs_time_integration call's device work (ms) */
