@@ -286,9 +286,30 @@ __device__ __forceinline__ const unsigned *active_mask(const int *blist, int nbl
   return reinterpret_cast<const unsigned *>(blist + nbl);
 }
 
+// Sum of a cell's face fluxes in the gather order: flux(f, fa) gives the flux *
+// area of the block's face f, speed(f) its wave speed * area (added with speeds).
+template <class Flux, class Speed>
+__device__ __forceinline__ void cell_gather(const int sv[4], Flux flux, Speed speed, bool speeds, double acc[4],
+                                            double &wacc) {
+  for (int v = 0; v < 4; ++v) acc[v] = 0.0;
+  wacc = 0.0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int s = sv[k];
+    if (s == 0) break;
+    const int f = (s > 0 ? s : -s) - 1;
+    double fa[4];
+    flux(f, fa);
+    if (s > 0)
+      for (int v = 0; v < 4; ++v) acc[v] = acc[v] + fa[v];
+    else
+      for (int v = 0; v < 4; ++v) acc[v] = acc[v] - fa[v];
+    if (speeds) wacc = wacc + speed(f);
+  }
+}
+
 // Gather, update and norm sums of cell i, one per thread (valid: i < N; whole
-// wavefronts call this): flux(f, fa) gives the flux * area of the block's face
-// f, speed(f) its wave speed * area.  amask (batches with masked instances): bit
+// wavefronts call this), with flux and speed as in cell_gather.  amask (batches with masked instances): bit
 // i of its words is set when cell i belongs to an active instance; a masked
 // cell keeps its state (the update is computed, nothing is stored) and
 // contributes zero increments.
@@ -301,20 +322,8 @@ __device__ __forceinline__ void cell_update(int N, int i, bool valid, const Upd 
   double d2[4] = {0, 0, 0, 0};
   const bool on = !amask || !valid || ((amask[i >> 5] >> (i & 31)) & 1u);
   if (valid) {
-    double acc[4] = {0.0, 0.0, 0.0, 0.0}, wacc = 0.0;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int s = in.sv[k];
-      if (s == 0) break;
-      const int f = (s > 0 ? s : -s) - 1;
-      double fa[4];
-      flux(f, fa);
-      if (s > 0)
-        for (int v = 0; v < 4; ++v) acc[v] = acc[v] + fa[v];
-      else
-        for (int v = 0; v < 4; ++v) acc[v] = acc[v] - fa[v];
-      if (A.steady && A.first) wacc = wacc + speed(f);
-    }
+    double acc[4], wacc;
+    cell_gather(in.sv, flux, speed, A.steady && A.first, acc, wacc);
     const double V = in.V;
     double R[4];
     const double iV = 1.0 / V;  // one division per cell (src/residual.f90:164-166 divides each)

@@ -82,6 +82,10 @@ struct StageIn {
   const int *blist;
   const unsigned *amask;
   const double *pinf_inst;
+  // residual evaluation (mode M_RESID): where the residual and the summed wave
+  // speeds go, in the caller's cell order (ref[device cell])
+  double *rout, *wsout;
+  const int *ref;
   // sweep direction: blocks in ascending or descending order.  Alternating
   // stages start where the last one ended, whose lists and states the 256 MB
   // memory-side cache still holds: 150 -> 139 us per stage on 2,097,152 cells
@@ -101,6 +105,7 @@ constexpr int kCodeRegs = 8;  // code words a thread holds in registers
 // own cells).  With cons (SSP-RK3 and the two-register form), Win holds
 // conservative states, converted once as they are staged, and the new stage
 // state goes to Ub (a buffer other than Win; no primitive state is written).
+// With mode M_RESID the block ends in the residual instead of an update.
 template <class SH, int LIM, int PMODE>
 __device__ __forceinline__ void stage_block(const StageIn &a, int lb, const Upd &A, const double *__restrict__ Win,
                                             double *__restrict__ Wout, int cons) {
@@ -242,7 +247,7 @@ __device__ __forceinline__ void stage_block(const StageIn &a, int lb, const Upd 
     if (!phi_one) at1(SH::P + 8 * tid) = ph;
   }
   __syncthreads();
-  const bool ws = A.steady && A.first;
+  const bool resid = A.mode == M_RESID, ws = resid || (A.steady && A.first);
   auto side = [&](unsigned o, double w[4], double gr[8], double &ph, double2 &c) __attribute__((always_inline)) {
     const double2 wa = at(o), wb = at(o + PS);
     c = at(o + 2 * PS);
@@ -284,7 +289,11 @@ __device__ __forceinline__ void stage_block(const StageIn &a, int lb, const Upd 
     if (ws) at1(SH::S + 8 * tid) = wsa;
   }
   UpdIn in;
-  if (mine) {
+  if (mine && resid) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) in.sv[k] = (k < a.gw) ? S.lgat[long(k) * N + id] : 0;
+    in.V = a.vol[id];
+  } else if (mine) {
     block_update_load(N, id, a.gw, A, S.lgat, a.vol, a.Ua, a.Ub, a.Facc, a.dtl, in, cons != 0);
     if (cons) {  // the stage input (the step-start state too on the first stage)
       for (int v = 0; v < 4; ++v) in.x[v] = u[v];
@@ -293,14 +302,25 @@ __device__ __forceinline__ void stage_block(const StageIn &a, int lb, const Upd 
     }
   }
   __syncthreads();
+  auto flux = [&](int f, double fa[4]) __attribute__((always_inline)) {
+    const double2 q0 = at(SH::F0 + 16 * f), q1 = at(SH::F1 + 16 * f);
+    fa[0] = q0.x; fa[1] = q0.y; fa[2] = q1.x; fa[3] = q1.y;
+  };
+  auto speed = [&](int f) __attribute__((always_inline)) { return at1(SH::S + 8 * f); };
+  if (resid) {
+    if (mine) {
+      double acc[4], wacc;
+      cell_gather(in.sv, flux, speed, true, acc, wacc);
+      const double iV = 1.0 / in.V;  // as in the stage update
+      for (int v = 0; v < 4; ++v) acc[v] = -acc[v] * iV;
+      const int c = a.ref[id];
+      st4(a.rout, c, acc);
+      a.wsout[c] = wacc;
+    }
+    return;
+  }
   if (tid < d.base)
-    cell_update(N, d.i0 + tid, mine, A, in,
-                [&](int f, double fa[4]) __attribute__((always_inline)) {
-                  const double2 q0 = at(SH::F0 + 16 * f), q1 = at(SH::F1 + 16 * f);
-                  fa[0] = q0.x; fa[1] = q0.y; fa[2] = q1.x; fa[3] = q1.y;
-                },
-                [&](int f) __attribute__((always_inline)) { return at1(SH::S + 8 * f); }, a.Ua, a.Ub, a.Facc, Wout,
-                a.dtl, a.norm, a.amask);
+    cell_update(N, d.i0 + tid, mine, A, in, flux, speed, a.Ua, a.Ub, a.Facc, Wout, a.dtl, a.norm, a.amask);
 }
 
 // four wavefronts per SIMD with the limiter (its registers spill at five, 154 ->

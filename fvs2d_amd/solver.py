@@ -287,7 +287,7 @@ class Solver:
     # -- state ------------------------------------------------------------
     @property
     def cvar(self) -> np.ndarray:
-        out = np.zeros((self.ncells, 4))
+        out = np.empty((self.ncells, 4))
         check(self._L.fvs_get_state(self._h, ptr(out)))
         return out
 
@@ -301,35 +301,35 @@ class Solver:
 
     # -- operators --------------------------------------------------------
     def cvar2pvar(self) -> np.ndarray:
-        out = np.zeros((self.ncells, 4))
+        out = np.empty((self.ncells, 4))
         check(self._L.fvs_primitives(self._h, ptr(out)))
         return out
 
     def compute_gradient_cellcntr(self) -> np.ndarray:
-        out = np.zeros((2, self.ncells, 4))
+        out = np.empty((2, self.ncells, 4))
         check(self._L.fvs_gradient(self._h, ptr(out)))
         return out
 
     def gradient_cellcntr_1var(self, fc) -> np.ndarray:
         fc = np.ascontiguousarray(fc, np.float64)
-        out = np.zeros((2, self.ncells))
+        out = np.empty((2, self.ncells))
         check(self._L.fvs_gradient_1var(self._h, ptr(fc), ptr(out)))
         return out
 
     def compute_gradient_limiter(self) -> np.ndarray:
-        out = np.zeros(self.ncells)
+        out = np.empty(self.ncells)
         check(self._L.fvs_limiter(self._h, ptr(out)))
         return out
 
     def compute_residual(self, time: float = 0.0):
-        r = np.zeros((self.ncells, 4))
-        w = np.zeros(self.ncells)
+        r = np.empty((self.ncells, 4))
+        w = np.empty(self.ncells)
         check(self._L.fvs_compute_residual(self._h, time, ptr(r), ptr(w)))
         self.resid, self.ws_nrml = r, w
         return r, w
 
     def compute_local_time(self) -> np.ndarray:
-        out = np.zeros(self.ncells)
+        out = np.empty(self.ncells)
         check(self._L.fvs_local_dt(self._h, ptr(out)))
         return out
 
