@@ -2,22 +2,21 @@
 //
 // Training step for a batch of M rows (M a multiple of 64), depth L hidden
 // layers of width 256:
-//   k_features       cell records -> bfloat16 input rows X0[M][128] (68 used)
-//   k_gemm_nt<FWD>   Z = X W + b, H = GELU(Z), one launch per hidden layer
+//   k_forward        cell records -> bfloat16 input rows X0[M][128] (68 used),
+//                    then for every hidden layer Z = X W + b, H = GELU(Z),
+//                    the activations of a row tile staying in LDS
 //   k_head           y = H W + b (float32), loss, dy, dZ of the last hidden
 //                    layer, output-layer weight/bias gradient partials
+//   k_backward       dZ_prev = (dZ W^T) * GELU'(Z_prev) down to the first
+//                    hidden layer, dZ of a row tile staying in LDS
 //   k_gemm_tn        weight-gradient partials X^T dZ (and bias partials)
-//   k_gemm_nt<BWD>   dZ_prev = (dZ W^T) * GELU'(Z_prev)
 //   k_adam           sums the partials in a fixed order, Adam update, and
 //                    refreshes the bfloat16 copies of the weights
-// The GEMMs run on v_mfma_f32_16x16x32_bf16: a workgroup of 4 wavefronts
-// owns 64 rows x all 256 columns (A read once), each wavefront a 64 x 64 tile
-// of 4 x 4 MFMA blocks.  Operands are staged through LDS with the reduction
-// index contiguous (rows padded to 40 elements, 80 bytes, so 16-byte
-// fragment reads hit distinct banks).  The weight gradient reduces over the
-// batch rows: each workgroup sums a contiguous slice of rows into one of S
-// partial copies, the Adam kernel adds the S copies in slice order, so the
-// result does not depend on scheduling (no float atomics).
+// Prediction is one k_forward launch with the output layer in it.
+// The matrix products run on v_mfma_f32_16x16x32_bf16.  The weight gradient
+// reduces over the batch rows: each workgroup sums a contiguous slice of rows
+// into one of S partial copies, the Adam kernel adds the S copies in slice
+// order, so the result does not depend on scheduling (no float atomics).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -28,6 +27,7 @@
 #include <memory>
 #include <new>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/fvs2d.h"
@@ -111,69 +111,49 @@ __host__ __device__ inline unsigned long long mix64(unsigned long long z) {
 }
 
 // ---------------------------------------------------------------- features
-// 16 threads per row, thread q writes input columns 8q..8q+7 (16 bytes):
-// q = 0..3 the radial harmonics 4q+1..4q+4, q = 4..7 the angular harmonics
-// 4(q-4)+1..+4 (one sincos of the base angle and one of the first harmonic,
-// then the angle-addition recurrence), q = 8 the four scalar channels.
-// sample != 0: row m takes record hash(seed, step, m) mod ndata; otherwise
-// record m, and rows m >= nvalid are zero.
-__global__ __launch_bounds__(256) void k_features(int M, long nvalid, const float *__restrict__ raw,
-                                                  const float *__restrict__ tgt, long ndata,
-                                                  unsigned long long seed, long step, int sample,
-                                                  u16 *__restrict__ X, float *__restrict__ T,
-                                                  float *__restrict__ F32) {
-  const long g = long(blockIdx.x) * 256 + threadIdx.x;
-  const long m = g >> 4;
-  const int q = int(g & 15);
-  if (m >= M) return;
-  bool valid;
-  long src;
-  if (sample) {
-    valid = true;
-    src = long(mix64(seed ^ mix64((unsigned long long)step * 0x100000001ull + (unsigned long long)m)) %
-               (unsigned long long)ndata);
-  } else {
-    valid = m < nvalid;
-    src = m;
-  }
-  float f[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  if (valid && q <= 8) {
-    const float *r = raw + src * kRaw;
-    if (q < 8) {
-      const double dx = double(r[0]) - 0.5, y = r[1];
-      double a;
-      if (q < 4) {
-        const double kPi = 3.14159265358979323846;
-        a = kPi * (log1p(4.0 * sqrt(dx * dx + y * y)) / log1p(200.0));
-      } else {
-        a = atan2(y, dx);
-      }
-      const int k0 = 4 * (q & 3) + 1;
-      double s1, c1, sk, ck;
-      sincos(a, &s1, &c1);
-      sincos(double(k0) * a, &sk, &ck);
-      for (int h = 0; h < 4; ++h) {
-        f[2 * h] = float(sk);
-        f[2 * h + 1] = float(ck);
-        const double sn = sk * c1 + ck * s1, cn = ck * c1 - sk * s1;
-        sk = sn;
-        ck = cn;
-      }
+// Input columns 8q..8q+7 of a cell record: q = 0..3 the radial harmonics
+// 4q+1..4q+4, q = 4..7 the angular harmonics 4(q-4)+1..+4 (one sincos of the
+// base angle and one of the first harmonic, then the angle-addition
+// recurrence), q = 8 the four scalar channels.
+constexpr int kFeatChunks = (kFeat + 7) / 8;
+__device__ __forceinline__ void features8(const float *__restrict__ r, int q, float f[8]) {
+  if (q < 8) {
+    const double dx = double(r[0]) - 0.5, y = r[1];
+    double a;
+    if (q < 4) {
+      const double kPi = 3.14159265358979323846;
+      a = kPi * (log1p(4.0 * sqrt(dx * dx + y * y)) / log1p(200.0));
     } else {
-      f[0] = float(log1p(100.0 * double(r[2])) / log1p(5000.0));
-      f[1] = float((double(r[3]) - 0.675) / 0.175);
-      f[2] = float((double(r[4]) - 1.0) / 3.0);
-      f[3] = float((double(r[5]) - 0.125) / 0.025);
+      a = atan2(y, dx);
     }
+    const int k0 = 4 * (q & 3) + 1;
+    double s1, c1, sk, ck;
+    sincos(a, &s1, &c1);
+    sincos(double(k0) * a, &sk, &ck);
+    for (int h = 0; h < 4; ++h) {
+      f[2 * h] = float(sk);
+      f[2 * h + 1] = float(ck);
+      const double sn = sk * c1 + ck * s1, cn = ck * c1 - sk * s1;
+      sk = sn;
+      ck = cn;
+    }
+  } else {
+    f[0] = float(log1p(100.0 * double(r[2])) / log1p(5000.0));
+    f[1] = float((double(r[3]) - 0.675) / 0.175);
+    f[2] = float((double(r[4]) - 1.0) / 3.0);
+    f[3] = float((double(r[5]) - 0.125) / 0.025);
+    f[4] = f[5] = f[6] = f[7] = 0.f;
   }
-  unsigned pk[4];
-  for (int c = 0; c < 4; ++c) pk[c] = unsigned(f2bf(f[2 * c])) | (unsigned(f2bf(f[2 * c + 1])) << 16);
-  *reinterpret_cast<uint4 *>(X + m * kInPad + 8 * q) = make_uint4(pk[0], pk[1], pk[2], pk[3]);
-  if (F32 && valid)
-    for (int c = 0; c < 8; ++c)
-      if (8 * q + c < kFeat) F32[m * kFeat + 8 * q + c] = f[c];
-  if (T && q == 0)
-    for (int o = 0; o < kOut; ++o) T[m * kOut + o] = valid ? tgt[src * kOut + o] : 0.0f;
+}
+
+// the feature map alone, float32: 256 rows per workgroup, blockIdx.y the columns
+__global__ __launch_bounds__(256) void k_features(int n, const float *__restrict__ raw, float *__restrict__ F32) {
+  const int m = blockIdx.x * 256 + threadIdx.x, q = blockIdx.y;
+  if (m >= n) return;
+  float f[8];
+  features8(raw + long(m) * kRaw, q, f);
+  for (int c = 0; c < 8; ++c)
+    if (8 * q + c < kFeat) F32[long(m) * kFeat + 8 * q + c] = f[c];
 }
 
 // ------------------------------------------------------------- GEMM core
@@ -199,146 +179,244 @@ __device__ __forceinline__ void mma_slab(const u16 *__restrict__ As, const u16 *
 }
 
 __device__ __forceinline__ unsigned pack2(float a, float b) {
-  return unsigned(f2bf(a)) | (unsigned(f2bf(b)) << 16);
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{a, b}, bf16x2));
 }
 
-// C[M][256] = A[M][K] * B[256][K]^T (both row-major, K a multiple of 32).
-// EPI 0 (forward): z = C + bias; Z = bf16(z), H = bf16(GELU(z)).
-// EPI 1 (backward data): dZ = bf16(C * GELU'(Zp)).
-// The next slab's global data is loaded into registers while the current
-// one is multiplied.
-template <int EPI>
-__global__ __launch_bounds__(256) void k_gemm_nt(int K, const u16 *__restrict__ A, const u16 *__restrict__ B,
-                                                 const float *__restrict__ bias, const u16 *__restrict__ Zp,
-                                                 u16 *__restrict__ O1, u16 *__restrict__ O2) {
-  __shared__ __attribute__((aligned(16))) u16 As[kRows * kLds];
-  __shared__ __attribute__((aligned(16))) u16 Bs[kW * kLds];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const long r0 = long(blockIdx.x) * kRows;
-  f32x4 acc[4][4];
+// ------------------------------------------------------ forward / backward
+// One launch for all layers: as one product per layer, 65,536 rows took 5 x 45
+// us forward in training (Z, H written, H read back) and prediction 397 us a
+// call; in this form 118 us forward, 132 us backward, and 246 us a call.
+// A workgroup of 4 wavefronts owns TR rows and all 256 columns of every layer:
+// the rows' activations stay in LDS from layer to layer, and only what the
+// weight gradient reads is written to HBM.  Each wavefront holds TR x 64
+// results.  Its weights are not shared with the other wavefronts, so they go
+// from L2 to registers without LDS, in the order the MFMA operand wants them
+// (pack_at): one contiguous KB per load.
+constexpr int kActLd = kW + 8;  // LDS row (elements): 16-byte accesses of 16 rows meet distinct banks
+constexpr int kSlabs0 = (kFeat + kBK - 1) / kBK;  // slabs of the input layer that are not padding
+
+// Element of the packed copy of B[n][k]: per slab of 32 k and 64 columns of a
+// wavefront four operand blocks of 16 columns x 32 k.  Row t of block j is
+// column 32 (j / 2) + 8 (t / 4) + 4 (j % 2) + t % 4, so that a lane's results
+// of blocks 2h and 2h + 1 are eight consecutive columns: activations leave as
+// 16-byte vectors, four lanes to a 64-byte segment.
+__host__ __device__ inline int pack_at(int n, int k) {
+  const int c = n & 31, t = 4 * (c >> 3) + (c & 3), j = 2 * ((n >> 5) & 1) + ((c >> 2) & 1);
+  return ((((k >> 5) * 4 + (n >> 6)) * 4 + j) * 64 + t + 16 * ((k & 31) >> 3)) * 8 + (k & 7);
+}
+
+// acc = rows of act (TR x 32 ns) times a wavefront's 64 columns, slab after
+// slab (Wp: the lane's place in the packed weights); D slabs of weights are in
+// registers or in flight (b; the caller has loaded the first D).
+template <int TR, int D>
+__device__ __forceinline__ void load_slab(const u16 *__restrict__ Wp, int s, bf16x8 (&b)[4]) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int j = 0; j < 4; ++j) b[j] = *reinterpret_cast<const bf16x8 *>(Wp + (s * 16 + j) * 512);
+}
+template <int TR, int D>
+__device__ __forceinline__ void chain_layer(const u16 *__restrict__ act, const u16 *__restrict__ Wp, int ns, int lane,
+                                            bf16x8 (&b)[D][4], f32x4 (&acc)[TR / 16][4]) {
+  const u16 *ap = act + (lane & 15) * kActLd + 8 * (lane >> 4);
+#pragma unroll
+  for (int i = 0; i < TR / 16; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int arow = tid >> 2, ac = (tid & 3) * 8;
-  const u16 *Ap = A + (r0 + arow) * K + ac;
-  uint4 ra = *reinterpret_cast<const uint4 *>(Ap), rb[4];
+  for (int s0 = 0; s0 < ns; s0 += D) {
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int ch = tid + 256 * q;
-    rb[q] = *reinterpret_cast<const uint4 *>(B + long(ch >> 2) * K + (ch & 3) * 8);
-  }
-  for (int k0 = 0; k0 < K; k0 += kBK) {
-    *reinterpret_cast<uint4 *>(As + arow * kLds + ac) = ra;
+    for (int u = 0; u < D; ++u) {
+      const int s = s0 + u;
+      if (s < ns) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int ch = tid + 256 * q;
-      *reinterpret_cast<uint4 *>(Bs + (ch >> 2) * kLds + (ch & 3) * 8) = rb[q];
-    }
-    __syncthreads();
-    if (k0 + kBK < K) {
-      ra = *reinterpret_cast<const uint4 *>(Ap + k0 + kBK);
+        for (int i = 0; i < TR / 16; ++i) {
+          const bf16x8 a = *reinterpret_cast<const bf16x8 *>(ap + 16 * i * kActLd + kBK * s);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int ch = tid + 256 * q;
-        rb[q] = *reinterpret_cast<const uint4 *>(B + long(ch >> 2) * K + k0 + kBK + (ch & 3) * 8);
-      }
-    }
-    mma_slab(As, Bs, lane, w, acc);
-    __syncthreads();
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const long row = r0 + 16 * i + (lane & 15);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n0 = 64 * w + 16 * j + 4 * (lane >> 4);
-      const long idx = row * kW + n0;
-      if (EPI == 0) {
-        const float4 bv = *reinterpret_cast<const float4 *>(bias + n0);
-        const float z0 = acc[i][j][0] + bv.x, z1 = acc[i][j][1] + bv.y, z2 = acc[i][j][2] + bv.z,
-                    z3 = acc[i][j][3] + bv.w;
-        *reinterpret_cast<uint2 *>(O1 + idx) = make_uint2(pack2(z0, z1), pack2(z2, z3));
-        *reinterpret_cast<uint2 *>(O2 + idx) = make_uint2(pack2(gelu(z0), gelu(z1)), pack2(gelu(z2), gelu(z3)));
-      } else {
-        const uint2 zz = *reinterpret_cast<const uint2 *>(Zp + idx);
-        const float z0 = bf2f(u16(zz.x & 0xffffu)), z1 = bf2f(u16(zz.x >> 16)), z2 = bf2f(u16(zz.y & 0xffffu)),
-                    z3 = bf2f(u16(zz.y >> 16));
-        *reinterpret_cast<uint2 *>(O1 + idx) =
-            make_uint2(pack2(acc[i][j][0] * gelu_grad(z0), acc[i][j][1] * gelu_grad(z1)),
-                       pack2(acc[i][j][2] * gelu_grad(z2), acc[i][j][3] * gelu_grad(z3)));
+          for (int j = 0; j < 4; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[u][j], a, acc[i][j], 0, 0, 0);
+        }
+        if (s + D < ns) load_slab<TR, D>(Wp, s + D, b[u]);
       }
     }
   }
 }
 
-// Large-tile form of k_gemm_nt for M a multiple of 256: 16 wavefronts own
-// 256 rows x 256 columns (wave w: rows 64(w/4).., columns 64(w%4)..), so a
-// workgroup reads each weight slab once per 256 rows instead of per 64
-// (weights are a quarter of the L2 traffic), and the slabs are double
-// buffered in LDS: one barrier per slab.  Same arithmetic as k_gemm_nt.
-constexpr int kBigRows = 256, kBigThreads = 1024;
+// the rows of a pass: records (and targets) given by the caller, rows from
+// nvalid on zero, or with ndata > 0 drawn from a set of that many: row m takes
+// record hash(seed, step, m) mod ndata
+struct Rows {
+  const float *raw, *tgt;
+  long nvalid, ndata;
+  unsigned long long seed;
+  long step;
+};
+__device__ __forceinline__ long row_source(const Rows &R, long m) {
+  if (R.ndata > 0)
+    return long(mix64(R.seed ^ mix64((unsigned long long)R.step * 0x100000001ull + (unsigned long long)m)) %
+                (unsigned long long)R.ndata);
+  return m < R.nvalid ? m : -1;
+}
 
-template <int EPI>
-__global__ __launch_bounds__(kBigThreads) void k_gemm_nt_big(int K, const u16 *__restrict__ A,
-                                                             const u16 *__restrict__ B, const float *__restrict__ bias,
-                                                             const u16 *__restrict__ Zp, u16 *__restrict__ O1,
-                                                             u16 *__restrict__ O2) {
-  __shared__ __attribute__((aligned(16))) u16 As[2][kBigRows * kLds];
-  __shared__ __attribute__((aligned(16))) u16 Bs[2][kW * kLds];
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, wm = wv >> 2, wn = wv & 3;
-  const long r0 = long(blockIdx.x) * kBigRows;
-  f32x4 acc[4][4];
+struct Chain {
+  int L;
+  long M;
+  const u16 *W[kMaxDepth];     // packed weights
+  const float *bias[kMaxDepth];
+  u16 *X0, *Z[kMaxDepth], *H[kMaxDepth];
+  const float *Wh, *bh;        // output layer
+  float *T, *Y;
+};
+
+// Wavefronts per SIMD the registers allow: 16 (TR / 16) accumulators, 16 D weights
+constexpr int chain_waves(int TR) { return TR >= 128 ? 2 : 3; }
+
+// Features and all hidden layers of TR rows.  TRAIN: X0, Z, H and the targets
+// go to HBM; otherwise only the network's output does.
+template <int TR, int D, bool TRAIN>
+__global__ __launch_bounds__(256, chain_waves(TR)) void k_forward(Chain c, Rows R) {
+  __shared__ __attribute__((aligned(16))) u16 act[TR * kActLd];
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const long r0 = long(blockIdx.x) * TR;
+  const int lp = (wv * 4 * 64 + lane) * 8;  // the lane's place in a slab of packed weights
+  bf16x8 b[D][4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // one 16-byte chunk of A and one of B per thread per slab (256 rows x 32)
-  const int row = tid >> 2, c8 = (tid & 3) * 8;
-  const u16 *Ap = A + (r0 + row) * K + c8;
-  const u16 *Bp = B + long(row) * K + c8;
-  uint4 ra = *reinterpret_cast<const uint4 *>(Ap);
-  uint4 rb = *reinterpret_cast<const uint4 *>(Bp);
-  *reinterpret_cast<uint4 *>(&As[0][row * kLds + c8]) = ra;
-  *reinterpret_cast<uint4 *>(&Bs[0][row * kLds + c8]) = rb;
+  for (int u = 0; u < D; ++u)
+    if (u < kSlabs0) load_slab<TR, D>(c.W[0] + lp, u, b[u]);
+  // consecutive lanes take the same columns of consecutive rows: a wavefront
+  // evaluates one kind of feature (the kinds differ in their functions)
+  for (int e = tid; e < TR * (4 * kSlabs0); e += 256) {
+    const int row = e % TR, q = e / TR;
+    const long m = r0 + row;
+    const long src = m < c.M ? row_source(R, m) : -1;
+    uint4 v = make_uint4(0, 0, 0, 0);
+    if (q < kFeatChunks && src >= 0) {
+      float f[8];
+      features8(R.raw + src * kRaw, q, f);
+      v = make_uint4(pack2(f[0], f[1]), pack2(f[2], f[3]), pack2(f[4], f[5]), pack2(f[6], f[7]));
+    }
+    *reinterpret_cast<uint4 *>(act + row * kActLd + 8 * q) = v;
+    if (TRAIN && q == 0 && m < c.M)
+      *reinterpret_cast<float4 *>(c.T + m * kOut) =
+          src >= 0 ? *reinterpret_cast<const float4 *>(R.tgt + src * kOut) : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
   __syncthreads();
-  const int ns = K / kBK;
-  for (int st = 0; st < ns; ++st) {
-    const int cur = st & 1;
-    const bool more = st + 1 < ns;
-    if (more) {
-      ra = *reinterpret_cast<const uint4 *>(Ap + (st + 1) * kBK);
-      rb = *reinterpret_cast<const uint4 *>(Bp + (st + 1) * kBK);
+  if (TRAIN) {
+    for (int e = tid; e < TR * (4 * kSlabs0); e += 256) {
+      const int row = e / (4 * kSlabs0), q = e % (4 * kSlabs0);
+      if (r0 + row < c.M)
+        *reinterpret_cast<uint4 *>(c.X0 + (r0 + row) * kInPad + 8 * q) =
+            *reinterpret_cast<const uint4 *>(act + row * kActLd + 8 * q);
     }
-    mma_slab(&As[cur][(64 * wm) * kLds], &Bs[cur][0], lane, wn, acc);
-    if (more) {
-      *reinterpret_cast<uint4 *>(&As[cur ^ 1][row * kLds + c8]) = ra;
-      *reinterpret_cast<uint4 *>(&Bs[cur ^ 1][row * kLds + c8]) = rb;
+  }
+  f32x4 acc[TR / 16][4];
+  for (int l = 0; l < c.L; ++l) {
+    chain_layer<TR, D>(act, c.W[l] + lp, l == 0 ? kSlabs0 : kW / kBK, lane, b, acc);
+    if (l + 1 < c.L)
+#pragma unroll
+      for (int u = 0; u < D; ++u) load_slab<TR, D>(c.W[l + 1] + lp, u, b[u]);
+    const int n0 = 64 * wv + 8 * (lane >> 4);
+    float bv[2][8];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) bv[h][e] = c.bias[l][n0 + 32 * h + e];
+    __syncthreads();  // every wavefront has read the layer's input
+#pragma unroll
+    for (int i = 0; i < TR / 16; ++i) {
+      const int row = 16 * i + (lane & 15);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        float z[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) z[e] = acc[i][2 * h + (e >> 2)][e & 3] + bv[h][e];
+        const uint4 hv = make_uint4(pack2(gelu(z[0]), gelu(z[1])), pack2(gelu(z[2]), gelu(z[3])),
+                                    pack2(gelu(z[4]), gelu(z[5])), pack2(gelu(z[6]), gelu(z[7])));
+        *reinterpret_cast<uint4 *>(act + row * kActLd + n0 + 32 * h) = hv;
+        if (TRAIN && r0 + 16 * i < c.M) {
+          const long idx = (r0 + row) * kW + n0 + 32 * h;
+          *reinterpret_cast<uint4 *>(c.Z[l] + idx) =
+              make_uint4(pack2(z[0], z[1]), pack2(z[2], z[3]), pack2(z[4], z[5]), pack2(z[6], z[7]));
+          *reinterpret_cast<uint4 *>(c.H[l] + idx) = hv;
+        }
+      }
     }
     __syncthreads();
   }
+  if (!TRAIN) {
+    // the output layer, 32 lanes per row as in k_head
+    const int q = tid & 31, rs = tid >> 5;
+    float w[8][kOut];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const long rr = r0 + 64 * wm + 16 * i + (lane & 15);
+    for (int e = 0; e < 8; ++e)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n0 = 64 * wn + 16 * j + 4 * (lane >> 4);
-      const long idx = rr * kW + n0;
-      if (EPI == 0) {
-        const float4 bv = *reinterpret_cast<const float4 *>(bias + n0);
-        const float z0 = acc[i][j][0] + bv.x, z1 = acc[i][j][1] + bv.y, z2 = acc[i][j][2] + bv.z,
-                    z3 = acc[i][j][3] + bv.w;
-        *reinterpret_cast<uint2 *>(O1 + idx) = make_uint2(pack2(z0, z1), pack2(z2, z3));
-        *reinterpret_cast<uint2 *>(O2 + idx) = make_uint2(pack2(gelu(z0), gelu(z1)), pack2(gelu(z2), gelu(z3)));
-      } else {
-        const uint2 zz = *reinterpret_cast<const uint2 *>(Zp + idx);
-        const float z0 = bf2f(u16(zz.x & 0xffffu)), z1 = bf2f(u16(zz.x >> 16)), z2 = bf2f(u16(zz.y & 0xffffu)),
-                    z3 = bf2f(u16(zz.y >> 16));
-        *reinterpret_cast<uint2 *>(O1 + idx) =
-            make_uint2(pack2(acc[i][j][0] * gelu_grad(z0), acc[i][j][1] * gelu_grad(z1)),
-                       pack2(acc[i][j][2] * gelu_grad(z2), acc[i][j][3] * gelu_grad(z3)));
+      for (int o = 0; o < kOut; ++o) w[e][o] = c.Wh[(8 * q + e) * kOut + o];
+    for (int row = rs; row < TR; row += 8) {
+      const uint4 hv = *reinterpret_cast<const uint4 *>(act + row * kActLd + 8 * q);
+      const unsigned hw[4] = {hv.x, hv.y, hv.z, hv.w};
+      float y[kOut] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float h = bf2f(u16((hw[e >> 1] >> (16 * (e & 1))) & 0xffffu));
+#pragma unroll
+        for (int o = 0; o < kOut; ++o) y[o] += h * w[e][o];
+      }
+      for (int off = 16; off >= 1; off >>= 1)
+        for (int o = 0; o < kOut; ++o) y[o] += __shfl_xor(y[o], off, 64);
+      if (q == 0 && r0 + row < R.nvalid)
+        *reinterpret_cast<float4 *>(c.Y + (r0 + row) * kOut) =
+            make_float4(y[0] + c.bh[0], y[1] + c.bh[1], y[2] + c.bh[2], y[3] + c.bh[3]);
+    }
+  }
+}
+
+// dZ of the hidden layers below the last, each in the place of its layer's Z
+// (c.W: the backward operands; Z of the last layer holds its dZ)
+template <int TR, int D>
+__global__ __launch_bounds__(256, chain_waves(TR)) void k_backward(Chain c) {
+  __shared__ __attribute__((aligned(16))) u16 act[TR * kActLd];
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const long r0 = long(blockIdx.x) * TR;
+  const int lp = (wv * 4 * 64 + lane) * 8;
+  bf16x8 b[D][4];
+#pragma unroll
+  for (int u = 0; u < D; ++u) load_slab<TR, D>(c.W[c.L - 1] + lp, u, b[u]);
+  const u16 *top = c.Z[c.L - 1];
+  for (int e = tid; e < TR * (kW / 8); e += 256) {
+    const int row = e / (kW / 8), q = e % (kW / 8);
+    *reinterpret_cast<uint4 *>(act + row * kActLd + 8 * q) =
+        r0 + row < c.M ? *reinterpret_cast<const uint4 *>(top + (r0 + row) * kW + 8 * q) : make_uint4(0, 0, 0, 0);
+  }
+  __syncthreads();
+  f32x4 acc[TR / 16][4];
+  for (int l = c.L - 1; l > 0; --l) {
+    chain_layer<TR, D>(act, c.W[l] + lp, kW / kBK, lane, b, acc);
+    if (l > 1)
+#pragma unroll
+      for (int u = 0; u < D; ++u) load_slab<TR, D>(c.W[l - 1] + lp, u, b[u]);
+    const int n0 = 64 * wv + 8 * (lane >> 4);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < TR / 16; ++i) {
+      const int row = 16 * i + (lane & 15);
+      __builtin_amdgcn_sched_barrier(0);  // Z of few rows at a time in registers
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        uint4 dv = make_uint4(0, 0, 0, 0);
+        if (r0 + 16 * i < c.M) {
+          u16 *zp = c.Z[l - 1] + (r0 + row) * kW + n0 + 32 * h;
+          const uint4 zv = *reinterpret_cast<const uint4 *>(zp);
+          const unsigned zw[4] = {zv.x, zv.y, zv.z, zv.w};
+          float d[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            d[e] = acc[i][2 * h + (e >> 2)][e & 3] * gelu_grad(bf2f(u16((zw[e >> 1] >> (16 * (e & 1))) & 0xffffu)));
+          dv = make_uint4(pack2(d[0], d[1]), pack2(d[2], d[3]), pack2(d[4], d[5]), pack2(d[6], d[7]));
+          *reinterpret_cast<uint4 *>(zp) = dv;
+        }
+        *reinterpret_cast<uint4 *>(act + row * kActLd + n0 + 32 * h) = dv;
       }
     }
+    __syncthreads();
   }
 }
 
@@ -555,14 +633,13 @@ constexpr int kHeadPart = kW * kOut + kOut;    // output-layer parameters
 
 // Workgroup b handles rows [128b, min(128b + 128, M)), 8 rows at a time (M is
 // a multiple of 64, so every lane of a row pair runs the same trips), 32 lanes per
-// row, 8 hidden columns per lane.  y = H Wh + bh in float32.  With dZ set:
+// row, 8 hidden columns per lane.  y = H Wh + bh in float32,
 // dy = 2 (y - t) / (nvalid * 4) for rows < nvalid (0 otherwise), the last
-// hidden layer's dZ = bf16((dy Wh^T) * GELU'(Z)), and this workgroup's
-// partial gradients of Wh and bh (Gh[b][...]) and loss sum (lossp[b]).
-__global__ __launch_bounds__(256) void k_head(long M, long nvalid, float inv_no, const u16 *__restrict__ H,
-                                              const u16 *__restrict__ Z, const float *__restrict__ Wh,
-                                              const float *__restrict__ bh, const float *__restrict__ T,
-                                              float *__restrict__ Y, u16 *__restrict__ dZ, float *__restrict__ Gh,
+// hidden layer's dZ = bf16((dy Wh^T) * GELU'(Z)) in the place of Z, and this
+// workgroup's partial gradients of Wh and bh (Gh[b][...]) and loss sum (lossp[b]).
+__global__ __launch_bounds__(256) void k_head(long M, long nvalid, float inv_no, const u16 *__restrict__ H, u16 *Z,
+                                              const float *__restrict__ Wh, const float *__restrict__ bh,
+                                              const float *__restrict__ T, float *__restrict__ Gh,
                                               float *__restrict__ lossp) {
   __shared__ float Ws[kW * kOut];
   __shared__ float red[4][32][8 * kOut + kOut + 1];
@@ -578,13 +655,13 @@ __global__ __launch_bounds__(256) void k_head(long M, long nvalid, float inv_no,
   uint4 hn{}, zn{};
   if (mbeg + rs < mend) {
     hn = *reinterpret_cast<const uint4 *>(H + (mbeg + rs) * kW + 8 * q);
-    if (dZ) zn = *reinterpret_cast<const uint4 *>(Z + (mbeg + rs) * kW + 8 * q);
+    zn = *reinterpret_cast<const uint4 *>(Z + (mbeg + rs) * kW + 8 * q);
   }
   for (long m = mbeg + rs; m < mend; m += 8) {
     const uint4 hv = hn, zv = zn;
     if (m + 8 < mend) {
       hn = *reinterpret_cast<const uint4 *>(H + (m + 8) * kW + 8 * q);
-      if (dZ) zn = *reinterpret_cast<const uint4 *>(Z + (m + 8) * kW + 8 * q);
+      zn = *reinterpret_cast<const uint4 *>(Z + (m + 8) * kW + 8 * q);
     }
     const unsigned hw[4] = {hv.x, hv.y, hv.z, hv.w};
     float h[8];
@@ -599,9 +676,6 @@ __global__ __launch_bounds__(256) void k_head(long M, long nvalid, float inv_no,
       for (int o = 0; o < kOut; ++o) y[o] += __shfl_xor(y[o], off, 64);
     for (int o = 0; o < kOut; ++o) y[o] += bh[o];
     const bool valid = m < nvalid;
-    if (Y && valid && q == 0)
-      for (int o = 0; o < kOut; ++o) Y[m * kOut + o] = y[o];
-    if (!dZ) continue;
     float dy[kOut];
     for (int o = 0; o < kOut; ++o) {
       const float r = valid ? y[o] - T[m * kOut + o] : 0.f;
@@ -617,11 +691,10 @@ __global__ __launch_bounds__(256) void k_head(long M, long nvalid, float inv_no,
       pk[c >> 1] |= unsigned(f2bf(g * gelu_grad(z))) << (16 * (c & 1));
       for (int o = 0; o < kOut; ++o) gw[c][o] += h[c] * dy[o];
     }
-    *reinterpret_cast<uint4 *>(dZ + m * kW + 8 * q) = make_uint4(pk[0], pk[1], pk[2], pk[3]);
+    *reinterpret_cast<uint4 *>(Z + m * kW + 8 * q) = make_uint4(pk[0], pk[1], pk[2], pk[3]);
     if (q == 0)
       for (int o = 0; o < kOut; ++o) gb[o] += dy[o];
   }
-  if (!dZ) return;
   // rows rs and rs^1 share a wavefront: add the two halves, then the 4 waves
   for (int c = 0; c < 8; ++c)
     for (int o = 0; o < kOut; ++o) gw[c][o] += __shfl_xor(gw[c][o], 32, 64);
@@ -671,8 +744,8 @@ __global__ __launch_bounds__(256) void k_head_reduce(int nhb, const float *__res
 struct LayerTab {
   long offW[kMaxLayers], offb[kMaxLayers];
   int in[kMaxLayers], out[kMaxLayers], inpad[kMaxLayers];
-  u16 *Wt[kMaxLayers];  // [out][inpad] copies (forward operand)
-  u16 *Wk[kMaxLayers];  // [in][out] copies (backward-data operand)
+  u16 *Wt[kMaxLayers];  // packed copies (pack_at): forward operand, reduction over the inputs
+  u16 *Wk[kMaxLayers];  // backward-data operand, reduction over the outputs
   int nl;
 };
 
@@ -733,8 +806,8 @@ __global__ __launch_bounds__(256) void k_adam(long P, int nsplit, int mode, cons
       const long e = p - tab.offW[l];
       const int k = int(e / tab.out[l]), n = int(e % tab.out[l]);
       const u16 v = f2bf(w[p]);
-      if (tab.Wt[l]) tab.Wt[l][long(n) * tab.inpad[l] + k] = v;
-      if (tab.Wk[l]) tab.Wk[l][long(k) * tab.out[l] + n] = v;
+      if (tab.Wt[l]) tab.Wt[l][pack_at(n, k)] = v;
+      if (tab.Wk[l]) tab.Wk[l][pack_at(k, n)] = v;
     }
   }
 }
@@ -752,8 +825,8 @@ struct fvs_mlp {
   float *w = nullptr, *m1 = nullptr, *m2 = nullptr, *G = nullptr, *Gh = nullptr, *gh = nullptr,
         *lossp = nullptr, *gtmp = nullptr;
   double *lossh = nullptr;
-  u16 *X0 = nullptr, *dZa = nullptr, *dZb = nullptr;
-  u16 *Z[kMaxDepth] = {}, *H[kMaxDepth] = {};
+  u16 *X0 = nullptr;
+  u16 *Z[kMaxDepth] = {}, *H[kMaxDepth] = {};  // the backward pass leaves dZ in Z
   float *T = nullptr, *Y = nullptr, *F32 = nullptr;
   float *raw = nullptr, *tgt = nullptr;  // training set
   long ndata = 0;
@@ -787,6 +860,7 @@ struct fvs_mlp {
 
 namespace {
 
+// MC_FEAT: part of MC_FWD
 enum { MC_FEAT, MC_FWD, MC_HEAD, MC_WGRAD, MC_BWD, MC_ADAM, MC_N };
 
 struct Prof {
@@ -813,52 +887,82 @@ int nsplit(int M) {
   return 1;
 }
 
-// forward (and with grad, backward) over the first M rows already in X0/T
-int run_pass(fvs_mlp &m, int M, long nvalid, bool grad, float *Y) {
+// f(tile rows): the row tile of a pass over M rows.  128 rows read the weights
+// least often and keep the matrix cores busiest, but need two tiles for each CU
+// (65,536 rows, forward with the output layer: 107 us in 128-row tiles); fewer
+// rows are cut into smaller tiles so that every CU has one.
+template <class F>
+void with_tile(long M, F f) {
+  if (M >= 128 * 512) f(std::integral_constant<int, 128>());
+  else if (M >= 64 * 256) f(std::integral_constant<int, 64>());
+  else f(std::integral_constant<int, 32>());
+}
+constexpr int chain_depth(int TR) { return TR >= 64 ? 2 : 4; }
+
+Chain chain_of(const fvs_mlp &m, long M, u16 *const *W) {
+  Chain c{};
+  c.L = m.L;
+  c.M = M;
+  for (int l = 0; l < m.L; ++l) {
+    c.W[l] = W[l];
+    c.bias[l] = m.w + m.tab.offb[l];
+    c.Z[l] = m.Z[l];
+    c.H[l] = m.H[l];
+  }
+  c.X0 = m.X0;
+  c.Wh = m.w + m.tab.offW[m.L];
+  c.bh = m.w + m.tab.offb[m.L];
+  c.T = m.T;
+  c.Y = m.Y;
+  return c;
+}
+
+template <bool TRAIN>
+void launch_forward(fvs_mlp &m, int M, const Rows &R) {
+  Prof pf(m, MC_FWD);
+  const Chain c = chain_of(m, M, m.tab.Wt);
+  with_tile(M, [&](auto tr) {
+    constexpr int TR = decltype(tr)::value;
+    hipLaunchKernelGGL((k_forward<TR, chain_depth(TR), TRAIN>), dim3((M + TR - 1) / TR), dim3(256), 0, m.stream, c, R);
+  });
+}
+
+// network output of M rows into Y
+int predict_pass(fvs_mlp &m, int M, const Rows &R) {
+  launch_forward<false>(m, M, R);
+  MLPC(hipGetLastError());
+  return 0;
+}
+
+// forward and backward over M rows: loss and weight-gradient partials
+int train_pass(fvs_mlp &m, int M, const Rows &R) {
   const int S = nsplit(M), chunk = M / S;
   const int L = m.L;
-  for (int l = 0; l < L; ++l) {
-    Prof pf(m, MC_FWD);
-    const u16 *A = (l == 0) ? m.X0 : m.H[l - 1];
-    if (M % kBigRows == 0)
-      hipLaunchKernelGGL(k_gemm_nt_big<0>, dim3(M / kBigRows), dim3(kBigThreads), 0, m.stream, m.tab.inpad[l], A,
-                         m.tab.Wt[l], m.w + m.tab.offb[l], nullptr, m.Z[l], m.H[l]);
-    else
-      hipLaunchKernelGGL(k_gemm_nt<0>, dim3(M / kRows), dim3(256), 0, m.stream, m.tab.inpad[l], A, m.tab.Wt[l],
-                         m.w + m.tab.offb[l], nullptr, m.Z[l], m.H[l]);
-  }
+  launch_forward<true>(m, M, R);
   {
     Prof pf(m, MC_HEAD);
-    const float inv_no = 1.0f / float(double(nvalid) * kOut);
-    hipLaunchKernelGGL(k_head, dim3((M + kHeadRows - 1) / kHeadRows), dim3(256), 0, m.stream, long(M), nvalid, inv_no,
-                       m.H[L - 1], m.Z[L - 1],
-                       m.w + m.tab.offW[L], m.w + m.tab.offb[L], m.T, Y, grad ? m.dZa : nullptr, m.Gh, m.lossp);
+    const float inv_no = 1.0f / float(double(R.nvalid) * kOut);
+    hipLaunchKernelGGL(k_head, dim3((M + kHeadRows - 1) / kHeadRows), dim3(256), 0, m.stream, long(M), R.nvalid,
+                       inv_no, m.H[L - 1], m.Z[L - 1], m.w + m.tab.offW[L], m.w + m.tab.offb[L], m.T, m.Gh, m.lossp);
   }
-  if (grad) {
-    u16 *cur = m.dZa, *oth = m.dZb;
-    for (int l = L - 1; l >= 0; --l) {
-      {
-        Prof pf(m, MC_WGRAD);
-        const u16 *A = (l == 0) ? m.X0 : m.H[l - 1];
-        const int K = m.tab.inpad[l];
-        if (chunk % (kTnGroups * kBK) == 0)
-          hipLaunchKernelGGL(k_gemm_tn_g, dim3((K / kRows) * S), dim3(256 * kTnGroups), 0, m.stream, K,
-                             m.tab.in[l], chunk, A, cur, m.G, m.P, m.tab.offW[l], m.tab.offb[l]);
-        else
-          hipLaunchKernelGGL(k_gemm_tn, dim3((K / kRows) * S), dim3(256), 0, m.stream, K, m.tab.in[l], chunk, A,
-                             cur, m.G, m.P, m.tab.offW[l], m.tab.offb[l]);
-      }
-      if (l > 0) {
-        Prof pf(m, MC_BWD);
-        if (M % kBigRows == 0)
-          hipLaunchKernelGGL(k_gemm_nt_big<1>, dim3(M / kBigRows), dim3(kBigThreads), 0, m.stream, kW, cur,
-                             m.tab.Wk[l], nullptr, m.Z[l - 1], oth, nullptr);
-        else
-          hipLaunchKernelGGL(k_gemm_nt<1>, dim3(M / kRows), dim3(256), 0, m.stream, kW, cur, m.tab.Wk[l], nullptr,
-                             m.Z[l - 1], oth, nullptr);
-        std::swap(cur, oth);
-      }
-    }
+  if (L > 1) {
+    Prof pf(m, MC_BWD);
+    const Chain c = chain_of(m, M, m.tab.Wk);
+    with_tile(M, [&](auto tr) {
+      constexpr int TR = decltype(tr)::value;
+      hipLaunchKernelGGL((k_backward<TR, chain_depth(TR)>), dim3((M + TR - 1) / TR), dim3(256), 0, m.stream, c);
+    });
+  }
+  for (int l = L - 1; l >= 0; --l) {
+    Prof pf(m, MC_WGRAD);
+    const u16 *A = (l == 0) ? m.X0 : m.H[l - 1];
+    const int K = m.tab.inpad[l];
+    if (chunk % (kTnGroups * kBK) == 0)
+      hipLaunchKernelGGL(k_gemm_tn_g, dim3((K / kRows) * S), dim3(256 * kTnGroups), 0, m.stream, K, m.tab.in[l], chunk,
+                         A, m.Z[l], m.G, m.P, m.tab.offW[l], m.tab.offb[l]);
+    else
+      hipLaunchKernelGGL(k_gemm_tn, dim3((K / kRows) * S), dim3(256), 0, m.stream, K, m.tab.in[l], chunk, A, m.Z[l],
+                         m.G, m.P, m.tab.offW[l], m.tab.offb[l]);
   }
   MLPC(hipGetLastError());
   return 0;
@@ -886,13 +990,6 @@ int stage_rows(fvs_mlp &m, int n, const float *raw, const float *target) {
   if (target)
     MLPC(hipMemcpyAsync(m.itgt, target, size_t(n) * kOut * sizeof(float), hipMemcpyHostToDevice, m.stream));
   return 0;
-}
-
-void launch_features(fvs_mlp &m, int M, long nvalid, const float *raw, const float *tgt, long ndata, long step,
-                     int sample, float *F32) {
-  Prof pf(m, MC_FEAT);
-  hipLaunchKernelGGL(k_features, dim3(unsigned((long(M) * 16 + 255) / 256)), dim3(256), 0, m.stream, M, nvalid, raw,
-                     tgt, ndata, m.opt.seed, step, sample, m.X0, tgt ? m.T : nullptr, F32);
 }
 
 int round64(long n) { return int((n + kRows - 1) / kRows * kRows); }
@@ -944,8 +1041,6 @@ int fvs_mlp_create(fvs_mlp **out, const fvs_mlp_options *opt) try {
   rc = rc ? rc : m->alloc(m->lossp, (M + kHeadRows - 1) / kHeadRows);
   rc = rc ? rc : m->alloc(m->lossh, 1);
   rc = rc ? rc : m->alloc(m->X0, M * kInPad);
-  rc = rc ? rc : m->alloc(m->dZa, M * kW);
-  rc = rc ? rc : m->alloc(m->dZb, M * kW);
   for (int l = 0; l < m->L && !rc; ++l) {
     rc = m->alloc(m->Z[l], M * kW);
     rc = rc ? rc : m->alloc(m->H[l], M * kW);
@@ -962,7 +1057,9 @@ int fvs_mlp_create(fvs_mlp **out, const fvs_mlp_options *opt) try {
   if (rc) return rc;
   tb.Wt[m->L] = tb.Wk[m->L] = nullptr;
   tb.Wk[0] = nullptr;
-  if (hipMemsetAsync(tb.Wt[0], 0, size_t(kW) * kInPad * sizeof(u16), m->stream) != hipSuccess)
+  // padding: input rows of the packed weights, columns of X0
+  if (hipMemsetAsync(tb.Wt[0], 0, size_t(kW) * kInPad * sizeof(u16), m->stream) != hipSuccess ||
+      hipMemsetAsync(m->X0, 0, M * kInPad * sizeof(u16), m->stream) != hipSuccess)
     return fail(FVS_EHIP, "memset");
   // Glorot-uniform weights from the seed, zero biases
   std::vector<float> w(m->P, 0.f);
@@ -1018,7 +1115,7 @@ int fvs_mlp_features(fvs_mlp *m, int n, const float *raw, float *feat) try {
   if (n < 0 || n > m->M) return fail(FVS_EINVAL, "n must be 0..batch");
   if (n == 0) return 0;
   if (int rc = stage_rows(*m, n, raw, nullptr)) return rc;
-  launch_features(*m, round64(n), n, m->iraw, nullptr, 0, 0, 0, m->F32);
+  hipLaunchKernelGGL(k_features, dim3((n + 255) / 256, kFeatChunks), dim3(256), 0, m->stream, n, m->iraw, m->F32);
   MLPC(hipGetLastError());
   MLPC(hipMemcpyAsync(feat, m->F32, size_t(n) * kFeat * sizeof(float), hipMemcpyDeviceToHost, m->stream));
   MLPC(hipStreamSynchronize(m->stream));
@@ -1060,8 +1157,7 @@ int fvs_mlp_train(fvs_mlp *m, int steps, double *loss) try {
   int rc = 0;
   if (hipEventRecord(m->ev0, m->stream) != hipSuccess) rc = fail(FVS_EHIP, "event");
   for (int s = 0; s < steps && !rc; ++s) {
-    launch_features(*m, m->M, m->M, m->raw, m->tgt, m->ndata, m->t + 1, 1, nullptr);
-    rc = run_pass(*m, m->M, m->M, true, nullptr);
+    rc = train_pass(*m, m->M, {m->raw, m->tgt, m->M, m->ndata, m->opt.seed, m->t + 1});
     if (!rc) rc = launch_adam(*m, 2, S, (m->M + kHeadRows - 1) / kHeadRows, inv_no, dl + s, nullptr);
   }
   if (!rc) {
@@ -1085,8 +1181,7 @@ static int grad_or_step(fvs_mlp *m, int n, const float *raw, const float *target
   const int M = round64(n);
   const int S = nsplit(M);
   if (int rc = stage_rows(*m, n, raw, target)) return rc;
-  launch_features(*m, M, n, m->iraw, m->itgt, 0, 0, 0, nullptr);
-  if (int rc = run_pass(*m, M, n, true, nullptr)) return rc;
+  if (int rc = train_pass(*m, M, {m->iraw, m->itgt, n, 0, 0, 0})) return rc;
   if (int rc = launch_adam(*m, update ? 2 : 1, S, (M + kHeadRows - 1) / kHeadRows, 1.0 / (double(n) * kOut), m->lossh,
                            update ? nullptr : m->gtmp))
     return rc;
@@ -1117,8 +1212,7 @@ int fvs_mlp_predict(fvs_mlp *m, long long n, const float *raw, float *out) try {
     const int nb = int(std::min<long long>(m->M, n - b));
     const int M = round64(nb);
     if (int rc = stage_rows(*m, nb, raw + b * kRaw, nullptr)) return rc;
-    launch_features(*m, M, nb, m->iraw, nullptr, 0, 0, 0, nullptr);
-    if (int rc = run_pass(*m, M, nb, false, m->Y)) return rc;
+    if (int rc = predict_pass(*m, M, {m->iraw, nullptr, nb, 0, 0, 0})) return rc;
     MLPC(hipMemcpyAsync(out + b * kOut, m->Y, size_t(nb) * kOut * sizeof(float), hipMemcpyDeviceToHost, m->stream));
     MLPC(hipStreamSynchronize(m->stream));
   }
@@ -1131,7 +1225,7 @@ int fvs_mlp_kernel_times(fvs_mlp *m, int steps, double *ms6, double *flop6, int 
   if (!m || !ms6 || !flop6 || !launches6) return fail(FVS_EINVAL, "null argument");
   if (!m->raw) return fail(FVS_ESTATE, "no training set (fvs_mlp_set_data)");
   if (steps < 1) return fail(FVS_EINVAL, "steps must be positive");
-  const int per_step = 2 * (1 + m->L + 1 + m->L + (m->L - 1) + 1);
+  const int per_step = 2 * (1 + 1 + m->L + 1 + 1);
   const int need = per_step * steps;
   while (int(m->evpool.size()) < need) {
     hipEvent_t e;
@@ -1151,7 +1245,7 @@ int fvs_mlp_kernel_times(fvs_mlp *m, int steps, double *ms6, double *flop6, int 
     ms[m->evclass[k]] += t;
     cnt[m->evclass[k]] += 1;
   }
-  // matrix-core flops per launch (2 per multiply-add), averaged over layers
+  // matrix-core flops per launch (2 per multiply-add; the weight gradient averaged over its layers)
   const double M = m->M;
   double fl[MC_N] = {0};
   double fwd = 0, wg = 0;
@@ -1159,9 +1253,9 @@ int fvs_mlp_kernel_times(fvs_mlp *m, int steps, double *ms6, double *flop6, int 
     fwd += 2.0 * M * m->tab.inpad[l] * kW;
     wg += 2.0 * M * m->tab.inpad[l] * kW;
   }
-  fl[MC_FWD] = fwd / m->L;
+  fl[MC_FWD] = fwd;
   fl[MC_WGRAD] = wg / m->L;
-  fl[MC_BWD] = 2.0 * M * kW * kW;
+  fl[MC_BWD] = 2.0 * M * kW * kW * (m->L - 1);
   fl[MC_HEAD] = 2.0 * M * kW * kOut * 3.0;
   for (int k = 0; k < MC_N; ++k) {
     ms6[k] = cnt[k] ? ms[k] / cnt[k] : 0.0;

@@ -1,0 +1,47 @@
+"""The all-layers forward and backward kernels at the edges of their row tiles
+(32, 64 and 128 rows), against the CPU oracle.
+
+Prediction: the oracle's bfloat16 form rounds the same activations, so a value
+differs by single flipped roundings (2^-9 of an activation) that travel on;
+1e-2 of the largest output, as in the parity tests.  The gradient of every row
+count: relative L2 error 2e-2 (the same reasoning, per whole gradient)."""
+import numpy as np
+import pytest
+
+from fvs2d_amd.mlp import WarmStartNet
+from oracle import mlp_oracle as mo
+
+pytestmark = pytest.mark.gpu
+
+
+def _data(n, seed):
+    rng = np.random.default_rng(seed)
+    raw = np.stack([rng.uniform(-20, 20, n), rng.uniform(-20, 20, n), rng.uniform(0, 20, n),
+                    rng.uniform(0.5, 0.85, n), rng.uniform(-2, 4, n), rng.uniform(0.1, 0.15, n)], 1)
+    return raw.astype(np.float32), rng.normal(0, 0.3, (n, 4)).astype(np.float32)
+
+
+def _rows(raw):
+    return mo.features(raw.astype(np.float64)).astype(np.float32).astype(np.float64)
+
+
+# tiles of 32, 64 (from 16,384 rows) and 128 (from 65,536), whole and ragged
+@pytest.mark.parametrize("depth,n", [(1, 1), (3, 31), (8, 97), (2, 16384), (2, 16449), (1, 65536), (2, 65601)])
+def test_predict_at_tile_edges(depth, n):
+    net = WarmStartNet(depth=depth, batch=66048, seed=depth)
+    raw, _ = _data(n, n)
+    y = net.predict(raw)
+    rows = np.unique(np.concatenate([np.arange(min(n, 200)), np.arange(max(0, n - 200), n)]))
+    ref, _ = mo.forward(net.get_params().astype(np.float64), _rows(raw[rows]), depth, bf16_mode=True)
+    assert np.max(np.abs(y[rows] - ref)) <= 1e-2 * np.max(np.abs(ref))
+
+
+@pytest.mark.parametrize("depth,n", [(1, 1), (2, 65), (3, 4097), (2, 16449)])
+def test_gradient_at_tile_edges(depth, n):
+    net = WarmStartNet(depth=depth, batch=16512, seed=depth)
+    raw, tgt = _data(n, n)
+    loss, g = net.grad(raw, tgt)
+    ref_loss, ref = mo.loss_and_grad(net.get_params().astype(np.float64), _rows(raw), tgt.astype(np.float64), depth,
+                                     bf16_mode=True)
+    assert abs(loss - ref_loss) <= 1e-3 * ref_loss
+    assert np.linalg.norm(g - ref) <= 2e-2 * np.linalg.norm(ref)
