@@ -2,14 +2,14 @@
 //
 // Training step for a batch of M rows (M a multiple of 64), depth L hidden
 // layers of width 256:
-//   k_forward        cell records -> bfloat16 input rows X0[M][128] (68 used),
+//   k_forward        cell records -> bfloat16 input rows X0[M][96] (68 used),
 //                    then for every hidden layer Z = X W + b, H = GELU(Z),
 //                    the activations of a row tile staying in LDS
 //   k_head           y = H W + b (float32), loss, dy, dZ of the last hidden
 //                    layer, output-layer weight/bias gradient partials
 //   k_backward       dZ_prev = (dZ W^T) * GELU'(Z_prev) down to the first
 //                    hidden layer, dZ of a row tile staying in LDS
-//   k_gemm_tn        weight-gradient partials X^T dZ (and bias partials)
+//   k_wgrad          weight-gradient partials X^T dZ (and bias partials)
 //   k_adam           sums the partials in a fixed order, Adam update, and
 //                    refreshes the bfloat16 copies of the weights
 // Prediction is one k_forward launch with the output layer in it.
@@ -47,13 +47,13 @@ constexpr int kW = FVS_MLP_WIDTH;
 constexpr int kOut = FVS_MLP_OUT;
 constexpr int kFeat = FVS_MLP_FEATURES;
 constexpr int kRaw = FVS_MLP_RAW;
-constexpr int kInPad = 128;
 constexpr int kMaxDepth = 8;
 constexpr int kMaxLayers = kMaxDepth + 1;
 constexpr int kMaxSplit = 64;
 constexpr int kBK = 32;        // reduction depth of one MFMA
-constexpr int kLds = kBK + 8;  // padded LDS row (elements)
-constexpr int kRows = 64;      // GEMM rows per workgroup
+constexpr int kSlabs0 = (kFeat + kBK - 1) / kBK;  // slabs of the input layer
+constexpr int kIn = kBK * kSlabs0;                // its columns, padded
+constexpr int kRows = 64;      // batch rows come in multiples of this
 
 static_assert(kW == 256, "the GEMM tiling assumes width 256");
 
@@ -176,28 +176,6 @@ __global__ __launch_bounds__(256) void k_features(int n, const float *__restrict
     if (8 * q + c < kFeat) F32[long(m) * kFeat + 8 * q + c] = f[c];
 }
 
-// ------------------------------------------------------------- GEMM core
-// One kBK slab of C[m][n] += sum_k A[m][k] B[n][k] with A_lds rows 16i..
-// (4 blocks) and B_lds rows 64w + 16j.. (4 blocks).  Fragment layout of
-// v_mfma_f32_16x16x32_bf16 for lane l: first operand row l%16, k
-// 8(l/16)..+7; second operand column l%16, same k; result rows
-// 4(l/16)..+3, column l%16.  The B fragment goes first, so the result is
-// C transposed: lane l holds C[16i + l%16][64w + 16j + 4(l/16) + e], four
-// consecutive columns, stored as one 8- or 16-byte vector.
-__device__ __forceinline__ void mma_slab(const u16 *__restrict__ As, const u16 *__restrict__ Bs, int lane, int w,
-                                         f32x4 (&acc)[4][4]) {
-  bf16x8 a[4], b[4];
-  const int r = lane & 15, kq = 8 * (lane >> 4);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) a[i] = *reinterpret_cast<const bf16x8 *>(As + (16 * i + r) * kLds + kq);
-#pragma unroll
-  for (int j = 0; j < 4; ++j) b[j] = *reinterpret_cast<const bf16x8 *>(Bs + (64 * w + 16 * j + r) * kLds + kq);
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[i], acc[i][j], 0, 0, 0);
-}
-
 __device__ __forceinline__ unsigned pack2(float a, float b) {
   typedef float f32x2 __attribute__((ext_vector_type(2)));
   typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -215,7 +193,6 @@ __device__ __forceinline__ unsigned pack2(float a, float b) {
 // from L2 to registers without LDS, in the order the MFMA operand wants them
 // (pack_at): one contiguous KB per load.
 constexpr int kActLd = kW + 8;  // LDS row (elements): 16-byte accesses of 16 rows meet distinct banks
-constexpr int kSlabs0 = (kFeat + kBK - 1) / kBK;  // slabs of the input layer that are not padding
 
 // Element of the packed copy of B[n][k]: per slab of 32 k and 64 columns of a
 // wavefront four operand blocks of 16 columns x 32 k.  Row t of block j is
@@ -277,6 +254,22 @@ __device__ __forceinline__ long row_source(const Rows &R, long m) {
   return m < R.nvalid ? m : -1;
 }
 
+// dW = A^T D reduces over the rows of the batch, so its operands want eight
+// rows of one column in a lane.  The forward and backward kernels write them
+// that way from LDS (pack_rows): per 32 rows and 16 columns one KB, lane by
+// lane, 16 bytes each; nothing is transposed here.
+__device__ __forceinline__ void pack_rows(const u16 *__restrict__ act, int rows, int cblocks, u16 *__restrict__ out,
+                                          int lane, int wv) {
+  const u16 *src = act + 8 * (lane >> 4) * kActLd + (lane & 15);
+  for (int q = wv; q < rows / kBK * cblocks; q += 4) {
+    const u16 *p = src + (q / cblocks) * kBK * kActLd + 16 * (q % cblocks);
+    unsigned v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = unsigned(p[2 * e * kActLd]) | unsigned(p[(2 * e + 1) * kActLd]) << 16;
+    *reinterpret_cast<uint4 *>(out + (long(q) * 64 + lane) * 8) = make_uint4(v[0], v[1], v[2], v[3]);
+  }
+}
+
 struct Chain {
   int L;
   long M;
@@ -291,7 +284,8 @@ struct Chain {
 constexpr int chain_waves(int TR) { return TR >= 128 ? 2 : 3; }
 
 // Features and all hidden layers of TR rows.  TRAIN: X0, Z, H and the targets
-// go to HBM; otherwise only the network's output does.
+// go to HBM (X0 and H in the weight gradient's order, the last H by rows for
+// k_head); otherwise only the network's output does.
 template <int TR, int D, bool TRAIN>
 __global__ __launch_bounds__(256, chain_waves(TR)) void k_forward(Chain c, Rows R) {
   __shared__ __attribute__((aligned(16))) u16 act[TR * kActLd];
@@ -332,14 +326,8 @@ __global__ __launch_bounds__(256, chain_waves(TR)) void k_forward(Chain c, Rows 
           src >= 0 ? *reinterpret_cast<const float4 *>(R.tgt + src * kOut) : make_float4(0.f, 0.f, 0.f, 0.f);
   }
   __syncthreads();
-  if (TRAIN) {
-    for (int e = tid; e < TR * (4 * kSlabs0); e += 256) {
-      const int row = e / (4 * kSlabs0), q = e % (4 * kSlabs0);
-      if (r0 + row < c.M)
-        *reinterpret_cast<uint4 *>(c.X0 + (r0 + row) * kInPad + 8 * q) =
-            *reinterpret_cast<const uint4 *>(act + row * kActLd + 8 * q);
-    }
-  }
+  const int rows = int(c.M - r0 < TR ? c.M - r0 : TR);
+  if (TRAIN) pack_rows(act, rows, 2 * kSlabs0, c.X0 + r0 * kIn, lane, wv);
   f32x4 acc[TR / 16][4];
   for (int l = 0; l < c.L; ++l) {
     chain_layer<TR, D>(act, c.W[l] + lp, l == 0 ? kSlabs0 : kW / kBK, lane, b, acc);
@@ -368,11 +356,12 @@ __global__ __launch_bounds__(256, chain_waves(TR)) void k_forward(Chain c, Rows 
           const long idx = (r0 + row) * kW + n0 + 32 * h;
           *reinterpret_cast<uint4 *>(c.Z[l] + idx) =
               make_uint4(pack2(z[0], z[1]), pack2(z[2], z[3]), pack2(z[4], z[5]), pack2(z[6], z[7]));
-          *reinterpret_cast<uint4 *>(c.H[l] + idx) = hv;
+          if (l + 1 == c.L) *reinterpret_cast<uint4 *>(c.H[l] + idx) = hv;
         }
       }
     }
     __syncthreads();
+    if (TRAIN && l + 1 < c.L) pack_rows(act, rows, kW / 16, c.H[l] + r0 * kW, lane, wv);
   }
   if (!TRAIN) {
     // the output layer, 32 lanes per row as in k_head
@@ -402,7 +391,8 @@ __global__ __launch_bounds__(256, chain_waves(TR)) void k_forward(Chain c, Rows 
 }
 
 // dZ of the hidden layers below the last, each in the place of its layer's Z
-// (c.W: the backward operands; Z of the last layer holds its dZ)
+// (c.W: the backward operands; Z of the last layer holds its dZ by rows), all of
+// them left in the weight gradient's order
 template <int TR, int D>
 __global__ __launch_bounds__(256, chain_waves(TR)) void k_backward(Chain c) {
   __shared__ __attribute__((aligned(16))) u16 act[TR * kActLd];
@@ -410,8 +400,9 @@ __global__ __launch_bounds__(256, chain_waves(TR)) void k_backward(Chain c) {
   const long r0 = long(blockIdx.x) * TR;
   const int lp = (wv * 4 * 64 + lane) * 8;
   bf16x8 b[D][4];
+  if (c.L > 1)
 #pragma unroll
-  for (int u = 0; u < D; ++u) load_slab<TR, D>(c.W[c.L - 1] + lp, u, b[u]);
+    for (int u = 0; u < D; ++u) load_slab<TR, D>(c.W[c.L - 1] + lp, u, b[u]);
   const u16 *top = c.Z[c.L - 1];
   for (int e = tid; e < TR * (kW / 8); e += 256) {
     const int row = e / (kW / 8), q = e % (kW / 8);
@@ -419,6 +410,8 @@ __global__ __launch_bounds__(256, chain_waves(TR)) void k_backward(Chain c) {
         r0 + row < c.M ? *reinterpret_cast<const uint4 *>(top + (r0 + row) * kW + 8 * q) : make_uint4(0, 0, 0, 0);
   }
   __syncthreads();
+  const int rows = int(c.M - r0 < TR ? c.M - r0 : TR);
+  pack_rows(act, rows, kW / 16, c.Z[c.L - 1] + r0 * kW, lane, wv);
   f32x4 acc[TR / 16][4];
   for (int l = c.L - 1; l > 0; --l) {
     chain_layer<TR, D>(act, c.W[l] + lp, kW / kBK, lane, b, acc);
@@ -435,228 +428,164 @@ __global__ __launch_bounds__(256, chain_waves(TR)) void k_backward(Chain c) {
       for (int h = 0; h < 2; ++h) {
         uint4 dv = make_uint4(0, 0, 0, 0);
         if (r0 + 16 * i < c.M) {
-          u16 *zp = c.Z[l - 1] + (r0 + row) * kW + n0 + 32 * h;
-          const uint4 zv = *reinterpret_cast<const uint4 *>(zp);
+          const uint4 zv = *reinterpret_cast<const uint4 *>(c.Z[l - 1] + (r0 + row) * kW + n0 + 32 * h);
           const unsigned zw[4] = {zv.x, zv.y, zv.z, zv.w};
           float d[8];
 #pragma unroll
           for (int e = 0; e < 8; ++e)
             d[e] = acc[i][2 * h + (e >> 2)][e & 3] * gelu_grad(bf2f(u16((zw[e >> 1] >> (16 * (e & 1))) & 0xffffu)));
           dv = make_uint4(pack2(d[0], d[1]), pack2(d[2], d[3]), pack2(d[4], d[5]), pack2(d[6], d[7]));
-          *reinterpret_cast<uint4 *>(zp) = dv;
         }
         *reinterpret_cast<uint4 *>(act + row * kActLd + n0 + 32 * h) = dv;
       }
     }
-    __syncthreads();
+    __syncthreads();  // all of Z is read, all of dZ in LDS
+    pack_rows(act, rows, kW / 16, c.Z[l - 1] + r0 * kW, lane, wv);
   }
 }
 
-// move rows (2mp, 2mp+1) x 8 columns, held as v0/v1, into a transposed LDS
-// tile T[col][m] as 32-bit pairs
-__device__ __forceinline__ void put_pairs(u16 *__restrict__ T, int col0, int mp, uint4 v0, uint4 v1) {
-  const unsigned a0[4] = {v0.x, v0.y, v0.z, v0.w}, a1[4] = {v1.x, v1.y, v1.z, v1.w};
-#pragma unroll
-  for (int c = 0; c < 8; ++c) {
-    const unsigned lo = (a0[c >> 1] >> (16 * (c & 1))) & 0xffffu, hi = (a1[c >> 1] >> (16 * (c & 1))) & 0xffffu;
-    *reinterpret_cast<unsigned *>(T + (col0 + c) * kLds + 2 * mp) = lo | (hi << 16);
-  }
-}
+// ------------------------------------------------------------ weight gradient
+// Row slices whose partials are kept apart (added by k_adam in their order): S
+// slices of cs slabs of 32 rows; a slice's slabs are summed in ng interleaved
+// groups, ((g0 + g1) + g2) + g3 with ng = 4.
+struct WGrad {
+  int L, S, cs, ng;
+  const u16 *A[kMaxDepth], *D[kMaxDepth];
+  long offW[kMaxDepth], offb[kMaxDepth], P;
+  float *G;
+};
+constexpr int kWgThreads = 512;
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(1))) const u32x4 *GlobalIn;
 
-// Workgroup -> (k-tile, row slice) of the weight-gradient kernels.  Workgroups
-// go to the eight XCDs round-robin by index; the nkt k-tiles of one slice read
-// the same D rows, so they are given indices eight apart (one XCD, whose L2
-// then serves D to all of them) and dispatched close together.  Needs the
-// slice count to be a multiple of 8, else the plain order is used.
-__device__ __forceinline__ void tn_tile(int nkt, int nsplit, int &kt, int &s) {
-  const int b = int(blockIdx.x);
-  if (nsplit % 8 == 0) {
-    const int r = b & 7, q = b >> 3;
-    kt = q % nkt;
-    s = (q / nkt) * 8 + r;
-  } else {
-    kt = b % nkt;
-    s = b / nkt;
-  }
-}
-
-// Weight-gradient partials: for k-tile kt (64 rows of dW) and row slice s,
-// dW[k][n] = sum over m in slice of A[m][k] * D[m][n], A[M][K], D[M][256].
-// Both operands are transposed into LDS (m contiguous); a thread moves two
-// rows' worth of 8 columns and writes 32-bit pairs; the next slab's global
-// data is loaded into registers while the current one is multiplied.
-// Workgroups of k-tile 0 also sum D's columns (the bias gradient).  Output
-// rows k >= Kreal (input padding) are not written.
-__global__ __launch_bounds__(256) void k_gemm_tn(int K, int Kreal, int chunk, const u16 *__restrict__ A,
-                                                 const u16 *__restrict__ D, float *__restrict__ G, long P,
-                                                 long offW, long offb) {
-  __shared__ __attribute__((aligned(16))) u16 As[kRows * kLds];
-  __shared__ __attribute__((aligned(16))) u16 Bs[kW * kLds];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int nkt = K / kRows;
-  int kt, s;
-  tn_tile(nkt, int(gridDim.x) / nkt, kt, s);
-  const long m0 = long(s) * chunk;
-  const int kb = kt * kRows;
-  f32x4 acc[4][4];
+// Partials of dW[k][n] for 16 NB inputs k, all 256 columns n and the slabs of a
+// slice, group after group.  A slab is 16 (NB + 16) KB of packed operands, read
+// into two LDS buffers (every fragment is a contiguous KB) with two more slabs
+// in registers on their way: the matrix cores need a quarter of the time that
+// these bytes take from HBM.  Wavefront (wk, wn) holds 8 NB x 64 results of the
+// group and as many of the groups before.  With Gb the first 256 threads also
+// sum a column of D each (the bias gradient).  All layers of 65,536 rows: 94 us;
+// as a launch per layer that transposed row-major operands into LDS, 64 inputs a
+// workgroup, 185 us.
+template <int NB>
+__device__ __forceinline__ void wgrad_tile(const u16 *A, int astride, const u16 *D, int s0, int cs, int ng, int Kreal,
+                                           float *__restrict__ GW, float *__restrict__ Gb, u16 *__restrict__ lds) {
+  constexpr int NI = NB / 2, kSlab = (NB + 16) * 512;
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), wk = wv >> 2, wn = wv & 3;
+  const bool own_a = tid < 64 * NB;  // A's 16-byte pieces of a slab; D's are two per thread
+  const GlobalIn Ap = (GlobalIn)A + (own_a ? tid : 0), Dp = (GlobalIn)D + tid;
+  int at = s0, g = 0;  // the next slab to load (past the end: the last one again)
+  auto load = [&](u32x4 &a, u32x4 &d0, u32x4 &d1) __attribute__((always_inline)) {
+    a = Ap[long(at) * astride];
+    d0 = Dp[long(at) * 1024];
+    d1 = Dp[long(at) * 1024 + 512];
+    if (at + ng < s0 + cs) at += ng;
+    else if (g + 1 < ng) at = s0 + ++g;
+  };
+  auto store = [&](int buf, u32x4 a, u32x4 d0, u32x4 d1) __attribute__((always_inline)) {
+    u32x4 *p = reinterpret_cast<u32x4 *>(lds + buf * kSlab) + tid;
+    if (own_a) p[0] = a;
+    p[64 * NB] = d0;
+    p[64 * NB + 512] = d1;
+  };
+  f32x4 acc[NI][4], sum[NI][4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < NI; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float db = 0.f;
-  const int amp = tid & 15, akg = tid >> 4;  // A: threads < 128, rows 2amp, 2amp+1, columns 8akg..
-  const u16 *Ap = A + (m0 + 2 * amp) * K + kb + 8 * akg;
-  const int bmp0 = tid & 15, bng0 = tid >> 4, bng1 = (tid + 256) >> 4;  // D: two chunks per thread
-  const u16 *Dp0 = D + (m0 + 2 * bmp0) * kW + 8 * bng0;
-  const u16 *Dp1 = D + (m0 + 2 * bmp0) * kW + 8 * bng1;
-  uint4 ra0{}, ra1{}, rb00, rb01, rb10, rb11;
-  if (tid < 128) {
-    ra0 = *reinterpret_cast<const uint4 *>(Ap);
-    ra1 = *reinterpret_cast<const uint4 *>(Ap + K);
-  }
-  rb00 = *reinterpret_cast<const uint4 *>(Dp0);
-  rb01 = *reinterpret_cast<const uint4 *>(Dp0 + kW);
-  rb10 = *reinterpret_cast<const uint4 *>(Dp1);
-  rb11 = *reinterpret_cast<const uint4 *>(Dp1 + kW);
-  for (int mm = 0; mm < chunk; mm += kBK) {
-    if (tid < 128) put_pairs(As, 8 * akg, amp, ra0, ra1);
-    put_pairs(Bs, 8 * bng0, bmp0, rb00, rb01);
-    put_pairs(Bs, 8 * bng1, bmp0, rb10, rb11);
-    __syncthreads();
-    if (mm + kBK < chunk) {
-      const long o = long(mm + kBK);
-      if (tid < 128) {
-        ra0 = *reinterpret_cast<const uint4 *>(Ap + o * K);
-        ra1 = *reinterpret_cast<const uint4 *>(Ap + (o + 1) * K);
+    for (int j = 0; j < 4; ++j) acc[i][j] = sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float db = 0.f, dbs = 0.f;
+  const int per = cs / ng;
+  int left = per;  // slabs of the group still to add
+  auto multiply = [&](const u16 *buf) __attribute__((always_inline)) {
+    const u16 *As = buf + wk * NI * 512 + lane * 8, *Ds = buf + (NB + 4 * wn) * 512 + lane * 8;
+    bf16x8 b[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) b[j] = *reinterpret_cast<const bf16x8 *>(Ds + j * 512);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const bf16x8 a = *reinterpret_cast<const bf16x8 *>(As + i * 512);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a, acc[i][j], 0, 0, 0);
+    }
+    if (Gb && tid < kW) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint4 v = *reinterpret_cast<const uint4 *>(buf + (NB + (tid >> 4)) * 512 + ((tid & 15) + 16 * q) * 8);
+        const unsigned w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) db += bf2f(u16((w[e >> 1] >> (16 * (e & 1))) & 0xffffu));
       }
-      rb00 = *reinterpret_cast<const uint4 *>(Dp0 + o * kW);
-      rb01 = *reinterpret_cast<const uint4 *>(Dp0 + (o + 1) * kW);
-      rb10 = *reinterpret_cast<const uint4 *>(Dp1 + o * kW);
-      rb11 = *reinterpret_cast<const uint4 *>(Dp1 + (o + 1) * kW);
     }
-    if (kt == 0) {
-      const u16 *row = Bs + tid * kLds;
-      for (int c = 0; c < kBK; ++c) db += bf2f(row[c]);
-    }
-    mma_slab(As, Bs, lane, w, acc);
-    __syncthreads();
-  }
-  float *Gs = G + long(s) * P;
+    if (--left == 0) {
+      left = per;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int k = kb + 16 * i + (lane & 15);
-    if (k >= Kreal) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n0 = 64 * w + 16 * j + 4 * (lane >> 4);
-      *reinterpret_cast<float4 *>(Gs + offW + long(k) * kW + n0) =
-          make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
-    }
-  }
-  if (kt == 0) Gs[offb + tid] = db;
-}
-
-// The same weight-gradient partials with four wave groups per workgroup
-// (1024 threads): group g multiplies slabs g, g + 4, g + 8, ... of the row
-// slice into its own accumulators and LDS buffers, so a CU keeps 16
-// wavefronts in flight instead of 4; the groups' sums are then added into
-// group 0's in group order (((g0 + g1) + g2) + g3), through LDS, one row
-// block at a time.  Needs chunk to be a multiple of 4 kBK.
-constexpr int kTnGroups = 4;
-constexpr int kTnBuf = (kRows + kW) * kLds;  // one group's A and D slabs (elements)
-__global__ __launch_bounds__(256 * kTnGroups) void k_gemm_tn_g(int K, int Kreal, int chunk, const u16 *__restrict__ A,
-                                                               const u16 *__restrict__ D, float *__restrict__ G,
-                                                               long P, long offW, long offb) {
-  __shared__ __attribute__((aligned(16))) u16 smem[kTnGroups * kTnBuf];
-  const int tid = threadIdx.x & 255, grp = threadIdx.x >> 8, lane = tid & 63, w = tid >> 6;
-  u16 *As = smem + grp * kTnBuf, *Bs = As + kRows * kLds;
-  const int nkt = K / kRows;
-  int kt, s;
-  tn_tile(nkt, int(gridDim.x) / nkt, kt, s);
-  const long m0 = long(s) * chunk + grp * kBK;
-  const int kb = kt * kRows;
-  f32x4 acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float db = 0.f;
-  const int amp = tid & 15, akg = tid >> 4;
-  const u16 *Ap = A + (m0 + 2 * amp) * K + kb + 8 * akg;
-  const int bmp0 = tid & 15, bng0 = tid >> 4, bng1 = (tid + 256) >> 4;
-  const u16 *Dp0 = D + (m0 + 2 * bmp0) * kW + 8 * bng0;
-  const u16 *Dp1 = D + (m0 + 2 * bmp0) * kW + 8 * bng1;
-  uint4 ra0{}, ra1{}, rb00, rb01, rb10, rb11;
-  if (tid < 128) {
-    ra0 = *reinterpret_cast<const uint4 *>(Ap);
-    ra1 = *reinterpret_cast<const uint4 *>(Ap + K);
-  }
-  rb00 = *reinterpret_cast<const uint4 *>(Dp0);
-  rb01 = *reinterpret_cast<const uint4 *>(Dp0 + kW);
-  rb10 = *reinterpret_cast<const uint4 *>(Dp1);
-  rb11 = *reinterpret_cast<const uint4 *>(Dp1 + kW);
-  constexpr int stride = kTnGroups * kBK;
-  for (int mm = 0; mm < chunk; mm += stride) {
-    if (tid < 128) put_pairs(As, 8 * akg, amp, ra0, ra1);
-    put_pairs(Bs, 8 * bng0, bmp0, rb00, rb01);
-    put_pairs(Bs, 8 * bng1, bmp0, rb10, rb11);
-    __syncthreads();
-    if (mm + stride < chunk) {
-      const long o = long(mm + stride);
-      if (tid < 128) {
-        ra0 = *reinterpret_cast<const uint4 *>(Ap + o * K);
-        ra1 = *reinterpret_cast<const uint4 *>(Ap + (o + 1) * K);
-      }
-      rb00 = *reinterpret_cast<const uint4 *>(Dp0 + o * kW);
-      rb01 = *reinterpret_cast<const uint4 *>(Dp0 + (o + 1) * kW);
-      rb10 = *reinterpret_cast<const uint4 *>(Dp1 + o * kW);
-      rb11 = *reinterpret_cast<const uint4 *>(Dp1 + (o + 1) * kW);
-    }
-    if (kt == 0) {
-      const u16 *row = Bs + tid * kLds;
-      for (int c = 0; c < kBK; ++c) db += bf2f(row[c]);
-    }
-    mma_slab(As, Bs, lane, w, acc);
-    __syncthreads();
-  }
-  // groups 1..3 hand their sums to group 0 through LDS, one row block i at a time
-  float *red = reinterpret_cast<float *>(smem);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    if (grp > 0)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        *reinterpret_cast<f32x4 *>(red + (long((grp - 1) * 256 + tid) * 16 + 4 * j)) = acc[i][j];
-    __syncthreads();
-    if (grp == 0)
-      for (int g2 = 1; g2 < kTnGroups; ++g2)
+      for (int i = 0; i < NI; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const f32x4 o = *reinterpret_cast<const f32x4 *>(red + (long((g2 - 1) * 256 + tid) * 16 + 4 * j));
-          acc[i][j] = acc[i][j] + o;
+          sum[i][j] = sum[i][j] + acc[i][j];
+          acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
+      dbs += db;
+      db = 0.f;
+    }
+  };
+  u32x4 x0, x1, x2, y0, y1, y2;
+  load(x0, x1, x2);
+  load(y0, y1, y2);
+  store(0, x0, x1, x2);
+  load(x0, x1, x2);
+  for (int t = 0; t < cs; t += 2) {
+    __syncthreads();  // slab t is in buffer 0, and buffer 1 has been read
+    store(1, y0, y1, y2);
+    load(y0, y1, y2);
+    multiply(lds);
+    if (t + 1 == cs) break;
     __syncthreads();
+    store(0, x0, x1, x2);
+    load(x0, x1, x2);
+    multiply(lds + kSlab);
   }
-  if (kt == 0) {
-    if (grp > 0) red[(grp - 1) * 256 + tid] = db;
-    __syncthreads();
-    if (grp == 0)
-      for (int g2 = 1; g2 < kTnGroups; ++g2) db += red[(g2 - 1) * 256 + tid];
-  }
-  if (grp != 0) return;
-  float *Gs = G + long(s) * P;
+  // lane l holds dW[16i + l%16][16j + 4(l/16)..+3]
+  const int n0 = 64 * wn + 4 * (lane >> 4);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int k = kb + 16 * i + (lane & 15);
+  for (int i = 0; i < NI; ++i) {
+    const int k = 16 * (wk * NI + i) + (lane & 15);
     if (k >= Kreal) continue;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n0 = 64 * w + 16 * j + 4 * (lane >> 4);
-      *reinterpret_cast<float4 *>(Gs + offW + long(k) * kW + n0) =
-          make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
-    }
+    for (int j = 0; j < 4; ++j) *reinterpret_cast<f32x4 *>(GW + long(k) * kW + n0 + 16 * j) = sum[i][j];
   }
-  if (kt == 0) Gs[offb + tid] = db;
+  if (Gb && tid < kW) Gb[tid] = dbs;
+}
+
+// Workgroups: per slice two 128-input tiles of each layer from the last to the
+// second, then the input layer's one tile.  The two tiles of a layer read the
+// same D; with the slices in eights they go to one XCD (workgroups are handed to
+// the eight XCDs in turn), whose L2 serves the second.
+__global__ __launch_bounds__(kWgThreads, 2) void k_wgrad(WGrad g) {
+  __shared__ __attribute__((aligned(16))) u16 lds[2 * 24 * 512];
+  const int hidden = 2 * (g.L - 1) * g.S;
+  int w = blockIdx.x;
+  if (w >= hidden) {
+    w -= hidden;
+    wgrad_tile<2 * kSlabs0>(g.A[0], 128 * kSlabs0, g.D[0], w * g.cs, g.cs, g.ng, kFeat, g.G + long(w) * g.P + g.offW[0],
+                            g.G + long(w) * g.P + g.offb[0], lds);
+    return;
+  }
+  const int l = g.L - 1 - w / (2 * g.S);
+  w %= 2 * g.S;
+  const int s = g.S % 8 == 0 ? (w >> 4) * 8 + (w & 7) : w >> 1, kt = g.S % 8 == 0 ? (w >> 3) & 1 : w & 1;
+  float *Gs = g.G + long(s) * g.P;
+  wgrad_tile<8>(g.A[l] + kt * 8 * 512, 1024, g.D[l], s * g.cs, g.cs, g.ng, 128, Gs + g.offW[l] + kt * 128L * kW,
+                kt == 0 ? Gs + g.offb[l] : nullptr, lds);
+}
+
+// largest divisor of M/32 that is at most kMaxSplit: row slices of the
+// gradient reduction, each a multiple of 32 rows
+int nsplit(int M) {
+  const int u = M / kBK;
+  for (int s = std::min(u, kMaxSplit); s >= 1; --s)
+    if (u % s == 0) return s;
+  return 1;
 }
 
 // ------------------------------------------------------------ output layer
@@ -775,7 +704,7 @@ __global__ __launch_bounds__(256) void k_head_reduce(int nhb, const float *__res
 // --------------------------------------------------------------- optimiser
 struct LayerTab {
   long offW[kMaxLayers], offb[kMaxLayers];
-  int in[kMaxLayers], out[kMaxLayers], inpad[kMaxLayers];
+  int in[kMaxLayers], out[kMaxLayers];
   u16 *Wt[kMaxLayers];  // packed copies (pack_at): forward operand, reduction over the inputs
   u16 *Wk[kMaxLayers];  // backward-data operand, reduction over the outputs
   int nl;
@@ -813,15 +742,13 @@ __global__ __launch_bounds__(256) void k_adam(long P, int nsplit, int mode, cons
       g = gh[p - offHead];
     } else {
       // the slices' partials in flight 16 at a time, summed in slice order
-      int k = 0;
-      for (; k + 16 <= nsplit; k += 16) {
+      for (int k = 0; k < nsplit; k += 16) {
         float v[16];
 #pragma unroll
-        for (int u = 0; u < 16; ++u) v[u] = G[long(k + u) * P + p];
+        for (int u = 0; u < 16; ++u) v[u] = k + u < nsplit ? G[long(k + u) * P + p] : 0.f;
 #pragma unroll
         for (int u = 0; u < 16; ++u) g += v[u];
       }
-      for (; k < nsplit; ++k) g += G[long(k) * P + p];
     }
     if (gout) gout[p] = g;
     if (mode == 2) {
@@ -910,15 +837,6 @@ struct Prof {
   }
 };
 
-// largest divisor of M/32 that is at most kMaxSplit: row slices of the
-// gradient reduction, each a multiple of 32 rows
-int nsplit(int M) {
-  const int u = M / kBK;
-  for (int s = std::min(u, kMaxSplit); s >= 1; --s)
-    if (u % s == 0) return s;
-  return 1;
-}
-
 // f(tile rows): the row tile of a pass over M rows.  128 rows read the weights
 // least often and keep the matrix cores busiest, but need two tiles for each CU
 // (65,536 rows, forward with the output layer: 107 us in 128-row tiles); fewer
@@ -968,7 +886,6 @@ int predict_pass(fvs_mlp &m, int M, const Rows &R) {
 
 // forward and backward over M rows: loss and weight-gradient partials
 int train_pass(fvs_mlp &m, int M, const Rows &R) {
-  const int S = nsplit(M), chunk = M / S;
   const int L = m.L;
   launch_forward<true>(m, M, R);
   {
@@ -977,7 +894,7 @@ int train_pass(fvs_mlp &m, int M, const Rows &R) {
     hipLaunchKernelGGL(k_head, dim3((M + kHeadRows - 1) / kHeadRows), dim3(256), 0, m.stream, long(M), R.nvalid,
                        inv_no, m.H[L - 1], m.Z[L - 1], m.w + m.tab.offW[L], m.w + m.tab.offb[L], m.T, m.Gh, m.lossp);
   }
-  if (L > 1) {
+  {
     Prof pf(m, MC_BWD);
     const Chain c = chain_of(m, M, m.tab.Wk);
     with_tile(M, [&](auto tr) {
@@ -985,16 +902,22 @@ int train_pass(fvs_mlp &m, int M, const Rows &R) {
       hipLaunchKernelGGL((k_backward<TR, chain_depth(TR)>), dim3((M + TR - 1) / TR), dim3(256), 0, m.stream, c);
     });
   }
-  for (int l = L - 1; l >= 0; --l) {
+  {
     Prof pf(m, MC_WGRAD);
-    const u16 *A = (l == 0) ? m.X0 : m.H[l - 1];
-    const int K = m.tab.inpad[l];
-    if (chunk % (kTnGroups * kBK) == 0)
-      hipLaunchKernelGGL(k_gemm_tn_g, dim3((K / kRows) * S), dim3(256 * kTnGroups), 0, m.stream, K, m.tab.in[l], chunk,
-                         A, m.Z[l], m.G, m.P, m.tab.offW[l], m.tab.offb[l]);
-    else
-      hipLaunchKernelGGL(k_gemm_tn, dim3((K / kRows) * S), dim3(256), 0, m.stream, K, m.tab.in[l], chunk, A, m.Z[l],
-                         m.G, m.P, m.tab.offW[l], m.tab.offb[l]);
+    WGrad g{};
+    for (int l = 0; l < L; ++l) {
+      g.A[l] = l == 0 ? m.X0 : m.H[l - 1];
+      g.D[l] = m.Z[l];
+      g.offW[l] = m.tab.offW[l];
+      g.offb[l] = m.tab.offb[l];
+    }
+    g.L = L;
+    g.S = nsplit(M);
+    g.cs = M / kBK / g.S;
+    g.ng = g.cs % 4 == 0 ? 4 : 1;
+    g.G = m.G;
+    g.P = m.P;
+    hipLaunchKernelGGL(k_wgrad, dim3((2 * L - 1) * g.S), dim3(kWgThreads), 0, m.stream, g);
   }
   MLPC(hipGetLastError());
   return 0;
@@ -1051,7 +974,6 @@ int fvs_mlp_create(fvs_mlp **out, const fvs_mlp_options *opt) try {
   for (int l = 0; l <= m->L; ++l) {
     tb.in[l] = (l == 0) ? kFeat : kW;
     tb.out[l] = (l == m->L) ? kOut : kW;
-    tb.inpad[l] = (l == 0) ? kInPad : kW;
     tb.offW[l] = off;
     off += long(tb.in[l]) * tb.out[l];
     tb.offb[l] = off;
@@ -1072,7 +994,7 @@ int fvs_mlp_create(fvs_mlp **out, const fvs_mlp_options *opt) try {
   rc = rc ? rc : m->alloc(m->gh, kHeadPart);
   rc = rc ? rc : m->alloc(m->lossp, (M + kHeadRows - 1) / kHeadRows);
   rc = rc ? rc : m->alloc(m->lossh, 1);
-  rc = rc ? rc : m->alloc(m->X0, M * kInPad);
+  rc = rc ? rc : m->alloc(m->X0, M * kIn);
   for (int l = 0; l < m->L && !rc; ++l) {
     rc = m->alloc(m->Z[l], M * kW);
     rc = rc ? rc : m->alloc(m->H[l], M * kW);
@@ -1083,15 +1005,14 @@ int fvs_mlp_create(fvs_mlp **out, const fvs_mlp_options *opt) try {
   rc = rc ? rc : m->alloc(m->iraw, M * kRaw);
   rc = rc ? rc : m->alloc(m->itgt, M * kOut);
   for (int l = 0; l < m->L && !rc; ++l) {
-    rc = m->alloc(tb.Wt[l], size_t(kW) * tb.inpad[l]);
+    rc = m->alloc(tb.Wt[l], size_t(kW) * (l == 0 ? kIn : kW));
     if (!rc && l > 0) rc = m->alloc(tb.Wk[l], size_t(kW) * kW);
   }
   if (rc) return rc;
   tb.Wt[m->L] = tb.Wk[m->L] = nullptr;
   tb.Wk[0] = nullptr;
-  // padding: input rows of the packed weights, columns of X0
-  if (hipMemsetAsync(tb.Wt[0], 0, size_t(kW) * kInPad * sizeof(u16), m->stream) != hipSuccess ||
-      hipMemsetAsync(m->X0, 0, M * kInPad * sizeof(u16), m->stream) != hipSuccess)
+  // padding input rows of the packed weights
+  if (hipMemsetAsync(tb.Wt[0], 0, size_t(kW) * kIn * sizeof(u16), m->stream) != hipSuccess)
     return fail(FVS_EHIP, "memset");
   // Glorot-uniform weights from the seed, zero biases
   std::vector<float> w(m->P, 0.f);
@@ -1257,7 +1178,7 @@ int fvs_mlp_kernel_times(fvs_mlp *m, int steps, double *ms6, double *flop6, int 
   if (!m || !ms6 || !flop6 || !launches6) return fail(FVS_EINVAL, "null argument");
   if (!m->raw) return fail(FVS_ESTATE, "no training set (fvs_mlp_set_data)");
   if (steps < 1) return fail(FVS_EINVAL, "steps must be positive");
-  const int per_step = 2 * (1 + 1 + m->L + 1 + 1);
+  const int per_step = 2 * (MC_N - 1);
   const int need = per_step * steps;
   while (int(m->evpool.size()) < need) {
     hipEvent_t e;
@@ -1277,16 +1198,15 @@ int fvs_mlp_kernel_times(fvs_mlp *m, int steps, double *ms6, double *flop6, int 
     ms[m->evclass[k]] += t;
     cnt[m->evclass[k]] += 1;
   }
-  // matrix-core flops per launch (2 per multiply-add; the weight gradient averaged over its layers)
+  // matrix-core flops per launch (2 per multiply-add)
   const double M = m->M;
   double fl[MC_N] = {0};
-  double fwd = 0, wg = 0;
+  double fwd = 0;
   for (int l = 0; l < m->L; ++l) {
-    fwd += 2.0 * M * m->tab.inpad[l] * kW;
-    wg += 2.0 * M * m->tab.inpad[l] * kW;
+    fwd += 2.0 * M * (l == 0 ? kIn : kW) * kW;
   }
   fl[MC_FWD] = fwd;
-  fl[MC_WGRAD] = wg / m->L;
+  fl[MC_WGRAD] = fwd;
   fl[MC_BWD] = 2.0 * M * kW * kW * (m->L - 1);
   fl[MC_HEAD] = 2.0 * M * kW * kOut * 3.0;
   for (int k = 0; k < MC_N; ++k) {

@@ -36,7 +36,9 @@ def test_predict_at_tile_edges(depth, n):
     assert np.max(np.abs(y[rows] - ref)) <= 1e-2 * np.max(np.abs(ref))
 
 
-@pytest.mark.parametrize("depth,n", [(1, 1), (2, 65), (3, 4097), (2, 16449)])
+# weight gradient: 1, 4, 26, 43 and 64 row slices of 2, 1, 5, 12 and 8 slabs, in
+# one group (slab counts not a multiple of 4) and in four
+@pytest.mark.parametrize("depth,n", [(1, 1), (2, 65), (3, 4097), (2, 16449), (3, 16384)])
 def test_gradient_at_tile_edges(depth, n):
     net = WarmStartNet(depth=depth, batch=16512, seed=depth)
     raw, tgt = _data(n, n)
