@@ -182,14 +182,31 @@ __device__ __forceinline__ unsigned pack2(float a, float b) {
   return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{a, b}, bf16x2));
 }
 
+// Sum over the 32 lanes of a half wavefront, the same in each: pairs 16 lanes
+// apart, then 8, 4, 2 and 1.  From 8 on by row rotation in the vector unit
+// instead of five trips through LDS: what a lane gets from the lane n further
+// on is what it would get from its partner, because the sums of the steps
+// before repeat every 2n lanes.
+__device__ __forceinline__ float row_sum(float y) {
+  y += __shfl_xor(y, 16, 64);
+  auto ror = [](float x, auto ctl) __attribute__((always_inline)) {
+    return __builtin_bit_cast(
+        float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(ctl)::value, 0xf, 0xf, true));
+  };
+  y += ror(y, std::integral_constant<int, 0x128>());
+  y += ror(y, std::integral_constant<int, 0x124>());
+  y += ror(y, std::integral_constant<int, 0x122>());
+  y += ror(y, std::integral_constant<int, 0x121>());
+  return y;
+}
+
 // ------------------------------------------------------ forward / backward
 // One launch for all layers: as one product per layer, 65,536 rows took 5 x 45
 // us forward in training (Z, H written, H read back) and prediction 397 us a
 // call; in this form 118 us forward, 132 us backward, and 246 us a call.
-// A workgroup of 4 wavefronts owns TR rows and all 256 columns of every layer:
-// the rows' activations stay in LDS from layer to layer, and only what the
-// weight gradient reads is written to HBM.  Each wavefront holds TR x 64
-// results.  Its weights are not shared with the other wavefronts, so they go
+// A workgroup owns TR rows and all 256 columns of every layer: the rows' activations stay in LDS from layer to layer, and only what the
+// weight gradient reads is written to HBM.  Each wavefront holds the results of
+// its columns; its weights are not shared with the other wavefronts, so they go
 // from L2 to registers without LDS, in the order the MFMA operand wants them
 // (pack_at): one contiguous KB per load.
 constexpr int kActLd = kW + 8;  // LDS row (elements): 16-byte accesses of 16 rows meet distinct banks
@@ -204,35 +221,45 @@ __host__ __device__ inline int pack_at(int n, int k) {
   return ((((k >> 5) * 4 + (n >> 6)) * 4 + j) * 64 + t + 16 * ((k & 31) >> 3)) * 8 + (k & 7);
 }
 
-// acc = rows of act (TR x 32 ns) times a wavefront's 64 columns, slab after
-// slab (Wp: the lane's place in the packed weights); D slabs of weights are in
-// registers or in flight (b; the caller has loaded the first D).
-template <int TR, int D>
-__device__ __forceinline__ void load_slab(const u16 *__restrict__ Wp, int s, bf16x8 (&b)[4]) {
+// Tile of a workgroup: TR rows, NJ operand blocks (16 NJ columns) for each of
+// its 16 / NJ wavefronts, D slabs of weights in registers or in flight.  W:
+// wavefronts per SIMD that the registers allow (4 (TR / 16) NJ accumulators,
+// 4 D NJ weights).
+template <int TR_, int NJ_, int D_, int W_>
+struct Tile {
+  static constexpr int TR = TR_, NJ = NJ_, D = D_, W = W_, NT = 1024 / NJ_, NR = TR_ / 16;
+  static_assert(NJ == 4 || NJ == 2, "results leave as pairs of blocks");
+};
+
+// acc = rows of act (TR x 32 ns) times a wavefront's columns, slab after slab
+// (Wp: the lane's place in the packed weights); the caller has loaded the first D
+// slabs of b.
+template <int NJ>
+__device__ __forceinline__ void load_slab(const u16 *__restrict__ Wp, int s, bf16x8 (&b)[NJ]) {
 #pragma unroll
-  for (int j = 0; j < 4; ++j) b[j] = *reinterpret_cast<const bf16x8 *>(Wp + (s * 16 + j) * 512);
+  for (int j = 0; j < NJ; ++j) b[j] = *reinterpret_cast<const bf16x8 *>(Wp + (s * 16 + j) * 512);
 }
-template <int TR, int D>
+template <class TL>
 __device__ __forceinline__ void chain_layer(const u16 *__restrict__ act, const u16 *__restrict__ Wp, int ns, int lane,
-                                            bf16x8 (&b)[D][4], f32x4 (&acc)[TR / 16][4]) {
+                                            bf16x8 (&b)[TL::D][TL::NJ], f32x4 (&acc)[TL::NR][TL::NJ]) {
   const u16 *ap = act + (lane & 15) * kActLd + 8 * (lane >> 4);
 #pragma unroll
-  for (int i = 0; i < TR / 16; ++i)
+  for (int i = 0; i < TL::NR; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int s0 = 0; s0 < ns; s0 += D) {
+    for (int j = 0; j < TL::NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < ns; s0 += TL::D) {
 #pragma unroll
-    for (int u = 0; u < D; ++u) {
+    for (int u = 0; u < TL::D; ++u) {
       const int s = s0 + u;
       if (s < ns) {
 #pragma unroll
-        for (int i = 0; i < TR / 16; ++i) {
+        for (int i = 0; i < TL::NR; ++i) {
           const bf16x8 a = *reinterpret_cast<const bf16x8 *>(ap + 16 * i * kActLd + kBK * s);
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
+          for (int j = 0; j < TL::NJ; ++j)
             acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[u][j], a, acc[i][j], 0, 0, 0);
         }
-        if (s + D < ns) load_slab<TR, D>(Wp, s + D, b[u]);
+        if (s + TL::D < ns) load_slab<TL::NJ>(Wp, s + TL::D, b[u]);
       }
     }
   }
@@ -259,9 +286,9 @@ __device__ __forceinline__ long row_source(const Rows &R, long m) {
 // that way from LDS (pack_rows): per 32 rows and 16 columns one KB, lane by
 // lane, 16 bytes each; nothing is transposed here.
 __device__ __forceinline__ void pack_rows(const u16 *__restrict__ act, int rows, int cblocks, u16 *__restrict__ out,
-                                          int lane, int wv) {
+                                          int lane, int wv, int waves) {
   const u16 *src = act + 8 * (lane >> 4) * kActLd + (lane & 15);
-  for (int q = wv; q < rows / kBK * cblocks; q += 4) {
+  for (int q = wv; q < rows / kBK * cblocks; q += waves) {
     const u16 *p = src + (q / cblocks) * kBK * kActLd + 16 * (q % cblocks);
     unsigned v[4];
 #pragma unroll
@@ -280,22 +307,20 @@ struct Chain {
   float *T, *Y;
 };
 
-// Wavefronts per SIMD the registers allow: 16 (TR / 16) accumulators, 16 D weights
-constexpr int chain_waves(int TR) { return TR >= 128 ? 2 : 3; }
-
 // Features and all hidden layers of TR rows.  TRAIN: X0, Z, H and the targets
 // go to HBM (X0 and H in the weight gradient's order, the last H by rows for
 // k_head); otherwise only the network's output does.
-template <int TR, int D, bool TRAIN>
-__global__ __launch_bounds__(256, chain_waves(TR)) void k_forward(Chain c, Rows R) {
+template <class TL, bool TRAIN>
+__global__ __launch_bounds__(TL::NT, TL::W) void k_forward(Chain c, Rows R) {
+  constexpr int TR = TL::TR, NJ = TL::NJ, D = TL::D, NT = TL::NT;
   __shared__ __attribute__((aligned(16))) u16 act[TR * kActLd];
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const long r0 = long(blockIdx.x) * TR;
-  const int lp = (wv * 4 * 64 + lane) * 8;  // the lane's place in a slab of packed weights
-  bf16x8 b[D][4];
+  const int lp = (wv * NJ * 64 + lane) * 8;  // the lane's place in a slab of packed weights
+  bf16x8 b[D][NJ];
 #pragma unroll
   for (int u = 0; u < D; ++u)
-    if (u < kSlabs0) load_slab<TR, D>(c.W[0] + lp, u, b[u]);
+    if (u < kSlabs0) load_slab<NJ>(c.W[0] + lp, u, b[u]);
   // Consecutive lanes take the same columns of consecutive rows: a wavefront
   // evaluates one kind of feature (the kinds differ in their functions).  The
   // base angles are formed once per row and wait behind the row's input columns.
@@ -303,13 +328,13 @@ __global__ __launch_bounds__(256, chain_waves(TR)) void k_forward(Chain c, Rows 
     return *reinterpret_cast<Angle *>(act + row * kActLd + kBK * kSlabs0 + kind * int(sizeof(Angle) / sizeof(u16)));
   };
   static_assert(kBK * kSlabs0 * sizeof(u16) + 2 * sizeof(Angle) <= kActLd * sizeof(u16), "room for the angles");
-  for (int e = tid; e < 2 * TR; e += 256) {
+  for (int e = tid; e < 2 * TR; e += NT) {
     const int row = e % TR, kind = e / TR;
     const long m = r0 + row, src = m < c.M ? row_source(R, m) : -1;
     if (src >= 0) angle(row, kind) = base_angle(R.raw + src * kRaw, kind);
   }
   __syncthreads();
-  for (int e = tid; e < TR * (4 * kSlabs0); e += 256) {
+  for (int e = tid; e < TR * (4 * kSlabs0); e += NT) {
     const int row = e % TR, q = e / TR;
     const long m = r0 + row;
     const long src = m < c.M ? row_source(R, m) : -1;
@@ -327,25 +352,25 @@ __global__ __launch_bounds__(256, chain_waves(TR)) void k_forward(Chain c, Rows 
   }
   __syncthreads();
   const int rows = int(c.M - r0 < TR ? c.M - r0 : TR);
-  if (TRAIN) pack_rows(act, rows, 2 * kSlabs0, c.X0 + r0 * kIn, lane, wv);
-  f32x4 acc[TR / 16][4];
+  if (TRAIN) pack_rows(act, rows, 2 * kSlabs0, c.X0 + r0 * kIn, lane, wv, NT / 64);
+  f32x4 acc[TL::NR][NJ];
   for (int l = 0; l < c.L; ++l) {
-    chain_layer<TR, D>(act, c.W[l] + lp, l == 0 ? kSlabs0 : kW / kBK, lane, b, acc);
+    chain_layer<TL>(act, c.W[l] + lp, l == 0 ? kSlabs0 : kW / kBK, lane, b, acc);
     if (l + 1 < c.L)
 #pragma unroll
-      for (int u = 0; u < D; ++u) load_slab<TR, D>(c.W[l + 1] + lp, u, b[u]);
-    const int n0 = 64 * wv + 8 * (lane >> 4);
-    float bv[2][8];
+      for (int u = 0; u < D; ++u) load_slab<NJ>(c.W[l + 1] + lp, u, b[u]);
+    const int n0 = 16 * NJ * wv + 8 * (lane >> 4);
+    float bv[NJ / 2][8];
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int h = 0; h < NJ / 2; ++h)
 #pragma unroll
       for (int e = 0; e < 8; ++e) bv[h][e] = c.bias[l][n0 + 32 * h + e];
     __syncthreads();  // every wavefront has read the layer's input
 #pragma unroll
-    for (int i = 0; i < TR / 16; ++i) {
+    for (int i = 0; i < TL::NR; ++i) {
       const int row = 16 * i + (lane & 15);
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
+      for (int h = 0; h < NJ / 2; ++h) {
         float z[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) z[e] = acc[i][2 * h + (e >> 2)][e & 3] + bv[h][e];
@@ -361,7 +386,7 @@ __global__ __launch_bounds__(256, chain_waves(TR)) void k_forward(Chain c, Rows 
       }
     }
     __syncthreads();
-    if (TRAIN && l + 1 < c.L) pack_rows(act, rows, kW / 16, c.H[l] + r0 * kW, lane, wv);
+    if (TRAIN && l + 1 < c.L) pack_rows(act, rows, kW / 16, c.H[l] + r0 * kW, lane, wv, NT / 64);
   }
   if (!TRAIN) {
     // the output layer, 32 lanes per row as in k_head
@@ -371,7 +396,7 @@ __global__ __launch_bounds__(256, chain_waves(TR)) void k_forward(Chain c, Rows 
     for (int e = 0; e < 8; ++e)
 #pragma unroll
       for (int o = 0; o < kOut; ++o) w[e][o] = c.Wh[(8 * q + e) * kOut + o];
-    for (int row = rs; row < TR; row += 8) {
+    for (int row = rs; row < TR; row += NT / 32) {
       const uint4 hv = *reinterpret_cast<const uint4 *>(act + row * kActLd + 8 * q);
       const unsigned hw[4] = {hv.x, hv.y, hv.z, hv.w};
       float y[kOut] = {0.f, 0.f, 0.f, 0.f};
@@ -381,8 +406,8 @@ __global__ __launch_bounds__(256, chain_waves(TR)) void k_forward(Chain c, Rows 
 #pragma unroll
         for (int o = 0; o < kOut; ++o) y[o] += h * w[e][o];
       }
-      for (int off = 16; off >= 1; off >>= 1)
-        for (int o = 0; o < kOut; ++o) y[o] += __shfl_xor(y[o], off, 64);
+#pragma unroll
+      for (int o = 0; o < kOut; ++o) y[o] = row_sum(y[o]);
       if (q == 0 && r0 + row < R.nvalid)
         *reinterpret_cast<float4 *>(c.Y + (r0 + row) * kOut) =
             make_float4(y[0] + c.bh[0], y[1] + c.bh[1], y[2] + c.bh[2], y[3] + c.bh[3]);
@@ -393,39 +418,40 @@ __global__ __launch_bounds__(256, chain_waves(TR)) void k_forward(Chain c, Rows 
 // dZ of the hidden layers below the last, each in the place of its layer's Z
 // (c.W: the backward operands; Z of the last layer holds its dZ by rows), all of
 // them left in the weight gradient's order
-template <int TR, int D>
-__global__ __launch_bounds__(256, chain_waves(TR)) void k_backward(Chain c) {
+template <class TL>
+__global__ __launch_bounds__(TL::NT, TL::W) void k_backward(Chain c) {
+  constexpr int TR = TL::TR, NJ = TL::NJ, D = TL::D, NT = TL::NT;
   __shared__ __attribute__((aligned(16))) u16 act[TR * kActLd];
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const long r0 = long(blockIdx.x) * TR;
-  const int lp = (wv * 4 * 64 + lane) * 8;
-  bf16x8 b[D][4];
+  const int lp = (wv * NJ * 64 + lane) * 8;
+  bf16x8 b[D][NJ];
   if (c.L > 1)
 #pragma unroll
-    for (int u = 0; u < D; ++u) load_slab<TR, D>(c.W[c.L - 1] + lp, u, b[u]);
+    for (int u = 0; u < D; ++u) load_slab<NJ>(c.W[c.L - 1] + lp, u, b[u]);
   const u16 *top = c.Z[c.L - 1];
-  for (int e = tid; e < TR * (kW / 8); e += 256) {
+  for (int e = tid; e < TR * (kW / 8); e += NT) {
     const int row = e / (kW / 8), q = e % (kW / 8);
     *reinterpret_cast<uint4 *>(act + row * kActLd + 8 * q) =
         r0 + row < c.M ? *reinterpret_cast<const uint4 *>(top + (r0 + row) * kW + 8 * q) : make_uint4(0, 0, 0, 0);
   }
   __syncthreads();
   const int rows = int(c.M - r0 < TR ? c.M - r0 : TR);
-  pack_rows(act, rows, kW / 16, c.Z[c.L - 1] + r0 * kW, lane, wv);
-  f32x4 acc[TR / 16][4];
+  pack_rows(act, rows, kW / 16, c.Z[c.L - 1] + r0 * kW, lane, wv, NT / 64);
+  f32x4 acc[TL::NR][NJ];
   for (int l = c.L - 1; l > 0; --l) {
-    chain_layer<TR, D>(act, c.W[l] + lp, kW / kBK, lane, b, acc);
+    chain_layer<TL>(act, c.W[l] + lp, kW / kBK, lane, b, acc);
     if (l > 1)
 #pragma unroll
-      for (int u = 0; u < D; ++u) load_slab<TR, D>(c.W[l - 1] + lp, u, b[u]);
-    const int n0 = 64 * wv + 8 * (lane >> 4);
+      for (int u = 0; u < D; ++u) load_slab<NJ>(c.W[l - 1] + lp, u, b[u]);
+    const int n0 = 16 * NJ * wv + 8 * (lane >> 4);
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < TR / 16; ++i) {
+    for (int i = 0; i < TL::NR; ++i) {
       const int row = 16 * i + (lane & 15);
       __builtin_amdgcn_sched_barrier(0);  // Z of few rows at a time in registers
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
+      for (int h = 0; h < NJ / 2; ++h) {
         uint4 dv = make_uint4(0, 0, 0, 0);
         if (r0 + 16 * i < c.M) {
           const uint4 zv = *reinterpret_cast<const uint4 *>(c.Z[l - 1] + (r0 + row) * kW + n0 + 32 * h);
@@ -440,7 +466,7 @@ __global__ __launch_bounds__(256, chain_waves(TR)) void k_backward(Chain c) {
       }
     }
     __syncthreads();  // all of Z is read, all of dZ in LDS
-    pack_rows(act, rows, kW / 16, c.Z[l - 1] + r0 * kW, lane, wv);
+    pack_rows(act, rows, kW / 16, c.Z[l - 1] + r0 * kW, lane, wv, NT / 64);
   }
 }
 
@@ -592,95 +618,103 @@ int nsplit(int M) {
 constexpr int kHeadRows = 128;                 // rows per workgroup
 constexpr int kHeadPart = kW * kOut + kOut;    // output-layer parameters
 
-// Workgroup b handles rows [128b, min(128b + 128, M)), 8 rows at a time (M is
-// a multiple of 64, so every lane of a row pair runs the same trips), 32 lanes per
-// row, 8 hidden columns per lane.  y = H Wh + bh in float32,
-// dy = 2 (y - t) / (nvalid * 4) for rows < nvalid (0 otherwise), the last
-// hidden layer's dZ = bf16((dy Wh^T) * GELU'(Z)) in the place of Z, and this
+// Workgroup b handles rows [128b, min(128b + 128, M)), 64 or 128: y = H Wh + bh in
+// float32, dy = 2 (y - t) / (nvalid * 4) for rows < nvalid (0 otherwise), the
+// last hidden layer's dZ = bf16((dy Wh^T) * GELU'(Z)) in the place of Z, and this
 // workgroup's partial gradients of Wh and bh (Gh[b][...]) and loss sum (lossp[b]).
-__global__ __launch_bounds__(256) void k_head(long M, long nvalid, float inv_no, const u16 *__restrict__ H, u16 *Z,
-                                              const float *__restrict__ Wh, const float *__restrict__ bh,
-                                              const float *__restrict__ T, float *__restrict__ Gh,
-                                              float *__restrict__ lossp) {
-  __shared__ float Ws[kW * kOut];
+// First 32 rows at a time with 32 lanes per row and 8 hidden columns per lane,
+// dy to LDS; then the sums over the rows, a quarter of the threads per output,
+// rows rs, rs + 8, ... in a thread.  (Both in one pass, 8 rows at a time: 4,096
+// rows 30 -> 19 us, 65,536 rows 48 -> 44; bound by vector instructions.)
+constexpr int kHeadThreads = 1024;
+__global__ __launch_bounds__(kHeadThreads, 4) void k_head(long M, long nvalid, float inv_no, const u16 *__restrict__ H,
+                                                       u16 *Z, const float *__restrict__ Wh,
+                                                       const float *__restrict__ bh, const float *__restrict__ T,
+                                                       float *__restrict__ Gh, float *__restrict__ lossp) {
   __shared__ float red[4][32][8 * kOut + kOut + 1];
-  const int tid = threadIdx.x, q = tid & 31, rs = tid >> 5, lane = tid & 63, wv = tid >> 6;
-  for (int e = tid; e < kW * kOut; e += 256) Ws[e] = Wh[e];
+  __shared__ __attribute__((aligned(16))) float res[kHeadRows][kOut];  // y - t
+  const int tid = threadIdx.x, q = tid & 31, lane = tid & 63, wv = (tid >> 6) & 3;
+  const long mbeg = long(blockIdx.x) * kHeadRows;
+  const int rows = int(M - mbeg < kHeadRows ? M - mbeg : kHeadRows);
+  {
+    float w[8][kOut], bo[kOut];
+    for (int c = 0; c < 8; ++c)
+      for (int o = 0; o < kOut; ++o) w[c][o] = Wh[(8 * q + c) * kOut + o];
+    for (int o = 0; o < kOut; ++o) bo[o] = bh[o];
+    for (int r0 = 0; r0 < rows; r0 += 64) {  // two rows per thread, their loads together
+      uint4 h2[2], z2[2];
+      float4 t2[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const long m = mbeg + r0 + 32 * u + (tid >> 5);
+        h2[u] = *reinterpret_cast<const uint4 *>(H + m * kW + 8 * q);
+        z2[u] = *reinterpret_cast<const uint4 *>(Z + m * kW + 8 * q);
+        t2[u] = *reinterpret_cast<const float4 *>(T + m * kOut);
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int r = r0 + 32 * u + (tid >> 5);
+        const long m = mbeg + r;
+        const uint4 hv = h2[u], zv = z2[u];
+        const float4 t4 = t2[u];
+        const float tv[kOut] = {t4.x, t4.y, t4.z, t4.w};
+        const unsigned hw[4] = {hv.x, hv.y, hv.z, hv.w};
+        float dy[kOut];
+        for (int o = 0; o < kOut; ++o) {
+          float t = 0.f;
+          for (int c = 0; c < 8; ++c) t += bf2f(u16((hw[c >> 1] >> (16 * (c & 1))) & 0xffffu)) * w[c][o];
+          const float y = row_sum(t) + bo[o];
+          const float d = m < nvalid ? y - tv[o] : 0.f;
+          dy[o] = 2.f * d * inv_no;
+          if (q == 0) res[r][o] = d;
+        }
+        const unsigned zw[4] = {zv.x, zv.y, zv.z, zv.w};
+        unsigned pk[4] = {0, 0, 0, 0};
+        for (int c = 0; c < 8; ++c) {
+          float g = 0.f;
+          for (int o = 0; o < kOut; ++o) g += dy[o] * w[c][o];
+          const float z = bf2f(u16((zw[c >> 1] >> (16 * (c & 1))) & 0xffffu));
+          pk[c >> 1] |= unsigned(f2bf(g * gelu_grad(z))) << (16 * (c & 1));
+        }
+        *reinterpret_cast<uint4 *>(Z + m * kW + 8 * q) = make_uint4(pk[0], pk[1], pk[2], pk[3]);
+      }
+    }
+  }
   __syncthreads();
-  float gw[8][kOut], gb[kOut], ls = 0.f;
-  for (int c = 0; c < 8; ++c)
-    for (int o = 0; o < kOut; ++o) gw[c][o] = 0.f;
-  for (int o = 0; o < kOut; ++o) gb[o] = 0.f;
-  const long mbeg = long(blockIdx.x) * kHeadRows, mend = mbeg + kHeadRows < M ? mbeg + kHeadRows : M;
-  // the next row's H and Z are in flight while this row is processed
-  uint4 hn{}, zn{};
-  if (mbeg + rs < mend) {
-    hn = *reinterpret_cast<const uint4 *>(H + (mbeg + rs) * kW + 8 * q);
-    zn = *reinterpret_cast<const uint4 *>(Z + (mbeg + rs) * kW + 8 * q);
+  const int rs = (tid >> 5) & 7, o = tid >> 8;
+  float gw[8] = {0, 0, 0, 0, 0, 0, 0, 0}, gb = 0.f, ls = 0.f;
+  for (int r0 = rs; r0 < rows; r0 += 64) {
+    uint4 h8[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) h8[u] = *reinterpret_cast<const uint4 *>(H + (mbeg + r0 + 8 * u) * kW + 8 * q);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const float *d = res[r0 + 8 * u];
+      const unsigned hw[4] = {h8[u].x, h8[u].y, h8[u].z, h8[u].w};
+      const float dy = 2.f * d[o] * inv_no;
+      for (int c = 0; c < 8; ++c) gw[c] += bf2f(u16((hw[c >> 1] >> (16 * (c & 1))) & 0xffffu)) * dy;
+      gb += dy;
+      if (o == 0)
+        for (int e = 0; e < kOut; ++e) ls += d[e] * d[e];
+    }
   }
-  for (long m = mbeg + rs; m < mend; m += 8) {
-    const uint4 hv = hn, zv = zn;
-    if (m + 8 < mend) {
-      hn = *reinterpret_cast<const uint4 *>(H + (m + 8) * kW + 8 * q);
-      zn = *reinterpret_cast<const uint4 *>(Z + (m + 8) * kW + 8 * q);
-    }
-    const unsigned hw[4] = {hv.x, hv.y, hv.z, hv.w};
-    float h[8];
-    for (int c = 0; c < 8; ++c) h[c] = bf2f(u16((hw[c >> 1] >> (16 * (c & 1))) & 0xffffu));
-    float y[kOut];
-    for (int o = 0; o < kOut; ++o) {
-      float t = 0.f;
-      for (int c = 0; c < 8; ++c) t += h[c] * Ws[(8 * q + c) * kOut + o];
-      y[o] = t;
-    }
-    for (int off = 16; off >= 1; off >>= 1)
-      for (int o = 0; o < kOut; ++o) y[o] += __shfl_xor(y[o], off, 64);
-    for (int o = 0; o < kOut; ++o) y[o] += bh[o];
-    const bool valid = m < nvalid;
-    float dy[kOut];
-    for (int o = 0; o < kOut; ++o) {
-      const float r = valid ? y[o] - T[m * kOut + o] : 0.f;
-      dy[o] = 2.f * r * inv_no;
-      if (q == 0) ls += r * r;
-    }
-    const unsigned zw[4] = {zv.x, zv.y, zv.z, zv.w};
-    unsigned pk[4] = {0, 0, 0, 0};
-    for (int c = 0; c < 8; ++c) {
-      float g = 0.f;
-      for (int o = 0; o < kOut; ++o) g += dy[o] * Ws[(8 * q + c) * kOut + o];
-      const float z = bf2f(u16((zw[c >> 1] >> (16 * (c & 1))) & 0xffffu));
-      pk[c >> 1] |= unsigned(f2bf(g * gelu_grad(z))) << (16 * (c & 1));
-      for (int o = 0; o < kOut; ++o) gw[c][o] += h[c] * dy[o];
-    }
-    *reinterpret_cast<uint4 *>(Z + m * kW + 8 * q) = make_uint4(pk[0], pk[1], pk[2], pk[3]);
-    if (q == 0)
-      for (int o = 0; o < kOut; ++o) gb[o] += dy[o];
-  }
-  // rows rs and rs^1 share a wavefront: add the two halves, then the 4 waves
-  for (int c = 0; c < 8; ++c)
-    for (int o = 0; o < kOut; ++o) gw[c][o] += __shfl_xor(gw[c][o], 32, 64);
-  for (int o = 0; o < kOut; ++o) gb[o] += __shfl_xor(gb[o], 32, 64);
+  // rows rs and rs^1 share a wavefront: add the two halves, then the 4 row groups
+  for (int c = 0; c < 8; ++c) gw[c] += __shfl_xor(gw[c], 32, 64);
+  gb += __shfl_xor(gb, 32, 64);
   ls += __shfl_xor(ls, 32, 64);
   if (lane < 32) {
-    for (int c = 0; c < 8; ++c)
-      for (int o = 0; o < kOut; ++o) red[wv][q][c * kOut + o] = gw[c][o];
-    for (int o = 0; o < kOut; ++o) red[wv][q][8 * kOut + o] = gb[o];
-    red[wv][q][8 * kOut + kOut] = ls;
+    for (int c = 0; c < 8; ++c) red[wv][q][c * kOut + o] = gw[c];
+    red[wv][q][8 * kOut + o] = gb;
+    if (o == 0) red[wv][q][8 * kOut + kOut] = ls;
   }
   __syncthreads();
   float *Gb = Gh + long(blockIdx.x) * kHeadPart;
-  for (int e = tid; e < kW * kOut; e += 256) {
-    const int k = e / kOut, o = e % kOut, qq = k / 8, c = k % 8;
-    Gb[e] = red[0][qq][c * kOut + o] + red[1][qq][c * kOut + o] + red[2][qq][c * kOut + o] +
-            red[3][qq][c * kOut + o];
-  }
-  if (tid < kOut)
-    Gb[kW * kOut + tid] = red[0][0][8 * kOut + tid] + red[1][0][8 * kOut + tid] + red[2][0][8 * kOut + tid] +
-                          red[3][0][8 * kOut + tid];
-  if (tid == 0)
-    lossp[blockIdx.x] = red[0][0][8 * kOut + kOut] + red[1][0][8 * kOut + kOut] + red[2][0][8 * kOut + kOut] +
-                        red[3][0][8 * kOut + kOut];
+  auto total = [&](int qq, int e) { return red[0][qq][e] + red[1][qq][e] + red[2][qq][e] + red[3][qq][e]; };
+  Gb[tid] = total(tid / (8 * kOut), tid % (8 * kOut));  // columns 8 qq + c, outputs o: tid = 32 qq + 4 c + o
+  if (tid < kOut) Gb[kW * kOut + tid] = total(0, 8 * kOut + tid);
+  if (tid == 0) lossp[blockIdx.x] = total(0, 8 * kOut + kOut);
 }
+static_assert(kHeadThreads == kW * kOut, "one weight of the output layer per thread");
 
 // Output-layer gradient: column c of the nhb partial rows, summed by 16
 // groups of rows (group g takes rows g, g+16, ...) and then the 16 group
@@ -691,7 +725,13 @@ __global__ __launch_bounds__(256) void k_head_reduce(int nhb, const float *__res
   const int c = blockIdx.x * 16 + t;
   float s = 0.f;
   if (c < kHeadPart)
-    for (int b = g; b < nhb; b += 16) s += Gh[long(b) * kHeadPart + c];
+    for (int b0 = g; b0 < nhb; b0 += 128) {  // eight loads in flight
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = b0 + 16 * u < nhb ? Gh[long(b0 + 16 * u) * kHeadPart + c] : 0.f;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) s += v[u];
+    }
   red[g][t] = s;
   __syncthreads();
   for (int h = 8; h >= 1; h >>= 1) {
@@ -837,17 +877,17 @@ struct Prof {
   }
 };
 
-// f(tile rows): the row tile of a pass over M rows.  128 rows read the weights
-// least often and keep the matrix cores busiest, but need two tiles for each CU
-// (65,536 rows, forward with the output layer: 107 us in 128-row tiles); fewer
-// rows are cut into smaller tiles so that every CU has one.
+// f(tile): the tile of a pass over M rows.  128 rows read the weights least
+// often and keep the matrix cores busiest, but need two tiles for each CU (32,768
+// rows, 10 training steps: 2728 us in tiles of 128, 2235 in tiles of 64); fewer
+// rows go in tiles of 32, each over 8 wavefronts (4,096 rows: 1258 us, over 4
+// wavefronts 1334; 16,384 rows: 1602, in tiles of 64 1775).
 template <class F>
 void with_tile(long M, F f) {
-  if (M >= 128 * 512) f(std::integral_constant<int, 128>());
-  else if (M >= 64 * 256) f(std::integral_constant<int, 64>());
-  else f(std::integral_constant<int, 32>());
+  if (M >= 128 * 512) f(Tile<128, 4, 2, 2>());
+  else if (M >= 64 * 512) f(Tile<64, 4, 2, 3>());
+  else f(Tile<32, 2, 4, 4>());
 }
-constexpr int chain_depth(int TR) { return TR >= 64 ? 2 : 4; }
 
 Chain chain_of(const fvs_mlp &m, long M, u16 *const *W) {
   Chain c{};
@@ -871,9 +911,9 @@ template <bool TRAIN>
 void launch_forward(fvs_mlp &m, int M, const Rows &R) {
   Prof pf(m, MC_FWD);
   const Chain c = chain_of(m, M, m.tab.Wt);
-  with_tile(M, [&](auto tr) {
-    constexpr int TR = decltype(tr)::value;
-    hipLaunchKernelGGL((k_forward<TR, chain_depth(TR), TRAIN>), dim3((M + TR - 1) / TR), dim3(256), 0, m.stream, c, R);
+  with_tile(M, [&](auto t) {
+    using TL = decltype(t);
+    hipLaunchKernelGGL((k_forward<TL, TRAIN>), dim3((M + TL::TR - 1) / TL::TR), dim3(TL::NT), 0, m.stream, c, R);
   });
 }
 
@@ -891,15 +931,15 @@ int train_pass(fvs_mlp &m, int M, const Rows &R) {
   {
     Prof pf(m, MC_HEAD);
     const float inv_no = 1.0f / float(double(R.nvalid) * kOut);
-    hipLaunchKernelGGL(k_head, dim3((M + kHeadRows - 1) / kHeadRows), dim3(256), 0, m.stream, long(M), R.nvalid,
+    hipLaunchKernelGGL(k_head, dim3((M + kHeadRows - 1) / kHeadRows), dim3(kHeadThreads), 0, m.stream, long(M), R.nvalid,
                        inv_no, m.H[L - 1], m.Z[L - 1], m.w + m.tab.offW[L], m.w + m.tab.offb[L], m.T, m.Gh, m.lossp);
   }
   {
     Prof pf(m, MC_BWD);
     const Chain c = chain_of(m, M, m.tab.Wk);
-    with_tile(M, [&](auto tr) {
-      constexpr int TR = decltype(tr)::value;
-      hipLaunchKernelGGL((k_backward<TR, chain_depth(TR)>), dim3((M + TR - 1) / TR), dim3(256), 0, m.stream, c);
+    with_tile(M, [&](auto t) {
+      using TL = decltype(t);
+      hipLaunchKernelGGL((k_backward<TL>), dim3((M + TL::TR - 1) / TL::TR), dim3(TL::NT), 0, m.stream, c);
     });
   }
   {
