@@ -297,6 +297,31 @@ __device__ __forceinline__ void stencil_minmax(int i, const int *__restrict__ so
 }
 
 // GGCB gradient (src/gradient_ggcb.f90:116-138):
+// Pieces of the Green-Gauss gradients, the same in every kernel: the own and one
+// neighbour's (or node's) term, the division by the volume, one cell's share of a
+// node value, and the limiter's bounds.
+__device__ __forceinline__ void gg_own(const double2 a, const double w[4], double gx[4], double gy[4]) {
+  for (int v = 0; v < 4; ++v) gx[v] = a.x * w[v], gy[v] = a.y * w[v];
+}
+__device__ __forceinline__ void gg_term(const double2 c, const double q[4], double gx[4], double gy[4]) {
+  for (int v = 0; v < 4; ++v) {
+    gx[v] = gx[v] + c.x * q[v];
+    gy[v] = gy[v] + c.y * q[v];
+  }
+}
+__device__ __forceinline__ void gg_divide(double V, double gx[4], double gy[4]) {
+  for (int v = 0; v < 4; ++v) gx[v] = gx[v] / V, gy[v] = gy[v] / V;
+}
+__device__ __forceinline__ void node_term(double c, const double q[4], double f[4]) {
+  for (int v = 0; v < 4; ++v) f[v] = f[v] + c * q[v];
+}
+__device__ __forceinline__ void stencil_bounds(const double q[4], double mn[4], double mx[4]) {
+  for (int v = 0; v < 4; ++v) {
+    mn[v] = (q[v] < mn[v]) ? q[v] : mn[v];
+    mx[v] = (q[v] > mx[v]) ? q[v] : mx[v];
+  }
+}
+
 // grad_i = (coef0 q_i + sum_f coefnb_f q_nb(f)) / vol
 template <int LIM>
 __global__ __launch_bounds__(kBlock) void k_grad_ggcb(int nbx, int N, int nfw, const double *__restrict__ W,
@@ -330,15 +355,11 @@ __global__ __launch_bounds__(kBlock) void k_grad_ggcb(int nbx, int N, int nfw, c
 #pragma unroll
   for (int k = 0; k < 4; ++k)
     if (k < nfw) make_prim(cv, gamma, q[k]);
-  for (int v = 0; v < 4; ++v) gx[v] = a.x * w[v], gy[v] = a.y * w[v];
+  gg_own(a, w, gx, gy);
 #pragma unroll
   for (int k = 0; k < 4; ++k)
-    if (k < nfw)
-      for (int v = 0; v < 4; ++v) {
-        gx[v] = gx[v] + c[k].x * q[k][v];
-        gy[v] = gy[v] + c[k].y * q[k][v];
-      }
-  for (int v = 0; v < 4; ++v) gx[v] = gx[v] / V, gy[v] = gy[v] / V;
+    if (k < nfw) gg_term(c[k], q[k], gx, gy);
+  gg_divide(V, gx, gy);
   double g8[8] = {gx[0], gx[1], gx[2], gx[3], gy[0], gy[1], gy[2], gy[3]};
   st8(grad, i, g8);
   if (LIM) {
@@ -381,10 +402,7 @@ __device__ __forceinline__ void gg_halo_minmax(const unsigned *__restrict__ lc, 
     const int j = int(((lc[(k >> 1) * kSlice] >> (16 * (k & 1))) & 0xffffu) >> 4);
     double q[4];
     ld4(lW, j, q);
-    for (int v = 0; v < 4; ++v) {
-      mn[v] = (q[v] < mn[v]) ? q[v] : mn[v];
-      mx[v] = (q[v] > mx[v]) ? q[v] : mx[v];
-    }
+    stencil_bounds(q, mn, mx);
   }
 }
 
@@ -434,15 +452,11 @@ __global__ __launch_bounds__(kBlock) void k_grad_ggcb_h(int nbx, int N, int nfw,
   __syncthreads();
   if (!act) return;
   double gx[4], gy[4];
-  for (int v = 0; v < 4; ++v) gx[v] = a.x * w[v], gy[v] = a.y * w[v];
+  gg_own(a, w, gx, gy);
 #pragma unroll
   for (int k = 0; k < 4; ++k)
-    if (k < nfw)
-      for (int v = 0; v < 4; ++v) {
-        gx[v] = gx[v] + c[k].x * q[k][v];
-        gy[v] = gy[v] + c[k].y * q[k][v];
-      }
-  for (int v = 0; v < 4; ++v) gx[v] = gx[v] / V, gy[v] = gy[v] / V;
+    if (k < nfw) gg_term(c[k], q[k], gx, gy);
+  gg_divide(V, gx, gy);
   double g8[8] = {gx[0], gx[1], gx[2], gx[3], gy[0], gy[1], gy[2], gy[3]};
   st8(grad, i, g8);
   const int s = i / kSlice;
@@ -486,8 +500,7 @@ __global__ __launch_bounds__(kBlock) void k_ggnb_nodes(int NV, const double *__r
     for (int u = 0; u < 4; ++u) make_prim(cons, gamma, q[u]);  // conservative states (SSP-RK3 stages)
 #pragma unroll
     for (int u = 0; u < 4; ++u)
-      if (k0 + u < wid)
-        for (int v2 = 0; v2 < 4; ++v2) f[v2] = f[v2] + c[u] * q[u][v2];
+      if (k0 + u < wid) node_term(c[u], q[u], f);
   }
   st4(F, v, f);
 }
@@ -519,13 +532,9 @@ __global__ __launch_bounds__(kBlock) void k_grad_ggnb(int nbx, int N, int gw, co
   double gx[4] = {0.0, 0.0, 0.0, 0.0}, gy[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
   for (int k = 0; k < 4; ++k)
-    if (k < gw)
-      for (int v = 0; v < 4; ++v) {
-        gx[v] = gx[v] + c[k].x * f[k][v];
-        gy[v] = gy[v] + c[k].y * f[k][v];
-      }
+    if (k < gw) gg_term(c[k], f[k], gx, gy);
   const double V = vol[i];
-  for (int v = 0; v < 4; ++v) gx[v] = gx[v] / V, gy[v] = gy[v] / V;
+  gg_divide(V, gx, gy);
   double g8[8] = {gx[0], gx[1], gx[2], gx[3], gy[0], gy[1], gy[2], gy[3]};
   st8(grad, i, g8);
   if (LIM) {
@@ -573,12 +582,8 @@ __global__ __launch_bounds__(kBlock) void k_grad_ggnb_h(int nbx, int N, int gw, 
   double gx[4] = {0.0, 0.0, 0.0, 0.0}, gy[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
   for (int k = 0; k < 4; ++k)
-    if (k < gw)
-      for (int v = 0; v < 4; ++v) {
-        gx[v] = gx[v] + c[k].x * f[k][v];
-        gy[v] = gy[v] + c[k].y * f[k][v];
-      }
-  for (int v = 0; v < 4; ++v) gx[v] = gx[v] / V, gy[v] = gy[v] / V;
+    if (k < gw) gg_term(c[k], f[k], gx, gy);
+  gg_divide(V, gx, gy);
   double g8[8] = {gx[0], gx[1], gx[2], gx[3], gy[0], gy[1], gy[2], gy[3]};
   st8(grad, i, g8);
   const int s = i / kSlice;
@@ -1161,7 +1166,7 @@ struct fvs_ctx {
   StageLists SL{};
   int stage_bs = 0, sweep = 0, nslist = 0;
   std::vector<int2> stage_cells;
-  long stage_words = 0, stage_faces = 0, stage_halo = 0;
+  long stage_words = 0, stage_faces = 0, stage_halo = 0, stage_incidences = 0;
   bool use_stage = true, two_kernel = false;
   int *slist = nullptr;
   bool halo = false;     // staged-halo lists built (k_grad_lsqh)
@@ -1721,14 +1726,19 @@ int two_kernel_lists(fvs_ctx &C) {
   HIPC(fetch(fbc, C.fb_cell, Fb));
   HIPC(fetch(fbt, C.fb_type, Fb));
   HIPC(fetch(fbg, C.fb_geo, 8 * Fb));
-  HIPC(fetch(off, C.soff, ns + 1));
-  HIPC(fetch(wid, C.swid, ns));
-  HIPC(hipStreamSynchronize(C.stream));
-  HIPC(fetch(code, C.sid, size_t(off[ns])));
+  // the stencil, with periodic shifts for a least-squares gradient; an unlimited
+  // Green-Gauss gradient has none
+  const void *ids = C.sid ? static_cast<const void *>(C.sid) : C.snb;
+  if (ids) {
+    HIPC(fetch(off, C.soff, ns + 1));
+    HIPC(fetch(wid, C.swid, ns));
+    HIPC(hipStreamSynchronize(C.stream));
+    HIPC(fetch(code, ids, size_t(off[ns])));
+  }
   HIPC(hipStreamSynchronize(C.stream));
   const StageMesh M{gat, fic, fig, fbc, fbt, fbg, off, wid, code};
   if (int rc = flux_lists(C, M)) return rc;
-  if (C.opt.kernel_path != 3)
+  if (C.opt.kernel_path != 3 && ids)
     if (int rc = setup_grad_halo(C, off, wid, code)) return rc;
   HIPC(hipStreamSynchronize(C.stream));
   C.two_kernel = true;
@@ -1848,6 +1858,8 @@ int setup_device(fvs_ctx &C) {
     if (int rc = C.upload(C.loff, lo)) return rc;
   }
   // LSQ stencil (gradient and/or limiter)
+  std::vector<int> boff, bwid;  // the bounds' stencil of a limited Green-Gauss gradient
+  std::vector<unsigned> bcode;
   if (!m.lsq_ptr.empty()) {
     std::vector<double> cw(2 * m.lsq_cell.size());
     parallel_for(long(m.lsq_cell.size()), 4096, [&](long, long k0, long k1) {
@@ -1944,24 +1956,22 @@ int setup_device(fvs_ctx &C) {
           if (int rc = setup_grad_halo(C, off, wid, code)) return rc;
       }
     }
-    // a limited Green-Gauss gradient takes its bounds from a staged halo of
-    // the same (node-neighbour) stencil: codes are the device ids (the
-    // bounds need no periodic shift)
+    // a limited Green-Gauss gradient takes its bounds from the same
+    // (node-neighbour) stencil: codes are the device ids (the bounds need no
+    // periodic shift)
     if ((C.opt.grad_method == 1 || C.opt.grad_method == 2) && C.opt.limiter > 0 && C.opt.recon != 1 &&
         C.opt.kernel_path != 3 && N < (1 << 27)) {
-      std::vector<unsigned> code(nb.begin(), nb.end());
-      if (int rc = setup_grad_halo(C, off, wid, code)) return rc;
+      bcode.assign(nb.begin(), nb.end());
+      boff = off;
+      bwid = wid;
     }
   }
-  if (C.fused && !C.stage_bs) {
-    const std::vector<int> none;
-    const std::vector<unsigned> nocode;
-    if (int rc = flux_lists(C, {gat, fic, fig, fbc, fbt, fbg, none, none, nocode})) return rc;
-    C.two_kernel = true;
-  }
+  StageMesh gm{gat, fic, fig, fbc, fbt, fbg, boff, bwid, bcode};
+  std::vector<int> nb, noff, nwid, ncell, cnode;
+  std::vector<double> ncoef;
   if (C.opt.grad_method == 1) {
     std::vector<double2> c0(N), cn(size_t(C.NFW) * N, make_double2(0.0, 0.0));
-    std::vector<int> nb(size_t(C.NFW) * N);
+    nb.resize(size_t(C.NFW) * N);
     for (int i = 0; i < N; ++i) {
       const int c = P[i];
       c0[i] = make_double2(m.ggcb_coef0[2 * c], m.ggcb_coef0[2 * c + 1]);
@@ -1977,6 +1987,8 @@ int setup_device(fvs_ctx &C) {
     if (int rc = C.upload(C.ggcb0, c0)) return rc;
     if (int rc = C.upload(C.ggcbnb, nb)) return rc;
     if (int rc = C.upload(C.ggcbc, cn)) return rc;
+    gm.fnb = &nb;
+    gm.ngg = C.NFW;
   }
   if (C.opt.grad_method == 2) {
     // nodes that touch a cell, ordered by their first device cell so that a
@@ -1994,7 +2006,8 @@ int setup_device(fvs_ctx &C) {
     for (int k = 0; k < NV; ++k) dnode[nodes[k]] = k;
     // node incidences in 64-node slices, the reference's cell order per node
     const int ns = (NV + kSlice - 1) / kSlice;
-    std::vector<int> noff(ns + 1, 0), nwid(ns, 0);
+    noff.assign(ns + 1, 0);
+    nwid.assign(ns, 0);
     long total = 0;
     for (int sl = 0; sl < ns; ++sl) {
       int w = 0;
@@ -2007,8 +2020,8 @@ int setup_device(fvs_ctx &C) {
       if (total > long(INT32_MAX)) return fail(FVS_EINVAL, "mesh too large: GGNB node incidences exceed 32-bit offsets");
       noff[sl + 1] = int(total);
     }
-    std::vector<int> ncell(size_t(total), 0);
-    std::vector<double> ncoef(size_t(total), 0.0);
+    ncell.assign(size_t(total), 0);
+    ncoef.assign(size_t(total), 0.0);
     for (int sl = 0; sl < ns; ++sl)
       for (int l = 0; l < kSlice; ++l) {
         const int k = sl * kSlice + l;
@@ -2023,7 +2036,7 @@ int setup_device(fvs_ctx &C) {
     // per cell: its nodes (the reference's local order) and coefedg
     int gwn = 0;
     for (int c = 0; c < N; ++c) gwn = std::max(gwn, m.nvrt[c]);
-    std::vector<int> cnode(size_t(gwn) * N, 0);
+    cnode.assign(size_t(gwn) * N, 0);
     std::vector<double2> cedg(size_t(gwn) * N, make_double2(0.0, 0.0));
     for (int i = 0; i < N; ++i) {
       const int c = P[i];
@@ -2043,6 +2056,20 @@ int setup_device(fvs_ctx &C) {
     if (int rc = C.upload(C.gcnode, cnode)) return rc;
     if (int rc = C.upload(C.gcedg, cedg)) return rc;
     if (int rc = C.alloc(C.gF, 4 * size_t(NV))) return rc;
+    gm.cnode = &cnode;
+    gm.ngg = gwn;
+    gm.noff = &noff;
+    gm.nwid = &nwid;
+    gm.ncell = &ncell;
+    gm.ncoef = &ncoef;
+  }
+  if (gm.ngg > 0 && C.fused && C.opt.recon != 1 && C.opt.kernel_path == 0 && C.ninst == 0 && N < (1 << 27))
+    if (int rc = setup_gg_stage(C, gm)) return rc;
+  if (!C.stage_bs && !bcode.empty())
+    if (int rc = setup_grad_halo(C, boff, bwid, bcode)) return rc;
+  if (C.fused && !C.stage_bs) {
+    if (int rc = flux_lists(C, gm)) return rc;
+    C.two_kernel = true;
   }
   // interior cells (vortex error), device ids, reference order
   std::vector<int> ci(m.cell_intr.size());
@@ -2337,6 +2364,9 @@ StageIn stage_in(const fvs_ctx &C, double t, double *uout) {
   a.S = C.SL;
   a.cxy = C.cxy;
   a.ginv = C.ginv;
+  a.gg0 = C.ggcb0;
+  a.ggc = C.opt.grad_method == 1 ? C.ggcbc : C.gcedg;
+  a.ngg = C.opt.grad_method == 1 ? C.NFW : C.gwn;
   a.st = C.shifts;
   a.p = C.opt.lsq_p;
   a.phisrc = C.opt.limiter > 0 ? 1 : 0;
@@ -2395,7 +2425,9 @@ int launch_stage(fvs_ctx &C, const Upd &A, double t, const double *uin = nullptr
     if (C.pmode == 0) FVS_STAGE(SH, L, 0);      \
     else if (C.pmode == 1) FVS_STAGE(SH, L, 1); \
     else if (C.pmode == 2) FVS_STAGE(SH, L, 2); \
-    else FVS_STAGE(SH, L, 3);                   \
+    else if (C.pmode == 3) FVS_STAGE(SH, L, 3); \
+    else if (C.pmode == kGGCB) FVS_STAGE(SH, L, kGGCB); \
+    else FVS_STAGE(SH, L, kGGNB);               \
   } while (0)
   if (C.stage_bs == StageLarge::BS) {
     if (lim) FVS_STAGE_PM(StageLarge, 1);
@@ -3335,7 +3367,9 @@ int fvs_phase_times(const fvs_ctx *C, double *sec4) try {
   // operations, about 18 per stencil entry against 300 per face and 60 per cell
   double share = 0.0;
   if (whole_stage(*C)) {
-    const double g = 36.0 * double(C->stage_words), f = 300.0 * double(C->stage_faces) + 60.0 * C->N;
+    double g = 36.0 * double(C->stage_words) + 8.0 * double(C->stage_incidences);
+    if (C->opt.grad_method != 3) g += 16.0 * (C->opt.grad_method == 1 ? C->NFW : C->gwn) * C->N;
+    const double f = 300.0 * double(C->stage_faces) + 60.0 * C->N;
     share = g / (g + f);
   }
   sec4[0] = (t[KC_GRAD] + share * t[KC_FUSED]) * 1e-3;  // gradient, limiter fused in
@@ -3605,9 +3639,10 @@ int fvs_kernel_times(fvs_ctx *C, double t1, int nsteps, double *ms, double *byte
     if (C->opt.steady) st3 += (8.0 + 8.0 * (nst - 1)) / nst;
     bfu = nlisted * (8 + 56) + N * (32 + 64 + (phi1 ? 0 : 8)) + N * (C->GW * 2.0 + 8 + st3);
   }
-  // whole stage: states, centres and G^-1 once, the block lists, limiter inputs,
+  // whole stage: states, centres and G^-1 or Green-Gauss coefficients once, the block lists, limiter inputs,
   // the update's cell-side traffic
-  double bst = N * (32 + 16 + 24 + C->GW * 2.0 + 8) + 4.0 * double(C->stage_words) + 4.0 * double(C->stage_halo) +
+  const double bcf = C->opt.grad_method == 3 ? 24.0 : C->opt.grad_method == 1 ? 16.0 + 16.0 * C->NFW : 16.0 * C->gwn;
+  double bst = N * (32 + 16 + bcf + C->GW * 2.0 + 8) + 10.0 * double(C->stage_incidences) + 4.0 * double(C->stage_words) + 4.0 * double(C->stage_halo) +
                44.0 * double(C->stage_faces) + (lim ? N * (8 + 4) + 16.0 * (3 * m.ntri + 4 * m.nquad) : 0.0);
   if (cons_stages(*C)) {
     double st3 = (32 + 64 + 64) / 3.0;  // new states, and the step-start state after the first stage

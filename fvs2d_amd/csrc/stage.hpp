@@ -32,14 +32,16 @@ struct StageShape {
   static constexpr int PS = 16 * C1, R2 = 3 * PS, FAR = 6 * PS;
   static constexpr int F0 = R2, F1 = R2 + 16 * F, G = 6 * PS, P = 10 * PS, S = P + 8 * C1, END = S + 8 * F;
   static constexpr int NSL = C1 / kSlice;  // stencil slices
+  static_assert(32 * NT <= 4 * PS, "the node values fit where the gradients go");
   static_assert(C1 % kSlice == 0 && C1 <= NT && F <= NT && 32 * F <= 3 * PS && BS % kSlice == 0, "block shape");
 };
 
 // One block: cells [i0, i0 + n0), base = n0 rounded up to whole slices, ring-1
 // cells at local indices base .. base + nr1 - 1, nh halo cells in all (ring 1,
 // ring 2; those past the C1 that ring 2 holds are far: read from HBM)
+// With node-based gradients nn nodes of up to 2 nkw cells each.
 struct StageBlock {
-  int i0, n0, base, nr1, nh, pad[3];
+  int i0, n0, base, nr1, nh, nn, nkw, pad;
 };
 
 // Per-block lists at fixed strides, so that a block's first loads wait on no
@@ -48,6 +50,9 @@ struct StageBlock {
 // faces as byte offsets of their two gradient cells (R side: | periodic shift of
 // its centre; 0xffff on a boundary; ~0 after the last) with 5 geometry values
 // (planes nx,ny | xf,yf | area); boundary code (type | instance << 2) of a face.
+// Green-Gauss gradients: four byte offsets per gradient cell in two words, of its
+// face neighbours' states or of its nodes' values (16 n for the block's node n);
+// nodes: the byte offsets of their cells two to a word, and the cells' weights.
 struct StageLists {
   const StageBlock *blk;
   const int *halo;
@@ -58,6 +63,9 @@ struct StageLists {
   const int *bcode;
   const short *lgat;
   int hs, cw, fs;  // strides: halo entries, code words per cell, faces
+  const unsigned *gcode, *ncode;
+  const double *nwt;
+  int ns, nkw;  // strides: nodes, words of cells per node
 };
 
 struct StageIn {
@@ -67,6 +75,8 @@ struct StageIn {
   StageLists S;
   const double2 *cxy;
   const double *ginv;
+  const double2 *gg0, *ggc;  // Green-Gauss: own coefficient (cell-based) and ngg per cell, planes
+  int ngg;
   ShiftTable st;
   double p;
   int phisrc;  // without LIM: 0 limiter values 1, 1 read phi (frozen)
@@ -100,17 +110,22 @@ using StageSmall = StageShape<128, 256, 192, 256, 5>;
 using StageLarge = StageShape<256, 512, 384, 512, 4>;
 
 constexpr int kCodeRegs = 8;  // code words a thread holds in registers
+constexpr int kNodeRegs = 3;  // words of a node's cells
 
 // Block lb of a whole stage.  LIM: the limiter is evaluated (and written for the
-// own cells).  With cons (SSP-RK3 and the two-register form), Win holds
+// own cells).  PMODE: the LSQ weights as in lsq_term, or a Green-Gauss gradient,
+// cell-based (kGGCB) or node-based (kGGNB).  With cons (SSP-RK3 and the two-register form), Win holds
 // conservative states, converted once as they are staged, and the new stage
 // state goes to Ub (a buffer other than Win; no primitive state is written).
 // With mode M_RESID the block ends in the residual instead of an update.
+constexpr int kGGCB = 4, kGGNB = 5;
+
 template <class SH, int LIM, int PMODE>
 __device__ __forceinline__ void stage_block(const StageIn &a, int lb, const Upd &A, const double *__restrict__ Win,
                                             double *__restrict__ Wout, int cons) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int NT = SH::NT, PS = SH::PS;
+  constexpr bool GG = PMODE >= kGGCB;
   auto at = [&](int o) __attribute__((always_inline)) -> double2 & { return *reinterpret_cast<double2 *>(smem + o); };
   auto at1 = [&](int o) __attribute__((always_inline)) -> double & { return *reinterpret_cast<double *>(smem + o); };
   const StageLists &S = a.S;
@@ -137,6 +152,26 @@ __device__ __forceinline__ void stage_block(const StageIn &a, int lb, const Upd 
   }
   const bool mine = tid < d.n0, act = mine || (tid >= d.base && tid < d.base + d.nr1);
   const int id = jd[0] & 0x07ffffff;
+  // Green-Gauss: the cell's four offsets, its coefficients and volume; the first
+  // cells of the thread's node
+  unsigned gc[2] = {0u, 0u}, nc[kNodeRegs];
+  double2 gk[4], gown = make_double2(0.0, 0.0);
+  double nw8[2 * kNodeRegs], GV = 1.0;
+  const unsigned *ncl = S.ncode + long(lb) * S.nkw * S.ns + tid;
+  const double *nwl = S.nwt + 2 * long(lb) * S.nkw * S.ns + tid;
+  if (GG && act) {
+    gc[0] = S.gcode[2 * long(lb) * SH::C1 + tid];
+    gc[1] = S.gcode[(2 * long(lb) + 1) * SH::C1 + tid];
+  }
+  if (PMODE == kGGNB) {
+#pragma unroll
+    for (int k = 0; k < kNodeRegs; ++k) {
+      const bool on = tid < d.nn && k < d.nkw;
+      nc[k] = on ? ncl[k * S.ns] : 0u;
+      nw8[2 * k] = on ? nwl[2 * k * S.ns] : 0.0;
+      nw8[2 * k + 1] = on ? nwl[(2 * k + 1) * S.ns] : 0.0;
+    }
+  }
   double g[8];
   g[7] = 0.0;
   if (rec != ~0u) {
@@ -162,7 +197,12 @@ __device__ __forceinline__ void stage_block(const StageIn &a, int lb, const Upd 
     double w[4];
     ld4(Win, j, w);
     if (r == 0) {
-      if (act) {
+      if (act && GG) {
+        if (PMODE == kGGCB) gown = a.gg0[j];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) gk[k] = (k < a.ngg) ? a.ggc[long(k) * N + j] : make_double2(0.0, 0.0);
+        GV = a.vol[j];
+      } else if (act) {
         Gi[0] = a.ginv[j];
         Gi[1] = a.ginv[N + j];
         Gi[2] = a.ginv[2 * long(N) + j];
@@ -191,6 +231,32 @@ __device__ __forceinline__ void stage_block(const StageIn &a, int lb, const Upd 
     if (keep) ph = a.phi[id];
   }
   __syncthreads();
+  if (PMODE == kGGNB) {
+    // node values where the gradients go afterwards: one node per thread
+    if (tid < d.nn) {
+      double f[4] = {0.0, 0.0, 0.0, 0.0};
+      auto add = [&](unsigned o, double c) __attribute__((always_inline)) {
+        const double2 qa = at(o), qb = at(o + PS);
+        const double q[4] = {qa.x, qa.y, qb.x, qb.y};
+        node_term(c, q, f);
+      };
+#pragma unroll
+      for (int k = 0; k < kNodeRegs; ++k)
+        if (k < d.nkw) {
+          add(nc[k] & 0xffffu, nw8[2 * k]);
+          add(nc[k] >> 16, nw8[2 * k + 1]);
+        }
+      for (int k = kNodeRegs; k < d.nkw; ++k) {
+        const unsigned w = ncl[k * S.ns];
+        add(w & 0xffffu, nwl[2 * k * S.ns]);
+        add(w >> 16, nwl[(2 * k + 1) * S.ns]);
+      }
+      at(SH::G + 16 * tid) = make_double2(f[0], f[1]);
+      at(SH::G + 16 * NT + 16 * tid) = make_double2(f[2], f[3]);
+    }
+    __syncthreads();
+  }
+  double gx[4] = {0.0, 0.0, 0.0, 0.0}, gy[4] = {0.0, 0.0, 0.0, 0.0};
   if (act) {
     const int o0 = 16 * tid;
     const double2 ci = at(o0 + 2 * PS), wa = at(o0), wb = at(o0 + PS);
@@ -200,9 +266,12 @@ __device__ __forceinline__ void stage_block(const StageIn &a, int lb, const Upd 
     auto term = [&](unsigned o) __attribute__((always_inline)) {
       const double2 cj = at(o + 2 * PS), qa = at(o), qb = at(o + PS);
       const double q[4] = {qa.x, qa.y, qb.x, qb.y};
-      lsq_term<LIM, PMODE>(cj.x, cj.y, ci, q, w, a.p, sx, sy, mn, mx);
+      if (GG) stencil_bounds(q, mn, mx);
+      else lsq_term<LIM, PMODE>(cj.x, cj.y, ci, q, w, a.p, sx, sy, mn, mx);
     };
-    if (d.nh <= d.nr1 + SH::C1) {
+    if (GG && !LIM) {
+      // no stencil beyond the faces or nodes
+    } else if (GG || d.nh <= d.nr1 + SH::C1) {
 #pragma unroll
       for (int k = 0; k < kCodeRegs; ++k)
         if (k < nw) {
@@ -234,17 +303,34 @@ __device__ __forceinline__ void stage_block(const StageIn &a, int lb, const Upd 
         lsq_term<LIM, PMODE>(xy.x, xy.y, ci, q, w, a.p, sx, sy, mn, mx);
       }
     }
-    double gx[4], gy[4];
-    lsq_apply_ginv(Gi[0], Gi[1], Gi[2], sx, sy, gx, gy);
-    at(SH::G + o0) = make_double2(gx[0], gx[1]);
-    at(SH::G + PS + o0) = make_double2(gx[2], gx[3]);
-    at(SH::G + 2 * PS + o0) = make_double2(gy[0], gy[1]);
-    at(SH::G + 3 * PS + o0) = make_double2(gy[2], gy[3]);
+    if (GG) {
+      constexpr int B = PMODE == kGGNB ? SH::G : 0, BP = PMODE == kGGNB ? 16 * NT : PS;
+      if (PMODE == kGGCB) gg_own(gown, w, gx, gy);
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (k < a.ngg) {
+          const int o = B + int((gc[k >> 1] >> (16 * (k & 1))) & 0xffffu);
+          const double2 qa = at(o), qb = at(o + BP);
+          const double q[4] = {qa.x, qa.y, qb.x, qb.y};
+          gg_term(gk[k], q, gx, gy);
+        }
+      gg_divide(GV, gx, gy);
+    } else {
+      lsq_apply_ginv(Gi[0], Gi[1], Gi[2], sx, sy, gx, gy);
+    }
     if (LIM && !keep) {
       ph = cell_limiter_v(a.lt, nf, fo, V, w, mn, mx, gx, gy);
       if (mine) a.phi[id] = ph;
     }
     if (!phi_one) at1(SH::P + 8 * tid) = ph;
+  }
+  if (PMODE == kGGNB) __syncthreads();  // the node values have been read
+  if (act) {
+    const int o0 = SH::G + 16 * tid;
+    at(o0) = make_double2(gx[0], gx[1]);
+    at(o0 + PS) = make_double2(gx[2], gx[3]);
+    at(o0 + 2 * PS) = make_double2(gy[0], gy[1]);
+    at(o0 + 3 * PS) = make_double2(gy[2], gy[3]);
   }
   __syncthreads();
   const bool resid = A.mode == M_RESID, ws = resid || (A.steady && A.first);

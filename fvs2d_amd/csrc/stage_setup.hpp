@@ -43,6 +43,12 @@ struct StageMesh {
   const std::vector<double> &fbg;
   const std::vector<int> &off, &wid;  // stencils in 64-cell slices
   const std::vector<unsigned> &code;  // id | periodic shift << 27
+  // Green-Gauss gradients: ngg face neighbours (planes) or nodes per cell; the
+  // nodes' cells and weights in 64-node slices
+  const std::vector<int> *fnb = nullptr, *cnode = nullptr;
+  int ngg = 0;
+  const std::vector<int> *noff = nullptr, *nwid = nullptr, *ncell = nullptr;
+  const std::vector<double> *ncoef = nullptr;
 };
 
 // the blocks cut from one contiguous part of the cells
@@ -53,8 +59,10 @@ struct StageCut {
   const int cw;       // code words of the widest stencil
   short *const lgat;  // gw x N signed 1-based local faces
   std::vector<StageBlock> blk;
-  std::vector<unsigned> halo, face, code;
+  std::vector<unsigned> halo, face, code, gcode;
   std::vector<int> slot, nf, width;
+  std::vector<unsigned short> ncode;  // per block nn x 2 nkw
+  std::vector<double> nwt;
   bool shift_ok = true;  // every periodic shift of a face is in the table
 
   // byte offset of the local cell with index q, of which the first n1 have gradients
@@ -85,7 +93,7 @@ struct StageCut {
     r1.erase(std::unique(r1.begin(), r1.end()), r1.end());
     const int base = nblk(i1 - i0, kSlice) * kSlice, n1 = base + int(r1.size());
     if (n1 > SH::C1) return false;
-    map.reset(size_t(n1) * (2 * cw + 1));
+    map.reset(size_t(n1) * (2 * cw + 5) + (M.cnode ? 8 * size_t(SH::NT) : 0));
     bool fresh;
     for (int i = i0; i < i1; ++i) map.at(unsigned(i), fresh) = i - i0;
     hal.assign(r1.begin(), r1.end());
@@ -98,7 +106,7 @@ struct StageCut {
       for (int l = 0; l < kSlice; ++l) {
         const int q = s * kSlice + l;
         const int i = q < base ? (i0 + q < i1 ? i0 + q : -1) : (q < n1 ? r1[q - base] : -1);
-        if (i < 0) continue;
+        if (i < 0 || cw == 0) continue;
         const int sg = i / kSlice, li = i % kSlice;
         w2[s] = std::max(w2[s], (M.wid[sg] + 1) / 2);
         for (int k = 0; k < 2 * cw; ++k) {
@@ -116,12 +124,19 @@ struct StageCut {
         }
       }
     }
+    int nn = 0, nkw = 0;
+    const size_t g0 = gcode.size();
+    if (M.ngg > 0 && !green_gauss(i0, i1, base, n1, nn, nkw)) {
+      code.resize(c0);
+      gcode.resize(g0);
+      return false;
+    }
     const int nl = base + int(hal.size());
     if (nl - n1 > SH::C1 && (i1 - i0 > kSlice || offset(nl - 1, n1) > 0xfff0)) {
       code.resize(c0);
       return false;
     }
-    blk.push_back({i0, i1 - i0, base, int(r1.size()), int(hal.size()), {0, 0, 0}});
+    blk.push_back({i0, i1 - i0, base, int(r1.size()), int(hal.size()), nn, nkw, 0});
     width.insert(width.end(), w2, w2 + SH::NSL);
     halo.insert(halo.end(), hal.begin(), hal.end());
     nf.push_back(int(loc.size()));
@@ -150,6 +165,64 @@ struct StageCut {
     return true;
   }
 
+  // offsets of the face neighbours or nodes of the block's gradient cells, and the
+  // nodes' cells; false when there are too many nodes or local cells
+  bool green_gauss(int i0, int i1, int base, int n1, int &nn, int &nkw) {
+    const int N = C.N;
+    const size_t g0 = gcode.size();
+    gcode.resize(g0 + 2 * SH::C1, 0u);
+    bool fresh;
+    auto local = [&](int j) {
+      int &x = map.at(unsigned(j), fresh);
+      if (fresh) {
+        x = base + int(hal.size());
+        hal.push_back(unsigned(j));
+      }
+      return x;
+    };
+    nodes.clear();
+    if (M.cnode) nmap.reset(4 * size_t(n1));
+    for (int q = 0; q < n1; ++q) {
+      const int i = q < base ? (i0 + q < i1 ? i0 + q : -1) : r1[q - base];
+      if (i < 0) continue;
+      for (int k = 0; k < M.ngg; ++k) {
+        unsigned v;
+        if (M.fnb) {
+          v = unsigned(offset(local((*M.fnb)[size_t(k) * N + i]), n1));
+        } else {
+          const int n = (*M.cnode)[size_t(k) * N + i];
+          int &x = nmap.at(unsigned(n), fresh);
+          if (fresh) {
+            x = int(nodes.size());
+            nodes.push_back(n);
+          }
+          v = 16u * unsigned(x);
+        }
+        gcode[g0 + size_t(k / 2) * SH::C1 + q] |= v << (16 * (k & 1));
+      }
+    }
+    if (int(nodes.size()) > SH::NT) return false;
+    nn = int(nodes.size());
+    cells.clear();
+    for (int n : nodes) {
+      const int sl = n / kSlice, at = (*M.noff)[sl] + n % kSlice;
+      int w = (*M.nwid)[sl];
+      while (w > 1 && (*M.ncoef)[size_t(at) + size_t(w - 1) * kSlice] == 0.0) --w;  // padding
+      cells.push_back(make_int2(at, w));
+      nkw = std::max(nkw, (w + 1) / 2);
+    }
+    for (int2 c : cells)
+      for (int k = 0; k < c.y; ++k) local((*M.ncell)[size_t(c.x) + size_t(k) * kSlice]);
+    if (base + int(hal.size()) - n1 > SH::C1) return false;  // every state in LDS
+    for (int2 c : cells)
+      for (int k = 0; k < 2 * nkw; ++k) {
+        const size_t e = size_t(c.x) + size_t(k < c.y ? k : 0) * kSlice;
+        ncode.push_back((unsigned short)(offset(local((*M.ncell)[e]), n1)));
+        nwt.push_back(k < c.y ? (*M.ncoef)[e] : 0.0);
+      }
+    return true;
+  }
+
   // cells [i0, i1) as one block or cut in two, down to one slice
   bool place(int i0, int i1) {
     if (block(i0, i1)) return true;
@@ -163,12 +236,15 @@ struct StageCut {
   StageCut(const fvs_ctx &c, const StageMesh &m, int w, short *g) : C(c), M(m), cw(w), lgat(g) {}
 
  private:
-  LocalMap map;
-  std::vector<int> loc, r1;
+  LocalMap map, nmap;
+  std::vector<int> loc, r1, nodes;
+  std::vector<int2> cells;
   std::vector<unsigned> hal;
 };
 
-int code_words(const StageMesh &M) { return std::max(1, (*std::max_element(M.wid.begin(), M.wid.end()) + 1) / 2); }
+int code_words(const StageMesh &M) {
+  return M.wid.empty() ? 0 : std::max(1, (*std::max_element(M.wid.begin(), M.wid.end()) + 1) / 2);
+}
 
 // Blocks per range of SH::BS cells, from up to 256 ranges spread over the cells
 // (a large number when one does not fit at all)
@@ -197,24 +273,31 @@ int setup_stage_blocks(fvs_ctx &C, const StageMesh &M) {
     for (long b = b0; b < b1 && ok[t]; ++b) ok[t] = parts[t].place_range(b) && parts[t].shift_ok;
   });
   std::vector<size_t> start(np + 1, 0);
-  int hs = 1, fs = 1;
+  int hs = 1, fs = 1, ns = 0, nkw = 0;
   for (long t = 0; t < np; ++t) {
     if (!ok[t]) return 0;
     start[t + 1] = start[t] + parts[t].blk.size();
-    for (const StageBlock &d : parts[t].blk) hs = std::max(hs, d.nh);
+    for (const StageBlock &d : parts[t].blk) {
+      hs = std::max(hs, d.nh);
+      ns = std::max(ns, d.nn);
+      nkw = std::max(nkw, d.nkw);
+    }
     for (int n : parts[t].nf) fs = std::max(fs, n);
   }
   const size_t nb = start[np];
   if (N > kStageSmallMesh && double(nb) > kStageMostBlocks * double(nr)) return 0;
   hs = (hs + 31) / 32 * 32;  // strides of whole cache lines
   fs = (fs + 15) / 16 * 16;
+  ns = (ns + 31) / 32 * 32;
   std::vector<StageBlock> blk(nb);
   std::vector<int> halo(nb * hs), bcode(nb * fs), width(nb * SH::NSL);
   std::vector<unsigned> code(nb * SH::NSL * cw * kSlice), face(nb * fs);
-  std::vector<double> geo(nb * fs * 5);
+  std::vector<double> geo(nb * fs * 5), nwt(nb * 2 * nkw * ns);
+  std::vector<unsigned> gcode(M.ngg > 0 ? nb * 2 * SH::C1 : 0), ncode(nb * nkw * ns);
   run_threads(int(np), [&](int t) {
     const StageCut<SH> &p = parts[t];
-    size_t ho = 0, fo = 0;
+    size_t ho = 0, fo = 0, no = 0;
+    std::copy(p.gcode.begin(), p.gcode.end(), gcode.begin() + (M.ngg > 0 ? start[t] * 2 * SH::C1 : 0));
     std::copy(p.blk.begin(), p.blk.end(), blk.begin() + start[t]);
     std::copy(p.width.begin(), p.width.end(), width.begin() + start[t] * SH::NSL);
     std::copy(p.code.begin(), p.code.end(), code.begin() + start[t] * SH::NSL * cw * kSlice);
@@ -237,14 +320,19 @@ int setup_stage_blocks(fvs_ctx &C, const StageMesh &M) {
         if (f >= Fi)
           bcode[b * fs + e] = M.fbt[bq] | ((C.ninst > 0 ? C.inst_of_real[C.perm[M.fbc[bq]]] : 0) << 2);
       }
+      for (int n = 0; n < p.blk[k].nn; ++n)
+        for (int e = 0; e < 2 * p.blk[k].nkw; ++e, ++no) {
+          ncode[(b * nkw + e / 2) * ns + n] |= unsigned(p.ncode[no]) << (16 * (e & 1));
+          nwt[(b * 2 * nkw + e) * ns + n] = p.nwt[no];
+        }
       ho += size_t(nh);
       fo += size_t(nf);
     }
   });
   StageBlock *dblk;
   int *dhalo, *dbcode, *dwidth;
-  unsigned *dcode, *dface;
-  double *dgeo;
+  unsigned *dcode, *dface, *dgcode, *dncode;
+  double *dgeo, *dnwt;
   short *dlgat;
   if (int rc = C.upload(dblk, blk)) return rc;
   if (int rc = C.upload(dhalo, halo)) return rc;
@@ -254,13 +342,17 @@ int setup_stage_blocks(fvs_ctx &C, const StageMesh &M) {
   if (int rc = C.upload(dface, face)) return rc;
   if (int rc = C.upload(dgeo, geo)) return rc;
   if (int rc = C.upload(dlgat, lgat)) return rc;
+  if (int rc = C.upload(dgcode, gcode)) return rc;
+  if (int rc = C.upload(dncode, ncode)) return rc;
+  if (int rc = C.upload(dnwt, nwt)) return rc;
   HIPC(hipStreamSynchronize(C.stream));  // the host arrays end here
-  C.SL = {dblk, dhalo, dcode, dwidth, dface, dgeo, dbcode, dlgat, hs, cw, fs};
+  C.SL = {dblk, dhalo, dcode, dwidth, dface, dgeo, dbcode, dlgat, hs, cw, fs, dgcode, dncode, dnwt, ns, nkw};
   C.stage_bs = SH::BS;
-  C.stage_words = C.stage_faces = C.stage_halo = 0;
+  C.stage_words = C.stage_faces = C.stage_halo = C.stage_incidences = 0;
   for (const StageCut<SH> &p : parts) {
     C.stage_faces += long(p.face.size());
     C.stage_halo += long(p.halo.size());
+    C.stage_incidences += long(p.nwt.size());
     for (int w : p.width) C.stage_words += long(w) * kSlice;
   }
   C.stage_cells.clear();
@@ -281,4 +373,26 @@ int setup_stage(fvs_ctx &C, const StageMesh &M) {
     if (C.stage_bs) return 0;
   }
   return setup_stage_blocks<StageSmall>(C, M);
+}
+
+// The same for a Green-Gauss gradient: the table of the faces' periodic shifts
+// and the centres come first; without room for the shifts stage_bs stays 0.
+int setup_gg_stage(fvs_ctx &C, const StageMesh &M) {
+  const MeshPrep &m = C.mp;
+  size_t n = 0;
+  for (int e : m.edge_intr) {
+    const double sx = m.esx[e], sy = m.esy[e];
+    if (sx == 0.0 && sy == 0.0) continue;
+    size_t q = 0;
+    while (q < n && !(C.shifts.sx[q] == sx && C.shifts.sy[q] == sy)) ++q;
+    if (q < n) continue;
+    if (n == 15) return 0;
+    C.shifts.sx[n] = sx;
+    C.shifts.sy[n++] = sy;
+  }
+  std::vector<double2> cxy(C.N);
+  for (int i = 0; i < C.N; ++i) cxy[i] = make_double2(m.cx[C.perm[i]], m.cy[C.perm[i]]);
+  if (int rc = C.upload(C.cxy, cxy)) return rc;
+  C.pmode = M.fnb ? kGGCB : kGGNB;
+  return setup_stage(C, M);
 }
