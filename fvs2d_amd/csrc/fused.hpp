@@ -41,8 +41,8 @@ __device__ __forceinline__ void lsq_term(double xj, double yj, const double2 ci,
     sx[v] = fma(t, dx, sx[v]);
     sy[v] = fma(t, dy, sy[v]);
     if (LIM) {
-      mn[v] = (q[v] < mn[v]) ? q[v] : mn[v];
-      mx[v] = (q[v] > mx[v]) ? q[v] : mx[v];
+      mn[v] = lesser(q[v], mn[v]);
+      mx[v] = greater(q[v], mx[v]);
     }
   }
 }
@@ -180,7 +180,7 @@ __device__ __forceinline__ void interior_flux_v(const Phys &P, const double g[8]
     pR[v] = fma(phR, fma(-k2, gC, k1 * dR), wR[v]);
   }
   double fl[4], ws;
-  roe_flux(P.gamma, pL, pR, g[0], g[1], fl, ws);
+  roe_flux(P.gamma, P.gi, pL, pR, g[0], g[1], fl, ws);
   const double A = g[2];
   for (int v = 0; v < 4; ++v) fa[v] = fl[v] * A;
   wsa = ws * A;
@@ -217,7 +217,7 @@ __device__ __forceinline__ void boundary_flux_v(const Phys &P, double t, int ty,
     mms_state(g[5], g[6], pR);
   }
   double fl[4], ws;
-  roe_flux(P.gamma, pL, pR, nx, ny, fl, ws);
+  roe_flux(P.gamma, P.gi, pL, pR, nx, ny, fl, ws);
   const double A = g[2];
   for (int v = 0; v < 4; ++v) fa[v] = fl[v] * A;
   wsa = ws * A;
@@ -326,7 +326,7 @@ __device__ __forceinline__ void cell_update(int N, int i, bool valid, const Upd 
     cell_gather(in.sv, flux, speed, A.steady && A.first, acc, wacc);
     const double V = in.V;
     double R[4];
-    const double iV = 1.0 / V;  // one division per cell (src/residual.f90:164-166 divides each)
+    const double iV = recip(V);  // one per cell (src/residual.f90:164-166 divides each)
     for (int v = 0; v < 4; ++v) R[v] = -acc[v] * iV;
     double hs = A.h;
     if (A.steady) {

@@ -26,6 +26,7 @@
 #include <thread>
 #include <numeric>
 #include <tuple>
+#include <type_traits>
 #include <string>
 #include <vector>
 
@@ -194,25 +195,27 @@ __device__ __forceinline__ double cell_limiter_v(int lt, int nf, const double2 o
     }
     return phi;
   }
+  // a face whose value equals the cell's gives the candidate 1 (or, with Barth,
+  // no smaller one), so that no test is needed
   const double eps2 = venkat_eps2(vol);
   double bn = 1.0, bd = 1.0;  // smallest candidate so far (the cap at 1 to start)
+  auto candidates = [&](auto venkat) __attribute__((always_inline)) {
 #pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    const double q = w[v], dmax = mx[v] - q, dmin = mn[v] - q;
+    for (int v = 0; v < 4; ++v) {
+      const double q = w[v], dmax = mx[v] - q, dmin = mn[v] - q;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      if (k >= nf) break;
-      const double pf = q + o[k].x * gx[v] + o[k].y * gy[v];
-      const double b = pf - q;
-      if (b != 0.0) {
+      for (int k = 0; k < 4; ++k) {
+        if (k >= nf) break;
+        const double pf = q + o[k].x * gx[v] + o[k].y * gy[v];
+        const double b = pf - q;
         const double a = (b > 0.0) ? dmax : dmin;
         double n, d;
-        if (lt == 1) {
+        if (decltype(venkat)::value) {
           n = (a * a + eps2) + 2.0 * b * a;
           d = a * a + 2.0 * (b * b) + a * b + eps2;
         } else {
           n = (b > 0.0) ? a : -a;
-          d = (b > 0.0) ? b : -b;
+          d = fabs(b);
         }
         if (n * bd < bn * d) {
           bn = n;
@@ -220,8 +223,10 @@ __device__ __forceinline__ double cell_limiter_v(int lt, int nf, const double2 o
         }
       }
     }
-  }
-  return bn / bd;
+  };
+  if (lt == 1) candidates(std::true_type());
+  else candidates(std::false_type());
+  return quotient(bn, bd, recip(bd));
 }
 
 // the same with the cell's face offsets loaded here (into registers: every
@@ -261,8 +266,8 @@ __global__ __launch_bounds__(kBlock) void k_grad_lsq(int nbx, int N, const doubl
       gx[v] = gx[v] + c.x * d;
       gy[v] = gy[v] + c.y * d;
       if (LIM) {
-        mn[v] = (q[v] < mn[v]) ? q[v] : mn[v];
-        mx[v] = (q[v] > mx[v]) ? q[v] : mx[v];
+        mn[v] = lesser(q[v], mn[v]);
+        mx[v] = greater(q[v], mx[v]);
       }
     }
   }
@@ -290,8 +295,8 @@ __device__ __forceinline__ void stencil_minmax(int i, const int *__restrict__ so
 #pragma unroll
     for (int u = 0; u < 4; ++u)
       for (int v = 0; v < 4; ++v) {
-        mn[v] = (q[u][v] < mn[v]) ? q[u][v] : mn[v];
-        mx[v] = (q[u][v] > mx[v]) ? q[u][v] : mx[v];
+        mn[v] = lesser(q[u][v], mn[v]);
+        mx[v] = greater(q[u][v], mx[v]);
       }
   }
 }
@@ -310,15 +315,16 @@ __device__ __forceinline__ void gg_term(const double2 c, const double q[4], doub
   }
 }
 __device__ __forceinline__ void gg_divide(double V, double gx[4], double gy[4]) {
-  for (int v = 0; v < 4; ++v) gx[v] = gx[v] / V, gy[v] = gy[v] / V;
+  const double r = recip(V);
+  for (int v = 0; v < 4; ++v) gx[v] = quotient(gx[v], V, r), gy[v] = quotient(gy[v], V, r);
 }
 __device__ __forceinline__ void node_term(double c, const double q[4], double f[4]) {
   for (int v = 0; v < 4; ++v) f[v] = f[v] + c * q[v];
 }
 __device__ __forceinline__ void stencil_bounds(const double q[4], double mn[4], double mx[4]) {
   for (int v = 0; v < 4; ++v) {
-    mn[v] = (q[v] < mn[v]) ? q[v] : mn[v];
-    mx[v] = (q[v] > mx[v]) ? q[v] : mx[v];
+    mn[v] = lesser(q[v], mn[v]);
+    mx[v] = greater(q[v], mx[v]);
   }
 }
 
@@ -618,7 +624,7 @@ __global__ __launch_bounds__(kBlock) void k_flux_int(int nbx, int Fi, Phys P, co
     pR[v] = fma(phR, fma(-k2, gC, k1 * dR), wR[v]);
   }
   double fl[4], ws;
-  roe_flux(P.gamma, pL, pR, g[0], g[1], fl, ws);
+  roe_flux(P.gamma, P.gi, pL, pR, g[0], g[1], fl, ws);
   const double A = g[2];
   double fa[4] = {fl[0] * A, fl[1] * A, fl[2] * A, fl[3] * A};
   st4(FA, f, fa);
@@ -660,7 +666,7 @@ __global__ __launch_bounds__(kBlock) void k_flux_bnd(int Fb, int Fi, Phys P, dou
     mms_state(g[5], g[6], pR);
   }
   double fl[4], ws;
-  roe_flux(P.gamma, pL, pR, nx, ny, fl, ws);
+  roe_flux(P.gamma, P.gi, pL, pR, nx, ny, fl, ws);
   const double A = g[2];
   double fa[4] = {fl[0] * A, fl[1] * A, fl[2] * A, fl[3] * A};
   st4(FA, Fi + b, fa);
@@ -1038,7 +1044,7 @@ __global__ void k_roe_batch(int n, double g, const double *__restrict__ pL, cons
   double a[4], b[4], f[4], w;
   ld4(pL, i, a);
   ld4(pR, i, b);
-  roe_flux(g, a, b, nxy[2 * i], nxy[2 * i + 1], f, w);
+  roe_flux(g, 1.0 / (g - 1.0), a, b, nxy[2 * i], nxy[2 * i + 1], f, w);
   st4(F, i, f);
   ws[i] = w;
 }
@@ -2389,7 +2395,6 @@ StageIn stage_in(const fvs_ctx &C, double t, double *uout) {
   a.phisrc = C.opt.limiter > 0 ? 1 : 0;
   a.phi = C.phi;
   a.lt = C.opt.limiter;
-  a.nvrt = C.nvrt;
   a.loff = C.loff;
   a.vol = C.vol;
   a.ioff = C.frz_some ? C.dinst_off : nullptr;
@@ -2597,6 +2602,7 @@ static int create_impl(fvs_ctx **out, int nnodes, const double *xy, int ntri, in
   const double kPi = 3.14159265358979323846;
   Phys &P = C->P;
   P.gamma = opt->gamma;
+  P.gi = 1.0 / (opt->gamma - 1.0);
   P.kappa = (opt->recon == 3) ? opt->kappa : 0.0;  // src/input.f90:258-271
   P.pinf[0] = 1.0;                                  // src/data_solution.f90:56-59
   P.pinf[1] = opt->mach * std::cos(opt->aoa_deg * (kPi / 180.0));

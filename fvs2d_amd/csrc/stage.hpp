@@ -82,7 +82,6 @@ struct StageIn {
   int phisrc;  // without LIM: 0 limiter values 1, 1 read phi (frozen)
   double *phi;
   int lt;
-  const int *nvrt;
   const double2 *loff;
   const double *vol;
   const int *ioff, *frz;
@@ -181,11 +180,11 @@ __device__ __forceinline__ void stage_block(const StageIn &a, int lb, const Upd 
     g[5] = x.x; g[6] = x.y;
     g[2] = b[4 * S.fs + tid];
   }
-  // limiter: the cell's face offsets, count and volume, or its frozen value
+  // limiter: the cell's face offsets (zero past its last face, where they give
+  // the candidate 1) and volume, or its frozen value
   const bool phi_one = !LIM && !a.phisrc;
   double2 fo[4];
   double V = 1.0, ph = 1.0;
-  int nf = 0;
   bool keep = !LIM;
   double Gi[3] = {0.0, 0.0, 0.0};
   double u[4] = {0.0, 0.0, 0.0, 0.0};
@@ -221,7 +220,6 @@ __device__ __forceinline__ void stage_block(const StageIn &a, int lb, const Upd 
   }
   if (!phi_one && act) {
     if (LIM) {
-      nf = a.nvrt[id];
       V = a.vol[id];
 #pragma unroll
       for (int k = 0; k < 4; ++k)
@@ -319,7 +317,7 @@ __device__ __forceinline__ void stage_block(const StageIn &a, int lb, const Upd 
       lsq_apply_ginv(Gi[0], Gi[1], Gi[2], sx, sy, gx, gy);
     }
     if (LIM && !keep) {
-      ph = cell_limiter_v(a.lt, nf, fo, V, w, mn, mx, gx, gy);
+      ph = cell_limiter_v(a.lt, a.gw, fo, V, w, mn, mx, gx, gy);
       if (mine) a.phi[id] = ph;
     }
     if (!phi_one) at1(SH::P + 8 * tid) = ph;
@@ -397,7 +395,7 @@ __device__ __forceinline__ void stage_block(const StageIn &a, int lb, const Upd 
     if (mine) {
       double acc[4], wacc;
       cell_gather(in.sv, flux, speed, true, acc, wacc);
-      const double iV = 1.0 / in.V;  // as in the stage update
+      const double iV = recip(in.V);  // as in the stage update
       for (int v = 0; v < 4; ++v) acc[v] = -acc[v] * iV;
       const int c = a.ref[id];
       st4(a.rout, c, acc);
