@@ -170,14 +170,22 @@ __global__ __launch_bounds__(kBlock) void k_grad_lsqc(int N, int nb, const doubl
 __device__ __forceinline__ void interior_flux_v(const Phys &P, const double g[8], const double wL[4],
                                                 const double wR[4], const double gL[8], const double gR[8],
                                                 double phL, double phR, double fa[4], double &wsa) {
-  const double k2 = P.kappa / 2.0, k1 = 1.0 - P.kappa;
   double pL[4], pR[4];
   for (int v = 0; v < 4; ++v) {
-    const double gC = wR[v] - wL[v];
-    const double dL = fma(g[3], gL[v], g[4] * gL[4 + v]);
-    const double dR = fma(g[5], gR[v], g[6] * gR[4 + v]);
-    pL[v] = fma(phL, fma(k2, gC, k1 * dL), wL[v]);
-    pR[v] = fma(phR, fma(-k2, gC, k1 * dR), wR[v]);
+    pL[v] = fma(g[3], gL[v], g[4] * gL[4 + v]);
+    pR[v] = fma(g[5], gR[v], g[6] * gR[4 + v]);
+  }
+  if (P.kappa != 0.0) {  // else the increments are the gradients' alone
+    const double k2 = P.kappa / 2.0, k1 = 1.0 - P.kappa;
+    for (int v = 0; v < 4; ++v) {
+      const double gC = wR[v] - wL[v];
+      pL[v] = fma(k2, gC, k1 * pL[v]);
+      pR[v] = fma(-k2, gC, k1 * pR[v]);
+    }
+  }
+  for (int v = 0; v < 4; ++v) {
+    pL[v] = fma(phL, pL[v], wL[v]);
+    pR[v] = fma(phR, pR[v], wR[v]);
   }
   double fl[4], ws;
   roe_flux(P.gamma, P.gi, pL, pR, g[0], g[1], fl, ws);

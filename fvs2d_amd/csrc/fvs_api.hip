@@ -195,37 +195,40 @@ __device__ __forceinline__ double cell_limiter_v(int lt, int nf, const double2 o
     }
     return phi;
   }
-  // a face whose value equals the cell's gives the candidate 1 (or, with Barth,
-  // no smaller one), so that no test is needed
+  // Of the faces where a variable rises (falls), the one where it does most has
+  // the smallest candidate: both forms, capped at 1, fall with |b| for a given
+  // bound.  So each variable has two candidates, not one per face (a variable
+  // that does not rise or fall gives the candidate 1, or none smaller).
   const double eps2 = venkat_eps2(vol);
   double bn = 1.0, bd = 1.0;  // smallest candidate so far (the cap at 1 to start)
-  auto candidates = [&](auto venkat) __attribute__((always_inline)) {
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const double q = w[v], dmax = mx[v] - q, dmin = mn[v] - q;
+  for (int v = 0; v < 4; ++v) {
+    const double q = w[v];
+    double up = 0.0, down = 0.0;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        if (k >= nf) break;
-        const double pf = q + o[k].x * gx[v] + o[k].y * gy[v];
-        const double b = pf - q;
-        const double a = (b > 0.0) ? dmax : dmin;
-        double n, d;
-        if (decltype(venkat)::value) {
-          n = (a * a + eps2) + 2.0 * b * a;
-          d = a * a + 2.0 * (b * b) + a * b + eps2;
-        } else {
-          n = (b > 0.0) ? a : -a;
-          d = fabs(b);
-        }
-        if (n * bd < bn * d) {
-          bn = n;
-          bd = d;
-        }
+    for (int k = 0; k < 4; ++k) {
+      if (k >= nf) break;
+      const double pf = q + o[k].x * gx[v] + o[k].y * gy[v];
+      up = greater(up, pf - q);
+      down = lesser(down, pf - q);
+    }
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const double b = e == 0 ? up : down, a = (e == 0 ? mx[v] : mn[v]) - q;
+      double n, d;
+      if (lt == 1) {
+        n = (a * a + eps2) + 2.0 * b * a;
+        d = a * a + 2.0 * (b * b) + a * b + eps2;
+      } else {
+        n = fabs(a);
+        d = fabs(b);
+      }
+      if (n * bd < bn * d) {
+        bn = n;
+        bd = d;
       }
     }
-  };
-  if (lt == 1) candidates(std::true_type());
-  else candidates(std::false_type());
+  }
   return quotient(bn, bd, recip(bd));
 }
 
