@@ -308,10 +308,8 @@ __device__ __forceinline__ void cell_gather(const int sv[4], Flux flux, Speed sp
     const int f = (s > 0 ? s : -s) - 1;
     double fa[4];
     flux(f, fa);
-    if (s > 0)
-      for (int v = 0; v < 4; ++v) acc[v] = acc[v] + fa[v];
-    else
-      for (int v = 0; v < 4; ++v) acc[v] = acc[v] - fa[v];
+    const double sign = s > 0 ? 1.0 : -1.0;  // adds or subtracts, exactly, without a branch per lane
+    for (int v = 0; v < 4; ++v) acc[v] = fma(sign, fa[v], acc[v]);
     if (speeds) wacc = wacc + speed(f);
   }
 }
