@@ -126,16 +126,16 @@ def mlp_bench(steps: int):
     kt = net.kernel_times(10)
     flops_step = sum(v[1] * v[2] for v in kt.values())
     # algorithmic HBM bytes per launch of the matrix-core kernels (bfloat16
-    # activations, each streamed once; weights are KBs): the forward layer reads
-    # its input (68 features padded to 128 columns for the first layer) and
-    # writes Z and GELU(Z); backward-data reads dZ and Z_prev and writes
-    # dZ_prev; the weight gradient reads its input and dZ and writes float32
-    # partials of 64 row slices
-    kin = [128] + [width] * (depth - 1)
+    # activations, each streamed once; weights are KBs): the forward pass writes
+    # its input (68 features padded to 96 columns) and Z and GELU(Z) of every
+    # layer; the backward pass reads the last dZ and every other layer's Z and
+    # writes every layer's dZ; the weight gradient reads every layer's input and
+    # dZ and writes float32 partials of 64 row slices
+    kin = [96] + [width] * (depth - 1)
     slices = 64
-    hbm = {"gemm_forward": sum(M * k * 2 + 2 * M * width * 2 for k in kin) / depth,
-           "gemm_backward_data": 3 * M * width * 2,
-           "gemm_weight_grad": sum(M * k * 2 + M * width * 2 + slices * (k + 1) * width * 4 for k in kin) / depth}
+    hbm = {"gemm_forward": M * (6 * 4 + kin[0] * 2) + depth * 2 * M * width * 2,
+           "gemm_backward_data": 2 * depth * M * width * 2,
+           "gemm_weight_grad": sum(M * k * 2 + M * width * 2 + slices * (k + 1) * width * 4 for k in kin)}
     gemm = {k: v for k, v in kt.items() if k.startswith("gemm")}
     dom = max(gemm, key=lambda k: gemm[k][0] * gemm[k][2])
     ms, fl, _ = kt[dom]
