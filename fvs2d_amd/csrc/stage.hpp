@@ -97,12 +97,12 @@ struct StageIn {
   const int *ref;
   // sweep direction: blocks in ascending or descending order.  Alternating
   // stages start where the last one ended, whose lists and states the 256 MB
-  // memory-side cache still holds: 150 -> 139 us per stage on 2,097,152 cells
+  // memory-side cache still holds: 7% of a stage on 2,097,152 cells (now 125 us)
   int down;
 };
 
 // The shapes in use.  128-cell blocks: five wavefronts per SIMD and five blocks on
-// a CU (390 us per step on 2,097,152 cells, 418 us at four).  256-cell blocks:
+// a CU (7% per step faster than four on 2,097,152 cells; now 375 us).  256-cell blocks:
 // two blocks of 8 wavefronts on a CU, for meshes whose 128-cell blocks exceed the shape
 // (the rule is with setup_stage).
 using StageSmall = StageShape<128, 256, 192, 256, 5>;
@@ -411,10 +411,11 @@ __device__ __forceinline__ void stage_block(const StageIn &a, int lb, const Upd 
     cell_update(N, d.i0 + tid, mine, A, in, flux, speed, a.Ua, a.Ub, a.Facc, Wout, a.dtl, a.norm, a.amask);
 }
 
-// four wavefronts per SIMD with the limiter (its registers spill at five, 154 ->
-// 171 us per step on 522,242 cells), SH::WAVES without it
+// four wavefronts per SIMD with the limiter (its registers spill at five, 11%
+// slower on 522,242 cells) and with the weights that need a division or pow,
+// SH::WAVES without them
 template <class SH, int LIM, int PMODE>
-__global__ __launch_bounds__(SH::NT, LIM || PMODE > 1 ? 4 : SH::WAVES) void k_stage(StageIn a, Upd A,
+__global__ __launch_bounds__(SH::NT, LIM || PMODE == 2 || PMODE == 3 ? 4 : SH::WAVES) void k_stage(StageIn a, Upd A,
                                                                        const double *__restrict__ Win,
                                                                        double *__restrict__ Wout, int cons) {
   const int nbl = a.nb < 0 ? -a.nb : a.nb;  // with a block list, its length

@@ -363,9 +363,11 @@ int setup_stage_blocks(fvs_ctx &C, const StageMesh &M) {
 // The block shape: 128-cell blocks, unless many of them do not fit (O-grids,
 // whose stretched blocks have large halos) and the mesh is large enough for a
 // 256-cell block on every CU.  Measured, us per step in 128- / 256-cell blocks:
-// 2,097,152-cell vortex (nothing cut) 390 / 410; O-grids, limited, 128x64 (11%
-// more blocks) 39 / 45, 256x128 69 / 70, 300x150 79 / 75, 512x256 (19% more) 153 /
-// 143; a batch of 12 O-grids (18% more) 443 / 396.
+// 2,097,152-cell vortex (nothing cut) 5% less / more; O-grids, limited, 128x64 (11%
+// more blocks) 13% less / more, 256x128 63 / 64, 300x150 72 / 69, 384x192 100 / 91,
+// 512x256 (19% more) 136 / 124; a batch of 12 O-grids (17% more) 416 / 371.  Room
+// for 448 local cells in the large shape cuts 9 ranges of 512x256 instead of 86 and
+// changes nothing.
 int setup_stage(fvs_ctx &C, const StageMesh &M) {
   const bool large = C.opt.kernel_path != 2 && C.N >= 256 * StageLarge::BS;
   if (large && stage_blocks_per_range<StageSmall>(C, M) > 1.05) {
