@@ -627,6 +627,11 @@ constexpr int kHeadPart = kW * kOut + kOut;    // output-layer parameters
 // rows rs, rs + 8, ... in a thread.  (Both in one pass, 8 rows at a time: 4,096
 // rows 30 -> 19 us, 65,536 rows 48 -> 44; bound by vector instructions.)
 constexpr int kHeadThreads = 1024;
+// a + b with b as it was rounded: not fused with the product it comes from
+__device__ __forceinline__ float add_rounded(float a, float b) {
+#pragma clang fp contract(off)
+  return a + b;
+}
 __global__ __launch_bounds__(kHeadThreads, 4) void k_head(long M, long nvalid, float inv_no, const u16 *__restrict__ H,
                                                        u16 *Z, const float *__restrict__ Wh,
                                                        const float *__restrict__ bh, const float *__restrict__ T,
@@ -693,7 +698,7 @@ __global__ __launch_bounds__(kHeadThreads, 4) void k_head(long M, long nvalid, f
       const unsigned hw[4] = {h8[u].x, h8[u].y, h8[u].z, h8[u].w};
       const float dy = 2.f * d[o] * inv_no;
       for (int c = 0; c < 8; ++c) gw[c] += bf2f(u16((hw[c >> 1] >> (16 * (c & 1))) & 0xffffu)) * dy;
-      gb += dy;
+      gb = add_rounded(gb, dy);
       if (o == 0)
         for (int e = 0; e < kOut; ++e) ls += d[e] * d[e];
     }

@@ -47,3 +47,35 @@ def test_gradient_at_tile_edges(depth, n):
                                      bf16_mode=True)
     assert abs(loss - ref_loss) <= 1e-3 * ref_loss
     assert np.linalg.norm(g - ref) <= 2e-2 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("n", [3, 100, 192, 1088, 4160])
+def test_output_bias_gradient_adds_rounded_terms(n):
+    """With a row count that is no power of two, 1/(4n) is inexact, and the output
+    layer's bias gradient shows whether each row's term was rounded before it was
+    added.  Terms recomputed in numpy's float32 from the device's own predictions,
+    added in the kernel's order: rows rs, rs + 8, ... of 128, pairs of the eight
+    sums, the four pairs; then the blocks' sums by 16 groups and a tree."""
+    net = WarmStartNet(depth=2, batch=4160, seed=4)
+    raw, tgt = _data(n, n)
+    _, g = net.grad(raw, tgt)
+    rows = (n + 63) // 64 * 64
+    f = np.float32
+    d = np.zeros(((rows + 127) // 128 * 128, 4), f)
+    d[:n] = net.predict(raw) - tgt
+    dy = (f(2) * d) * f(1.0 / (4.0 * n))
+    part = []
+    for b in range(0, len(d), 128):
+        s = np.zeros((8, 4), f)
+        for k in range(0, 128, 8):
+            s = s + dy[b + k:b + k + 8]
+        s = s[0::2] + s[1::2]
+        part.append(((s[0] + s[1]) + s[2]) + s[3])
+    red = np.zeros((16, 4), f)
+    for b, p in enumerate(part):
+        red[b % 16] = red[b % 16] + p
+    h = 8
+    while h:
+        red[:h] = red[:h] + red[h:2 * h]
+        h //= 2
+    assert np.array_equal(g[-4:], red[0])
