@@ -259,17 +259,19 @@ double stage_blocks_per_range(const fvs_ctx &C, const StageMesh &M) {
   return double(cut.blk.size()) / double(std::max(1L, ranges));
 }
 
+constexpr long kStageGrain = 8;  // ranges per worker thread at least (some 50 us each)
+
 // Cuts all cells into blocks of shape SH and uploads the lists; C.stage_bs stays
 // 0 when a slice does not fit, or when so many ranges had to be cut that the
 // two-kernel path is faster.
 template <class SH>
 int setup_stage_blocks(fvs_ctx &C, const StageMesh &M) {
   const int N = C.N, Fi = C.Fi, cw = code_words(M);
-  const long nr = nblk(N, SH::BS), np = parallel_parts(nr, 64);
+  const long nr = nblk(N, SH::BS), np = parallel_parts(nr, kStageGrain);
   std::vector<short> lgat(size_t(C.GW) * N, 0);
   std::vector<StageCut<SH>> parts(np, StageCut<SH>(C, M, cw, lgat.data()));
   std::vector<char> ok(np, 1);
-  parallel_for(nr, 64, [&](long t, long b0, long b1) {
+  parallel_for(nr, kStageGrain, [&](long t, long b0, long b1) {
     for (long b = b0; b < b1 && ok[t]; ++b) ok[t] = parts[t].place_range(b) && parts[t].shift_ok;
   });
   std::vector<size_t> start(np + 1, 0);
