@@ -72,7 +72,8 @@ int fvs_mlp_predict(fvs_mlp *m, long long n, const float *raw, float *out);
 /* Times steps training steps with events around every launch.  Per kernel
  * class [features, forward GEMM, output layer + loss, weight-gradient GEMM,
  * backward-data GEMM, Adam]: mean ms per launch, matrix-core flops per launch
- * and launch count. */
+ * and launch count.  The features are formed in the forward launch (their class
+ * has no launches), and each GEMM class is one launch for all layers. */
 int fvs_mlp_kernel_times(fvs_mlp *m, int steps, double *ms6, double *flop6, int *launches6);
 /* device time of the last fvs_mlp_train call (ms) */
 double fvs_mlp_last_elapsed_ms(const fvs_mlp *m);
