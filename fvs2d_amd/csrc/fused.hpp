@@ -687,8 +687,9 @@ __global__ __launch_bounds__(BS, LIM ? 1 : 7) void k_grad_lsqh(int N, int nb, in
 
 // Residual norms of one step of instance k from the step's partials (fixed
 // order: kBlock threads over the whole slices of its cells, its cells in
-// slices shared with other instances, then a tree).  red: 4 kBlock doubles of
-// LDS; threads past kBlock only keep the barriers.
+// slices shared with other instances, then a tree) to out, if anyone asked (not
+// NULL).  red: 4 kBlock doubles of LDS; threads past kBlock only keep the
+// barriers.
 struct InstNorms {
   int ninst, ng, nsplit;     // instances, slices and shared slices
   const int *off;            // first cell of each instance
@@ -702,7 +703,7 @@ __device__ __forceinline__ void inst_norm_row(const InstNorms &I, int k, const d
   const int t = threadIdx.x;
   // an instance that is masked out repeats the norms of its last step
   if (I.act && !I.act[k]) {
-    if (t < 4) out[t] = I.last[4 * k + t];
+    if (out && t < 4) out[t] = I.last[4 * k + t];
     return;
   }
   const int a = I.off[k], b = I.off[k + 1];
@@ -742,20 +743,21 @@ __device__ __forceinline__ void inst_norm_row(const InstNorms &I, int k, const d
   }
   if (t < 4) {
     const double n = sqrt(red[t * kBlock] / double(b - a));
-    out[t] = n;
+    if (out) out[t] = n;
     if (keep_last) I.last[4 * k + t] = n;
   }
   __syncthreads();
 }
 
-// per-instance norms of the pending steps: one workgroup per instance and step
-__global__ __launch_bounds__(kBlock) void k_inst_norms(InstNorms I, int rows, const double *__restrict__ part,
+// per-instance norms of the pending steps from row r0 on (out NULL: only kept as
+// the instances' last): one workgroup per instance and step
+__global__ __launch_bounds__(kBlock) void k_inst_norms(InstNorms I, int r0, int rows, const double *__restrict__ part,
                                                        const double *__restrict__ d2, const int *__restrict__ ctr,
                                                        double *__restrict__ out) {
   __shared__ double red[4 * kBlock];
-  const int k = blockIdx.x, r = blockIdx.y;
+  const int k = blockIdx.x, r = r0 + blockIdx.y;
   inst_norm_row(I, k, part + 4 * long(r) * I.ng, d2 + 4 * long(r) * I.nsplit * kSlice, r == rows - 1,
-                out + 4 * ((long(ctr[0]) + r) * I.ninst + k), red);
+                out ? out + 4 * ((long(ctr[0]) + r) * I.ninst + k) : nullptr, red);
 }
 
 __global__ void k_counter(int *__restrict__ ctr, int value, int add) {

@@ -3136,16 +3136,19 @@ int launch_step(fvs_ctx &C, double told) {
 // output rows from the device's step counter on, which then advances.  One
 // launch of one workgroup per step (and instance): a reduction of its own after
 // every step left the chip idle meanwhile, 3.2 of 47 us per step on 8,192
-// cells and 70 of 580 us on a batch of 12 O-grids (983,040 cells).
+// cells and 70 of 580 us on a batch of 12 O-grids (983,040 cells).  In a batch
+// the last step's per-instance norms are formed also when nobody asked: an
+// instance masked out afterwards repeats them.
 int launch_norms(fvs_ctx &C, int rows, double *dn, double *dinst) {
   if (rows <= 0) return 0;
   {
     ProfScope ps(C, KC_NORM);
     if (dn && !C.nact)
       hipLaunchKernelGGL(k_norms, dim3(rows), dim3(kNormThreads), 0, C.stream, C.ng, C.N, C.part, C.dctr, dn);
-    if (dinst && C.ninst > 0)
-      hipLaunchKernelGGL(k_inst_norms, dim3(C.ninst, rows), dim3(kBlock), 0, C.stream, inst_norms_of(C), rows, C.part,
-                         C.d2s, C.dctr, dinst);
+    const int r0 = dinst ? 0 : rows - 1;
+    if (C.ninst > 0)
+      hipLaunchKernelGGL(k_inst_norms, dim3(C.ninst, rows - r0), dim3(kBlock), 0, C.stream, inst_norms_of(C), r0, rows,
+                         C.part, C.d2s, C.dctr, dinst);
   }
   hipLaunchKernelGGL(k_counter, dim3(1), dim3(1), 0, C.stream, C.dctr, rows, 1);
   HIPC(hipGetLastError());

@@ -474,8 +474,8 @@ struct PersistCtl {
   double *W0, *W1;          // primitive states: stage k of the launch reads W0 when k is even
   double *dn;               // whole-mesh norms, one row per step (NULL: none)
   int ng;                   // 64-cell slices
-  double *dinst;            // per-instance norms (NULL: none)
-  InstNorms inst;
+  double *dinst;            // per-instance norms (NULL: the last step's are only kept)
+  InstNorms inst;           // no instances on a single mesh
   int *ctr;                 // output row of the first step; advanced by nsteps at the end
   unsigned *bar;
   int *err;
@@ -509,10 +509,10 @@ __global__ __launch_bounds__(StageSmall::NT, 3) void k_steps_persistent(StageIn 
     // written by the last stage of the next step, two or more barriers later
     const long row = long(row0) + s;
     if (c.dn && blockIdx.x == 0) norm_row<StageSmall::NT>(c.ng, a.N, a.norm.part, c.dn + 4 * row, lds);
-    if (c.dinst)
+    if (c.dinst || s == c.nsteps - 1)
       for (int k = blockIdx.x; k < c.inst.ninst; k += gridDim.x)
         inst_norm_row(c.inst, k, a.norm.part, a.norm.d2, s == c.nsteps - 1,
-                      c.dinst + 4 * (row * c.inst.ninst + k), lds);
+                      c.dinst ? c.dinst + 4 * (row * c.inst.ninst + k) : nullptr, lds);
   }
   if (ok) ok = grid_barrier(c.bar, gridDim.x, gen, c.spin, c.err);
   if (ok && blockIdx.x == 0 && threadIdx.x == 0) c.ctr[0] = row0 + c.nsteps;
