@@ -2113,7 +2113,7 @@ int setup_device(fvs_ctx &C) {
   if (int rc = C.alloc(C.grad, 2 * n4)) return rc;
   if (int rc = C.alloc(C.phi, N)) return rc;
   if (int rc = C.alloc(C.dtl, N)) return rc;
-  if (int rc = C.alloc(C.FA, 4 * size_t(Fi + Fb))) return rc;
+  if (int rc = C.alloc(C.FA, 4 * std::max(size_t(Fi + Fb), size_t(N)))) return rc;
   if (int rc = C.alloc(C.WSA, size_t(Fi + Fb))) return rc;
   if (int rc = C.alloc(C.rout, n4)) return rc;
   if (int rc = C.alloc(C.wsout, N)) return rc;
@@ -2412,8 +2412,8 @@ StageIn stage_in(const fvs_ctx &C, double t, double *uout) {
   // the active-cell bits follow the list of 256-cell blocks, one per device cell
   a.amask = C.nact ? reinterpret_cast<const unsigned *>(C.blist + nblk(C.N)) : nullptr;
   a.pinf_inst = C.ninst > 0 ? C.dpinf_inst : nullptr;
-  a.rout = C.Uc;
-  a.wsout = C.Ub;
+  a.rout = C.rout;
+  a.wsout = C.wsout;
   a.ref = C.dperm;
   const int nb = int(C.stage_cells.size());
   a.nb = C.nact ? C.nslist : xcd_arg(nb, C.xcd_fused);
@@ -2489,17 +2489,19 @@ int finish_vortex_err(fvs_ctx &C, int rows, double *dst) {
 }
 
 // n values of the caller's array `out`, in its cell order, from device records:
-// reordered into tmp (a stage buffer, free between calls), then copied
-int give4(fvs_ctx &C, const double *src, int stride, double *tmp, double *out) {
-  hipLaunchKernelGGL(k_give4, dim3(nblk(C.N)), dim3(256), 0, C.stream, C.N, C.dip, src, stride, tmp);
+// reordered into FA (face fluxes live within one residual evaluation; the stage
+// states do not serve, a masked batch instance's launches still read them), then
+// copied
+int give4(fvs_ctx &C, const double *src, int stride, double *out) {
+  hipLaunchKernelGGL(k_give4, dim3(nblk(C.N)), dim3(256), 0, C.stream, C.N, C.dip, src, stride, C.FA);
   HIPC(hipGetLastError());
-  HIPC(hipMemcpyAsync(out, tmp, 4 * size_t(C.N) * sizeof(double), hipMemcpyDeviceToHost, C.stream));
+  HIPC(hipMemcpyAsync(out, C.FA, 4 * size_t(C.N) * sizeof(double), hipMemcpyDeviceToHost, C.stream));
   return 0;
 }
-int give1(fvs_ctx &C, const double *src, int stride, double *tmp, double *out) {
-  hipLaunchKernelGGL(k_give1, dim3(nblk(C.N)), dim3(256), 0, C.stream, C.N, C.dip, src, stride, tmp);
+int give1(fvs_ctx &C, const double *src, int stride, double *out) {
+  hipLaunchKernelGGL(k_give1, dim3(nblk(C.N)), dim3(256), 0, C.stream, C.N, C.dip, src, stride, C.FA);
   HIPC(hipGetLastError());
-  HIPC(hipMemcpyAsync(out, tmp, size_t(C.N) * sizeof(double), hipMemcpyDeviceToHost, C.stream));
+  HIPC(hipMemcpyAsync(out, C.FA, size_t(C.N) * sizeof(double), hipMemcpyDeviceToHost, C.stream));
   return 0;
 }
 
@@ -2828,8 +2830,8 @@ int fvs_mesh_lsq(const fvs_mesh *M, int *ptr, int *cell, double *w, double *coef
 
 int fvs_set_state(fvs_ctx *C, const double *cvar) try {
   if (!C || !cvar) return fail(FVS_EINVAL, "null argument");
-  HIPC(hipMemcpyAsync(C->Uc, cvar, 4 * size_t(C->N) * sizeof(double), hipMemcpyHostToDevice, C->stream));
-  hipLaunchKernelGGL(k_take_state, dim3(nblk(C->N)), dim3(256), 0, C->stream, C->N, C->opt.gamma, C->dip, C->Uc, C->U0,
+  HIPC(hipMemcpyAsync(C->FA, cvar, 4 * size_t(C->N) * sizeof(double), hipMemcpyHostToDevice, C->stream));
+  hipLaunchKernelGGL(k_take_state, dim3(nblk(C->N)), dim3(256), 0, C->stream, C->N, C->opt.gamma, C->dip, C->FA, C->U0,
                      C->W);
   HIPC(hipGetLastError());
   C->w_stale = false;
@@ -2843,7 +2845,7 @@ int fvs_set_state(fvs_ctx *C, const double *cvar) try {
 int fvs_get_state(fvs_ctx *C, double *cvar) try {
   if (int rc = need_state(C)) return rc;
   if (!cvar) return fail(FVS_EINVAL, "null argument");
-  if (int rc = give4(*C, C->U0, 4, C->Uc, cvar)) return rc;
+  if (int rc = give4(*C, C->U0, 4, cvar)) return rc;
   HIPC(hipStreamSynchronize(C->stream));
   return 0;
 } catch (...) {
@@ -2894,7 +2896,7 @@ int fvs_primitives(fvs_ctx *C, double *pvar) try {
   refresh_prim(*C);
   HIPC(hipGetLastError());
   if (pvar)
-    if (int rc = give4(*C, C->W, 4, C->Uc, pvar)) return rc;
+    if (int rc = give4(*C, C->W, 4, pvar)) return rc;
   HIPC(hipStreamSynchronize(C->stream));
   return 0;
 } catch (...) {
@@ -2908,8 +2910,8 @@ int fvs_gradient(fvs_ctx *C, double *grad) try {
     if (int rc = launch_gradient(*C, false)) return rc;
   if (grad) {
     // device record [x0..x3, y0..y3] -> Fortran grad(4,N,2)
-    if (int rc = give4(*C, C->grad, 8, C->Uc, grad)) return rc;
-    if (int rc = give4(*C, C->grad + 4, 8, C->Ub, grad + 4 * size_t(C->N))) return rc;
+    if (int rc = give4(*C, C->grad, 8, grad)) return rc;
+    if (int rc = give4(*C, C->grad + 4, 8, grad + 4 * size_t(C->N))) return rc;
   }
   HIPC(hipStreamSynchronize(C->stream));
   return 0;
@@ -2922,15 +2924,15 @@ int fvs_gradient_1var(fvs_ctx *C, const double *fc, double *dfc) try {
   // the scalar rides in slot 0 of a scratch primitive record; the gradient
   // kernels treat the four slots independently
   const size_t N = size_t(C->N);
-  HIPC(hipMemcpyAsync(C->Uc, fc, N * sizeof(double), hipMemcpyHostToDevice, C->stream));
-  hipLaunchKernelGGL(k_take1, dim3(nblk(C->N)), dim3(256), 0, C->stream, C->N, C->dip, C->Uc, C->rout);
+  HIPC(hipMemcpyAsync(C->FA, fc, N * sizeof(double), hipMemcpyHostToDevice, C->stream));
+  hipLaunchKernelGGL(k_take1, dim3(nblk(C->N)), dim3(256), 0, C->stream, C->N, C->dip, C->FA, C->rout);
   HIPC(hipGetLastError());
   std::swap(C->W, C->rout);
   int rc = launch_gradient(*C, false);
   std::swap(C->W, C->rout);
   if (rc) return rc;
-  if ((rc = give1(*C, C->grad, 8, C->Uc, dfc))) return rc;
-  if ((rc = give1(*C, C->grad + 4, 8, C->Ub, dfc + N))) return rc;
+  if ((rc = give1(*C, C->grad, 8, dfc))) return rc;
+  if ((rc = give1(*C, C->grad + 4, 8, dfc + N))) return rc;
   HIPC(hipStreamSynchronize(C->stream));
   return 0;
 } catch (...) {
@@ -2943,7 +2945,7 @@ int fvs_limiter(fvs_ctx *C, double *phi) try {
   if (C->opt.recon != 1 && C->opt.limiter > 0)
     if (int rc = launch_gradient(*C, true)) return rc;
   if (phi)
-    if (int rc = give1(*C, C->phi, 1, C->Uc, phi)) return rc;
+    if (int rc = give1(*C, C->phi, 1, phi)) return rc;
   HIPC(hipStreamSynchronize(C->stream));
   return 0;
 } catch (...) {
@@ -2961,15 +2963,15 @@ int fvs_compute_residual(fvs_ctx *C, double time, double *resid, double *ws) try
     // one launch, straight into the caller's order (five launches and two
     // reorderings without it: 55 us of device time on 221,778 limited cells)
     if (int rc = launch_stage(*C, A, time)) return rc;
-    if (resid) HIPC(hipMemcpyAsync(resid, C->Uc, 4 * N * sizeof(double), hipMemcpyDeviceToHost, C->stream));
-    if (ws) HIPC(hipMemcpyAsync(ws, C->Ub, N * sizeof(double), hipMemcpyDeviceToHost, C->stream));
+    if (resid) HIPC(hipMemcpyAsync(resid, C->rout, 4 * N * sizeof(double), hipMemcpyDeviceToHost, C->stream));
+    if (ws) HIPC(hipMemcpyAsync(ws, C->wsout, N * sizeof(double), hipMemcpyDeviceToHost, C->stream));
   } else {
     if (int rc = launch_fluxes(*C, time)) return rc;
     if (int rc = launch_update(*C, A)) return rc;
     if (resid)
-      if (int rc = give4(*C, C->rout, 4, C->Uc, resid)) return rc;
+      if (int rc = give4(*C, C->rout, 4, resid)) return rc;
     if (ws)
-      if (int rc = give1(*C, C->wsout, 1, C->Ub, ws)) return rc;
+      if (int rc = give1(*C, C->wsout, 1, ws)) return rc;
   }
   HIPC(hipStreamSynchronize(C->stream));
   return 0;
