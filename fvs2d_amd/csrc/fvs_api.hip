@@ -3260,12 +3260,12 @@ int launch_persistent(fvs_ctx &C, double t1, int nsteps, double *dn, double *din
 int run_steps(fvs_ctx &C, double t1, int nsteps, double *dn, double *dv, double *dinst, bool graph_ok = true) {
   const double dt = C.opt.dt;
   const int nst = (C.opt.rk_scheme == FVS_RK_SSP3) ? 3 : 4;
-  const bool cons = cons_stages(C);
-  if (!cons) ensure_prim(C);  // the stages read W
+  const bool persistent = graph_ok && C.use_persistent && !C.profiling && !dv && !time_dependent(C);
+  const bool cons = !persistent && cons_stages(C);  // persistent stages are primitive ones
+  if (!cons) ensure_prim(C);                        // the stages read W
   hipLaunchKernelGGL(k_counter, dim3(1), dim3(1), 0, C.stream, C.dctr, 0, 0);
   HIPC(hipGetLastError());
-  if (graph_ok && C.use_persistent && !C.profiling && !dv && !time_dependent(C))
-    return launch_persistent(C, t1, nsteps, dn, dinst);
+  if (persistent) return launch_persistent(C, t1, nsteps, dn, dinst);
   int s = 0;
   // graph replay: one captured graph covers an even number of stages so the
   // primitive-state buffers are back in place after each replay, and as many
