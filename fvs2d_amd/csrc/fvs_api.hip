@@ -220,8 +220,12 @@ __device__ __forceinline__ double cell_limiter_v(int lt, int nf, const double2 o
         n = (a * a + eps2) + 2.0 * b * a;
         d = a * a + 2.0 * (b * b) + a * b + eps2;
       } else {
-        n = fabs(a);
-        d = fabs(b);
+        // |a| / |b| with |b| scaled to [0.5, 1): increments may be as small as
+        // the variable (a velocity that is zero but for a distant disturbance),
+        // where products of them vanish and 1 / |b| is not representable
+        const int e2 = -__builtin_amdgcn_frexp_exp(b);
+        n = ldexp(fabs(a), e2);
+        d = ldexp(fabs(b), e2);
       }
       if (n * bd < bn * d) {
         bn = n;
