@@ -32,6 +32,7 @@
 
 #include "../../include/fvs2d.h"
 #include "kernels.hpp"
+#include "local_map.hpp"
 #include "mesh_prep.hpp"
 
 using namespace fvs;

@@ -1,39 +1,6 @@
 // Host side of the whole-stage kernel: its block lists (included by fvs_api.hip
 // after the context).
 
-// local index of a cell in a block (keys: id | periodic shift << 27), open
-// addressing
-class LocalMap {
-  std::vector<unsigned> key;
-  std::vector<int> val, used;
-  unsigned mask = 0;
-
- public:
-  void reset(size_t most) {
-    size_t n = 256;
-    while (n < 2 * most) n *= 2;
-    if (n > key.size()) {
-      key.assign(n, ~0u);
-      val.resize(n);
-      mask = unsigned(n - 1);
-    } else {
-      for (int h : used) key[h] = ~0u;
-    }
-    used.clear();
-  }
-  // the entry of k, created (fresh) if there is none
-  int &at(unsigned k, bool &fresh) {
-    unsigned h = (k * 2654435761u >> 8) & mask;
-    while (key[h] != ~0u && key[h] != k) h = (h + 1) & mask;
-    fresh = key[h] == ~0u;
-    if (fresh) {
-      key[h] = k;
-      used.push_back(int(h));
-    }
-    return val[h];
-  }
-};
-
 // the mesh as the block lists read it (device cell order)
 struct StageMesh {
   const std::vector<int> &gat;       // gw x N signed face slots
@@ -93,7 +60,7 @@ struct StageCut {
     r1.erase(std::unique(r1.begin(), r1.end()), r1.end());
     const int base = nblk(i1 - i0, kSlice) * kSlice, n1 = base + int(r1.size());
     if (n1 > SH::C1) return false;
-    map.reset(size_t(n1) * (2 * cw + 5) + (M.cnode ? 8 * size_t(SH::NT) : 0));
+    map.clear();
     bool fresh;
     for (int i = i0; i < i1; ++i) map.at(unsigned(i), fresh) = i - i0;
     hal.assign(r1.begin(), r1.end());
@@ -181,7 +148,7 @@ struct StageCut {
       return x;
     };
     nodes.clear();
-    if (M.cnode) nmap.reset(4 * size_t(n1));
+    nmap.clear();
     for (int q = 0; q < n1; ++q) {
       const int i = q < base ? (i0 + q < i1 ? i0 + q : -1) : r1[q - base];
       if (i < 0) continue;
@@ -211,9 +178,13 @@ struct StageCut {
       cells.push_back(make_int2(at, w));
       nkw = std::max(nkw, (w + 1) / 2);
     }
+    const auto fits = [&] { return base + int(hal.size()) - n1 <= SH::C1; };  // every state in LDS
     for (int2 c : cells)
-      for (int k = 0; k < c.y; ++k) local((*M.ncell)[size_t(c.x) + size_t(k) * kSlice]);
-    if (base + int(hal.size()) - n1 > SH::C1) return false;  // every state in LDS
+      for (int k = 0; k < c.y; ++k) {
+        local((*M.ncell)[size_t(c.x) + size_t(k) * kSlice]);
+        if (!fits()) return false;
+      }
+    if (!fits()) return false;
     for (int2 c : cells)
       for (int k = 0; k < 2 * nkw; ++k) {
         const size_t e = size_t(c.x) + size_t(k < c.y ? k : 0) * kSlice;
