@@ -39,10 +39,15 @@ struct StageShape {
 // One block: cells [i0, i0 + n0), base = n0 rounded up to whole slices, ring-1
 // cells at local indices base .. base + nr1 - 1, nh halo cells in all (ring 1,
 // ring 2; those past the C1 that ring 2 holds are far: read from HBM)
-// With node-based gradients nn nodes of up to 2 nkw cells each.
+// With node-based gradients nn nodes of up to 2 nkw cells each.  more: where the
+// block's far cells start, or its nodes' words past the first kNodeRegs (a block
+// with the one has none of the other).
 struct StageBlock {
-  int i0, n0, base, nr1, nh, nn, nkw, pad;
+  int i0, n0, base, nr1, nh, nn, nkw, more;
 };
+
+constexpr int kCodeRegs = 8;  // code words a thread holds in registers
+constexpr int kNodeRegs = 3;  // words of a node's cells
 
 // Per-block lists at fixed strides, so that a block's first loads wait on no
 // offset: halo cells id | periodic shift << 27 (-1 after the last); stencil
@@ -53,11 +58,16 @@ struct StageBlock {
 // Green-Gauss gradients: four byte offsets per gradient cell in two words, of its
 // face neighbours' states or of its nodes' values (16 n for the block's node n);
 // nodes: the byte offsets of their cells two to a word, and the cells' weights.
+// What a thread does not load at the start is packed instead, so that one node of
+// many cells does not widen the lists of every block: a slice's code words past
+// the first kCodeRegs, a block's far cells, its nodes' words (planes of nn) past
+// the first kNodeRegs with their weights.
 struct StageLists {
   const StageBlock *blk;
   const int *halo;
   const unsigned *code;
   const int *width;  // per slice: words used
+  const int *mstart;  // where its packed ones start, in 64s
   const unsigned *face;
   const double *geo;
   const int *bcode;
@@ -66,6 +76,9 @@ struct StageLists {
   const unsigned *gcode, *ncode;
   const double *nwt;
   int ns, nkw;  // strides: nodes, words of cells per node
+  const unsigned *morecode, *morenode;
+  const double *morewt;
+  const int *far;
 };
 
 struct StageIn {
@@ -107,9 +120,6 @@ struct StageIn {
 // (the rule is with setup_stage).
 using StageSmall = StageShape<128, 256, 192, 256, 5>;
 using StageLarge = StageShape<256, 512, 384, 512, 4>;
-
-constexpr int kCodeRegs = 8;  // code words a thread holds in registers
-constexpr int kNodeRegs = 3;  // words of a node's cells
 
 // Block lb of a whole stage.  LIM: the limiter is evaluated (and written for the
 // own cells).  PMODE: the LSQ weights as in lsq_term, or a Green-Gauss gradient,
@@ -249,9 +259,10 @@ __device__ __forceinline__ void stage_block(const StageIn &a, int lb, const Upd 
           add(nc[k] >> 16, nw8[2 * k + 1]);
         }
       for (int k = kNodeRegs; k < d.nkw; ++k) {
-        const unsigned w = ncl[k * S.ns];
-        add(w & 0xffffu, nwl[2 * k * S.ns]);
-        add(w >> 16, nwl[(2 * k + 1) * S.ns]);
+        const long q = d.more + long(k - kNodeRegs) * d.nn;
+        const unsigned w = S.morenode[q + tid];
+        add(w & 0xffffu, S.morewt[2 * q + tid]);
+        add(w >> 16, S.morewt[2 * q + d.nn + tid]);
       }
       at(SH::G + 16 * tid) = make_double2(f[0], f[1]);
       at(SH::G + 16 * NT + 16 * tid) = make_double2(f[2], f[3]);
@@ -271,6 +282,11 @@ __device__ __forceinline__ void stage_block(const StageIn &a, int lb, const Upd 
       if (GG) stencil_bounds(q, mn, mx);
       else lsq_term<LIM, PMODE>(cj.x, cj.y, ci, q, w, a.p, sx, sy, mn, mx);
     };
+    // the code words past those in registers (the offset is loaded only here: with
+    // the widths at the start it cost every small stage 0.2 us)
+    const auto packed = [&]() __attribute__((always_inline)) {
+      return S.morecode + (long(S.mstart[lb * SH::NSL + wv]) - kCodeRegs) * kSlice + (tid & 63);
+    };
     if (GG && !LIM) {
       // no stencil beyond the faces or nodes
     } else if (GG || d.nh <= d.nr1 + SH::C1) {
@@ -280,20 +296,25 @@ __device__ __forceinline__ void stage_block(const StageIn &a, int lb, const Upd 
           term(cr[k] & 0xffffu);
           term(cr[k] >> 16);
         }
-      for (int k = kCodeRegs; k < nw; ++k) {
-        const unsigned c = lc[k * kSlice];
-        term(c & 0xffffu);
-        term(c >> 16);
+      if (nw > kCodeRegs) {
+        const unsigned *lm = packed();
+        for (int k = kCodeRegs; k < nw; ++k) {
+          const unsigned c = lm[k * kSlice];
+          term(c & 0xffffu);
+          term(c >> 16);
+        }
       }
     } else {
       // ring 2 does not fit: the codes past it are far cells, from HBM
+      const unsigned *lm = packed();
       for (int k = 0; k < 2 * nw; ++k) {
-        const unsigned o = (lc[(k >> 1) * kSlice] >> (16 * (k & 1))) & 0xffffu;
+        const int word = k >> 1;
+        const unsigned o = ((word < kCodeRegs ? lc : lm)[word * kSlice] >> (16 * (k & 1))) & 0xffffu;
         if (o < unsigned(SH::FAR)) {
           term(o);
           continue;
         }
-        const int e = hl[d.nr1 + SH::C1 + int((o - SH::FAR) >> 4)], j = e & 0x07ffffff, sh = unsigned(e) >> 27;
+        const int e = S.far[d.more + int((o - SH::FAR) >> 4)], j = e & 0x07ffffff, sh = unsigned(e) >> 27;
         double2 xy = a.cxy[j];
         double q[4];
         ld4(Win, j, q);

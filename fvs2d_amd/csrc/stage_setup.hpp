@@ -23,11 +23,12 @@ template <class SH>
 struct StageCut {
   const fvs_ctx &C;
   const StageMesh &M;
-  const int cw;       // code words of the widest stencil
+  const int cw;       // code words per cell at a fixed stride
   short *const lgat;  // gw x N signed 1-based local faces
   std::vector<StageBlock> blk;
-  std::vector<unsigned> halo, face, code, gcode;
-  std::vector<int> slot, nf, width;
+  std::vector<unsigned> halo, face, code, morecode, gcode;
+  std::vector<int> slot, nf;
+  std::vector<int2> width;
   std::vector<unsigned short> ncode;  // per block nn x 2 nkw
   std::vector<double> nwt;
   bool shift_ok = true;  // every periodic shift of a face is in the table
@@ -65,18 +66,26 @@ struct StageCut {
     for (int i = i0; i < i1; ++i) map.at(unsigned(i), fresh) = i - i0;
     hal.assign(r1.begin(), r1.end());
     for (size_t k = 0; k < r1.size(); ++k) map.at(unsigned(r1[k]), fresh) = base + int(k);
-    const size_t c0 = code.size();
+    const size_t c0 = code.size(), m0 = morecode.size();
+    const auto drop_codes = [&] { code.resize(c0), morecode.resize(m0); };
     code.resize(c0 + size_t(SH::NSL) * cw * kSlice, 0u);
-    int w2[SH::NSL];
+    int2 w2[SH::NSL];
     for (int s = 0; s < SH::NSL; ++s) {
-      w2[s] = 0;
-      for (int l = 0; l < kSlice; ++l) {
+      const auto cell = [&](int l) {
         const int q = s * kSlice + l;
-        const int i = q < base ? (i0 + q < i1 ? i0 + q : -1) : (q < n1 ? r1[q - base] : -1);
-        if (i < 0 || cw == 0) continue;
+        return q < base ? (i0 + q < i1 ? i0 + q : -1) : (q < n1 ? r1[q - base] : -1);
+      };
+      w2[s] = make_int2(0, int(morecode.size() / kSlice));
+      for (int l = 0; l < kSlice && cw > 0; ++l)
+        if (cell(l) >= 0) w2[s].x = std::max(w2[s].x, (M.wid[cell(l) / kSlice] + 1) / 2);
+      morecode.resize(morecode.size() + size_t(std::max(0, w2[s].x - cw)) * kSlice, 0u);
+      unsigned *const fixed = code.data() + c0 + size_t(s) * cw * kSlice;
+      unsigned *const more = morecode.data() + size_t(w2[s].y) * kSlice;
+      for (int l = 0; l < kSlice && cw > 0; ++l) {
+        const int q = s * kSlice + l, i = cell(l);
+        if (i < 0) continue;
         const int sg = i / kSlice, li = i % kSlice;
-        w2[s] = std::max(w2[s], (M.wid[sg] + 1) / 2);
-        for (int k = 0; k < 2 * cw; ++k) {
+        for (int k = 0; k < 2 * w2[s].x; ++k) {
           int v = q;  // past the cell's own stencil: the cell itself (a zero term)
           if (k < M.wid[sg]) {
             const unsigned key = M.code[M.off[sg] + long(k) * kSlice + li];
@@ -87,20 +96,21 @@ struct StageCut {
             }
             v = x;
           }
-          code[c0 + (size_t(s) * cw + k / 2) * kSlice + l] |= unsigned(offset(v, n1)) << (16 * (k & 1));
+          unsigned *const word = k / 2 < cw ? fixed + k / 2 * kSlice : more + (k / 2 - cw) * kSlice;
+          word[l] |= unsigned(offset(v, n1)) << (16 * (k & 1));
         }
       }
     }
     int nn = 0, nkw = 0;
     const size_t g0 = gcode.size();
     if (M.ngg > 0 && !green_gauss(i0, i1, base, n1, nn, nkw)) {
-      code.resize(c0);
+      drop_codes();
       gcode.resize(g0);
       return false;
     }
     const int nl = base + int(hal.size());
     if (nl - n1 > SH::C1 && (i1 - i0 > kSlice || offset(nl - 1, n1) > 0xfff0)) {
-      code.resize(c0);
+      drop_codes();
       return false;
     }
     blk.push_back({i0, i1 - i0, base, int(r1.size()), int(hal.size()), nn, nkw, 0});
@@ -214,7 +224,8 @@ struct StageCut {
 };
 
 int code_words(const StageMesh &M) {
-  return M.wid.empty() ? 0 : std::max(1, (*std::max_element(M.wid.begin(), M.wid.end()) + 1) / 2);
+  if (M.wid.empty()) return 0;
+  return std::min(kCodeRegs, std::max(1, (*std::max_element(M.wid.begin(), M.wid.end()) + 1) / 2));
 }
 
 // Blocks per range of SH::BS cells, from up to 256 ranges spread over the cells
@@ -245,25 +256,34 @@ int setup_stage_blocks(fvs_ctx &C, const StageMesh &M) {
   parallel_for(nr, kStageGrain, [&](long t, long b0, long b1) {
     for (long b = b0; b < b1 && ok[t]; ++b) ok[t] = parts[t].place_range(b) && parts[t].shift_ok;
   });
-  std::vector<size_t> start(np + 1, 0);
+  std::vector<size_t> start(np + 1, 0), mstart(np + 1, 0);
   int hs = 1, fs = 1, ns = 0, nkw = 0;
+  size_t nmore = 0, nfar = 0;  // packed words of nodes and far cells so far
   for (long t = 0; t < np; ++t) {
     if (!ok[t]) return 0;
     start[t + 1] = start[t] + parts[t].blk.size();
-    for (const StageBlock &d : parts[t].blk) {
-      hs = std::max(hs, d.nh);
+    mstart[t + 1] = mstart[t] + parts[t].morecode.size() / kSlice;
+    for (StageBlock &d : parts[t].blk) {
+      hs = std::max(hs, std::min(d.nh, d.nr1 + SH::C1));
       ns = std::max(ns, d.nn);
-      nkw = std::max(nkw, d.nkw);
+      nkw = std::max(nkw, std::min(d.nkw, kNodeRegs));
+      d.more = int(d.nn ? nmore : nfar);
+      nmore += size_t(d.nn) * std::max(0, d.nkw - kNodeRegs);
+      nfar += std::max(0, d.nh - d.nr1 - SH::C1);
     }
     for (int n : parts[t].nf) fs = std::max(fs, n);
   }
   const size_t nb = start[np];
+  if (std::max({mstart[np], nmore, nfar}) > size_t(INT32_MAX)) return 0;
   if (N > kStageSmallMesh && double(nb) > kStageMostBlocks * double(nr)) return 0;
   hs = (hs + 31) / 32 * 32;  // strides of whole cache lines
   fs = (fs + 15) / 16 * 16;
   ns = (ns + 31) / 32 * 32;
   std::vector<StageBlock> blk(nb);
-  std::vector<int> halo(nb * hs), bcode(nb * fs), width(nb * SH::NSL);
+  std::vector<int> halo(nb * hs), far(nfar), bcode(nb * fs);
+  std::vector<int> width(nb * SH::NSL), wstart(nb * SH::NSL);
+  std::vector<unsigned> morecode(mstart[np] * kSlice), morenode(nmore);
+  std::vector<double> morewt(2 * nmore);
   std::vector<unsigned> code(nb * SH::NSL * cw * kSlice), face(nb * fs);
   std::vector<double> geo(nb * fs * 5), nwt(nb * 2 * nkw * ns);
   std::vector<unsigned> gcode(M.ngg > 0 ? nb * 2 * SH::C1 : 0), ncode(nb * nkw * ns);
@@ -272,13 +292,19 @@ int setup_stage_blocks(fvs_ctx &C, const StageMesh &M) {
     size_t ho = 0, fo = 0, no = 0;
     std::copy(p.gcode.begin(), p.gcode.end(), gcode.begin() + (M.ngg > 0 ? start[t] * 2 * SH::C1 : 0));
     std::copy(p.blk.begin(), p.blk.end(), blk.begin() + start[t]);
-    std::copy(p.width.begin(), p.width.end(), width.begin() + start[t] * SH::NSL);
+    for (size_t k = 0; k < p.width.size(); ++k) {
+      width[start[t] * SH::NSL + k] = p.width[k].x;
+      wstart[start[t] * SH::NSL + k] = p.width[k].y + int(mstart[t]);
+    }
+    std::copy(p.morecode.begin(), p.morecode.end(), morecode.begin() + mstart[t] * kSlice);
     std::copy(p.code.begin(), p.code.end(), code.begin() + start[t] * SH::NSL * cw * kSlice);
     for (size_t k = 0; k < p.blk.size(); ++k) {
       const size_t b = start[t] + k;
-      const int nh = p.blk[k].nh, nf = p.nf[k];
-      std::fill(std::copy(p.halo.begin() + ho, p.halo.begin() + ho + nh, halo.begin() + b * hs),
-                halo.begin() + (b + 1) * hs, -1);
+      const StageBlock &d = p.blk[k];
+      const int nh = d.nh, nf = p.nf[k];
+      const auto h0 = p.halo.begin() + ho, h1 = h0 + std::min(nh, d.nr1 + SH::C1);
+      std::fill(std::copy(h0, h1, halo.begin() + b * hs), halo.begin() + (b + 1) * hs, -1);
+      if (h1 != h0 + nh) std::copy(h1, h0 + nh, far.begin() + d.more);
       std::fill(std::copy(p.face.begin() + fo, p.face.begin() + fo + nf, face.begin() + b * fs),
                 face.begin() + (b + 1) * fs, ~0u);
       double *q = &geo[b * fs * 5];
@@ -293,24 +319,32 @@ int setup_stage_blocks(fvs_ctx &C, const StageMesh &M) {
         if (f >= Fi)
           bcode[b * fs + e] = M.fbt[bq] | ((C.ninst > 0 ? C.inst_of_real[C.perm[M.fbc[bq]]] : 0) << 2);
       }
-      for (int n = 0; n < p.blk[k].nn; ++n)
-        for (int e = 0; e < 2 * p.blk[k].nkw; ++e, ++no) {
-          ncode[(b * nkw + e / 2) * ns + n] |= unsigned(p.ncode[no]) << (16 * (e & 1));
-          nwt[(b * 2 * nkw + e) * ns + n] = p.nwt[no];
+      for (int n = 0; n < d.nn; ++n)
+        for (int e = 0; e < 2 * d.nkw; ++e, ++no) {
+          const unsigned v = unsigned(p.ncode[no]) << (16 * (e & 1));
+          if (e / 2 < nkw) {
+            ncode[(b * nkw + e / 2) * ns + n] |= v;
+            nwt[(b * 2 * nkw + e) * ns + n] = p.nwt[no];
+          } else {
+            morenode[size_t(d.more) + size_t(e / 2 - nkw) * d.nn + n] |= v;
+            morewt[2 * size_t(d.more) + size_t(e - 2 * nkw) * d.nn + n] = p.nwt[no];
+          }
         }
       ho += size_t(nh);
       fo += size_t(nf);
     }
   });
   StageBlock *dblk;
-  int *dhalo, *dbcode, *dwidth;
-  unsigned *dcode, *dface, *dgcode, *dncode;
-  double *dgeo, *dnwt;
+  int *dhalo, *dbcode, *dfar;
+  int *dwidth, *dwstart;
+  unsigned *dcode, *dface, *dgcode, *dncode, *dmorecode, *dmorenode;
+  double *dgeo, *dnwt, *dmorewt;
   short *dlgat;
   if (int rc = C.upload(dblk, blk)) return rc;
   if (int rc = C.upload(dhalo, halo)) return rc;
   if (int rc = C.upload(dbcode, bcode)) return rc;
   if (int rc = C.upload(dwidth, width)) return rc;
+  if (int rc = C.upload(dwstart, wstart)) return rc;
   if (int rc = C.upload(dcode, code)) return rc;
   if (int rc = C.upload(dface, face)) return rc;
   if (int rc = C.upload(dgeo, geo)) return rc;
@@ -318,15 +352,20 @@ int setup_stage_blocks(fvs_ctx &C, const StageMesh &M) {
   if (int rc = C.upload(dgcode, gcode)) return rc;
   if (int rc = C.upload(dncode, ncode)) return rc;
   if (int rc = C.upload(dnwt, nwt)) return rc;
+  if (int rc = C.upload(dmorecode, morecode)) return rc;
+  if (int rc = C.upload(dmorenode, morenode)) return rc;
+  if (int rc = C.upload(dmorewt, morewt)) return rc;
+  if (int rc = C.upload(dfar, far)) return rc;
   HIPC(hipStreamSynchronize(C.stream));  // the host arrays end here
-  C.SL = {dblk, dhalo, dcode, dwidth, dface, dgeo, dbcode, dlgat, hs, cw, fs, dgcode, dncode, dnwt, ns, nkw};
+  C.SL = {dblk, dhalo, dcode, dwidth, dwstart, dface, dgeo, dbcode, dlgat, hs, cw, fs, dgcode, dncode, dnwt, ns, nkw,
+          dmorecode, dmorenode, dmorewt, dfar};
   C.stage_bs = SH::BS;
   C.stage_words = C.stage_faces = C.stage_halo = C.stage_incidences = 0;
   for (const StageCut<SH> &p : parts) {
     C.stage_faces += long(p.face.size());
     C.stage_halo += long(p.halo.size());
     C.stage_incidences += long(p.nwt.size());
-    for (int w : p.width) C.stage_words += long(w) * kSlice;
+    for (int2 w : p.width) C.stage_words += long(w.x) * kSlice;
   }
   C.stage_cells.clear();
   for (const StageBlock &d : blk) C.stage_cells.push_back(make_int2(d.i0, d.n0));
