@@ -1983,7 +1983,7 @@ int setup_device(fvs_ctx &C) {
         // the whole stage in one kernel, or the lists of two kernels per stage
         if (C.fused && C.opt.recon != 1 && C.opt.kernel_path != 3)
           if (int rc = setup_stage(C, {gat, fic, fig, fbc, fbt, fbg, off, wid, code})) return rc;
-        if (!C.stage_bs && C.opt.recon != 1 && C.opt.kernel_path != 3)
+        if (!whole_stage(C) && C.opt.recon != 1 && C.opt.kernel_path != 3)
           if (int rc = setup_grad_halo(C, off, wid, code)) return rc;
       }
     }
@@ -2096,9 +2096,9 @@ int setup_device(fvs_ctx &C) {
   }
   if (gm.ngg > 0 && C.fused && C.opt.recon != 1 && C.opt.kernel_path == 0 && C.ninst == 0 && N < (1 << 27))
     if (int rc = setup_gg_stage(C, gm)) return rc;
-  if (!C.stage_bs && !bcode.empty())
+  if (!whole_stage(C) && !bcode.empty())
     if (int rc = setup_grad_halo(C, boff, bwid, bcode)) return rc;
-  if (C.fused && !C.stage_bs) {
+  if (C.fused && !whole_stage(C)) {
     if (int rc = flux_lists(C, gm)) return rc;
     C.two_kernel = true;
   }
@@ -3234,29 +3234,35 @@ int launch_persistent(fvs_ctx &C, double t1, int nsteps, double *dn, double *din
   c.spin = 1u << 22;
   C.norm_row = 0;
   StageIn a = stage_in(C, t1, nullptr);
-  const size_t lds = std::max(size_t(StageSmall::END), size_t(4) * kNormThreads * sizeof(double));
   const bool lim = o.limiter > 0 && !C.limiter_frozen;
+  const bool large = C.stage_bs == StageLarge::BS;
+  const int nt = large ? StageLarge::NT : StageSmall::NT;
+  const size_t lds = std::max(size_t(large ? StageLarge::END : StageSmall::END), size_t(4) * kNormThreads * sizeof(double));
   const void *fn = nullptr;
-#define FVS_PK(L, PM) fn = reinterpret_cast<const void *>(&k_steps_persistent<L, PM>)
-  if (lim) {
-    if (C.pmode == 0) FVS_PK(1, 0);
-    else if (C.pmode == 1) FVS_PK(1, 1);
-    else if (C.pmode == 2) FVS_PK(1, 2);
-    else FVS_PK(1, 3);
+#define FVS_PK(SH, L, PM) fn = reinterpret_cast<const void *>(&k_steps_persistent<SH, L, PM>)
+#define FVS_PK_PM(SH, L)                     \
+  do {                                       \
+    if (C.pmode == 0) FVS_PK(SH, L, 0);      \
+    else if (C.pmode == 1) FVS_PK(SH, L, 1); \
+    else if (C.pmode == 2) FVS_PK(SH, L, 2); \
+    else FVS_PK(SH, L, 3);                   \
+  } while (0)
+  if (large) {
+    if (lim) FVS_PK_PM(StageLarge, 1);
+    else FVS_PK_PM(StageLarge, 0);
   } else {
-    if (C.pmode == 0) FVS_PK(0, 0);
-    else if (C.pmode == 1) FVS_PK(0, 1);
-    else if (C.pmode == 2) FVS_PK(0, 2);
-    else FVS_PK(0, 3);
+    if (lim) FVS_PK_PM(StageSmall, 1);
+    else FVS_PK_PM(StageSmall, 0);
   }
+#undef FVS_PK_PM
 #undef FVS_PK
   int per_cu = 0;
-  HIPC(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, StageSmall::NT, lds));
+  HIPC(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, nt, lds));
   if (per_cu < 1) return fail(FVS_ESTATE, "persistent launch: the whole-stage kernel does not fit on a compute unit");
   const int grid = std::min(c.nlaunch, per_cu * C.ncu);
   hipLaunchKernelGGL(k_barrier_reset, dim3(1), dim3(64), 0, C.stream, C.pbar, C.perr);
   void *args[] = {&a, &c};
-  HIPC(hipLaunchCooperativeKernel(fn, dim3(grid), dim3(StageSmall::NT), args, unsigned(lds), C.stream));
+  HIPC(hipLaunchCooperativeKernel(fn, dim3(grid), dim3(nt), args, unsigned(lds), C.stream));
   C.persist_ran = true;
   if ((nsteps * c.nst) % 2) std::swap(C.W, C.Walt);
   return 0;
@@ -3429,7 +3435,7 @@ int fvs_phase_times(const fvs_ctx *C, double *sec4) try {
 
 int fvs_set_persistent(fvs_ctx *C, int on) try {
   if (!C) return fail(FVS_EINVAL, "null context");
-  if (on && !(C->opt.kernel_path == 2 && C->stage_bs == StageSmall::BS))
+  if (on && !(C->opt.kernel_path == 2 && C->stage_bs))
     return fail(FVS_ESTATE, "persistent launches run the whole-stage kernel: create the context with kernel_path 2 "
                             "(LSQ gradient)");
   C->use_persistent = on != 0;

@@ -449,7 +449,7 @@ __global__ __launch_bounds__(SH::NT, LIM || PMODE == 2 || PMODE == 3 ? 4 : SH::W
 
 // ---------------------------------------------------------------------------
 // Persistent whole-step kernel: one cooperative launch runs nsteps time steps
-// of the whole-stage block body (128-cell blocks) over the launch-block list (the ragged batch's
+// of the whole-stage block body over the launch-block list (the ragged batch's
 // active blocks, or every block), with a grid-wide barrier after each stage
 // and the step's residual norms reduced in the same launch.
 // ---------------------------------------------------------------------------
@@ -503,8 +503,8 @@ struct PersistCtl {
   unsigned spin;
 };
 
-template <int LIM, int PMODE>
-__global__ __launch_bounds__(StageSmall::NT, 3) void k_steps_persistent(StageIn a, PersistCtl c) {
+template <class SH, int LIM, int PMODE>
+__global__ __launch_bounds__(SH::NT, SH::NT > 256 ? 4 : 3) void k_steps_persistent(StageIn a, PersistCtl c) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   double *lds = reinterpret_cast<double *>(smem);
   unsigned gen = 0;
@@ -519,7 +519,7 @@ __global__ __launch_bounds__(StageSmall::NT, 3) void k_steps_persistent(StageIn 
       double *Wout = par ? c.W0 : c.W1;
       for (int q = blockIdx.x; q < c.nlaunch; q += gridDim.x) {
         const int lb = a.blist ? a.blist[q] : q;
-        stage_block<StageSmall, LIM, PMODE>(a, lb, A, Win, Wout, 0);
+        stage_block<SH, LIM, PMODE>(a, lb, A, Win, Wout, 0);
         __syncthreads();  // the next block's staging overwrites this one's LDS
       }
       ok = grid_barrier(c.bar, gridDim.x, gen, c.spin, c.err);
@@ -529,7 +529,7 @@ __global__ __launch_bounds__(StageSmall::NT, 3) void k_steps_persistent(StageIn 
     // this step's norms; the partials and increments they read are next
     // written by the last stage of the next step, two or more barriers later
     const long row = long(row0) + s;
-    if (c.dn && blockIdx.x == 0) norm_row<StageSmall::NT>(c.ng, a.N, a.norm.part, c.dn + 4 * row, lds);
+    if (c.dn && blockIdx.x == 0) norm_row<SH::NT>(c.ng, a.N, a.norm.part, c.dn + 4 * row, lds);
     if (c.dinst || s == c.nsteps - 1)
       for (int k = blockIdx.x; k < c.inst.ninst; k += gridDim.x)
         inst_norm_row(c.inst, k, a.norm.part, a.norm.d2, s == c.nsteps - 1,

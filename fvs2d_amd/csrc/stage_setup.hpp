@@ -245,7 +245,8 @@ constexpr long kStageGrain = 8;  // ranges per worker thread at least (some 50 u
 
 // Cuts all cells into blocks of shape SH and uploads the lists; C.stage_bs stays
 // 0 when a slice does not fit, or when so many ranges had to be cut that the
-// two-kernel path is faster.
+// two-kernel path is faster.  With kernel_path 2 there are lists in that case too,
+// for persistent launches, and C.use_stage is false.
 template <class SH>
 int setup_stage_blocks(fvs_ctx &C, const StageMesh &M) {
   const int N = C.N, Fi = C.Fi, cw = code_words(M);
@@ -275,7 +276,8 @@ int setup_stage_blocks(fvs_ctx &C, const StageMesh &M) {
   }
   const size_t nb = start[np];
   if (std::max({mstart[np], nmore, nfar}) > size_t(INT32_MAX)) return 0;
-  if (N > kStageSmallMesh && double(nb) > kStageMostBlocks * double(nr)) return 0;
+  const bool cut = N > kStageSmallMesh && double(nb) > kStageMostBlocks * double(nr);
+  if (cut && C.opt.kernel_path != 2) return 0;
   hs = (hs + 31) / 32 * 32;  // strides of whole cache lines
   fs = (fs + 15) / 16 * 16;
   ns = (ns + 31) / 32 * 32;
@@ -360,6 +362,7 @@ int setup_stage_blocks(fvs_ctx &C, const StageMesh &M) {
   C.SL = {dblk, dhalo, dcode, dwidth, dwstart, dface, dgeo, dbcode, dlgat, hs, cw, fs, dgcode, dncode, dnwt, ns, nkw,
           dmorecode, dmorenode, dmorewt, dfar};
   C.stage_bs = SH::BS;
+  C.use_stage = !cut;
   C.stage_words = C.stage_faces = C.stage_halo = C.stage_incidences = 0;
   for (const StageCut<SH> &p : parts) {
     C.stage_faces += long(p.face.size());
@@ -386,7 +389,13 @@ int setup_stage(fvs_ctx &C, const StageMesh &M) {
     if (int rc = setup_stage_blocks<StageLarge>(C, M)) return rc;
     if (C.stage_bs) return 0;
   }
-  return setup_stage_blocks<StageSmall>(C, M);
+  if (int rc = setup_stage_blocks<StageSmall>(C, M)) return rc;
+  if (C.stage_bs || C.opt.kernel_path != 2) return 0;
+  // persistent launches of cells whose 64-cell blocks exceed the small shape
+  // (quadrilaterals in rows): 64 cells and their up to 256 neighbours fit the large
+  if (int rc = setup_stage_blocks<StageLarge>(C, M)) return rc;
+  C.use_stage = false;
+  return 0;
 }
 
 // The same for a Green-Gauss gradient: the table of the faces' periodic shifts

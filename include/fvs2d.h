@@ -74,8 +74,10 @@ typedef struct {
                               one);
                            1: face-flux buffer kernels only;
                            2: the whole stage in one kernel on primitive states
-                              (LSQ, centroid form; falls back to 0 where it does not
-                              apply), which fvs_set_persistent needs;
+                              (LSQ, centroid form), which fvs_set_persistent needs;
+                              single launches take two kernels per stage where the
+                              cell order gives no compact blocks, and those of 0
+                              where the kernel does not apply;
                            3: two kernels per stage without the per-block halo data
                               (the LSQ gradient gathers its stencil cell by cell) and
                               with SSP-RK3 stages on primitive states */

@@ -1,6 +1,8 @@
-"""Persistent whole-step launches next to the other routes of a context: one that
-changes between them and two kernels per stage continues from its current state,
-bit for bit the kernels of kernel_path 3."""
+"""Persistent whole-step launches next to the other routes of a context: meshes
+whose block ranges are cut (the reference order on many cells, quadrilaterals in
+the reference order) take them, and a context that changes between them and two
+kernels per stage continues from its current state.  Bit for bit the kernels of
+kernel_path 3."""
 import numpy as np
 import pytest
 
@@ -9,6 +11,37 @@ from fvs2d_amd.solver import Solver
 from tests.common import vortex_scheme
 
 pytestmark = pytest.mark.gpu
+
+
+def quads(nx, ny):
+    """nx x ny quadrilaterals on a sheared rectangle, periodic in both directions."""
+    i, j = (a.ravel() for a in np.meshgrid(np.arange(nx + 1), np.arange(ny + 1)))
+    xy = np.stack([-5 + 10 * i / nx + 0.3 * j / ny, -5 + 10 * j / ny], 1).astype(float)
+    qi, qj = (a.ravel() for a in np.meshgrid(np.arange(nx), np.arange(ny)))
+    bl = qj * (nx + 1) + qi
+    cells = np.stack([bl, bl + 1, bl + nx + 2, bl + nx + 1], 1)
+    canon = ((j % ny) * (nx + 1) + i % nx).astype(np.int32)
+    return meshgen.Mesh(xy, 0, nx * ny, cells.ravel().astype(np.int32), [], canon=canon, period=(10.0, 10.0))
+
+
+MESHES = {
+    "many triangles": lambda: meshgen.jittered_square(132, periodic=True, seed=2),
+    "quads": lambda: quads(96, 70),
+}
+
+
+@pytest.mark.parametrize("limiter", [0, 1])
+@pytest.mark.parametrize("mesh", list(MESHES))
+def test_reference_order_takes_persistent_launches(mesh, limiter):
+    m, sch = MESHES[mesh](), vortex_scheme(dt=1e-3, limiter=limiter, reorder=0)
+    a, b, c = Solver(m, sch, kernel_path=3), Solver(m, sch, kernel_path=2), Solver(m, sch, kernel_path=2)
+    c.set_persistent(True)
+    for s in (a, b, c):
+        s.initialize_solution(1, 0.0)
+    for n in (5, 4):
+        na, nb, nc = (s.time_integration(0.0, n) for s in (a, b, c))
+        assert np.array_equal(na, nb) and np.array_equal(na, nc)
+    assert np.array_equal(a.cvar, b.cvar) and np.array_equal(a.cvar, c.cvar)
 
 
 @pytest.mark.parametrize("rk", [_lib.RK_SSP3, _lib.RK_SSP42_SO, _lib.RK_SSP42])
