@@ -2129,7 +2129,7 @@ int setup_device(fvs_ctx &C) {
   if (int rc = C.alloc(C.vpart, 13 * size_t(nblk(std::max(C.ncell_intr, 1))) * C.norm_rows)) return rc;
   if (int rc = C.alloc(C.small, 64)) return rc;
   if (int rc = C.alloc(C.dctr, 1)) return rc;
-  if (int rc = C.alloc(C.pbar, 2)) return rc;
+  if (int rc = C.alloc(C.pbar, kBarWords)) return rc;
   if (int rc = C.alloc(C.perr, 1)) return rc;
   if (C.ninst > 0) {
     // per-instance ranges in device order, free streams, wall-face ranges
