@@ -1280,7 +1280,9 @@ struct fvs_ctx {
   bool profiling = false;
   // phase timers (fvs_set_phase_timers): device ms per kernel class, summed
   // over the time-integration calls made while they are on
-  bool phase_timing = false;
+  // (timing_stage: in the call at hand; clk: the whole-stage blocks' clocks)
+  bool phase_timing = false, timing_stage = false;
+  unsigned long long *clk = nullptr;
   double phase_ms[6] = {0, 0, 0, 0, 0, 0};
   std::vector<hipEvent_t> evpool;
   std::vector<int> evclass;
@@ -2423,6 +2425,7 @@ StageIn stage_in(const fvs_ctx &C, double t, double *uout) {
   const int nb = int(C.stage_cells.size());
   a.nb = C.nact ? C.nslist : xcd_arg(nb, C.xcd_fused);
   a.down = C.sweep;
+  a.clk = C.clk;
   return a;
 }
 
@@ -2447,9 +2450,14 @@ int launch_stage(fvs_ctx &C, const Upd &A, double t, const double *uin = nullptr
   const dim3 g(C.nact && !resid ? C.nslist : xcd_grid(int(C.stage_cells.size())));
   const double *in = cons ? uin : C.W;
   double *out = cons ? nullptr : C.Walt;
-#define FVS_STAGE(SH, L, PM)                                                                                     \
-  hipLaunchKernelGGL((k_stage<SH, L, PM>), g, dim3(SH::NT), stage_lds<SH>(C, resid || (A.steady && A.first)), C.stream, \
-                     a, A, in, out, cons ? 1 : 0)
+#define FVS_STAGE_T(SH, L, PM, T)                                                                                \
+  hipLaunchKernelGGL((k_stage<SH, L, PM, T>), g, dim3(SH::NT), stage_lds<SH>(C, resid || (A.steady && A.first)), \
+                     C.stream, a, A, in, out, cons ? 1 : 0)
+#define FVS_STAGE(SH, L, PM)                          \
+  do {                                                \
+    if (C.timing_stage) FVS_STAGE_T(SH, L, PM, true); \
+    else FVS_STAGE_T(SH, L, PM, false);               \
+  } while (0)
 #define FVS_STAGE_PM(SH, L)                     \
   do {                                          \
     if (C.pmode == 0) FVS_STAGE(SH, L, 0);      \
@@ -2468,6 +2476,7 @@ int launch_stage(fvs_ctx &C, const Upd &A, double t, const double *uin = nullptr
   }
 #undef FVS_STAGE_PM
 #undef FVS_STAGE
+#undef FVS_STAGE_T
   HIPC(hipGetLastError());
   if (!cons && !resid) std::swap(C.W, C.Walt);
   return 0;
@@ -3330,12 +3339,21 @@ int integrate(fvs_ctx *C, double t1, int nsteps, double *norms, double *verr, do
     C->profiling = true;
     C->evused = 0;
     C->evclass.clear();
+    C->timing_stage = whole_stage(*C) && C->clk;
   }
   HIPC(hipEventRecord(C->ev0, C->stream));
   const int rc_run = run_steps(*C, t1, nsteps, dn, dv, di);
-  if (timers) C->profiling = false;
+  const bool split = timers && C->timing_stage;
+  if (timers) C->profiling = C->timing_stage = false;
   if (rc_run) return rc_run;
   HIPC(hipEventRecord(C->ev1, C->stream));
+  double clocks[2] = {0.0, 0.0};
+  if (split) {
+    hipLaunchKernelGGL(k_phase_clocks, dim3(1), dim3(256), 0, C->stream, int(C->stage_cells.size()), C->clk,
+                       C->small + 32);
+    HIPC(hipGetLastError());
+    HIPC(hipMemcpyAsync(clocks, C->small + 32, sizeof(clocks), hipMemcpyDeviceToHost, C->stream));
+  }
   // the small outputs queue behind the steps; one wait for all of them
   int perr = 0;
   if (C->persist_ran) HIPC(hipMemcpyAsync(&perr, C->perr, sizeof(int), hipMemcpyDeviceToHost, C->stream));
@@ -3354,7 +3372,10 @@ int integrate(fvs_ctx *C, double t1, int nsteps, double *norms, double *verr, do
     for (size_t k = 0; k < C->evclass.size(); ++k) {
       float t = 0.f;
       HIPC(hipEventElapsedTime(&t, C->evpool[2 * k], C->evpool[2 * k + 1]));
-      C->phase_ms[C->evclass[k]] += t;
+      // a whole stage: gradient time is its blocks' part of their clock cycles
+      const double part = split && C->evclass[k] == KC_FUSED && clocks[1] > 0.0 ? clocks[0] / clocks[1] : 0.0;
+      C->phase_ms[KC_GRAD] += part * t;
+      C->phase_ms[C->evclass[k]] += (1.0 - part) * t;
     }
   return 0;
 }
@@ -3406,6 +3427,11 @@ int fvs_time_integration_noalloc(fvs_ctx *C, double t1, int nsteps, double *norm
 
 int fvs_set_phase_timers(fvs_ctx *C, int on) try {
   if (!C) return fail(FVS_EINVAL, "null context");
+  if (on && C->stage_bs && !C->clk) {
+    const size_t n = 2 * C->stage_cells.size();
+    if (int rc = C->upload(C->clk, std::vector<unsigned long long>(n, 0))) return rc;
+    HIPC(hipStreamSynchronize(C->stream));
+  }
   C->phase_timing = on != 0;
   return 0;
 } catch (...) {
@@ -3415,18 +3441,9 @@ int fvs_set_phase_timers(fvs_ctx *C, int on) try {
 int fvs_phase_times(const fvs_ctx *C, double *sec4) try {
   if (!C || !sec4) return fail(FVS_EINVAL, "null argument");
   const double *t = C->phase_ms;
-  // whole-stage launches: their time in the proportion of the floating-point
-  // operations, about 18 per stencil entry against 300 per face and 60 per cell
-  double share = 0.0;
-  if (whole_stage(*C)) {
-    double g = 36.0 * double(C->stage_words) + 8.0 * double(C->stage_incidences);
-    if (C->opt.grad_method != 3) g += 16.0 * (C->opt.grad_method == 1 ? C->NFW : C->gwn) * C->N;
-    const double f = 300.0 * double(C->stage_faces) + 60.0 * C->N;
-    share = g / (g + f);
-  }
-  sec4[0] = (t[KC_GRAD] + share * t[KC_FUSED]) * 1e-3;  // gradient, limiter fused in
-  sec4[1] = 0.0;                                        // limiter: inside the gradient phase
-  sec4[2] = (t[KC_FLUX_INT] + t[KC_FLUX_BND] + (1.0 - share) * t[KC_FUSED]) * 1e-3;  // face fluxes (+ fused update)
+  sec4[0] = t[KC_GRAD] * 1e-3;                                       // gradient, limiter fused in
+  sec4[1] = 0.0;                                                     // limiter: inside the gradient phase
+  sec4[2] = (t[KC_FLUX_INT] + t[KC_FLUX_BND] + t[KC_FUSED]) * 1e-3;  // face fluxes (+ fused stage update)
   sec4[3] = (t[KC_UPDATE] + t[KC_NORM]) * 1e-3;                   // stage updates, residual norms
   return 0;
 } catch (...) {

@@ -112,6 +112,9 @@ struct StageIn {
   // stages start where the last one ended, whose lists and states the 256 MB
   // memory-side cache still holds: 7% of a stage on 2,097,152 cells (now 125 us)
   int down;
+  // phase timers: per block the clock cycles its launches spent until the gradients
+  // were there, and in all
+  unsigned long long *clk;
 };
 
 // The shapes in use.  128-cell blocks: five wavefronts per SIMD and five blocks on
@@ -133,7 +136,8 @@ using StageLarge = StageShape<256, 512, 384, 512, 4>;
 // it on every size that was measured (3,200 to 819,200 cells).
 constexpr int kGGCB = 4, kGGNB = 5;
 
-template <class SH, int LIM, int PMODE>
+// TIMED: the phase timers are on (a run-time switch cost 2,097,152 cells 1.3%).
+template <class SH, int LIM, int PMODE, bool TIMED = false>
 __device__ __forceinline__ void stage_block(const StageIn &a, int lb, const Upd &A, const double *__restrict__ Win,
                                             double *__restrict__ Wout, int cons) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -144,6 +148,8 @@ __device__ __forceinline__ void stage_block(const StageIn &a, int lb, const Upd 
   const StageLists &S = a.S;
   const StageBlock d = S.blk[lb];
   const int tid = threadIdx.x, N = a.N;
+  unsigned long long t0 = 0, t1 = 0;
+  if (TIMED) t0 = __builtin_readcyclecounter();
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   // face record and geometry, stencil codes
   const int *hl = S.halo + long(lb) * S.hs;
@@ -356,6 +362,7 @@ __device__ __forceinline__ void stage_block(const StageIn &a, int lb, const Upd 
     at(o0 + 3 * PS) = make_double2(gy[2], gy[3]);
   }
   __syncthreads();
+  if (TIMED) t1 = __builtin_readcyclecounter();
   const bool resid = A.mode == M_RESID, ws = resid || (A.steady && A.first);
   auto side = [&](unsigned o, double w[4], double gr[8], double &ph, double2 &c) __attribute__((always_inline)) {
     const double2 wa = at(o), wb = at(o + PS);
@@ -430,12 +437,16 @@ __device__ __forceinline__ void stage_block(const StageIn &a, int lb, const Upd 
   }
   if (tid < d.base)
     cell_update(N, d.i0 + tid, mine, A, in, flux, speed, a.Ua, a.Ub, a.Facc, Wout, a.dtl, a.norm, a.amask);
+  if (TIMED && tid == 0) {
+    a.clk[2 * lb] += t1 - t0;
+    a.clk[2 * lb + 1] += __builtin_readcyclecounter() - t0;
+  }
 }
 
 // four wavefronts per SIMD with the limiter (its registers spill at five, 11%
 // slower on 522,242 cells) and with the weights that need a division or pow,
 // SH::WAVES without them
-template <class SH, int LIM, int PMODE>
+template <class SH, int LIM, int PMODE, bool TIMED>
 __global__ __launch_bounds__(SH::NT, LIM || PMODE == 2 || PMODE == 3 ? 4 : SH::WAVES) void k_stage(StageIn a, Upd A,
                                                                        const double *__restrict__ Win,
                                                                        double *__restrict__ Wout, int cons) {
@@ -444,7 +455,7 @@ __global__ __launch_bounds__(SH::NT, LIM || PMODE == 2 || PMODE == 3 ? 4 : SH::W
   if (lb >= nbl) return;  // the whole workgroup leaves before any barrier
   if (a.down) lb = nbl - 1 - lb;
   if (a.blist) lb = a.blist[lb];
-  stage_block<SH, LIM, PMODE>(a, lb, A, Win, Wout, cons);
+  stage_block<SH, LIM, PMODE, TIMED>(a, lb, A, Win, Wout, cons);
 }
 
 // ---------------------------------------------------------------------------
@@ -544,6 +555,27 @@ __global__ __launch_bounds__(SH::NT, SH::NT > 256 ? 4 : 3) void k_steps_persiste
   }
   if (ok) ok = grid_barrier(c.bar, gridDim.x, gen, c.spin, c.err);
   if (ok && blockIdx.x == 0 && threadIdx.x == 0) c.ctr[0] = row0 + c.nsteps;
+}
+
+// the blocks' clocks, added up and set to zero
+__global__ __launch_bounds__(256) void k_phase_clocks(int nb, unsigned long long *__restrict__ clk,
+                                                      double *__restrict__ out) {
+  __shared__ double red[2][256];
+  const int t = threadIdx.x;
+  double s[2] = {0.0, 0.0};
+  for (int b = t; b < nb; b += 256)
+    for (int k = 0; k < 2; ++k) {
+      s[k] += double(clk[2 * b + k]);
+      clk[2 * b + k] = 0;
+    }
+  for (int k = 0; k < 2; ++k) red[k][t] = s[k];
+  __syncthreads();
+  for (int h = 128; h > 0; h >>= 1) {
+    if (t < h)
+      for (int k = 0; k < 2; ++k) red[k][t] += red[k][t + h];
+    __syncthreads();
+  }
+  if (t < 2) out[t] = red[t][0];
 }
 
 __global__ void k_barrier_reset(unsigned *bar, int *err) {

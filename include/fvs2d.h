@@ -135,8 +135,9 @@ int fvs_set_phase_timers(fvs_ctx *ctx, int on);
  * evaluated inside the gradient launches, so its time is here), limiter
  * (always 0 for that reason), face fluxes (with the stage update where it is
  * fused into the flux launch), Runge-Kutta (separate stage-update launches
- * and the residual-norm reduction).  A launch of a whole stage is divided
- * between gradient and face fluxes in the proportion of their operations. */
+ * and the residual-norm reduction).  The blocks of a whole-stage launch read
+ * the clock when their gradients are complete, and the launch is divided between
+ * gradient and face fluxes by their cycles before and after. */
 int fvs_phase_times(const fvs_ctx *ctx, double *sec4);
 /* Launch mode, no reference counterpart: on != 0 runs each
  * fvs_time_integration call (or batch call) as one persistent cooperative
