@@ -187,8 +187,8 @@ __device__ __forceinline__ double cell_limiter_v(int lt, int nf, const double2 o
         const double pf = q + o[k].x * gx[v] + o[k].y * gy[v];
         const double diff = pf - q;
         double e = 1.0;
-        if (diff > 0.0) e = limiter_fn(lt, dmax, diff, vol);
-        else if (diff < 0.0) e = limiter_fn(lt, dmin, diff, vol);
+        if (diff > 0.0) e = van_albada(dmax, diff, vol);
+        else if (diff < 0.0) e = van_albada(dmin, diff, vol);
         pe = (e < pe) ? e : pe;
       }
       const double pv = (1.0 < pe) ? 1.0 : pe;
@@ -309,7 +309,6 @@ __device__ __forceinline__ void stencil_minmax(int i, const int *__restrict__ so
   }
 }
 
-// GGCB gradient (src/gradient_ggcb.f90:116-138):
 // Pieces of the Green-Gauss gradients, the same in every kernel: the own and one
 // neighbour's (or node's) term, the division by the volume, one cell's share of a
 // node value, and the limiter's bounds.
@@ -336,6 +335,7 @@ __device__ __forceinline__ void stencil_bounds(const double q[4], double mn[4], 
   }
 }
 
+// GGCB gradient (src/gradient_ggcb.f90:116-138):
 // grad_i = (coef0 q_i + sum_f coefnb_f q_nb(f)) / vol
 template <int LIM>
 __global__ __launch_bounds__(kBlock) void k_grad_ggcb(int nbx, int N, int nfw, const double *__restrict__ W,
@@ -691,19 +691,6 @@ struct Upd {
   int use_acc;   // CLASSIC final stage: update with the accumulator
   double cfl, gamma;
 };
-
-__device__ __forceinline__ void block_sum4(double v[4], double *red) {
-  // fixed-shape tree over the block: deterministic
-  const int t = threadIdx.x;
-  for (int k = 0; k < 4; ++k) red[k * kBlock + t] = v[k];
-  __syncthreads();
-  for (int s = kBlock / 2; s > 0; s >>= 1) {
-    if (t < s)
-      for (int k = 0; k < 4; ++k) red[k * kBlock + t] = red[k * kBlock + t] + red[k * kBlock + t + s];
-    __syncthreads();
-  }
-  for (int k = 0; k < 4; ++k) v[k] = red[k * kBlock];
-}
 
 // Where a step's last stage leaves the squared increments of the residual
 // norm: one sum of four per 64-cell slice (a wavefront's cells, added by a
@@ -1164,7 +1151,7 @@ struct fvs_ctx {
   // fused flux + update (k_flux_update): per-block face lists, local gather
   bool fused = false;
   int maxf = 0;
-  int *boff = nullptr, *bfaces = nullptr;
+  int *boff = nullptr;
   short *lgat = nullptr;  // signed 1-based index into the block's face list
   // the same per-block lists for blocks of kSmallBlock cells (single meshes),
   // used by the fused flux kernel when small_blocks is set (autotuned)

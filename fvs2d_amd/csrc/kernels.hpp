@@ -38,9 +38,10 @@ struct Phys {
 // root spends about half of its instructions on operands whose quotient or
 // residual leaves the exponent range and on special values; states, areas and
 // volumes are far from that.  These give the same correctly rounded results for
-// operands and results within 2^-900 .. 2^900 (compared with the general
-// operations on 2^33 pairs), 0 for a zero numerator or root, and a value that is
-// not finite for those that are not, or for a zero divisor.
+// operands and results within 2^-900 .. 2^900 (equal to the general operations on
+// 2^31 pairs each with exponents up to 3, 40 and 440), 0 for a zero numerator or
+// root, and a value that is not finite for those that are not, or for a zero
+// divisor.
 
 // 1 / d: an approximation, two Newton steps, and a third whose residual is exact
 __device__ __forceinline__ double recip(double d) {
@@ -177,21 +178,13 @@ __device__ __forceinline__ double venkat_eps2(double vol) {
   return t * t * t;
 }
 
-// limiter function: src/gradient_limiter.f90:103-134
-__device__ __forceinline__ double limiter_fn(int lt, double a, double b, double vol) {
-  if (lt == 1) {
-    const double eps2 = venkat_eps2(vol);
-    return ((a * a + eps2) + 2.0 * b * a) / (a * a + 2.0 * (b * b) + a * b + eps2);
-  } else if (lt == 2) {
-    const double r = a / b;
-    return (1.0 < r) ? 1.0 : r;
-  } else {
-    const double h = 2.0 * sqrt(vol / kPiD);
-    const double t = 0.3 * h;
-    const double eps2 = t * t * t;
-    const double l = ((b * b + eps2) * a + (a * a + eps2) * b) / (a * a + b * b + 2.0 * eps2);
-    return l / (b + eps2);
-  }
+// the Van Albada form of src/gradient_limiter.f90:122-127
+__device__ __forceinline__ double van_albada(double a, double b, double vol) {
+  const double h = 2.0 * sqrt(vol / kPiD);
+  const double t = 0.3 * h;
+  const double eps2 = t * t * t;
+  const double l = ((b * b + eps2) * a + (a * a + eps2) * b) / (a * a + b * b + 2.0 * eps2);
+  return l / (b + eps2);
 }
 
 }  // namespace fvs
