@@ -33,8 +33,8 @@ struct Phys {
 // ---------------------------------------------------------------------------
 // division, square root, minimum
 // ---------------------------------------------------------------------------
-// The stage kernels are bound by vector instructions (69% of the issue cycles on
-// 2,097,152 cells, the rest mostly waits).  A general FP64 division or square
+// The stage kernels are bound by vector instructions (64% of the issue cycles on
+// 2,097,152 unlimited cells, the rest mostly waits).  A general FP64 division or square
 // root spends about half of its instructions on operands whose quotient or
 // residual leaves the exponent range and on special values; states, areas and
 // volumes are far from that.  These give the same correctly rounded results for

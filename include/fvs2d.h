@@ -66,12 +66,12 @@ typedef struct {
   int reorder;          /* device cell order: 0 reference order, 1 Morton (Z-curve)
                            blocks, 2 recursive coordinate bisection (compact
                            blocks on graded meshes); results are the same  */
-  int kernel_path;      /* 0: fastest available (LSQ gradients: the whole stage in one
-                              kernel where the cell order gives compact blocks, else a
-                              gradient and a fused flux+update kernel; SSP-RK3 stages
-                              read conservative stage states and write no primitive
-                              state, with the LSQ gradient or an unlimited Green-Gauss
-                              one);
+  int kernel_path;      /* 0: fastest available (LSQ gradients, and Green-Gauss ones of
+                              single meshes: the whole stage in one kernel where the
+                              cell order gives compact blocks, else a gradient and a
+                              fused flux+update kernel; stages of SSP-RK3 and of the
+                              two-register SSP-RK(4,2) read conservative stage states
+                              and write no primitive state where their kernels can);
                            1: face-flux buffer kernels only;
                            2: the whole stage in one kernel on primitive states
                               (LSQ, centroid form), which fvs_set_persistent needs;
@@ -118,9 +118,9 @@ int fvs_batch_time_integration(fvs_ctx *ctx, double t1, int nsteps, double *inst
 int fvs_batch_set_active(fvs_ctx *ctx, const int *active);
 /* C_L, C_D, C_L(cell), C_D(cell) per instance (4*ninst), src/io.f90:340-449 */
 int fvs_batch_wall_forces(fvs_ctx *ctx, double *out);
-/* Launch mode, no reference counterpart: on != 0 captures the launches of one
- * time step (two for three-stage schemes) in a HIP graph and replays it; the
- * instantiated graph is kept for later fvs_time_integration calls until a call
+/* Launch mode, no reference counterpart: on != 0 captures the launches of
+ * one to eight time steps (an even number of stages, at most half the steps of
+ * the call) in a HIP graph and replays it; the instantiated graph is kept for later fvs_time_integration calls until a call
  * changes what a step launches (time step, limiter freezing, active
  * instances, autotuned choices).  Time-dependent boundary data (the
  * Dirichlet vortex) always use stream launches. */
