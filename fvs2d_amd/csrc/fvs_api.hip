@@ -152,6 +152,12 @@ __global__ __launch_bounds__(256) void k_give1(int N, const int *__restrict__ ip
   const int c = blockIdx.x * 256 + threadIdx.x;
   if (c < N) out[c] = in[long(stride) * ip[c]];
 }
+// v of the cells whose bit is clear, as it was saved
+__global__ __launch_bounds__(256) void k_keep_masked(int N, const unsigned *__restrict__ bits,
+                                                     const double *__restrict__ saved, double *__restrict__ v) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < N && !((bits[i >> 5] >> (i & 31)) & 1u)) v[i] = saved[i];
+}
 // the caller's scalars into slot 0 of device-order records, the others 0
 __global__ __launch_bounds__(256) void k_take1(int N, const int *__restrict__ ip, const double *__restrict__ in,
                                                double *__restrict__ out) {
@@ -2429,12 +2435,8 @@ int launch_stage(fvs_ctx &C, const Upd &A, double t, const double *uin = nullptr
   const bool cons = uin != nullptr, lim = C.opt.limiter > 0 && !C.limiter_frozen;
   const bool resid = A.mode == M_RESID;
   C.sweep ^= 1;
-  StageIn a = stage_in(C, t, uout);
-  if (resid) {  // every cell's
-    a.blist = nullptr;
-    a.nb = xcd_arg(int(C.stage_cells.size()), C.xcd_fused);
-  }
-  const dim3 g(C.nact && !resid ? C.nslist : xcd_grid(int(C.stage_cells.size())));
+  const StageIn a = stage_in(C, t, uout);
+  const dim3 g(C.nact ? C.nslist : xcd_grid(int(C.stage_cells.size())));
   const double *in = cons ? uin : C.W;
   double *out = cons ? nullptr : C.Walt;
 #define FVS_STAGE_T(SH, L, PM, T)                                                                                \
@@ -2521,6 +2523,35 @@ void refresh_prim(fvs_ctx &C) {
 void ensure_prim(fvs_ctx &C) {
   if (C.w_stale) refresh_prim(C);
 }
+
+// For the length of a query every instance of a batch counts as active: gradients,
+// limiter values, residuals and forces are those of each cell's current state.
+// The launches of the time loop leave masked instances' primitive states,
+// gradients and limiter values where they were; a query leaves the limiter
+// values so too (an instance may resume with them frozen).
+class AllCells {
+  fvs_ctx &C;
+  const int nact;
+
+ public:
+  explicit AllCells(fvs_ctx &c) : C(c), nact(c.nact) {
+    if (!nact) return;
+    refresh_prim(C);
+    // (the accumulator is dead between steps)
+    if (C.opt.limiter > 0)
+      (void)hipMemcpyAsync(C.Facc, C.phi, size_t(C.N) * sizeof(double), hipMemcpyDeviceToDevice, C.stream);
+    C.nact = 0;
+  }
+  ~AllCells() {
+    if (!nact) return;
+    C.nact = nact;
+    if (C.opt.limiter > 0)
+      hipLaunchKernelGGL(k_keep_masked, dim3(nblk(C.N)), dim3(256), 0, C.stream, C.N,
+                         reinterpret_cast<const unsigned *>(C.blist + nblk(C.N)), C.Facc, C.phi);
+  }
+  AllCells(const AllCells &) = delete;
+  AllCells &operator=(const AllCells &) = delete;
+};
 
 }  // namespace
 
@@ -2907,6 +2938,7 @@ int fvs_primitives(fvs_ctx *C, double *pvar) try {
 int fvs_gradient(fvs_ctx *C, double *grad) try {
   if (int rc = need_state(C)) return rc;
   ensure_prim(*C);
+  const AllCells all(*C);
   if (C->opt.recon != 1)
     if (int rc = launch_gradient(*C, false)) return rc;
   if (grad) {
@@ -2924,6 +2956,7 @@ int fvs_gradient_1var(fvs_ctx *C, const double *fc, double *dfc) try {
   if (!C || !fc || !dfc) return fail(FVS_EINVAL, "null argument");
   // the scalar rides in slot 0 of a scratch primitive record; the gradient
   // kernels treat the four slots independently
+  const AllCells all(*C);
   const size_t N = size_t(C->N);
   HIPC(hipMemcpyAsync(C->FA, fc, N * sizeof(double), hipMemcpyHostToDevice, C->stream));
   hipLaunchKernelGGL(k_take1, dim3(nblk(C->N)), dim3(256), 0, C->stream, C->N, C->dip, C->FA, C->rout);
@@ -2943,6 +2976,7 @@ int fvs_gradient_1var(fvs_ctx *C, const double *fc, double *dfc) try {
 int fvs_limiter(fvs_ctx *C, double *phi) try {
   if (int rc = need_state(C)) return rc;
   ensure_prim(*C);
+  const AllCells all(*C);
   if (C->opt.recon != 1 && C->opt.limiter > 0)
     if (int rc = launch_gradient(*C, true)) return rc;
   if (phi)
@@ -2956,6 +2990,7 @@ int fvs_limiter(fvs_ctx *C, double *phi) try {
 int fvs_compute_residual(fvs_ctx *C, double time, double *resid, double *ws) try {
   if (int rc = need_state(C)) return rc;
   refresh_prim(*C);
+  const AllCells all(*C);
   Upd A{};
   A.mode = M_RESID;
   A.gamma = C->opt.gamma;
@@ -3563,6 +3598,7 @@ int fvs_wall_forces(fvs_ctx *C, double *out4) try {
   if (!out4) return fail(FVS_EINVAL, "null argument");
   const double kPi = 3.14159265358979323846;
   refresh_prim(*C);
+  const AllCells all(*C);
   if (int rc = launch_gradient(*C, false)) return rc;
   const double al = C->opt.aoa_deg * (kPi / 180.0);
   hipLaunchKernelGGL(k_wall_forces, dim3(1), dim3(64), 0, C->stream, C->nwall, C->wall, C->fb_cell, C->fb_geo, C->W,

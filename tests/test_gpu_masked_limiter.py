@@ -16,17 +16,21 @@ ASK = {
     "gradient": lambda s: s.compute_gradient_cellcntr(),
     "scalar gradient": lambda s: s.gradient_cellcntr_1var(np.linspace(-1.0, 1.0, s.ncells)),
     "forces": lambda s: s.wall_forces_batch(),
+    "limiter": lambda s: s.compute_gradient_limiter(),
+    "residual": lambda s: s.compute_residual(0.0),
 }
+ROUTES = {"whole-stage": (0, None), "two-kernels": (0, {"gradient": 2}), "primitive": (2, None), "gather": (3, None)}
 
 
-@pytest.mark.parametrize("choices", [None, {"gradient": 2}], ids=["whole-stage", "two-kernels"])
+@pytest.mark.parametrize("route", list(ROUTES))
 @pytest.mark.parametrize("rk", [_lib.RK_SSP3, _lib.RK_SSP42_SO, _lib.RK_SSP42])
 @pytest.mark.parametrize("ask", list(ASK))
-def test_queries_leave_frozen_limiters_alone(ask, rk, choices):
+def test_queries_leave_frozen_limiters_alone(ask, rk, route):
+    path, choices = ROUTES[route]
     meshes = [cases.naca(n, l)[0] for n, l in [(24, 12), (20, 11)]]
     out = []
     for query in (None, ASK[ask]):
-        b = BatchSolver(meshes, [(0.7, 1.0), (0.6, -1.0)], cases.naca(16, 8, cfl=0.5, rk_scheme=rk)[1])
+        b = BatchSolver(meshes, [(0.7, 1.0), (0.6, -1.0)], cases.naca(16, 8, cfl=0.5, rk_scheme=rk, kernel_path=path)[1])
         if choices:
             b.set_launch_choices(choices)
         b.initialize_freestream()
