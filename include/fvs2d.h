@@ -114,7 +114,9 @@ int fvs_create_batch(fvs_ctx **out, int ninst, const int *cell_offsets, const do
 int fvs_batch_time_integration(fvs_ctx *ctx, double t1, int nsteps, double *inst_norms);
 /* active[k] != 0 keeps instance k stepping; the others are left out of the
  * launches (blocks holding only inactive instances are skipped, and a block
- * shared with an active instance leaves their cells untouched) */
+ * shared with an active instance leaves their cells untouched).  Queries
+ * (gradients, limiter, residual, forces) answer for every instance's current
+ * state and leave the limiter values of inactive ones as they were */
 int fvs_batch_set_active(fvs_ctx *ctx, const int *active);
 /* C_L, C_D, C_L(cell), C_D(cell) per instance (4*ninst), src/io.f90:340-449 */
 int fvs_batch_wall_forces(fvs_ctx *ctx, double *out);
