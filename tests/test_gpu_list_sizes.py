@@ -1,6 +1,8 @@
 """The whole-stage kernel's block lists do not grow with the widest stencil of the
 mesh: the device memory of a context on a mesh with one node of many cells stays
 within a quarter of the same mesh's without it."""
+import gc
+
 import pytest
 import torch
 
@@ -13,6 +15,7 @@ pytestmark = pytest.mark.gpu
 
 
 def device_bytes(m, sch):
+    gc.collect()  # contexts that earlier tests left behind
     torch.cuda.synchronize()
     free = torch.cuda.mem_get_info()[0]
     s = Solver(m, sch)
